@@ -293,6 +293,100 @@ def work(case):
     return {"bytes": (used + shared) * H * I * bits / 8 + rows, "flops": 2.0 * (P + shared * T) * 3 * H * I}
 
 
+# ------------------------------------------------------------- the same pass in 64 bits, from the formats' definitions
+def _nibbles(b):
+    return torch.stack([b & 15, b >> 4], -1).flatten(-2)                  # low nibble first
+
+
+def _fields(b, bits, tile):
+    """High bits: byte t of a tile of 512 values holds values p x tile + t in its fields p; tile 0: consecutive values."""
+    f = torch.stack([b >> s & (1 << bits) - 1 for s in range(0, 8, bits)], -1)
+    return f.flatten(-2) if not tile else f.unflatten(-2, (-1, tile)).transpose(-1, -2).flatten(-3)
+
+
+def _scaled(u, s, m=None):
+    s = s.double().repeat_interleave(u.shape[-1] // s.shape[-1], -1)
+    return u * s if m is None else u * s - m.double().repeat_interleave(u.shape[-1] // m.shape[-1], -1)
+
+
+def _blocks(q, s):
+    s = s.double().repeat_interleave(128, -2)[..., :q.shape[-2], :]
+    return _scaled(q.float().double(), s)
+
+
+def _weight64(fmt, w, shuffled=True):
+    if fmt in ("int4", "int4_zp"):
+        z = w[2].double().repeat_interleave(128, -1) if fmt == "int4_zp" else 8.0
+        return _scaled(_nibbles(w[0]).double() - z, w[1])
+    if fmt == "fp8_block":
+        return _blocks(*w)
+    if fmt.startswith("fp8"):
+        return w[0].float().double() * w[1].double()[:, None]
+    if fmt == "q8_0":
+        return _scaled(w[0].double(), w[1])
+    u = _nibbles(w[0])
+    if fmt == "q4_0":
+        return _scaled(u.double() - 8.0, w[1])
+    if fmt == "q4_k":
+        return _scaled(u.double(), *w[1:])
+    if fmt == "q5_k":
+        return _scaled((u + 16 * _fields(w[1], 1, 64 * shuffled)).double(), *w[2:])
+    return _scaled((u + 16 * _fields(w[1], 2, 128 * shuffled)).double() - 32.0, w[2])
+
+
+def _quant64(a):
+    """One scale = absmax / 448 per 128 values, e4m3 codes, and back."""
+    b = a.unflatten(-1, (-1, 128))
+    s = b.abs().amax(-1, keepdim=True).clamp(min=1e-12) / 448.0
+    return ((b / s).float().to(torch.float8_e4m3fn).double() * s).flatten(-2)
+
+
+def _act(g, u):
+    return g * torch.sigmoid(g) * u
+
+
+def _experts64(st, x, ids, w, quant):
+    """sum over the routes of weight x expert(x), from block-FP8 stacks."""
+    f = (lambda a: _quant64(a.to(_DT[st["dtype"]]).double())) if quant else (lambda a: a)
+    xq, y = f(x), torch.zeros_like(x)
+    for e in range(E):
+        t, j = (ids == e).nonzero(as_tuple=True)
+        if t.numel():
+            gu = xq[t] @ _blocks(st["w13"][e], st["s13"][e]).t()
+            y.index_add_(0, t, w[t, j, None] * (f(_act(*gu.chunk(2, 1))) @ _blocks(st["w2"][e], st["s2"][e]).t()))
+    return y
+
+
+def exact(case, seed):
+    st, fam = prepare(case, seed), case["family"]
+    x = st["x"].double()
+    if fam == "linear":
+        return x @ _weight64(st["fmt"], st["w"]).t()
+    if fam == "norm_linear":
+        a = x + st["residual"].double()
+        n = a * torch.rsqrt(a.pow(2).mean(-1, keepdim=True) + 1e-6) * st["norm_w"].double()
+        return n @ _weight64(st["fmt"], st["w"]).t(), n, a
+    if fam == "moe_gguf":
+        P, tok = st["T"] * TOPK, st["tok_ids"].long()
+        gate, inter = torch.empty(P, 2 * I, dtype=torch.float64, device="cuda"), torch.empty(P, I, dtype=torch.float64, device="cuda")
+        routes = torch.empty(P, H, dtype=torch.float64, device="cuda")
+        for e, at, n in st["chunks"].tolist():
+            r = slice(at, at + n)
+            for h, k in enumerate(("gate", "up")):
+                gate[r, h * I:(h + 1) * I] = x[tok[r]] @ _weight64("q4_k", [t[e] for t in st[k]]).t()
+            inter[r] = _act(*gate[r].chunk(2, 1))
+            routes[r] = inter[r] @ _weight64("q6_k", [t[e] for t in st["down"]], shuffled=False).t()
+        pos = st["pos"].long()
+        return (routes[pos] * st["w_sorted"].double()[pos][..., None]).sum(1), gate, routes
+    order = torch.sort(st["logits"].double(), dim=1, descending=True, stable=True)
+    ids, w = order.indices[:, :TOPK], torch.softmax(order.values[:, :TOPK], 1)
+    y = _experts64(st, x, ids, w, case.get("act_quant", False))
+    if fam == "moe_full":
+        gu = x @ _blocks(st["sw13"], st["ss13"]).t()
+        y += torch.sigmoid(x @ st["gate"].double().t()) * (_act(*gu.chunk(2, 1)) @ _blocks(st["sw2"], st["ss2"]).t())
+    return y
+
+
 # Four times the largest relative error (2-norm of the difference) seen against the same formula in 64 bits on the
 # dequantized weights, over the listed cases and 24 drawn ones: linear fp16 4.2e-4, bf16 2.4e-3 (the output's rounding,
 # and the weights' where the matrix cores take them); experts fp16 6.6e-4, bf16 4.4e-3 (the intermediate's rounding as
