@@ -30,6 +30,7 @@
 #pragma once
 #include "qlinear_common.hpp"
 #include <type_traits>
+#include <utility>
 
 namespace qlin {
 
@@ -37,7 +38,8 @@ struct GemmArgs {
   const void* x;              // activations re-tiled into MFMA operand order (the workspace)
   const void* w;
   const void* scale;
-  const void* zp;             // int4: zero-points (may be null); Q4_K: mins
+  const void* zp;             // int4: zero-points (may be null); Q4_K / Q5_K: mins
+  const void* qh;             // Q5_K / Q6_K: high bits
   void* out;
   int M, N, K;
   int tiles_m, tiles_n;
@@ -124,7 +126,7 @@ struct WInt4 {
     return r;
   }
   // byte offset of chunk kc of row n at k = 0, and the row's first side-table entry
-  static __device__ __forceinline__ void chunk_addr(const Res& r, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
+  static __device__ __forceinline__ void chunk_addr(Res& r, int, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
     boff = (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * 16);
     soff = (uint32_t)n * (uint32_t)r.Kg;              // in groups; x2 for the fp16 scale
   }
@@ -226,7 +228,7 @@ struct WQ4K {
     r.mr = make_rsrc(p.zp, (uint32_t)p.N * (uint32_t)r.Kc * 2u);
     return r;
   }
-  static __device__ __forceinline__ void chunk_addr(const Res& r, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
+  static __device__ __forceinline__ void chunk_addr(Res& r, int, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
     boff = (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * 16);
     soff = ((uint32_t)n * (uint32_t)r.Kc + (uint32_t)kc) * 2u;   // bytes: one fp16 per 32 k
   }
@@ -277,6 +279,160 @@ struct WQ4K {
   static __device__ __forceinline__ float out_scale(const Res&, const GemmArgs&, int) { return 1.0f; }
 };
 
+// ------------------------------------------------------------------ GGUF Q4_0 / Q8_0 / Q5_K / Q6_K (repacked)
+// fp16 activations only.  Q4_0 is the int4 layout with one scale per 32 k and zero-point 8: the
+// E4M3 trick of WInt4.  The others bring a byte per weight into place and take it to fp32 with
+// v_cvt_f32_ubyte (exact):
+//   Q8_0: code + 128 (sign bit flipped); fma(u, s, -128 s) is exact (8 x 11 significant bits);
+//   Q6_K: nibble | 2 high bits << 4;     fma(u, s, -32 s) is exact; two scales per chunk of 32 k;
+//   Q5_K: nibble | high bit << 4;        fp16(fp16(u s) - min), two roundings, as Q4_K;
+// each with the rounding(s) of the dense dequantization.  The high bits are tile-shuffled: inside
+// 512 k, byte t holds element p * 128 + t in its 2-bit field p (Q6_K), element p * 64 + t in bit p
+// (Q5_K), so the 32 weights of a chunk take one field of 32 consecutive bytes, the same field for
+// the whole 64-wide step; the bytes come through L1 again for the other fields.
+enum { GT_Q40 = 3, GT_Q80 = 4, GT_Q5K = 5, GT_Q6K = 6 };    // the format numbers of gemv_rows.hpp
+template <class Act, int BN, int F>
+struct WGguf {
+  static_assert(Act::dt == DT_F16, "GGUF formats run in fp16");
+  static constexpr bool kHigh = F == GT_Q5K || F == GT_Q6K;
+  static constexpr int CPR = F == GT_Q80 ? 4 : 2;
+  static constexpr double kWeightBytesPerK = F == GT_Q80 ? 1.0 : F == GT_Q6K ? 0.75 : F == GT_Q5K ? 0.625 : 0.5;
+  static constexpr int B_CH = (BN * CPR + 255) / 256;
+  static constexpr int LPC = F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2;
+  static constexpr int PPD = F == GT_Q5K ? 17 : F == GT_Q6K ? 13 : F == GT_Q40 ? 8 : 5;   // pieces per dword (8 nibbles / 4 bytes)
+  static constexpr int kPieces = B_CH * 4 * PPD;
+  static constexpr bool kOutScale = false;
+  static constexpr bool kPermK = false;
+  struct Res {
+    __amdgpu_buffer_rsrc_t wr, sr, mr, hr;
+    int Ks;                                           // bytes of scales per row
+    uint32_t hoff[kHigh ? B_CH : 1];
+  };
+  struct Stage {
+    u32x4 b[B_CH];
+    uint32_t s[B_CH];
+    uint32_t m[F == GT_Q5K ? B_CH : 1];
+    u32x4 h[kHigh ? B_CH : 1][2];
+    uint32_t sh;                                      // shift of this step's field of the high-bit bytes (uniform)
+  };
+  struct Dq {
+    uint32_t e, o, h0, h1;
+    float a, b;
+    f32x2 fe, fo;
+    u32x4 outv;
+    float sf[B_CH][F == GT_Q6K ? 2 : 1], nz[B_CH][F == GT_Q6K ? 2 : 1];
+    f16x2 mv[F == GT_Q5K ? B_CH : 1];
+  };
+  static __device__ __forceinline__ Res make(const GemmArgs& p, int = 0) {
+    Res r;
+    const uint32_t nk = (uint32_t)p.N * (uint32_t)p.K;      // < 2^31 (checked by the host)
+    r.Ks = (F == GT_Q6K ? p.K >> 4 : p.K >> 5) * 2;
+    r.wr = make_rsrc(p.w, F == GT_Q80 ? nk : nk / 2);
+    r.sr = make_rsrc(p.scale, (uint32_t)p.N * (uint32_t)r.Ks);
+    r.mr = make_rsrc(p.zp, F == GT_Q5K ? (uint32_t)p.N * (uint32_t)r.Ks : 0u);
+    r.hr = make_rsrc(p.qh, F == GT_Q6K ? nk / 4 : F == GT_Q5K ? nk / 8 : 0u);
+    return r;
+  }
+  static __device__ __forceinline__ void chunk_addr(Res& r, int i, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
+    boff = (uint32_t)n * (F == GT_Q80 ? (uint32_t)K : (uint32_t)K >> 1) + (uint32_t)(kc * 16);
+    soff = (uint32_t)n * (uint32_t)r.Ks + (uint32_t)(F == GT_Q80 ? (kc >> 1) * 2 : F == GT_Q6K ? kc * 4 : kc * 2);
+    if constexpr (kHigh) r.hoff[i] = (uint32_t)n * (F == GT_Q6K ? (uint32_t)K >> 2 : (uint32_t)K >> 3) + (uint32_t)(kc * 32);
+  }
+  static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
+                                               const uint32_t (&soff)[B_CH], int kt, uint32_t dead, int idx) {
+    const uint32_t k0 = (uint32_t)kt * kBK;
+    const int i = idx / LPC, kind = idx % LPC;
+    if (kind == 0) st.b[i] = __builtin_amdgcn_raw_buffer_load_b128(r.wr, boff[i] | dead, F == GT_Q80 ? k0 : k0 >> 1, 0);
+    else if (kind == 1) {
+      if constexpr (F == GT_Q6K) st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, k0 >> 3, 0);
+      else st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, k0 >> 4, 0);
+    } else if (kind == 4) {
+      if constexpr (F == GT_Q5K) st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, k0 >> 4, 0);
+    } else if constexpr (kHigh) {
+      const uint32_t tile = F == GT_Q6K ? (k0 >> 9) * 128u + (k0 & 127u) : (k0 >> 9) * 64u;
+      st.h[i][kind - 2] = __builtin_amdgcn_raw_buffer_load_b128(r.hr, r.hoff[i] | dead, tile + (uint32_t)(kind - 2) * 16u, 0);
+      st.sh = F == GT_Q6K ? (k0 >> 7 & 3u) * 2u : k0 >> 6 & 7u;
+    }
+  }
+  static __device__ __forceinline__ void begin(const Res&, const Stage& st, Dq& q) {
+#pragma unroll
+    for (int i = 0; i < B_CH; ++i) {
+#pragma unroll
+      for (int t = 0; t < (F == GT_Q6K ? 2 : 1); ++t) {
+        const float s = (float)__builtin_bit_cast(_Float16, (uint16_t)(st.s[i] >> 16 * t));
+        q.sf[i][t] = F == GT_Q40 ? s * 512.0f : s;            // exact: a power of two
+        q.nz[i][t] = s * (F == GT_Q80 ? -128.0f : F == GT_Q6K ? -32.0f : -8.0f);
+      }
+      if constexpr (F == GT_Q5K) {
+        const _Float16 mn = __builtin_bit_cast(_Float16, (uint16_t)st.m[i]);
+        q.mv[i] = f16x2{mn, mn};
+      }
+    }
+  }
+  static __device__ __forceinline__ uint32_t pack2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)a, (_Float16)b});
+  }
+  static __device__ __forceinline__ float byte_f(uint32_t v, int i) { return (float)(v >> 8 * i & 0xffu); }   // v_cvt_f32_ubyte
+  static __device__ __forceinline__ void piece(const Stage& st, Dq& q, int I, unsigned char* const (&dst)[B_CH]) {
+#pragma clang fp contract(off)
+    const int dword = I / PPD, part = I % PPD;
+    const int i = dword / 4, dw = dword % 4;
+    const uint32_t w = st.b[i][dw];
+    if constexpr (F == GT_Q40) {
+      auto pair = [&](float a, float b) {
+        return pack2(__builtin_fmaf(a, q.sf[i][0], q.nz[i][0]), __builtin_fmaf(b, q.sf[i][0], q.nz[i][0]));
+      };
+      if (part == 0) {
+        q.e = w & 0x0F0F0F0Fu;
+        q.o = (w >> 4) & 0x0F0F0F0Fu;
+      } else if (part == 1 || part == 4) {
+        q.fe = part == 1 ? __builtin_amdgcn_cvt_pk_f32_fp8((int)q.e, false) : __builtin_amdgcn_cvt_pk_f32_fp8((int)q.e, true);
+        q.fo = part == 1 ? __builtin_amdgcn_cvt_pk_f32_fp8((int)q.o, false) : __builtin_amdgcn_cvt_pk_f32_fp8((int)q.o, true);
+      } else if (part == 7) *reinterpret_cast<u32x4*>(dst[i] + dw * 16) = q.outv;
+      else q.outv[part < 4 ? part - 2 : part - 3] = part == 2 || part == 5 ? pair(q.fe[0], q.fo[0]) : pair(q.fe[1], q.fo[1]);
+    } else if constexpr (F == GT_Q80) {
+      // one dword = 4 weights = half of a 16-byte LDS write
+      if (part == 0) q.e = w ^ 0x80808080u;
+      else if (part == 1 || part == 3) {
+        q.a = byte_f(q.e, part - 1);
+        q.b = byte_f(q.e, part);
+      } else {
+        q.outv[(dw & 1) * 2 + (part == 4)] = pack2(__builtin_fmaf(q.a, q.sf[i][0], q.nz[i][0]), __builtin_fmaf(q.b, q.sf[i][0], q.nz[i][0]));
+        if (part == 4 && (dw & 1)) *reinterpret_cast<u32x4*>(dst[i] + (dw >> 1) * 16) = q.outv;
+      }
+    } else {
+      constexpr uint32_t kField = F == GT_Q6K ? 0x03030303u : 0x01010101u;
+      constexpr int kPair = F == GT_Q6K ? 2 : 3;              // pieces per pair of weights
+      if (part == 0) {
+        q.e = w & 0x0F0F0F0Fu;
+        q.o = (w >> 4) & 0x0F0F0F0Fu;
+      } else if (part == 1) {
+        q.h0 = st.h[i][dw >> 1][(dw & 1) * 2] >> st.sh & kField;         // elements 0 1 2 3 of the dword's 8
+        q.h1 = st.h[i][dw >> 1][(dw & 1) * 2 + 1] >> st.sh & kField;     // elements 4 5 6 7
+      } else if (part == 2) {
+        const uint32_t he = __builtin_amdgcn_perm(q.h1, q.h0, 0x06040200u);
+        q.h1 = __builtin_amdgcn_perm(q.h1, q.h0, 0x07050301u);
+        q.h0 = he;
+      } else if (part == 3) {
+        q.e |= q.h0 << 4;
+        q.o |= q.h1 << 4;
+      } else if (part == PPD - 1) *reinterpret_cast<u32x4*>(dst[i] + dw * 16) = q.outv;
+      else {
+        const int pr = (part - 4) / kPair, sub = (part - 4) % kPair;
+        if (sub == 0) {
+          q.a = byte_f(q.e, pr);
+          q.b = byte_f(q.o, pr);
+        } else if constexpr (F == GT_Q6K) {
+          const int t = dw >> 1;                               // 16-wide group of the chunk
+          q.outv[pr] = pack2(__builtin_fmaf(q.a, q.sf[i][t], q.nz[i][t]), __builtin_fmaf(q.b, q.sf[i][t], q.nz[i][t]));
+        } else if (sub == 1) q.h0 = pack2(q.a * q.sf[i][0], q.b * q.sf[i][0]);
+        else q.outv[pr] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, q.h0) - q.mv[i]);
+      }
+    }
+  }
+  static __device__ __forceinline__ float out_scale(const Res&, const GemmArgs&, int) { return 1.0f; }
+};
+
 // ------------------------------------------------------------------ FP8 E4M3
 // 16 codes per 16-byte chunk, four chunks per row and step.  BLOCK = false: the decode is exact
 // (every E4M3 value is a 16-bit float) and the per-channel or per-tensor scale multiplies the
@@ -315,7 +471,7 @@ struct WFp8 {
     r.se = (const char*)p.scale + (long long)e * p.g_s_stride;
     return r;
   }
-  static __device__ __forceinline__ void chunk_addr(const Res& r, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
+  static __device__ __forceinline__ void chunk_addr(Res& r, int, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
     boff = (uint32_t)n * (uint32_t)K + (uint32_t)(kc * 16);
     soff = (uint32_t)(n >> 7) * (uint32_t)r.Kb * 4u;  // bytes: the row block's first scale
   }
@@ -372,6 +528,11 @@ struct WFp8 {
     return p.scale_f16 ? (float)((const _Float16*)r.se)[n] : ((const float*)r.se)[n];
   }
 };
+
+template <int... I, class F>
+__device__ __forceinline__ void fold_pieces(std::integer_sequence<int, I...>, F f) {
+  (f(I), ...);
+}
 
 // ------------------------------------------------------------------ kernel
 // GROUPED: the M-tiles come from a device-built table of (expert, rows) instead of a regular grid
@@ -441,7 +602,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   const int Mp = (p.M + 15) & ~15;
   const uint32_t xtiles = GROUPED ? (uint32_t)p.x_blocks : (uint32_t)(Mp >> 4);
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, xtiles * 16u * (uint32_t)K * 2u);
-  const typename Fmt::Res res = Fmt::make(p, expert);
+  typename Fmt::Res res = Fmt::make(p, expert);
   // 16-row activation tile b of this wavefront inside the BM-row tile.  GROUPED: the two wavefront
   // rows take the tiles alternately and a wavefront multiplies only the first TM, TM / 2 or TM / 4 of
   // its tiles, whichever covers the `live` ones with rows of the expert in them (the K loop exists
@@ -490,7 +651,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
     const int n = tile_row(row);
     const bool live = FUSE ? (n0 + (row >> 5) * 16 + (row & 15) < p.n_half) : (n < N);
     const uint32_t dead = (uint32_t)(!(live && row < BN)) << 31;
-    Fmt::chunk_addr(res, n, kc, K, boff[i], soff[i]);
+    Fmt::chunk_addr(res, i, n, kc, K, boff[i], soff[i]);
     boff[i] |= dead;
     soff[i] |= dead;
     blds[i] = smem + (row * kPitch + kc * (kBK / CPR)) * 2;
@@ -579,8 +740,9 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   {
     DqState q;
     Fmt::begin(res, s0, q);
-#pragma unroll
-    for (int I = 0; I < kPieces; ++I) dq_piece(s0, 0, I, q);
+    // a fold, not a loop: the pieces of the longer formats exceed what "#pragma unroll" expands, and a rolled
+    // loop would keep the stage on the stack
+    fold_pieces(std::make_integer_sequence<int, kPieces>{}, [&](int I) __attribute__((always_inline)) { dq_piece(s0, 0, I, q); });
   }
   __syncthreads();
   auto k_loop = [&](auto live_c) __attribute__((always_inline)) {

@@ -400,6 +400,18 @@ def _chk_f16(t, numel, nm, who):
          f"{who}: {nm} must be contiguous fp16 with {numel} elements")
 
 
+def _gguf_tiled(fmt, x, w, qh, scale, qmin, out, M, N, K):
+    """The prefill route of these formats; False where the weight-streaming kernel takes the call: K that does not fill
+    the tiles' K steps, operands beyond the 2 Gi that the tiled kernel addresses, or up to 128 rows, which two passes of
+    the streaming kernel cover (Q6_K 5120 x 5120: M=128 45 against 64 us, M=192 68 against 65 us)."""
+    if M <= 128 or not _prefill_route(M, K) or (M + 15) * K * 2 >= 1 << 31 or N * K >= 1 << 31 or N == 0:
+        return False
+    buf, nbytes = _tiled_workspace(x, M, K)
+    capi.call("mi_gemm_gguf_tiled_ws", x, fmt, capi.ptr(x), capi.ptr(w), capi.ptr(qh), capi.ptr(scale), capi.ptr(qmin),
+              capi.ptr(out), capi.ptr(buf), nbytes, M, N, K)
+    return True
+
+
 def _gemv_q4_0(input, weight, weight_scale, output, who):
     _chk(weight.dtype == torch.uint8 and weight.dim() == 2 and weight.is_contiguous(),
          f"{who}: weight must be contiguous uint8 [N, K/2]")
@@ -407,6 +419,8 @@ def _gemv_q4_0(input, weight, weight_scale, output, who):
     _chk(K % 32 == 0, f"{who}: K={K} must be a multiple of 32")
     _chk_f16(weight_scale, N * (K // 32), "weight_scale [N, K/32]", who)
     M = _chk_gguf_io(input, output, N, K, who)
+    if _gguf_tiled(3, input, weight, None, weight_scale, None, output, M, N, K):
+        return output
     capi.call("mi_gemv_q4_0", input, capi.ptr(input), capi.ptr(weight), capi.ptr(weight_scale), capi.ptr(output), M, N, K)
     return output
 
@@ -428,6 +442,8 @@ def _gemv_q8_0(input, weight, weight_scale, output, who):
     _chk(K % 32 == 0, f"{who}: K={K} must be a multiple of 32")
     _chk_f16(weight_scale, N * (K // 32), "weight_scale [N, K/32]", who)
     M = _chk_gguf_io(input, output, N, K, who)
+    if _gguf_tiled(4, input, weight, None, weight_scale, None, output, M, N, K):
+        return output
     capi.call("mi_gemv_q8_0", input, capi.ptr(input), capi.ptr(weight), capi.ptr(weight_scale), capi.ptr(output), M, N, K)
     return output
 
@@ -451,6 +467,8 @@ def esimd_gemv_q5_k(input, ql, qh, weight_scale, weight_min, output):
     _chk_f16(weight_scale, N * (K // 32), "weight_scale [N, K/32]", who)
     _chk_f16(weight_min, N * (K // 32), "weight_min [N, K/32]", who)
     M = _chk_gguf_io(input, output, N, K, who)
+    if _gguf_tiled(5, input, ql, qh, weight_scale, weight_min, output, M, N, K):
+        return output
     capi.call("mi_gemv_q5k", input, capi.ptr(input), capi.ptr(ql), capi.ptr(qh), capi.ptr(weight_scale),
               capi.ptr(weight_min), capi.ptr(output), M, N, K)
     return output
@@ -636,6 +654,8 @@ def _gemv_q6_k(input, ql, qh, weight_scale, output, who):
     _chk_u8(qh, (N, K // 4), "qh", who)
     _chk_f16(weight_scale, N * (K // 16), "weight_scale [N, K/16]", who)
     M = _chk_gguf_io(input, output, N, K, who)
+    if _gguf_tiled(6, input, ql, qh, weight_scale, None, output, M, N, K):
+        return output
     capi.call("mi_gemv_q6k", input, capi.ptr(input), capi.ptr(ql), capi.ptr(qh), capi.ptr(weight_scale),
               capi.ptr(output), M, N, K)
     return output

@@ -255,6 +255,30 @@ def test_one_hot_activations_return_the_dequantized_weights(ops, dev, kind, M, K
     assert torch.equal(out.cpu().float(), wd[:, ks].t())
 
 
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("M,N,K", [(129, 8, 512),                 # 128 x 128 tiles, a last row tile of one row
+                                   (144, 257, 1024),              # odd N: element-wise stores
+                                   (300, 9000, 512),              # 256-row tiles
+                                   (130, 72, 1536),               # three high-bit tiles of 512
+                                   (140, 64, 640), (131, 40, 96)])  # Q4_0 / Q8_0 only: K % 128 == 0 (tiled), K % 32 == 0 (streaming)
+def test_prefill_one_hot_rows_return_the_dequantized_weights(ops, dev, kind, M, N, K):
+    """More than 128 rows take the tiled matrix-core GEMM: one 1.0 per row returns the oracle's dequantized fp16
+    weights value for value (decode, high bits of every field, scales, tile and K-step edges)."""
+    if kind in ("q5_k", "q6_k") and K % 512:
+        pytest.skip("K must be a multiple of 512")
+    _, s = ops
+    rep = _repack_oracle(kind, _raw_case(kind, N, -(-K // 512) * 512, seed=M + K))
+    if K % 512:
+        rep = tuple(np.ascontiguousarray(a[:, :a.shape[1] * K // (-(-K // 512) * 512)]) for a in rep)
+    wd = torch.from_numpy(_dequant_oracle(kind, rep).astype(np.float32))
+    ks = (9 + 37 * torch.arange(M)) % K
+    x = torch.zeros(M, K, dtype=torch.float16)
+    x[torch.arange(M), ks] = 1.0
+    out = torch.empty(M, N, dtype=torch.float16, device=dev)
+    _gemv(s, kind, x.to(dev), [_t(a).to(dev) for a in rep], out)
+    assert torch.equal(out.cpu().float(), wd[:, ks].t())
+
+
 @pytest.mark.parametrize("name,kind", [("esimd_gemm_q4_0", "q4_0"), ("esimd_gemv_q8_0_m", "q8_0"), ("esimd_gemv_q6_k_m", "q6_k")])
 def test_small_m_variants(ops, dev, name, kind):
     _, s = ops
