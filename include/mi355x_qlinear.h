@@ -457,6 +457,11 @@ int mi_moe_mlp_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_d
  * route of the block-scaled linear (vllm/patches/vllm_for_multi_arc.patch:2671-2691) and the
  * M > 1 dense route of Q4_K (sglang/patches/sglang_for_multi_arc.patch:3211-3213). */
 int mi_gemm_tiled_workspace(int M, int K, long long* bytes);
+/* The bytes with which every *_ws entry of the dense tiled GEMM (mi_gemm_int4_ws, mi_gemm_fp8_tiled_ws,
+ * mi_gemm_q4k_tiled_ws, mi_gemm_gguf_tiled_ws) may also spread the K range of a problem with few tiles over
+ * the chip: the re-tiled activations and the slices' fp32 sums.  With less (down to the sizes above)
+ * the same entries run in one piece. */
+int mi_gemm_tiled_workspace_split(int M, int N, int K, long long* bytes);
 int mi_gemm_fp8_tiled_ws(const void* x, const void* w, const void* scale, int scale_mode, int scale_is_f16,
                          void* out, void* workspace, long long workspace_bytes, int M, int N, int K,
                          int act_dtype, void* stream);

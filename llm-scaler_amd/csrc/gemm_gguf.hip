@@ -32,10 +32,10 @@ int mi_gemm_gguf_tiled_ws(int fmt, const void* x, const void* w, const void* qh,
   p.w = w; p.qh = qh; p.scale = scale; p.zp = qmin; p.out = out; p.M = M; p.N = N; p.K = K;
   hipStream_t st = (hipStream_t)stream;
   switch (fmt) {
-    case GT_Q40: return run_gemm_tiled<ActF16, WQ40>(p, x, workspace, st);
-    case GT_Q80: return run_gemm_tiled<ActF16, WQ80>(p, x, workspace, st);
-    case GT_Q5K: return run_gemm_tiled<ActF16, WQ5K>(p, x, workspace, st);
-    default: return run_gemm_tiled<ActF16, WQ6K>(p, x, workspace, st);
+    case GT_Q40: return run_gemm_tiled<ActF16, WQ40>(p, x, workspace, workspace_bytes, st);
+    case GT_Q80: return run_gemm_tiled<ActF16, WQ80>(p, x, workspace, workspace_bytes, st);
+    case GT_Q5K: return run_gemm_tiled<ActF16, WQ5K>(p, x, workspace, workspace_bytes, st);
+    default: return run_gemm_tiled<ActF16, WQ6K>(p, x, workspace, workspace_bytes, st);
   }
 }
 

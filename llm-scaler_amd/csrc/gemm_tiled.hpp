@@ -29,6 +29,7 @@
 // chunk as a sequence of small pieces, and an optional factor on the finished sums.
 #pragma once
 #include "qlinear_common.hpp"
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -62,6 +63,8 @@ struct GemmArgs {
   int n_half;                 // FUSE: weight row n (gate) pairs with row n + n_half (up); N = 2 n_half
   int gelu;                   // FUSE: tanh-GELU instead of SiLU
   int out_rows;               // rows of out (bounds mapped rows)
+  int splits, split_steps;    // SPLIT: the 64-wide steps of K go to `splits` workgroups per tile, split_steps (even) each
+  float* partial;             // SPLIT: fp32 sums, [split][tile][wave][column tile][row tile][lane][4]
   int out_packed;             // GROUPED: out is written in the re-tiled operand order of x (16-row blocks of the
                               // tile table, n_out / 32 steps each) for a following grouped GEMM; out_rows = 16 x blocks
 };
@@ -539,7 +542,9 @@ __device__ __forceinline__ void fold_pieces(std::integer_sequence<int, I...>, F 
 // (MoE: rows sorted by expert, one weight matrix per expert).  FUSE: the tile's weight rows
 // alternate, 16 at a time, between a gate block and the up block n_half rows further on, and the
 // epilogue writes act(gate) * up (N / 2 output columns).
-template <class Act, class Fmt, int BM, int BN, bool GROUPED = false, bool FUSE = false>
+// SPLIT: blockIdx.y takes one slice of K and the fp32 sums go to a workspace in accumulator order (1 KiB
+// per store); split_reduce_kernel adds the slices and writes the output.
+template <class Act, class Fmt, int BM, int BN, bool GROUPED = false, bool FUSE = false, bool SPLIT = false>
 __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   using Elem = typename Act::elem;
   constexpr int WM = BM / 2, WN = BN / 2;             // wave sub-tile
@@ -587,8 +592,13 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   const int n0 = FUSE ? tn * (BN / 2) : tn * BN;      // FUSE: first gate row of the tile
   int M = p.M;
   const int N = p.N, K = p.K;
-  const int KT = K / kBK;                             // 64-wide steps (even: K % 128 == 0)
   const int Q = K / 32;                               // 32-wide MFMA steps
+  int kt0 = 0, KT = K / kBK;                          // 64-wide steps of this workgroup (even: K % 128 == 0)
+  if constexpr (SPLIT) {
+    kt0 = blockIdx.y * p.split_steps;
+    KT = kt0 + p.split_steps < KT ? kt0 + p.split_steps : KT;
+  }
+  const int Qe = 2 * KT;
   int expert = 0, row0 = 0, xblk0 = 0;
   if constexpr (GROUPED) {
     if (tm >= p.g_count[0]) return;                   // the grid is an upper bound of the tile count
@@ -633,7 +643,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
     xtoff[b] = __builtin_amdgcn_readfirstlane(t * (uint32_t)Q * 1024u);
   }
   auto load_x1 = [&](int slot, int b, int q) {        // a step beyond the last re-reads the last (never used)
-    const uint32_t qc = (uint32_t)(q < Q ? q : Q - 1);
+    const uint32_t qc = (uint32_t)(q < Qe ? q : Qe - 1);
     xring[slot][b] = __builtin_amdgcn_raw_buffer_load_b128(xr, xlane, xtoff[b] + qc * 1024u, 0);
   };
   auto load_x = [&](int slot, int q) {
@@ -729,13 +739,13 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   };
 
   StageB s0, s1;
-  load_b(s0, 0);
+  load_b(s0, kt0);
   __builtin_amdgcn_sched_barrier(0);
-  load_b(s1, 1);
+  load_b(s1, kt0 + 1);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     __builtin_amdgcn_sched_barrier(0);               // keep the ring's loads in issue order
-    load_x(r, r);
+    load_x(r, 2 * kt0 + r);
   }
   {
     DqState q;
@@ -746,7 +756,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   }
   __syncthreads();
   auto k_loop = [&](auto live_c) __attribute__((always_inline)) {
-    for (int kt = 0; kt < KT; kt += 2) {
+    for (int kt = kt0; kt < KT; kt += 2) {
       step64(live_c, kt, 0, 0, s1, s0);
       step64(live_c, kt + 1, 1, 2, s0, s1);
     }
@@ -762,6 +772,16 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   // the last MFMAs are still in the matrix pipe: wait before reading their results
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
   // D = W-tile (rows n) x X-tile^T: lane holds n = 4 g + v (v = 0..3), m = j
+  if constexpr (SPLIT) {
+    f32x4* dst = reinterpret_cast<f32x4*>(p.partial) +
+                 (((size_t)blockIdx.y * (size_t)(p.tiles_m * p.tiles_n) + (size_t)(tn * p.tiles_m + tm)) * 4 + wave) * (TN * TM * 64) + lane;
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+      for (int b = 0; b < TM; ++b)
+        if (m0 + mtile(b) * 16 < M) dst[(a * TM + b) * 64] = acc[a][b];       // uniform: row tiles with rows of x in them
+    return;
+  }
   Elem* out = (Elem*)p.out;
   const int n_out = FUSE ? p.n_half : N;              // output columns
   // output row of this lane's row of activation tile b, or -1
@@ -938,7 +958,42 @@ static __global__ __launch_bounds__(256) void pack_x_kernel(const uint16_t* __re
   xp[((size_t)t * Q + q) * 64 + l] = v;
 }
 
+// Adds the K slices of a SPLIT launch (in slice order), scales, rounds and writes the output.  A wavefront
+// takes one 16 x 16 accumulator tile: lane 16 g + j holds row j, columns 4 g .. 4 g + 3.  grid (tiles, 4 TN TM / 4).
 template <class Act, class Fmt, int BM, int BN>
+__global__ __launch_bounds__(256) void split_reduce_kernel(const GemmArgs p) {
+  using Elem = typename Act::elem;
+  constexpr int TM = BM / 32, TN = BN / 32;
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+  const int tile = blockIdx.x;
+  const int at = __builtin_amdgcn_readfirstlane(blockIdx.y * 4 + (threadIdx.x >> 6));   // [wave][column tile][row tile]
+  const int wave = at / (TN * TM), a = at / TM % TN, b = at % TM;
+  const int tn = tile / p.tiles_m, tm = tile - tn * p.tiles_m;
+  const int m = tm * BM + (wave >> 1) * (BM / 2) + b * 16, n = tn * BN + (wave & 1) * (BN / 2) + a * 16 + g * 4;
+  if (m >= p.M) return;                               // uniform
+  const size_t slice = (size_t)p.tiles_m * p.tiles_n * (BM * BN / 4);                   // in f32x4
+  const f32x4* src = reinterpret_cast<const f32x4*>(p.partial) + (size_t)tile * (BM * BN / 4) + (size_t)at * 64 + lane;
+  f32x4 sum = src[0];
+#pragma unroll 4
+  for (int i = 1; i < p.splits; ++i) sum += src[(size_t)i * slice];
+  if (m + j >= p.M) return;
+  if constexpr (Fmt::kOutScale) {
+    const typename Fmt::Res res = Fmt::make(p);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) sum[v] *= Fmt::out_scale(res, p, n + v < p.N ? n + v : p.N - 1);
+  }
+  Elem* out = (Elem*)p.out + (size_t)(m + j) * p.N + n;
+  if (n + 3 < p.N && (p.N & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0) {
+    Elem r[4] = {Act::from_f32(sum[0]), Act::from_f32(sum[1]), Act::from_f32(sum[2]), Act::from_f32(sum[3])};
+    *reinterpret_cast<u32x2*>(out) = __builtin_bit_cast(u32x2, r);
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (n + v < p.N) out[v] = Act::from_f32(sum[v]);
+  }
+}
+
+template <class Act, class Fmt, int BM, int BN, bool SPLIT = false>
 static int launch_gemm_tiled(GemmArgs p, hipStream_t st) {
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
@@ -955,7 +1010,7 @@ static int launch_gemm_tiled(GemmArgs p, hipStream_t st) {
     }
   }
   const size_t lds = (size_t)2 * (Fmt::B_CH * 256 / Fmt::CPR) * kPitch * 2;
-  auto kern = gemm_tiled_kernel<Act, Fmt, BM, BN>;
+  auto kern = gemm_tiled_kernel<Act, Fmt, BM, BN, false, false, SPLIT>;
   if (lds > 64 * 1024) {
     static bool raised = false;                       // opt in to > 64 KiB of dynamic LDS once
     if (!raised) {
@@ -965,7 +1020,9 @@ static int launch_gemm_tiled(GemmArgs p, hipStream_t st) {
       raised = true;
     }
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(256), lds, st, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)(SPLIT ? p.splits : 1)), dim3(256), lds, st, p);
+  if constexpr (SPLIT)
+    hipLaunchKernelGGL((split_reduce_kernel<Act, Fmt, BM, BN>), dim3((unsigned)(p.tiles_m * p.tiles_n), BM * BN / 1024), dim3(256), 0, st, p);
   return launch_status();
 }
 
@@ -986,13 +1043,41 @@ static inline long device_cu_count_gemm() {
   return cus;
 }
 
+static inline bool gemm_big_tiles(long M, long N) {
+  return M > 128 && ((M + 255) / 256) * ((N + 255) / 256) * 2 > device_cu_count_gemm();
+}
+
+// K slices of a problem on 128 x 128 tiles.  A tile is a chain of K / 64 steps of about 0.65 us whether its
+// neighbours' CUs are busy or not, so a problem with few tiles leaves the chip idle: slices up to one workgroup
+// per CU (two per CU share the path from L2 to the CU and gain nothing: Q8_0 1000 x 4096 x 4096, 256 tiles:
+// 61 us in one piece, 65 in two).  Every slice writes and reads fp32 sums of the whole output, 8 bytes per
+// element at about 5 TB/s, which sets the best number where tiles are few.  One slice against this rule's:
+// INT4 128 x 4096 x 4096 44 -> 22 us, Q4_K 100 x 5120 x 5120 63 -> 26 us, Q6_K 129 x 5120 x 5120 71 -> 38 us, INT4
+// 1024 x 6144 x 2048 72 -> 51 us, FP8 70 x 1024 x 1024 13.6 -> 10 us.
+static inline int gemm_splits(long M, long N, long K) {
+  if (M <= 64 || N <= 0 || gemm_big_tiles(M, N)) return 1;
+  const long tiles = ((M + 127) / 128) * ((N + 127) / 128);
+  const long most = std::min(device_cu_count_gemm() / tiles, K / 128);
+  const double chain = 0.65 * (double)(K / 64), sums = (double)((M + 15) / 16 * 16) * (double)N * 8.0 / 5e6;   // us
+  int best = 1;
+  for (long s = 2; s <= most; ++s)
+    if (chain / s + sums * s < chain / best + (best > 1 ? sums * best : -2.0)) best = (int)s;     // the second launch: 2 us
+  return best;
+}
+
+// bytes of the re-tiled activations and, behind them, of the slices' sums
+static inline long long gemm_workspace(long M, long N, long K, int splits) {
+  const long long packed = ((M + 15) & ~15LL) * K * 2;
+  return splits < 2 ? packed : packed + (long long)splits * ((M + 127) / 128) * ((N + 127) / 128) * (128 * 128 * 4);
+}
+
 // Re-tiles x into `workspace` and runs the tile shape that fits the problem: 128 x 128 tiles
 // while 256-row tiles would leave more than half of the chip idle, else 256 rows x 256 / 224 /
 // 192 / 160 columns, whichever needs the least time over its rounds of resident workgroups (a
 // 5120-column weight is 32 tiles of 160: with 8 row tiles exactly one round of 256 workgroups,
 // where 256-column tiles fill 160 of the 256 CUs).  FMT is a template taking (Act, BN).
 template <class Act, template <class, int> class FMT>
-static int run_gemm_tiled(GemmArgs p, const void* x, void* workspace, hipStream_t st) {
+static int run_gemm_tiled(GemmArgs p, const void* x, void* workspace, long long workspace_bytes, hipStream_t st) {
   const int Mp = (p.M + 15) & ~15;
   const int Q = p.K / 32;
   hipLaunchKernelGGL(pack_x_kernel, dim3((unsigned)(((Q + 3) / 4) * (Mp / 16))), dim3(256), 0, st, (const uint16_t*)x,
@@ -1002,8 +1087,17 @@ static int run_gemm_tiled(GemmArgs p, const void* x, void* workspace, hipStream_
   // work per weight and activation byte it moves and runs at about a third of the rate)
   const long cus = device_cu_count_gemm();
   const long tiles_m = (p.M + 255) / 256;
-  const bool big = p.M > 128 && tiles_m * ((p.N + 255) / 256) * 2 > cus;
-  if (!big) return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128>(p, st);
+  const bool big = gemm_big_tiles(p.M, p.N);
+  if (!big) {
+    const int splits = gemm_splits(p.M, p.N, p.K);
+    if (splits > 1 && workspace_bytes >= gemm_workspace(p.M, p.N, p.K, splits)) {
+      p.split_steps = ((p.K / 128 + splits - 1) / splits) * 2;
+      p.splits = (p.K / 64 + p.split_steps - 1) / p.split_steps;
+      p.partial = (float*)((char*)workspace + gemm_workspace(p.M, p.N, p.K, 1));
+      return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128, true>(p, st);
+    }
+    return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128>(p, st);
+  }
   // time ~ rounds of resident workgroups x (columns of a tile + a fixed part per K step)
   auto cost = [&](long bn) { return ((tiles_m * ((p.N + bn - 1) / bn) + cus - 1) / cus) * (bn + kTileFixedCols); };
   long best = 256;

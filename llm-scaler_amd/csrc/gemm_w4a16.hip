@@ -30,8 +30,8 @@ int mi_gemm_int4_ws(const void* x, const void* w, const void* scale, const void*
   if (!workspace || workspace_bytes < (long long)Mp * K * 2) return MI_ERR_ARG;
   GemmArgs p{};
   p.w = w; p.scale = scale; p.zp = zp; p.out = out; p.M = M; p.N = N; p.K = K;
-  return act_dtype == DT_F16 ? run_gemm_tiled<ActF16, WInt4>(p, x, workspace, (hipStream_t)stream)
-                             : run_gemm_tiled<ActBF16, WInt4>(p, x, workspace, (hipStream_t)stream);
+  return act_dtype == DT_F16 ? run_gemm_tiled<ActF16, WInt4>(p, x, workspace, workspace_bytes, (hipStream_t)stream)
+                             : run_gemm_tiled<ActBF16, WInt4>(p, x, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int mi_gemm_int4(const void* x, const void* w, const void* scale, const void* zp, void* out, int M, int N,
@@ -40,7 +40,8 @@ int mi_gemm_int4(const void* x, const void* w, const void* scale, const void* zp
   const int rc = mi_gemm_int4_workspace(M, N, K, &bytes);
   if (rc != MI_OK) return rc;
   if (!bytes) return mi_gemm_int4_ws(x, w, scale, zp, out, nullptr, 0, M, N, K, act_dtype, stream);
-  // scratch for the re-tiled activations: this stream's grow-only buffer (the first
+  if (mi_gemm_tiled_workspace_split(M, N, K, &bytes) != MI_OK) return MI_ERR_SHAPE;
+  // scratch for the re-tiled activations and the K slices' sums: this stream's grow-only buffer (the first
   // call of a size allocates; callers that must never allocate pass their own
   // workspace through mi_gemm_int4_ws)
   void* ws = scratch_get((hipStream_t)stream, (size_t)bytes);

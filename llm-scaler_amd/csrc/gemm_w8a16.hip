@@ -30,6 +30,13 @@ int mi_gemm_tiled_workspace(int M, int K, long long* bytes) {
   return MI_OK;
 }
 
+int mi_gemm_tiled_workspace_split(int M, int N, int K, long long* bytes) {
+  if (!bytes) return MI_ERR_ARG;
+  if (M < 0 || N < 0 || K <= 0) return MI_ERR_SHAPE;
+  *bytes = gemm_workspace(M, N, K, gemm_splits(M, N, K));
+  return MI_OK;
+}
+
 int mi_gemm_fp8_tiled_ws(const void* x, const void* w, const void* scale, int scale_mode, int scale_is_f16,
                          void* out, void* workspace, long long workspace_bytes, int M, int N, int K,
                          int act_dtype, void* stream) {
@@ -45,10 +52,10 @@ int mi_gemm_fp8_tiled_ws(const void* x, const void* w, const void* scale, int sc
   p.scale_mode = scale_mode; p.scale_f16 = scale_is_f16;
   hipStream_t st = (hipStream_t)stream;
   if (scale_mode == 2)
-    return act_dtype == DT_F16 ? run_gemm_tiled<ActF16, WFp8Block>(p, x, workspace, st)
-                               : run_gemm_tiled<ActBF16, WFp8Block>(p, x, workspace, st);
-  return act_dtype == DT_F16 ? run_gemm_tiled<ActF16, WFp8Plain>(p, x, workspace, st)
-                             : run_gemm_tiled<ActBF16, WFp8Plain>(p, x, workspace, st);
+    return act_dtype == DT_F16 ? run_gemm_tiled<ActF16, WFp8Block>(p, x, workspace, workspace_bytes, st)
+                               : run_gemm_tiled<ActBF16, WFp8Block>(p, x, workspace, workspace_bytes, st);
+  return act_dtype == DT_F16 ? run_gemm_tiled<ActF16, WFp8Plain>(p, x, workspace, workspace_bytes, st)
+                             : run_gemm_tiled<ActBF16, WFp8Plain>(p, x, workspace, workspace_bytes, st);
 }
 
 int mi_gemm_q4k_tiled_ws(const void* x, const void* ql, const void* scale, const void* qmin, void* out,
@@ -60,7 +67,7 @@ int mi_gemm_q4k_tiled_ws(const void* x, const void* ql, const void* scale, const
   if (!workspace || workspace_bytes < (long long)((M + 15) & ~15) * K * 2) return MI_ERR_ARG;
   GemmArgs p{};
   p.w = ql; p.scale = scale; p.zp = qmin; p.out = out; p.M = M; p.N = N; p.K = K;
-  return run_gemm_tiled<ActF16, WQ4K>(p, x, workspace, (hipStream_t)stream);
+  return run_gemm_tiled<ActF16, WQ4K>(p, x, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -88,8 +88,11 @@ static int run(SkinnyArgs a, int act_dtype, hipStream_t st) {
   // prefill: the tiled matrix-core GEMM reads the weight once per 256 rows instead of once per 64
   if constexpr (FMT == 0 || FMT == 2) {
     if (a.M > 64 && a.K % 128 == 0) {
-      long long bytes = 0;
-      if (mi_gemm_tiled_workspace(a.M, a.K, &bytes) != MI_OK) return MI_ERR_SHAPE;
+      long long bytes = 0, need = 0;
+      for (int i = 0; i < a.nmat; ++i) {
+        if (mi_gemm_tiled_workspace_split(a.M, a.N[i], a.K, &need) != MI_OK) return MI_ERR_SHAPE;
+        if (need > bytes) bytes = need;
+      }
       void* ws = scratch_get(st, (size_t)bytes);
       if (!ws) return MI_ERR_LAUNCH;
       for (int i = 0; i < a.nmat; ++i) {

@@ -72,12 +72,15 @@ def _chk_act(x: torch.Tensor, out: torch.Tensor, who: str):
 _SC_PERN, _SC_PERT, _SC_BLOCK = 0, 1, 2
 
 
-def _tiled_workspace(x, M, K):
-    need = ctypes.c_longlong(0)
-    rc = capi.lib().mi_gemm_tiled_workspace(M, K, ctypes.byref(need))
-    if rc != 0:
-        raise RuntimeError(f"mi_gemm_tiled_workspace: {capi.MI_ERRORS.get(rc, rc)}")
-    return torch.empty(need.value, dtype=torch.uint8, device=x.device), need.value
+def _tiled_workspace(x, M, Ns, K):
+    """Workspace of one call per N in Ns: re-tiled activations and, behind them, the sums of the K slices."""
+    need, most = ctypes.c_longlong(0), 0
+    for N in Ns:
+        rc = capi.lib().mi_gemm_tiled_workspace_split(M, int(N), K, ctypes.byref(need))
+        if rc != 0:
+            raise RuntimeError(f"mi_gemm_tiled_workspace_split: {capi.MI_ERRORS.get(rc, rc)}")
+        most = max(most, need.value)
+    return torch.empty(most, dtype=torch.uint8, device=x.device), most
 
 
 def _prefill_route(M, K):
@@ -85,7 +88,7 @@ def _prefill_route(M, K):
 
 
 def _fp8_tiled_multi(x, ws, ss, os_, Ns, M, K, mode, scale_f16):
-    buf, nbytes = _tiled_workspace(x, M, K)
+    buf, nbytes = _tiled_workspace(x, M, Ns, K)
     for w, s, o, N in zip(ws, ss, os_, Ns):
         capi.call("mi_gemm_fp8_tiled_ws", x, capi.ptr(x), capi.ptr(w), capi.ptr(s), mode, 1 if scale_f16 else 0,
                   capi.ptr(o), capi.ptr(buf), nbytes, M, int(N), K, capi.act_dtype(x))
@@ -299,13 +302,9 @@ def _gemm_int4(x, w, s, zp, o, who):
     M, N, K = _chk_int4(x, w, s, zp, o, who)
     # the prefill kernel re-tiles the activations into a workspace; it comes from torch's
     # caching allocator so that the op stays capturable in a HIP graph
-    need = ctypes.c_longlong(0)
-    rc = capi.lib().mi_gemm_int4_workspace(M, N, K, ctypes.byref(need))
-    if rc != 0:
-        raise RuntimeError(f"{who}: {capi.MI_ERRORS.get(rc, rc)}")
-    ws = torch.empty(need.value, dtype=torch.uint8, device=x.device) if need.value else None
+    ws, nbytes = _tiled_workspace(x, M, [N], K) if M > 64 and N else (None, 0)
     capi.call("mi_gemm_int4_ws", x, capi.ptr(x), capi.ptr(w), capi.ptr(s), capi.ptr(zp), capi.ptr(o),
-              capi.ptr(ws), need.value, M, N, K, capi.act_dtype(x))
+              capi.ptr(ws), nbytes, M, N, K, capi.act_dtype(x))
     return o
 
 
@@ -340,7 +339,7 @@ def _chk_q4k(x, w, s, mn, o, who):
 def esimd_gemv_q4_k(input, weight, weight_scale, weight_min, output):
     M, N, K = _chk_q4k(input, weight, weight_scale, weight_min, output, "esimd_gemv_q4_k")
     if _prefill_route(M, K):
-        buf, nbytes = _tiled_workspace(input, M, K)
+        buf, nbytes = _tiled_workspace(input, M, [N], K)
         capi.call("mi_gemm_q4k_tiled_ws", input, capi.ptr(input), capi.ptr(weight), capi.ptr(weight_scale),
                   capi.ptr(weight_min), capi.ptr(output), capi.ptr(buf), nbytes, M, N, K)
         return output
@@ -401,12 +400,16 @@ def _chk_f16(t, numel, nm, who):
 
 
 def _gguf_tiled(fmt, x, w, qh, scale, qmin, out, M, N, K):
-    """The prefill route of these formats; False where the weight-streaming kernel takes the call: K that does not fill
-    the tiles' K steps, operands beyond the 2 Gi that the tiled kernel addresses, or up to 128 rows, which two passes of
-    the streaming kernel cover (Q6_K 5120 x 5120: M=128 45 against 64 us, M=192 68 against 65 us)."""
-    if M <= 128 or not _prefill_route(M, K) or (M + 15) * K * 2 >= 1 << 31 or N * K >= 1 << 31 or N == 0:
+    """The prefill route of these formats; False where the weight-streaming kernels take the call: K that does not fill
+    the tiles' K steps, operands beyond the 2 Gi that the tiled kernel addresses, or up to 128 rows of Q4_0 and Q8_0 with K
+    within the K-sliced kernel's reach, which covers them in two passes (Q4_0 128 x 1024 x 12000: 14 against 17 us, 66 x
+    5120 x 1024: 22 against 14; Q8_0 100 x 1024 x 1024: 10 against 11, 80 x 4096 x 4096: 24 against 21; Q6_K 120 x 5120 x
+    12288: 74 against 52)."""
+    if M <= 128 and K <= {3: 3072, 4: 2048}.get(fmt, 0):
         return False
-    buf, nbytes = _tiled_workspace(x, M, K)
+    if not _prefill_route(M, K) or (M + 15) * K * 2 >= 1 << 31 or N * K >= 1 << 31 or N == 0:
+        return False
+    buf, nbytes = _tiled_workspace(x, M, [N], K)
     capi.call("mi_gemm_gguf_tiled_ws", x, fmt, capi.ptr(x), capi.ptr(w), capi.ptr(qh), capi.ptr(scale), capi.ptr(qmin),
               capi.ptr(out), capi.ptr(buf), nbytes, M, N, K)
     return True
