@@ -16,6 +16,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 _PKG_ROOT = os.path.dirname(_HERE)
 HEADER = os.path.join(os.path.dirname(_PKG_ROOT), "include", "mi355x_qlinear.h")
 LIB_PATH = os.path.join(_PKG_ROOT, "lib", "libmi355x_qlinear.so")
+TORCH_OPS_PATH = os.path.join(_PKG_ROOT, "lib", "libmi355x_torch_ops.so")
 
 MI_ERRORS = {-1: "invalid argument (null pointer or bad enum)",
              -2: "unsupported shape or divisibility",
@@ -76,6 +77,14 @@ def lib():
             fn.restype = ctypes.c_int
         _lib = handle
     return _lib
+
+
+def load_torch_ops():
+    """Registers the native host path of the hot operators (csrc/torch_ops.cpp)."""
+    if not os.path.exists(TORCH_OPS_PATH):
+        raise ImportError(f"mi355x_qlinear: {TORCH_OPS_PATH} is missing - build it with "
+                          f"`make -C {os.path.join(_PKG_ROOT, 'csrc')}`. There is no fallback path.")
+    torch.ops.load_library(TORCH_OPS_PATH)
 
 
 def _device_ptr(t) -> int:

@@ -35,14 +35,23 @@ def _library(ns: str) -> torch.library.Library:
 
 
 _DEFINED = {}        # namespace -> names of the operators defined here
+_CHECKED = {}        # operators with a native host path -> their Python implementation
 
 
 def _define(ns: str, schema: str, impl, meta=None):
+    """Declares an operator.  Where the native host path implements it (csrc/torch_ops.cpp), `impl` is what that hands
+    the calls it does not take to, under the name mi355x_checked::<name>."""
     lib = _library(ns)
     lib.define(schema)
     name = schema.split("(", 1)[0]
     _DEFINED.setdefault(ns, []).append(name)
-    lib.impl(name, impl, "CUDA")
+    if not torch._C._dispatch_has_kernel_for_dispatch_key(f"{ns}::{name}", "CUDA"):
+        lib.impl(name, impl, "CUDA")
+    elif name not in _CHECKED:
+        _CHECKED[name] = impl
+        checked = _library("mi355x_checked")
+        checked.define(schema)
+        checked.impl(name, impl, "CUDA")
     if meta is not None:
         lib.impl(name, meta, "Meta")
 
@@ -2168,6 +2177,7 @@ def register():
     if _registered:
         return
     _registered = True
+    capi.load_torch_ops()
     for ns in (_V, _S):
         _define(ns, "esimd_gemv_fp8_pern(Tensor input, Tensor weight, Tensor weight_scale, "
                     "Tensor output, int N, int K) -> Tensor", esimd_gemv_fp8_pern, _ret(3))

@@ -1,0 +1,131 @@
+"""The native host path of the hot operators against their Python implementations (mi355x_checked::<name>): the same
+schema, the same results bit for bit over the forms that both accept, the same refusals."""
+import pytest
+import torch
+
+from mi355x_qlinear import ops as _ops
+
+_V, _S = torch.ops.custom_esimd_kernels_vllm, torch.ops.custom_esimd_kernels_sglang
+
+
+def test_every_native_operator_has_its_python_implementation():
+    assert len(_ops._CHECKED) == 25
+    for ns, names in _ops._DEFINED.items():
+        for name in names:
+            if name in _ops._CHECKED:
+                own = getattr(getattr(torch.ops, ns), name).default._schema
+                other = getattr(torch.ops.mi355x_checked, name).default._schema
+                assert str(own).split("::", 1)[1] == str(other).split("::", 1)[1]
+                assert torch._C._dispatch_has_kernel_for_dispatch_key(f"mi355x_checked::{name}", "CUDA")
+
+
+def _u8(*s):
+    return torch.randint(0, 256, s, dtype=torch.uint8, device="cuda")
+
+
+def _h(*s):
+    return (torch.rand(*s, device="cuda") * 0.01 + 0.005).half()
+
+
+def _args(name, M, K, N, dt):
+    """(arguments, index of the output) of one call."""
+    x = torch.randn(M, K, device="cuda").to(dt)
+    o = torch.empty(M, N, device="cuda", dtype=dt)
+    f8 = (torch.randn(N, K, device="cuda") * 4).to(torch.float8_e4m3fn)
+    one = torch.full((1,), 0.01, device="cuda")
+    if name == "esimd_gemv_fp8_pern":
+        return [x, f8, torch.rand(N, device="cuda") * 0.01, o, N, K], 3
+    if name.startswith("esimd_gemv_fp8_pern_fused"):
+        n = int(name[-1])
+        sc = [_h(N) for _ in range(n)]
+        return [x] + [a for i in range(n) for a in (f8, sc[i], o if i == 0 else torch.empty_like(o), N)] + [K], 3
+    if "blockscale" in name:
+        bs = torch.rand(-(-N // 128), K // 128, device="cuda") * 0.01
+        more = [f8.view(torch.uint8), bs, torch.empty_like(o)] if name.endswith("fused2") else []
+        return [x, f8, bs, o] + more + [128, 128], 3
+    if "resadd" in name:
+        K1 = K
+        xs = [torch.randn(1, K1, device="cuda").to(dt) for _ in range(3)]
+        w = [_u8(N, K // 2), _h(N, K // 128)] if "int4" in name else [f8, one]
+        return xs[:2] + [xs[2].view(-1)] + w + [torch.empty(1, N, device="cuda", dtype=dt), torch.empty_like(xs[0]), 1e-6], 5
+    if "fp8_pert" in name:
+        n = int(name[-1]) if "fused" in name else 1
+        return [x] + [a for i in range(n) for a in (f8, one, o if i == 0 else torch.empty_like(o))], 3
+    if "int4" in name:
+        w, sc = _u8(N, K // 2), _h(N, K // 128)
+        if name.endswith("_zp"):
+            return [x, w, sc, _u8(N, K // 128) & 15, o], 4
+        more = [w, sc, torch.empty_like(o)] if name.endswith("fused2") else []
+        return [x.view(1, M, K), w.view(torch.int32), sc, o] + more, 3      # 3-D input, int32 view of the weight
+    if name == "esimd_gemv_q4_k":
+        return [x, _u8(N, K // 2), _h(N, K // 32), _h(N, K // 32), o], 4
+    if "q4_0" in name:
+        return [x, _u8(N, K // 2), _h(N, K // 32), o], 3
+    if "q8_0" in name:
+        return [x, _u8(N, K).view(torch.int8), _h(N, K // 32), o], 3
+    if "q5_k" in name:
+        return [x, _u8(N, K // 2), _u8(N, K // 8), _h(N, K // 32), _h(N, K // 32), o], 5
+    return [x, _u8(N, K // 2), _u8(N, K // 4), _h(N, K // 16), o], 4
+
+
+_LINEAR = sorted(n for n in _ops._CHECKED if not n.startswith("moe_"))
+
+
+def _own(name):
+    return getattr(_V, name) if name in _ops._DEFINED["custom_esimd_kernels_vllm"] else getattr(_S, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", _LINEAR)
+def test_same_results_and_same_refusals(dev, name):
+    checked = getattr(torch.ops.mi355x_checked, name)
+    for dt in (torch.float16, torch.bfloat16):
+        if dt == torch.bfloat16 and "_q" in name and "_k" in name or dt == torch.bfloat16 and ("q4_0" in name or "q8_0" in name):
+            continue                                      # GGUF formats run in fp16
+        for M, K, N in ((1, 512, 40), (3, 1024, 257), (65, 512, 136), (130, 1024, 264)):
+            torch.manual_seed(M + N)
+            args, at = _args(name, M, K, N, dt)
+            clone = [a.clone() if torch.is_tensor(a) else a for a in args]
+            assert _own(name)(*args) is args[at] and checked(*clone) is clone[at]
+            for a, b in zip(args, clone):                 # outputs, and the residual that the norm updates
+                assert not torch.is_tensor(a) or torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8))
+    args, at = _args(name, 2, 512, 24, torch.float16)
+    bad = [(0, args[0].cpu()), (0, args[0].double()), (1, args[1][..., :-1]), (at, args[at].float()),
+           (at, torch.empty(3, 7, dtype=torch.float16, device=dev))]
+    for i, v in bad:
+        broken = list(args)
+        broken[i] = v
+        said = []
+        for op in (_own(name), checked):
+            with pytest.raises((RuntimeError, NotImplementedError)) as e:
+                op(*broken)
+            said.append(str(e.value).split("\n")[0])
+        if i or v.is_cuda:
+            assert said[0] == said[1]
+
+
+@pytest.mark.gpu
+def test_calls_that_need_preparation_still_run(dev):
+    """Accepted before although not as the kernels want it: a per-channel scale that is a strided view."""
+    args, at = _args("esimd_gemv_fp8_pern", 2, 512, 24, torch.float16)
+    args[2] = args[2].repeat_interleave(2)[::2]
+    out = _V.esimd_gemv_fp8_pern(*args).clone()
+    assert torch.equal(out, torch.ops.mi355x_checked.esimd_gemv_fp8_pern(*args))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 3, 12, 13])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_moe_decode_is_the_same(dev, T, dt):
+    """Both sides of the largest batch with one GEMV per route (96 pairs)."""
+    torch.manual_seed(T)
+    E, k, H, I = 16, 8, 256, 128
+    f8 = lambda *s: (torch.randn(*s, device=dev) * 4).to(torch.float8_e4m3fn)
+    sc = lambda *s: torch.rand(*s, device=dev) * 0.01
+    x, logits = torch.randn(T, H, device=dev).to(dt), torch.randn(T, E, device=dev).to(dt)
+    w = [f8(E, 2 * I, H), sc(E, 2 * I // 128, H // 128), f8(2 * I, H), sc(2 * I // 128, H // 128), f8(E, H, I),
+         sc(E, H // 128, I // 128), f8(H, I), sc(H // 128, I // 128), torch.randn(1, H, device=dev).to(dt)]
+    outs = [torch.empty_like(x) for _ in range(2)]
+    for op, o in zip((torch.ops.moe_ops, torch.ops.mi355x_checked), outs):
+        assert op.moe_forward_full_fp8_block(x, logits, o, *w, k, 1, E) is o
+    assert torch.equal(outs[0], outs[1])
