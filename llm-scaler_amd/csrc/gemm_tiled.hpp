@@ -85,6 +85,19 @@ __device__ __forceinline__ void mfma_agpr(f32x4& acc, u32x4 a, u32x4 b) {
 constexpr int kBK = 64;
 constexpr int kPitch = kBK + 8;                      // elements per LDS row (144 bytes)
 
+// Exact integers as fp16 pairs, one instruction per pair.  Nibbles in bytes: a byte 0..15 read as an E4M3 code is
+// n * 2^-9 (the subnormals and the first binade, same spacing).  Bytes: 0x6400 | u is 1024 + u.
+__device__ __forceinline__ f16x2 nibbles_f16(uint32_t bytes, bool high) {
+  return __builtin_bit_cast(f16x2, high ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(bytes, 512.0f, true)
+                                        : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(bytes, 512.0f, false));
+}
+__device__ __forceinline__ f16x2 planted_f16(uint32_t bytes, bool high) {
+  return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, bytes, high ? 0x04030402u : 0x04010400u));
+}
+__device__ __forceinline__ f16x2 both(float v) { return f16x2{(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ f16x2 both_bits(uint32_t v) { return __builtin_bit_cast(f16x2, (v & 0xffffu) * 0x10001u); }
+__device__ __forceinline__ uint32_t bits(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+
 // ------------------------------------------------------------------ INT4 group 128
 // 32 nibbles per 16-byte chunk, two chunks per row and step; fp16 scale and optional zero-point
 // byte per group of 128.  A nibble 0..15 read as an E4M3 code is nib * 2^-9 (codes below 16 are
@@ -92,9 +105,8 @@ constexpr int kPitch = kBK + 8;                      // elements per LDS row (14
 // into floats; fma(nib * 2^-9, 512 s, -z s) in fp32 is exact ((nib - z) * s has at most 16
 // significant bits), then one RNE to the activation type: the same value as rne((nib - z) * s),
 // only the sign of a zero can differ from the subtract-then-multiply form, which no product
-// notices.  (A packed-fp16 formulation — plant the nibble in the mantissa of 1024, v_pk_add_f16,
-// v_pk_mul_f16 — measured 1.5x slower for the whole kernel, with or without v_perm_b32: the
-// packed 16-bit instructions do not hide behind the MFMAs the way the fp32 ones do.)
+// notices.  fp16 activations take the same value from packed fp16: n - z is exact and the product is
+// rounded once; the pairs are (0 2)(1 3)(4 6)(5 7) of a dword's 8 nibbles, and x is re-tiled in that order.
 template <class Act, int BN>
 struct WInt4 {
   static constexpr int CPR = 2;                       // chunks per row and 64-wide step
@@ -103,7 +115,8 @@ struct WInt4 {
   static constexpr int LPC = 3;                       // load instructions per chunk
   static constexpr int kPieces = B_CH * 4 * 8;        // 8 pieces per packed dword of 8 nibbles
   static constexpr bool kOutScale = false;
-  static constexpr bool kPermK = false;
+  static constexpr bool kHalf = Act::dt == DT_F16;
+  static constexpr bool kPermK = kHalf;
   struct Res {
     __amdgpu_buffer_rsrc_t wr, sr, zr;
     bool has_zp;
@@ -116,8 +129,9 @@ struct WInt4 {
   struct Dq {
     uint32_t e, o;
     f32x2 fe, fo;
+    f16x2 te, to, sh[B_CH], nz[B_CH];                 // fp16: scale and -z
     u32x4 outv;
-    float sf[B_CH], nzs[B_CH];                        // 512 * scale and -z * scale (exact)
+    float sf[B_CH], nzs[B_CH];                        // bf16: 512 * scale and -z * scale (exact)
   };
   static __device__ __forceinline__ Res make(const GemmArgs& p, int = 0) {
     Res r;
@@ -150,8 +164,13 @@ struct WInt4 {
     for (int i = 0; i < B_CH; ++i) {
       const _Float16 sc = __builtin_bit_cast(_Float16, (uint16_t)st.s[i]);
       const float z = r.has_zp ? (float)st.z[i] : 8.0f;
-      q.sf[i] = (float)sc * 512.0f;
-      q.nzs[i] = -z * (float)sc;
+      if constexpr (kHalf) {
+        q.sh[i] = f16x2{sc, sc};
+        q.nz[i] = both(-z);
+      } else {
+        q.sf[i] = (float)sc * 512.0f;
+        q.nzs[i] = -z * (float)sc;
+      }
     }
   }
   static __device__ __forceinline__ uint32_t pack2(float a, float b) {
@@ -176,6 +195,13 @@ struct WInt4 {
       q.o = (w >> 4) & 0x0F0F0F0Fu;
     } else if (part == 7) {
       *reinterpret_cast<u32x4*>(dst[i] + dw * 16) = q.outv;
+    } else if constexpr (kHalf) {
+      const f16x2 s = q.sh[i], nz = q.nz[i];
+      if (part == 1 || part == 4) {
+        q.te = nibbles_f16(q.e, part == 4);
+        q.to = nibbles_f16(q.o, part == 4);
+      } else if (part == 2 || part == 5) q.outv[part == 5 ? 2 : 0] = bits((q.te + nz) * s);
+      else q.outv[part == 6 ? 3 : 1] = bits((q.to + nz) * s);
     } else if (part == 1) {
       q.fe = __builtin_amdgcn_cvt_pk_f32_fp8((int)q.e, false);
       q.fo = __builtin_amdgcn_cvt_pk_f32_fp8((int)q.o, false);
@@ -193,10 +219,8 @@ struct WInt4 {
 // ------------------------------------------------------------------ GGUF Q4_K (repacked)
 // The int4 nibble layout with an fp16 scale and an fp16 min per 32 k = per chunk:
 // w = fp16(fp16(nib * scale) - min), the product rounded before the subtraction (two roundings,
-// as the dense dequantization does).  The product is formed in fp32 (exact: 4 x 11 significant
-// bits) and rounded once to fp16, which is the fp16 product; the subtraction is the one packed
-// fp16 instruction left per pair (packed 16-bit arithmetic does not hide behind the MFMAs, see
-// INT4 above).  fp16 activations only.
+// as the dense dequantization does): one conversion, one packed product and one packed difference per
+// pair of weights.  fp16 activations only; pairs and x in the order of INT4's fp16 form.
 template <class Act, int BN>
 struct WQ4K {
   static_assert(Act::dt == DT_F16, "Q4_K runs in fp16");
@@ -204,10 +228,10 @@ struct WQ4K {
   static constexpr double kWeightBytesPerK = 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
   static constexpr int LPC = 3;
-  static constexpr int PPD = 12;                      // pieces per dword of 8 nibbles
+  static constexpr int PPD = 8;                       // pieces per dword of 8 nibbles
   static constexpr int kPieces = B_CH * 4 * PPD;
   static constexpr bool kOutScale = false;
-  static constexpr bool kPermK = false;
+  static constexpr bool kPermK = true;
   struct Res {
     __amdgpu_buffer_rsrc_t wr, sr, mr;
     int Kc;
@@ -217,11 +241,10 @@ struct WQ4K {
     uint32_t s[B_CH], m[B_CH];                        // fp16 bits (32-bit slots: 16-bit members end up on the stack)
   };
   struct Dq {
-    uint32_t e, o, t;
-    f32x2 fe, fo;
+    uint32_t e, o;
+    f16x2 te, to;
     u32x4 outv;
-    float sf[B_CH];                                   // 512 * scale
-    f16x2 mv[B_CH];
+    f16x2 sv[B_CH], mv[B_CH];
   };
   static __device__ __forceinline__ Res make(const GemmArgs& p, int = 0) {
     Res r;
@@ -246,49 +269,35 @@ struct WQ4K {
   static __device__ __forceinline__ void begin(const Res&, const Stage& st, Dq& q) {
 #pragma unroll
     for (int i = 0; i < B_CH; ++i) {
-      const _Float16 mn = __builtin_bit_cast(_Float16, (uint16_t)st.m[i]);
-      q.sf[i] = (float)__builtin_bit_cast(_Float16, (uint16_t)st.s[i]) * 512.0f;   // exact: a power of two
-      q.mv[i] = f16x2{mn, mn};
+      q.sv[i] = both_bits(st.s[i]);
+      q.mv[i] = both_bits(st.m[i]);
     }
   }
   static __device__ __forceinline__ void piece(const Stage& st, Dq& q, int I, unsigned char* const (&dst)[B_CH]) {
 #pragma clang fp contract(off)
     const int dword = I / PPD, part = I % PPD;
     const int i = dword / 4, dw = dword % 4;
-    // nib * 2^-9 times 512 s = nib * s exactly in fp32; one RNE to fp16 = the fp16 product
-    auto prod = [&](float a, float b) {
-      const f16x2 r = {(_Float16)(a * q.sf[i]), (_Float16)(b * q.sf[i])};
-      return __builtin_bit_cast(uint32_t, r);
-    };
-    auto sub_min = [&](uint32_t v) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v) - q.mv[i]); };
     if (part == 0) {
       const uint32_t w = st.b[i][dw];
       q.e = w & 0x0F0F0F0Fu;
       q.o = (w >> 4) & 0x0F0F0F0Fu;
-    } else if (part == 1) {
-      q.fe = __builtin_amdgcn_cvt_pk_f32_fp8((int)q.e, false);
-      q.fo = __builtin_amdgcn_cvt_pk_f32_fp8((int)q.o, false);
-    } else if (part == 6) {
-      q.fe = __builtin_amdgcn_cvt_pk_f32_fp8((int)q.e, true);
-      q.fo = __builtin_amdgcn_cvt_pk_f32_fp8((int)q.o, true);
-    } else if (part == 2 || part == 7) q.t = prod(q.fe[0], q.fo[0]);
-    else if (part == 4 || part == 9) q.t = prod(q.fe[1], q.fo[1]);
-    else if (part == 3) q.outv[0] = sub_min(q.t);
-    else if (part == 5) q.outv[1] = sub_min(q.t);
-    else if (part == 8) q.outv[2] = sub_min(q.t);
-    else if (part == 10) q.outv[3] = sub_min(q.t);
+    } else if (part == 1 || part == 4) {
+      q.te = nibbles_f16(q.e, part == 4);
+      q.to = nibbles_f16(q.o, part == 4);
+    } else if (part == 2 || part == 5) q.outv[part == 5 ? 2 : 0] = bits(q.te * q.sv[i] - q.mv[i]);
+    else if (part == 3 || part == 6) q.outv[part == 6 ? 3 : 1] = bits(q.to * q.sv[i] - q.mv[i]);
     else *reinterpret_cast<u32x4*>(dst[i] + dw * 16) = q.outv;
   }
   static __device__ __forceinline__ float out_scale(const Res&, const GemmArgs&, int) { return 1.0f; }
 };
 
 // ------------------------------------------------------------------ GGUF Q4_0 / Q8_0 / Q5_K / Q6_K (repacked)
-// fp16 activations only.  Q4_0 is the int4 layout with one scale per 32 k and zero-point 8: the
-// E4M3 trick of WInt4.  The others bring a byte per weight into place and take it to fp32 with
-// v_cvt_f32_ubyte (exact):
-//   Q8_0: code + 128 (sign bit flipped); fma(u, s, -128 s) is exact (8 x 11 significant bits);
-//   Q6_K: nibble | 2 high bits << 4;     fma(u, s, -32 s) is exact; two scales per chunk of 32 k;
-//   Q5_K: nibble | high bit << 4;        fp16(fp16(u s) - min), two roundings, as Q4_K;
+// fp16 activations only, packed fp16 arithmetic (an MFMA hides two vector instructions, so their number sets the
+// time).  Q4_0 is the int4 layout with one scale per 32 k and zero-point 8.  The others bring a byte u per weight
+// into place and plant it in 1024 + u:
+//   Q8_0: u = code + 128 (sign bit flipped); w = fp16((1024 + u - 1152) s);
+//   Q6_K: u = nibble | 2 high bits << 4;     w = fp16((1024 + u - 1056) s); two scales per chunk of 32 k;
+//   Q5_K: u = nibble | high bit << 4;        w = fp16(fp16(u s) - min), two roundings, as Q4_K;
 // each with the rounding(s) of the dense dequantization.  The high bits are tile-shuffled: inside
 // 512 k, byte t holds element p * 128 + t in its 2-bit field p (Q6_K), element p * 64 + t in bit p
 // (Q5_K), so the 32 weights of a chunk take one field of 32 consecutive bytes, the same field for
@@ -302,10 +311,10 @@ struct WGguf {
   static constexpr double kWeightBytesPerK = F == GT_Q80 ? 1.0 : F == GT_Q6K ? 0.75 : F == GT_Q5K ? 0.625 : 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
   static constexpr int LPC = F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2;
-  static constexpr int PPD = F == GT_Q5K ? 17 : F == GT_Q6K ? 13 : F == GT_Q40 ? 8 : 5;   // pieces per dword (8 nibbles / 4 bytes)
+  static constexpr int PPD = F == GT_Q5K ? 13 : F == GT_Q6K ? 9 : F == GT_Q40 ? 8 : 3;   // pieces per dword (8 nibbles / 4 bytes)
   static constexpr int kPieces = B_CH * 4 * PPD;
   static constexpr bool kOutScale = false;
-  static constexpr bool kPermK = false;
+  static constexpr bool kPermK = F != GT_Q80;            // pairs (0 2)(1 3)(4 6)(5 7); Q8_0 in order
   struct Res {
     __amdgpu_buffer_rsrc_t wr, sr, mr, hr;
     int Ks;                                           // bytes of scales per row
@@ -320,11 +329,9 @@ struct WGguf {
   };
   struct Dq {
     uint32_t e, o, h0, h1;
-    float a, b;
-    f32x2 fe, fo;
+    f16x2 te, to;
     u32x4 outv;
-    float sf[B_CH][F == GT_Q6K ? 2 : 1], nz[B_CH][F == GT_Q6K ? 2 : 1];
-    f16x2 mv[F == GT_Q5K ? B_CH : 1];
+    f16x2 sv[B_CH][F == GT_Q6K ? 2 : 1], mv[F == GT_Q5K ? B_CH : 1];
   };
   static __device__ __forceinline__ Res make(const GemmArgs& p, int = 0) {
     Res r;
@@ -360,52 +367,36 @@ struct WGguf {
   static __device__ __forceinline__ void begin(const Res&, const Stage& st, Dq& q) {
 #pragma unroll
     for (int i = 0; i < B_CH; ++i) {
-#pragma unroll
-      for (int t = 0; t < (F == GT_Q6K ? 2 : 1); ++t) {
-        const float s = (float)__builtin_bit_cast(_Float16, (uint16_t)(st.s[i] >> 16 * t));
-        q.sf[i][t] = F == GT_Q40 ? s * 512.0f : s;            // exact: a power of two
-        q.nz[i][t] = s * (F == GT_Q80 ? -128.0f : F == GT_Q6K ? -32.0f : -8.0f);
-      }
-      if constexpr (F == GT_Q5K) {
-        const _Float16 mn = __builtin_bit_cast(_Float16, (uint16_t)st.m[i]);
-        q.mv[i] = f16x2{mn, mn};
-      }
+      q.sv[i][0] = both_bits(st.s[i]);
+      if constexpr (F == GT_Q6K) q.sv[i][1] = both_bits(st.s[i] >> 16);
+      if constexpr (F == GT_Q5K) q.mv[i] = both_bits(st.m[i]);
     }
   }
-  static __device__ __forceinline__ uint32_t pack2(float a, float b) {
-    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)a, (_Float16)b});
-  }
-  static __device__ __forceinline__ float byte_f(uint32_t v, int i) { return (float)(v >> 8 * i & 0xffu); }   // v_cvt_f32_ubyte
   static __device__ __forceinline__ void piece(const Stage& st, Dq& q, int I, unsigned char* const (&dst)[B_CH]) {
 #pragma clang fp contract(off)
     const int dword = I / PPD, part = I % PPD;
     const int i = dword / 4, dw = dword % 4;
     const uint32_t w = st.b[i][dw];
     if constexpr (F == GT_Q40) {
-      auto pair = [&](float a, float b) {
-        return pack2(__builtin_fmaf(a, q.sf[i][0], q.nz[i][0]), __builtin_fmaf(b, q.sf[i][0], q.nz[i][0]));
-      };
+      const f16x2 s = q.sv[i][0], m8 = both(-8.0f);
       if (part == 0) {
         q.e = w & 0x0F0F0F0Fu;
         q.o = (w >> 4) & 0x0F0F0F0Fu;
       } else if (part == 1 || part == 4) {
-        q.fe = part == 1 ? __builtin_amdgcn_cvt_pk_f32_fp8((int)q.e, false) : __builtin_amdgcn_cvt_pk_f32_fp8((int)q.e, true);
-        q.fo = part == 1 ? __builtin_amdgcn_cvt_pk_f32_fp8((int)q.o, false) : __builtin_amdgcn_cvt_pk_f32_fp8((int)q.o, true);
+        q.te = nibbles_f16(q.e, part == 4);
+        q.to = nibbles_f16(q.o, part == 4);
       } else if (part == 7) *reinterpret_cast<u32x4*>(dst[i] + dw * 16) = q.outv;
-      else q.outv[part < 4 ? part - 2 : part - 3] = part == 2 || part == 5 ? pair(q.fe[0], q.fo[0]) : pair(q.fe[1], q.fo[1]);
+      else if (part == 2 || part == 5) q.outv[part == 5 ? 2 : 0] = bits((q.te + m8) * s);
+      else q.outv[part == 6 ? 3 : 1] = bits((q.to + m8) * s);
     } else if constexpr (F == GT_Q80) {
       // one dword = 4 weights = half of a 16-byte LDS write
       if (part == 0) q.e = w ^ 0x80808080u;
-      else if (part == 1 || part == 3) {
-        q.a = byte_f(q.e, part - 1);
-        q.b = byte_f(q.e, part);
-      } else {
-        q.outv[(dw & 1) * 2 + (part == 4)] = pack2(__builtin_fmaf(q.a, q.sf[i][0], q.nz[i][0]), __builtin_fmaf(q.b, q.sf[i][0], q.nz[i][0]));
-        if (part == 4 && (dw & 1)) *reinterpret_cast<u32x4*>(dst[i] + (dw >> 1) * 16) = q.outv;
+      else {
+        q.outv[(dw & 1) * 2 + part - 1] = bits((planted_f16(q.e, part == 2) + both(-1152.0f)) * q.sv[i][0]);
+        if (part == 2 && (dw & 1)) *reinterpret_cast<u32x4*>(dst[i] + (dw >> 1) * 16) = q.outv;
       }
     } else {
       constexpr uint32_t kField = F == GT_Q6K ? 0x03030303u : 0x01010101u;
-      constexpr int kPair = F == GT_Q6K ? 2 : 3;              // pieces per pair of weights
       if (part == 0) {
         q.e = w & 0x0F0F0F0Fu;
         q.o = (w >> 4) & 0x0F0F0F0Fu;
@@ -421,15 +412,11 @@ struct WGguf {
         q.o |= q.h1 << 4;
       } else if (part == PPD - 1) *reinterpret_cast<u32x4*>(dst[i] + dw * 16) = q.outv;
       else {
-        const int pr = (part - 4) / kPair, sub = (part - 4) % kPair;
-        if (sub == 0) {
-          q.a = byte_f(q.e, pr);
-          q.b = byte_f(q.o, pr);
-        } else if constexpr (F == GT_Q6K) {
-          const int t = dw >> 1;                               // 16-wide group of the chunk
-          q.outv[pr] = pack2(__builtin_fmaf(q.a, q.sf[i][t], q.nz[i][t]), __builtin_fmaf(q.b, q.sf[i][t], q.nz[i][t]));
-        } else if (sub == 1) q.h0 = pack2(q.a * q.sf[i][0], q.b * q.sf[i][0]);
-        else q.outv[pr] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, q.h0) - q.mv[i]);
+        const int pr = F == GT_Q6K ? part - 4 : (part - 4) >> 1;       // outv[pr]: pairs of e, o, e, o
+        const bool first = F == GT_Q6K || (part & 1) == 0;
+        if (first) q.te = planted_f16(pr & 1 ? q.o : q.e, pr >> 1) + both(F == GT_Q6K ? -1056.0f : -1024.0f);
+        if constexpr (F == GT_Q6K) q.outv[pr] = bits(q.te * q.sv[i][dw >> 1]);   // dw >> 1: 16-wide group of the chunk
+        else if (!first) q.outv[pr] = bits(q.te * q.sv[i][0] - q.mv[i]);
       }
     }
   }
@@ -935,7 +922,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
 // zero.  One workgroup writes four blocks, contiguously.  (Reading the rows contiguously and
 // turning them through an LDS tile, as the grouped variant does, was measured slower here:
 // 9.1 against 7.3 us for 2048 x 4096.)
-// perm_k: the 8 elements of a lane leave in the order 0 4 1 5 2 6 3 7 (weight formats whose
+// perm_k: the 8 elements of a lane leave in the order 0 2 1 3 4 6 5 7 (weight formats whose
 // dequantization produces that order).
 constexpr int kPackQ = 16;                            // grouped variant: 32-wide steps per workgroup
 constexpr int kPackPitch = kPackQ * 64 + 16;          // and its LDS row pitch (operand reads hit distinct banks)
@@ -950,10 +937,10 @@ static __global__ __launch_bounds__(256) void pack_x_kernel(const uint16_t* __re
   u32x4 v = {0u, 0u, 0u, 0u};
   if (m < M) v = *reinterpret_cast<const u32x4*>(x + (size_t)m * K + q * 32 + (l >> 4) * 8);
   if (perm_k) {
-    // dwords hold (x0 x1)(x2 x3)(x4 x5)(x6 x7) -> (x0 x4)(x1 x5)(x2 x6)(x3 x7)
+    // dwords hold (x0 x1)(x2 x3)(x4 x5)(x6 x7) -> (x0 x2)(x1 x3)(x4 x6)(x5 x7)
     const uint32_t d0 = v[0], d1 = v[1], d2 = v[2], d3 = v[3];
-    v = u32x4{__builtin_amdgcn_perm(d2, d0, 0x05040100u), __builtin_amdgcn_perm(d2, d0, 0x07060302u),
-              __builtin_amdgcn_perm(d3, d1, 0x05040100u), __builtin_amdgcn_perm(d3, d1, 0x07060302u)};
+    v = u32x4{__builtin_amdgcn_perm(d1, d0, 0x05040100u), __builtin_amdgcn_perm(d1, d0, 0x07060302u),
+              __builtin_amdgcn_perm(d3, d2, 0x05040100u), __builtin_amdgcn_perm(d3, d2, 0x07060302u)};
   }
   xp[((size_t)t * Q + q) * 64 + l] = v;
 }
