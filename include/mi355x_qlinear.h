@@ -222,6 +222,15 @@ int mi_moe_gguf_grouped(int fmt, const void* x, int x_rows, const int32_t* tok_i
                         const void* const* qh, const void* const* scale, const void* const* qmin, void* out,
                         long long out_stride, int out_rows, const int32_t* chunks, int num_chunks, int num_experts,
                         int N, int K, int rows16, void* stream);
+/* The same for prompts, through the tiled matrix-core GEMM: chunks of one expert that follow each other without a
+ * gap are merged into tiles of 256 rows, the rows of x are gathered and re-tiled once.  The operands and results of
+ * mi_moe_gguf_grouped with rows16 = 0; K % 128 == 0, x and the stacks 16-byte aligned, two matrices for fmt 2 only,
+ * num_chunks x 64 x K x 2 below 2 GiB.  workspace: mi_moe_gguf_grouped_tiled_workspace bytes. */
+int mi_moe_gguf_grouped_tiled_workspace(int num_chunks, int K, long long* bytes);
+int mi_moe_gguf_grouped_tiled_ws(int fmt, const void* x, int x_rows, const int32_t* tok_ids, int nmat, const void* const* ql,
+                                 const void* const* qh, const void* const* scale, const void* const* qmin, void* out,
+                                 long long out_stride, int out_rows, const int32_t* chunks, int num_chunks, int num_experts,
+                                 int N, int K, void* workspace, long long workspace_bytes, void* stream);
 int mi_q4_0_repack(const void* raw, void* packed, void* scale, int N, int K, void* stream);
 int mi_q8_0_repack(const void* raw, void* qs, void* scale, int N, int K, void* stream);
 int mi_q5k_repack(const void* raw, void* ql, void* qh, void* scale, void* qmin, int N, int K,

@@ -57,6 +57,9 @@ struct GemmArgs {
   const int32_t* g_tile;
   const int32_t* g_count;
   long long g_w_stride, g_s_stride;
+  long long g_z_stride, g_h_stride;   // GGUF stacks: mins, high bits
+  const void *w1, *scale1, *zp1;      // a second stack of matrices (w1 set): N-tiles from tiles_n / 2 on take it, output columns N ..
+  int out_ld;                 // GROUPED: columns of a row of out (0: the output columns)
   const int32_t* out_map;
   const void* row_weight;
   int x_blocks;               // 16-row blocks in the re-tiled activations
@@ -246,12 +249,12 @@ struct WQ4K {
     u32x4 outv;
     f16x2 sv[B_CH], mv[B_CH];
   };
-  static __device__ __forceinline__ Res make(const GemmArgs& p, int = 0) {
+  static __device__ __forceinline__ Res make(const GemmArgs& p, int e = 0) {
     Res r;
     r.Kc = p.K >> 5;
-    r.wr = make_rsrc(p.w, (uint32_t)p.N * ((uint32_t)p.K >> 1));
-    r.sr = make_rsrc(p.scale, (uint32_t)p.N * (uint32_t)r.Kc * 2u);
-    r.mr = make_rsrc(p.zp, (uint32_t)p.N * (uint32_t)r.Kc * 2u);
+    r.wr = make_rsrc((const char*)p.w + (long long)e * p.g_w_stride, (uint32_t)p.N * ((uint32_t)p.K >> 1));
+    r.sr = make_rsrc((const char*)p.scale + (long long)e * p.g_s_stride, (uint32_t)p.N * (uint32_t)r.Kc * 2u);
+    r.mr = make_rsrc((const char*)p.zp + (long long)e * p.g_z_stride, (uint32_t)p.N * (uint32_t)r.Kc * 2u);
     return r;
   }
   static __device__ __forceinline__ void chunk_addr(Res& r, int, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
@@ -302,15 +305,19 @@ struct WQ4K {
 // 512 k, byte t holds element p * 128 + t in its 2-bit field p (Q6_K), element p * 64 + t in bit p
 // (Q5_K), so the 32 weights of a chunk take one field of 32 consecutive bytes, the same field for
 // the whole 64-wide step; the bytes come through L1 again for the other fields.
-enum { GT_Q40 = 3, GT_Q80 = 4, GT_Q5K = 5, GT_Q6K = 6 };    // the format numbers of gemv_rows.hpp
-template <class Act, int BN, int F>
+// GT_Q5P / GT_Q6P: the high bits in element order (the MoE down stacks): a dword's 8 weights take one / two
+// consecutive bytes, spread to one field per byte with shifts and masks.
+enum { GT_Q40 = 3, GT_Q80 = 4, GT_Q5K = 5, GT_Q6K = 6, GT_Q5P = 7, GT_Q6P = 8 };    // the format numbers of gemv_rows.hpp, skinny_kernel.hpp
+template <class Act, int BN, int FMT>
 struct WGguf {
+  static constexpr int F = FMT == GT_Q5P ? GT_Q5K : FMT == GT_Q6P ? GT_Q6K : FMT;
+  static constexpr bool kPlainH = FMT == GT_Q5P || FMT == GT_Q6P;
   static_assert(Act::dt == DT_F16, "GGUF formats run in fp16");
   static constexpr bool kHigh = F == GT_Q5K || F == GT_Q6K;
   static constexpr int CPR = F == GT_Q80 ? 4 : 2;
   static constexpr double kWeightBytesPerK = F == GT_Q80 ? 1.0 : F == GT_Q6K ? 0.75 : F == GT_Q5K ? 0.625 : 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
-  static constexpr int LPC = F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2;
+  static constexpr int LPC = (F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2) - (kPlainH ? 1 : 0);
   static constexpr int PPD = F == GT_Q5K ? 13 : F == GT_Q6K ? 9 : F == GT_Q40 ? 8 : 3;   // pieces per dword (8 nibbles / 4 bytes)
   static constexpr int kPieces = B_CH * 4 * PPD;
   static constexpr bool kOutScale = false;
@@ -324,7 +331,8 @@ struct WGguf {
     u32x4 b[B_CH];
     uint32_t s[B_CH];
     uint32_t m[F == GT_Q5K ? B_CH : 1];
-    u32x4 h[kHigh ? B_CH : 1][2];
+    u32x4 h[kHigh && !kPlainH ? B_CH : 1][2];
+    u32x2 hp[kPlainH ? B_CH : 1];
     uint32_t sh;                                      // shift of this step's field of the high-bit bytes (uniform)
   };
   struct Dq {
@@ -333,20 +341,21 @@ struct WGguf {
     u32x4 outv;
     f16x2 sv[B_CH][F == GT_Q6K ? 2 : 1], mv[F == GT_Q5K ? B_CH : 1];
   };
-  static __device__ __forceinline__ Res make(const GemmArgs& p, int = 0) {
+  static __device__ __forceinline__ Res make(const GemmArgs& p, int e = 0) {
     Res r;
     const uint32_t nk = (uint32_t)p.N * (uint32_t)p.K;      // < 2^31 (checked by the host)
     r.Ks = (F == GT_Q6K ? p.K >> 4 : p.K >> 5) * 2;
-    r.wr = make_rsrc(p.w, F == GT_Q80 ? nk : nk / 2);
-    r.sr = make_rsrc(p.scale, (uint32_t)p.N * (uint32_t)r.Ks);
-    r.mr = make_rsrc(p.zp, F == GT_Q5K ? (uint32_t)p.N * (uint32_t)r.Ks : 0u);
-    r.hr = make_rsrc(p.qh, F == GT_Q6K ? nk / 4 : F == GT_Q5K ? nk / 8 : 0u);
+    r.wr = make_rsrc((const char*)p.w + (long long)e * p.g_w_stride, F == GT_Q80 ? nk : nk / 2);
+    r.sr = make_rsrc((const char*)p.scale + (long long)e * p.g_s_stride, (uint32_t)p.N * (uint32_t)r.Ks);
+    r.mr = make_rsrc((const char*)p.zp + (long long)e * p.g_z_stride, F == GT_Q5K ? (uint32_t)p.N * (uint32_t)r.Ks : 0u);
+    r.hr = make_rsrc((const char*)p.qh + (long long)e * p.g_h_stride, F == GT_Q6K ? nk / 4 : F == GT_Q5K ? nk / 8 : 0u);
     return r;
   }
   static __device__ __forceinline__ void chunk_addr(Res& r, int i, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
     boff = (uint32_t)n * (F == GT_Q80 ? (uint32_t)K : (uint32_t)K >> 1) + (uint32_t)(kc * 16);
     soff = (uint32_t)n * (uint32_t)r.Ks + (uint32_t)(F == GT_Q80 ? (kc >> 1) * 2 : F == GT_Q6K ? kc * 4 : kc * 2);
-    if constexpr (kHigh) r.hoff[i] = (uint32_t)n * (F == GT_Q6K ? (uint32_t)K >> 2 : (uint32_t)K >> 3) + (uint32_t)(kc * 32);
+    if constexpr (kHigh) r.hoff[i] = (uint32_t)n * (F == GT_Q6K ? (uint32_t)K >> 2 : (uint32_t)K >> 3) +
+                                     (uint32_t)(kc * (!kPlainH ? 32 : F == GT_Q6K ? 8 : 4));
   }
   static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
                                                const uint32_t (&soff)[B_CH], int kt, uint32_t dead, int idx) {
@@ -356,9 +365,12 @@ struct WGguf {
     else if (kind == 1) {
       if constexpr (F == GT_Q6K) st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, k0 >> 3, 0);
       else st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, k0 >> 4, 0);
-    } else if (kind == 4) {
+    } else if (kPlainH && kind == 2) {
+      if constexpr (kPlainH && F == GT_Q6K) st.hp[i] = __builtin_amdgcn_raw_buffer_load_b64(r.hr, r.hoff[i] | dead, k0 >> 2, 0);
+      else if constexpr (kPlainH) st.hp[i][0] = __builtin_amdgcn_raw_buffer_load_b32(r.hr, r.hoff[i] | dead, k0 >> 3, 0);
+    } else if (kind == LPC - 1 && F == GT_Q5K) {
       if constexpr (F == GT_Q5K) st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, k0 >> 4, 0);
-    } else if constexpr (kHigh) {
+    } else if constexpr (kHigh && !kPlainH) {
       const uint32_t tile = F == GT_Q6K ? (k0 >> 9) * 128u + (k0 & 127u) : (k0 >> 9) * 64u;
       st.h[i][kind - 2] = __builtin_amdgcn_raw_buffer_load_b128(r.hr, r.hoff[i] | dead, tile + (uint32_t)(kind - 2) * 16u, 0);
       st.sh = F == GT_Q6K ? (k0 >> 7 & 3u) * 2u : k0 >> 6 & 7u;
@@ -400,9 +412,25 @@ struct WGguf {
       if (part == 0) {
         q.e = w & 0x0F0F0F0Fu;
         q.o = (w >> 4) & 0x0F0F0F0Fu;
-      } else if (part == 1) {
+      } else if (kPlainH && part == 1) {
+        if constexpr (kPlainH && F == GT_Q6K) {
+          const uint32_t v = st.hp[i][dw >> 1] >> (16 * (dw & 1)) & 0xffffu;    // field t: element t
+          q.h0 = (v | v << 8) & 0x00FF00FFu;
+        } else if constexpr (kPlainH) {
+          const uint32_t v = st.hp[i][0] >> (8 * dw) & 0xffu;                   // bit t: element t
+          q.h0 = (v | v << 12) & 0x000F000Fu;
+        }
+      } else if (kPlainH && part == 2) {
+        q.h0 = F == GT_Q6K ? (q.h0 | q.h0 << 4) & 0x0F0F0F0Fu : (q.h0 | q.h0 << 6) & 0x03030303u;   // byte m: elements 2 m, 2 m + 1
+        q.h1 = F == GT_Q6K ? (q.h0 & 0x0C0C0C0Cu) << 2 : (q.h0 & 0x02020202u) << 3;
+      } else if (kPlainH && part == 3) {
+        q.e |= (q.h0 & kField) << 4;
+        q.o |= q.h1;
+      } else if (!kPlainH && part == 1) {
+        if constexpr (!kPlainH) {
         q.h0 = st.h[i][dw >> 1][(dw & 1) * 2] >> st.sh & kField;         // elements 0 1 2 3 of the dword's 8
         q.h1 = st.h[i][dw >> 1][(dw & 1) * 2 + 1] >> st.sh & kField;     // elements 4 5 6 7
+        }
       } else if (part == 2) {
         const uint32_t he = __builtin_amdgcn_perm(q.h1, q.h0, 0x06040200u);
         q.h1 = __builtin_amdgcn_perm(q.h1, q.h0, 0x07050301u);
@@ -576,7 +604,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
     tm = blockIdx.x - tn * p.tiles_m;
   }
   int m0 = tm * BM;
-  const int n0 = FUSE ? tn * (BN / 2) : tn * BN;      // FUSE: first gate row of the tile
+  const int n0 = FUSE ? tn * (BN / 2) : (GROUPED && p.w1 && tn >= p.tiles_n >> 1 ? tn - (p.tiles_n >> 1) : tn) * BN;   // FUSE: first gate row
   int M = p.M;
   const int N = p.N, K = p.K;
   const int Q = K / 32;                               // 32-wide MFMA steps
@@ -599,7 +627,17 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   const int Mp = (p.M + 15) & ~15;
   const uint32_t xtiles = GROUPED ? (uint32_t)p.x_blocks : (uint32_t)(Mp >> 4);
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(p.x, xtiles * 16u * (uint32_t)K * 2u);
-  typename Fmt::Res res = Fmt::make(p, expert);
+  int col0 = 0;                                       // first output column of this workgroup's matrix
+  const void *mw = p.w, *ms = p.scale, *mz = p.zp;
+  if constexpr (GROUPED && !FUSE) {
+    if (p.w1 && tn >= p.tiles_n >> 1) {
+      mw = p.w1; ms = p.scale1; mz = p.zp1;
+      col0 = N;
+    }
+  }
+  GemmArgs mat = p;
+  mat.w = mw; mat.scale = ms; mat.zp = mz;
+  typename Fmt::Res res = Fmt::make(mat, expert);
   // 16-row activation tile b of this wavefront inside the BM-row tile.  GROUPED: the two wavefront
   // rows take the tiles alternately and a wavefront multiplies only the first TM, TM / 2 or TM / 4 of
   // its tiles, whichever covers the `live` ones with rows of the expert in them (the K loop exists
@@ -771,6 +809,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   }
   Elem* out = (Elem*)p.out;
   const int n_out = FUSE ? p.n_half : N;              // output columns
+  const int ld = GROUPED && p.out_ld ? p.out_ld : n_out;
   // output row of this lane's row of activation tile b, or -1
   int orow[TM];
   float rw[TM];
@@ -824,14 +863,14 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
       if constexpr (GROUPED) r[v] *= rw[b];
     }
   };
-  const size_t out_bytes = (size_t)(GROUPED ? p.out_rows : p.M) * (size_t)n_out * 2u;
+  const size_t out_bytes = (size_t)(GROUPED ? p.out_rows : p.M) * (size_t)ld * 2u;
   constexpr int WNO = FUSE ? WN / 2 : WN;             // output columns of this wavefront
   constexpr int LPR = WNO / 8;                        // lanes, 16 bytes each, per output row of the wave tile
   constexpr int RPP = 64 / LPR;                       // rows per store instruction
   constexpr int PASSES = (16 + RPP - 1) / RPP;
   constexpr int OPITCH = WNO * 2 + 16;                // a row of the wave tile + a slot for the row's offset
   static_assert(WNO % 8 == 0 && 4 * 16 * OPITCH <= 2 * BNP * kPitch * 2, "output staging tile");
-  if ((n_out & 7) == 0 && out_bytes < (1ull << 31) && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0) {
+  if (((n_out | ld) & 7) == 0 && out_bytes < (1ull << 31) && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0) {
     // Each 16-row tile of results is rounded, turned through a tile in LDS that belongs to this
     // wavefront alone (the weight tiles are free after the K loop's last barrier; the LDS queue of a
     // wavefront runs in order, so no barrier) and leaves as 16 bytes per lane, a row's columns in
@@ -849,7 +888,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
       for (int b = 0; b < TM; ++b) {
         if (GROUPED && b >= live) break;              // uniform: the tiles past the expert's rows
         *reinterpret_cast<uint32_t*>(otile + j * OPITCH + WNO * 2) =
-            orow[b] >= 0 ? (uint32_t)orow[b] * (uint32_t)n_out * 2u : kOOB;
+            orow[b] >= 0 ? (uint32_t)orow[b] * (uint32_t)ld * 2u : kOOB;
 #pragma unroll
         for (int ao = 0; ao < TNO; ++ao) {
           float r[4];
@@ -888,7 +927,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
           const u32x4 v = *reinterpret_cast<const u32x4*>(src + cc * 16);
           const uint32_t ro = *reinterpret_cast<const uint32_t*>(src + WNO * 2);
           const bool ok = lane_ok && row < 16;
-          __builtin_amdgcn_raw_buffer_store_b128(v, orsrc, ok ? ro + (uint32_t)colr * 2u : kOOB, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b128(v, orsrc, ok ? ro + (uint32_t)(colr + col0) * 2u : kOOB, 0, 0);
         }
       }
     };
@@ -904,7 +943,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
           const int n = col_of(ao);
           float r[4];
           result4(gelu_c, b, ao, r);
-          Elem* dst = out + (size_t)orow[b] * n_out + n;
+          Elem* dst = out + (size_t)orow[b] * ld + col0 + n;
 #pragma unroll
           for (int v = 0; v < 4; ++v)
             if (n + v < n_out) dst[v] = Act::from_f32(r[v]);
@@ -926,6 +965,11 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
 // dequantization produces that order).
 constexpr int kPackQ = 16;                            // grouped variant: 32-wide steps per workgroup
 constexpr int kPackPitch = kPackQ * 64 + 16;          // and its LDS row pitch (operand reads hit distinct banks)
+// dwords (x0 x1)(x2 x3)(x4 x5)(x6 x7) -> (x0 x2)(x1 x3)(x4 x6)(x5 x7)
+__device__ __forceinline__ u32x4 perm_k8(u32x4 v) {
+  return u32x4{__builtin_amdgcn_perm(v[1], v[0], 0x05040100u), __builtin_amdgcn_perm(v[1], v[0], 0x07060302u),
+               __builtin_amdgcn_perm(v[3], v[2], 0x05040100u), __builtin_amdgcn_perm(v[3], v[2], 0x07060302u)};
+}
 static __global__ __launch_bounds__(256) void pack_x_kernel(const uint16_t* __restrict__ x, u32x4* __restrict__ xp,
                                                             int M, int K, int Q, int perm_k) {
   const int l = threadIdx.x & 63;
@@ -936,13 +980,60 @@ static __global__ __launch_bounds__(256) void pack_x_kernel(const uint16_t* __re
   const int m = t * 16 + (l & 15);
   u32x4 v = {0u, 0u, 0u, 0u};
   if (m < M) v = *reinterpret_cast<const u32x4*>(x + (size_t)m * K + q * 32 + (l >> 4) * 8);
-  if (perm_k) {
-    // dwords hold (x0 x1)(x2 x3)(x4 x5)(x6 x7) -> (x0 x2)(x1 x3)(x4 x6)(x5 x7)
-    const uint32_t d0 = v[0], d1 = v[1], d2 = v[2], d3 = v[3];
-    v = u32x4{__builtin_amdgcn_perm(d1, d0, 0x05040100u), __builtin_amdgcn_perm(d1, d0, 0x07060302u),
-              __builtin_amdgcn_perm(d3, d2, 0x05040100u), __builtin_amdgcn_perm(d3, d2, 0x07060302u)};
-  }
+  if (perm_k) v = perm_k8(v);
   xp[((size_t)t * Q + q) * 64 + l] = v;
+}
+
+// Gather + re-tile: block b of the table -> MFMA operand order (see pack_x_kernel); rows past the
+// block's count are zero.  One workgroup re-tiles 16 consecutive 32-wide steps of one block: each
+// wavefront reads 1 KiB of each of four (gathered) rows, the rows meet in an LDS tile and leave
+// as 16 contiguous blocks.
+template <bool PERM = false>
+__global__ __launch_bounds__(256) void pack_x_grouped_kernel(const uint16_t* __restrict__ x,
+                                                             const int32_t* __restrict__ row_map,
+                                                             const int32_t* __restrict__ blk,
+                                                             const int32_t* __restrict__ counts,
+                                                             u32x4* __restrict__ xp, int a_rows, int K, int Q,
+                                                             int row_div) {
+  __shared__ __attribute__((aligned(16))) unsigned char tile[16 * kPackPitch];
+  const int nq = (Q + kPackQ - 1) / kPackQ;           // flat grid: kPackQ steps of one block per workgroup
+  const int b = blockIdx.x / nq;
+  if (b >= counts[1]) return;
+  const int l = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int q0 = (blockIdx.x - b * nq) * kPackQ;
+  const int live = blk[2 * b + 1], first = blk[2 * b];
+  // Unconditional loads with indices held in range, the surplus zeroed afterwards: a branch around
+  // each (map entry, row piece) pair would make the four pairs eight dependent round trips.
+  u32x4 v[4];
+  unsigned row[4];
+  const int k = q0 * 32 + l * 8;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = wave * 4 + i;
+    const int pos = first + (r < live ? r : 0);
+    row[i] = row_map ? (unsigned)row_map[pos] : (unsigned)pos;
+  }
+  if (row_map && row_div != 1) {                      // after all four entries have been requested
+#pragma unroll
+    for (int i = 0; i < 4; ++i) row[i] /= (unsigned)row_div;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const bool ok = wave * 4 + i < live && k < K && row[i] < (unsigned)a_rows;
+    v[i] = *reinterpret_cast<const u32x4*>(x + (ok ? (size_t)row[i] * K + k : (size_t)0));
+    if (!ok) v[i] = u32x4{0u, 0u, 0u, 0u};
+    if constexpr (PERM) v[i] = perm_k8(v[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(tile + (wave * 4 + i) * kPackPitch + l * 16) = v[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int q = q0 + wave * 4 + i;
+    if (q < Q)
+      xp[((size_t)b * Q + q) * 64 + l] =
+          *reinterpret_cast<const u32x4*>(tile + (l & 15) * kPackPitch + (wave * 4 + i) * 64 + (l >> 4) * 16);
+  }
 }
 
 // Adds the K slices of a SPLIT launch (in slice order), scales, rounds and writes the output.  A wavefront

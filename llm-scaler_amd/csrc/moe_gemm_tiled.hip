@@ -94,56 +94,6 @@ __global__ __launch_bounds__(kMapThreads) void moe_tile_map_kernel(const int32_t
   }
 }
 
-// Gather + re-tile: block b of the table -> MFMA operand order (see pack_x_kernel); rows past the
-// block's count are zero.  One workgroup re-tiles 16 consecutive 32-wide steps of one block: each
-// wavefront reads 1 KiB of each of four (gathered) rows, the rows meet in an LDS tile and leave
-// as 16 contiguous blocks.
-__global__ __launch_bounds__(256) void pack_x_grouped_kernel(const uint16_t* __restrict__ x,
-                                                             const int32_t* __restrict__ row_map,
-                                                             const int32_t* __restrict__ blk,
-                                                             const int32_t* __restrict__ counts,
-                                                             u32x4* __restrict__ xp, int a_rows, int K, int Q,
-                                                             int row_div) {
-  __shared__ __attribute__((aligned(16))) unsigned char tile[16 * kPackPitch];
-  const int nq = (Q + kPackQ - 1) / kPackQ;           // flat grid: kPackQ steps of one block per workgroup
-  const int b = blockIdx.x / nq;
-  if (b >= counts[1]) return;
-  const int l = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int q0 = (blockIdx.x - b * nq) * kPackQ;
-  const int live = blk[2 * b + 1], first = blk[2 * b];
-  // Unconditional loads with indices held in range, the surplus zeroed afterwards: a branch around
-  // each (map entry, row piece) pair would make the four pairs eight dependent round trips.
-  u32x4 v[4];
-  unsigned row[4];
-  const int k = q0 * 32 + l * 8;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = wave * 4 + i;
-    const int pos = first + (r < live ? r : 0);
-    row[i] = row_map ? (unsigned)row_map[pos] : (unsigned)pos;
-  }
-  if (row_map && row_div != 1) {                      // after all four entries have been requested
-#pragma unroll
-    for (int i = 0; i < 4; ++i) row[i] /= (unsigned)row_div;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const bool ok = wave * 4 + i < live && k < K && row[i] < (unsigned)a_rows;
-    v[i] = *reinterpret_cast<const u32x4*>(x + (ok ? (size_t)row[i] * K + k : (size_t)0));
-    if (!ok) v[i] = u32x4{0u, 0u, 0u, 0u};
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(tile + (wave * 4 + i) * kPackPitch + l * 16) = v[i];
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int q = q0 + wave * 4 + i;
-    if (q < Q)
-      xp[((size_t)b * Q + q) * 64 + l] =
-          *reinterpret_cast<const u32x4*>(tile + (l & 15) * kPackPitch + (wave * 4 + i) * 64 + (l >> 4) * 16);
-  }
-}
-
 struct TiledMoeLayout {
   long long x_bytes, tile_off, blk_off, cnt_off, total;
   int max_blocks, max_tiles;
@@ -230,7 +180,7 @@ int mi_moe_gemm_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_
   int32_t* counts = (int32_t*)(ws + L.cnt_off);
   hipLaunchKernelGGL(moe_tile_map_kernel, dim3(1), dim3(kMapThreads), 0, st, expert_start, E, bm, g_tile, blk, counts);
   const int Q = K / 32;
-  hipLaunchKernelGGL(pack_x_grouped_kernel, dim3((unsigned)(((Q + kPackQ - 1) / kPackQ) * L.max_blocks)), dim3(256), 0, st, (const uint16_t*)a,
+  hipLaunchKernelGGL(pack_x_grouped_kernel<false>, dim3((unsigned)(((Q + kPackQ - 1) / kPackQ) * L.max_blocks)), dim3(256), 0, st, (const uint16_t*)a,
                      row_map, blk, counts, (u32x4*)ws, a_rows, K, Q, row_map_div);
   GemmArgs p{};
   p.x = ws; p.w = w; p.scale = w_scale; p.out = out; p.M = total_rows; p.N = N; p.K = K;
@@ -282,7 +232,7 @@ int mi_moe_mlp_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_d
   char* inter = ws + L.total;                          // [blocks][I / 32][1 KiB], operand order
   hipLaunchKernelGGL(moe_tile_map_kernel, dim3(1), dim3(kMapThreads), 0, st, expert_start, E, bm, g_tile, blk, counts);
   const int Q = H / 32;
-  hipLaunchKernelGGL(pack_x_grouped_kernel, dim3((unsigned)(((Q + kPackQ - 1) / kPackQ) * L.max_blocks)), dim3(256), 0, st,
+  hipLaunchKernelGGL(pack_x_grouped_kernel<false>, dim3((unsigned)(((Q + kPackQ - 1) / kPackQ) * L.max_blocks)), dim3(256), 0, st,
                      (const uint16_t*)a, row_map, blk, counts, (u32x4*)ws, a_rows, H, Q, row_map_div);
   GemmArgs p{};
   p.x = ws; p.w = w13; p.scale = w13_scale; p.out = inter; p.M = total_rows; p.N = 2 * I; p.K = H;

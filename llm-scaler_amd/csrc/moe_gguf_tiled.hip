@@ -1,0 +1,186 @@
+// Grouped GGUF MoE GEMMs over chunks (mi_moe_gguf_grouped's operands) for prompts: the chunks of an expert that
+// follow each other are merged into M-tiles and run through the tiled matrix-core GEMM, which dequantizes a weight
+// once per tile; the chunk kernel (moe_gguf_grouped.hip) does it once per 64 rows and wavefront.
+//   1. one workgroup turns the chunk list into a table of M-tiles {expert, first row, rows, first 16-row
+//      activation block} and a table of activation blocks;
+//   2. the rows of x are gathered (token list) and re-tiled into MFMA operand order per block;
+//   3. the GEMM runs one workgroup per (M-tile, N-tile); gate and up are two stacks of one launch.
+#include "gemm_tiled.hpp"
+#include "../../include/mi355x_qlinear.h"
+
+namespace qlin {
+
+// 256 x 256 like the FP8 experts' tiles (a wavefront skips the row tiles past the chunk's last): 2048 tokens, top 8 of
+// 128 experts, H = 2048, I = 768: 404 us for the layer against 445 on 128 x 128 and 510 with the chunk kernel.
+constexpr int kGgufBM = 256, kGgufBN = 256;
+constexpr int kChunkRows = 64;                        // rows of a chunk that count
+constexpr int kChunkMapThreads = 1024;
+
+template <class Act, int BN> using WQ5P = WGguf<Act, BN, GT_Q5P>;
+template <class Act, int BN> using WQ6P = WGguf<Act, BN, GT_Q6P>;
+
+// Chunk i continues chunk i - 1 when that one is full and i goes on behind it with the same expert; a run of
+// continuing chunks is cut into tiles of kGgufBM rows.  Thread t owns `per` consecutive chunks; runs across threads
+// are found with a running maximum of the run starts, the places of tiles and blocks with two exclusive scans.
+__global__ __launch_bounds__(kChunkMapThreads) void chunk_tile_map_kernel(const int32_t* __restrict__ chunks, int n, int E,
+                                                                          int out_rows, int32_t* __restrict__ g_tile,
+                                                                          int32_t* __restrict__ blk, int32_t* __restrict__ counts) {
+  constexpr int kPerTile = kGgufBM / kChunkRows;
+  __shared__ int s_a[kChunkMapThreads / 64], s_b[kChunkMapThreads / 64], s_c[kChunkMapThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int per = (n + kChunkMapThreads - 1) / kChunkMapThreads;
+  const int i0 = tid * per, i1 = min(i0 + per, n);
+  auto rows = [&](int i) {                            // 0: the chunk is skipped
+    const int e = chunks[3 * i], t0 = chunks[3 * i + 1], nt = chunks[3 * i + 2];
+    return nt <= 0 || e < 0 || e >= E || t0 < 0 || t0 >= out_rows ? 0 : min(min(nt, kChunkRows), out_rows - t0);
+  };
+  auto continues = [&](int i) {
+    return i > 0 && rows(i) > 0 && rows(i - 1) == kChunkRows && chunks[3 * i] == chunks[3 * i - 3] &&
+           chunks[3 * i + 1] == chunks[3 * i - 2] + kChunkRows;
+  };
+  // last run start in the own chunks, then the last one before them
+  int last = -1;
+  for (int i = i0; i < i1; ++i)
+    if (!continues(i)) last = i;
+  int m = last;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int o = __shfl_up(m, off);
+    if (lane >= off) m = max(m, o);
+  }
+  if (lane == 63) s_a[w] = m;
+  int before = __shfl_up(m, 1);
+  if (lane == 0) before = -1;
+  __syncthreads();
+  for (int i = 0; i < w; ++i) before = max(before, s_a[i]);
+  // tiles and blocks that start in the own chunks
+  auto tile_rows = [&](int i) {
+    int r = rows(i);
+    for (int k = 1; k < kPerTile && i + k < n && continues(i + k); ++k) r += rows(i + k);
+    return r;
+  };
+  auto starts = [&](int i, int& run) {
+    if (!continues(i)) run = i;
+    return rows(i) > 0 && (i - run) % kPerTile == 0;
+  };
+  int tiles = 0, blocks = 0, run = before;
+  for (int i = i0; i < i1; ++i)
+    if (starts(i, run)) {
+      ++tiles;
+      blocks += (tile_rows(i) + 15) >> 4;
+    }
+  int it = tiles, ib = blocks;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int ot = __shfl_up(it, off), ob = __shfl_up(ib, off);
+    if (lane >= off) { it += ot; ib += ob; }
+  }
+  if (lane == 63) { s_b[w] = it; s_c[w] = ib; }
+  __syncthreads();
+  int at = it - tiles, ab = ib - blocks, all_t = 0, all_b = 0;
+  for (int i = 0; i < kChunkMapThreads / 64; ++i) {
+    if (i < w) { at += s_b[i]; ab += s_c[i]; }
+    all_t += s_b[i]; all_b += s_c[i];
+  }
+  run = before;
+  for (int i = i0; i < i1; ++i)
+    if (starts(i, run)) {
+      const int r = tile_rows(i), t0 = chunks[3 * i + 1];
+      int32_t* t = g_tile + 4 * at;
+      t[0] = chunks[3 * i]; t[1] = t0; t[2] = r; t[3] = ab;
+      ++at;
+      for (int b = 0; b * 16 < r; ++b, ++ab) {
+        blk[2 * ab] = t0 + 16 * b;
+        blk[2 * ab + 1] = min(16, r - 16 * b);
+      }
+    }
+  if (tid == 0) { counts[0] = all_t; counts[1] = all_b; }
+}
+
+// {re-tiled x, tile table, block table, counts}: at most one tile per chunk, four blocks per chunk
+struct ChunkLayout { long long tile_off, blk_off, cnt_off, total; };
+static inline ChunkLayout chunk_layout(long long n, long long K) {
+  ChunkLayout L;
+  L.tile_off = (n * kChunkRows * K * 2 + 255) & ~255LL;
+  L.blk_off = L.tile_off + ((n * 16 + 255) & ~255LL);
+  L.cnt_off = L.blk_off + ((n * (kChunkRows / 16) * 8 + 255) & ~255LL);
+  L.total = L.cnt_off + 256;
+  return L;
+}
+
+template <template <class, int> class FMT>
+static int launch_chunk_gemm(GemmArgs p, int nmat, int max_tiles, hipStream_t st) {
+  using F = FMT<ActF16, kGgufBN>;
+  p.tiles_m = (max_tiles + 7) / 8 * 8;                // whole rounds of the 8 XCDs (surplus workgroups exit)
+  p.tiles_n = nmat * ((p.N + kGgufBN - 1) / kGgufBN);
+  if ((long long)p.tiles_m * p.tiles_n >= (1LL << 31)) return MI_ERR_SHAPE;
+  auto kern = gemm_tiled_kernel<ActF16, F, kGgufBM, kGgufBN, true, false>;
+  constexpr size_t lds = (size_t)2 * (F::B_CH * 256 / F::CPR) * kPitch * 2;
+  if (lds > 64 * 1024) {
+    static const int raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess ? MI_OK : MI_ERR_LAUNCH;
+    if (raised != MI_OK) return raised;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(256), lds, st, p);
+  return launch_status();
+}
+
+}  // namespace qlin
+
+using namespace qlin;
+
+extern "C" {
+
+int mi_moe_gguf_grouped_tiled_workspace(int num_chunks, int K, long long* bytes) {
+  if (!bytes) return MI_ERR_ARG;
+  if (num_chunks < 0 || K <= 0 || (K % 128)) return MI_ERR_SHAPE;
+  if ((long long)num_chunks * kChunkRows * K * 2 >= (1LL << 31)) return MI_ERR_SHAPE;
+  *bytes = chunk_layout(num_chunks, K).total;
+  return MI_OK;
+}
+
+int mi_moe_gguf_grouped_tiled_ws(int fmt, const void* x, int x_rows, const int32_t* tok_ids, int nmat, const void* const* ql,
+                                 const void* const* qh, const void* const* scale, const void* const* qmin, void* out,
+                                 long long out_stride, int out_rows, const int32_t* chunks, int num_chunks, int num_experts,
+                                 int N, int K, void* workspace, long long workspace_bytes, void* stream) {
+  if (!x || !ql || !scale || !out || !chunks) return MI_ERR_ARG;
+  if (fmt != 2 && fmt != 5 && fmt != 6) return MI_ERR_ARG;
+  if (nmat < 1 || nmat > 2 || (nmat == 2 && fmt != 2) || num_experts < 1) return MI_ERR_ARG;
+  if (x_rows < 0 || out_rows < 0 || num_chunks < 0 || N < 0) return MI_ERR_SHAPE;
+  long long need = 0;
+  if (const int rc = mi_moe_gguf_grouped_tiled_workspace(num_chunks, K, &need)) return rc;
+  if (out_stride < (long long)nmat * N || out_stride >= (1LL << 31)) return MI_ERR_SHAPE;
+  if ((uint64_t)N * (uint64_t)K >= (1ull << 31)) return MI_ERR_SHAPE;
+  for (int i = 0; i < nmat; ++i) {
+    if (!ql[i] || !scale[i]) return MI_ERR_ARG;
+    if (fmt != 6 && (!qmin || !qmin[i])) return MI_ERR_ARG;
+    if (fmt != 2 && (!qh || !qh[i])) return MI_ERR_ARG;
+  }
+  if (!num_chunks || !N || !out_rows || !x_rows) return MI_OK;
+  if (!workspace || workspace_bytes < need) return MI_ERR_ARG;
+  const ChunkLayout L = chunk_layout(num_chunks, K);
+  char* ws = (char*)workspace;
+  int32_t *tile = (int32_t*)(ws + L.tile_off), *blk = (int32_t*)(ws + L.blk_off), *cnt = (int32_t*)(ws + L.cnt_off);
+  hipStream_t st = (hipStream_t)stream;
+  hipLaunchKernelGGL(chunk_tile_map_kernel, dim3(1), dim3(kChunkMapThreads), 0, st, chunks, num_chunks, num_experts, out_rows, tile,
+                     blk, cnt);
+  const int Q = K / 32, max_blocks = num_chunks * (kChunkRows / 16);
+  hipLaunchKernelGGL(pack_x_grouped_kernel<true>, dim3((unsigned)max_blocks * ((Q + kPackQ - 1) / kPackQ)), dim3(256), 0, st,
+                     (const uint16_t*)x, tok_ids, blk, cnt, (u32x4*)ws, x_rows, K, Q, 1);
+  GemmArgs p{};
+  const long long nk = (long long)N * K;
+  p.x = ws; p.w = ql[0]; p.scale = scale[0]; p.out = out; p.M = out_rows; p.N = N; p.K = K;
+  p.zp = fmt != 6 ? qmin[0] : nullptr;
+  p.qh = fmt != 2 ? qh[0] : nullptr;
+  if (nmat == 2) { p.w1 = ql[1]; p.scale1 = scale[1]; p.zp1 = qmin[1]; }
+  p.g_tile = tile; p.g_count = cnt;
+  p.g_w_stride = nk / 2;
+  p.g_s_stride = fmt == 6 ? nk / 8 : nk / 16;
+  p.g_z_stride = nk / 16;
+  p.g_h_stride = fmt == 5 ? nk / 8 : nk / 4;
+  p.x_blocks = max_blocks; p.out_rows = out_rows; p.out_ld = (int)out_stride;
+  if (fmt == 2) return launch_chunk_gemm<WQ4K>(p, nmat, num_chunks, st);
+  return fmt == 5 ? launch_chunk_gemm<WQ5P>(p, nmat, num_chunks, st) : launch_chunk_gemm<WQ6P>(p, nmat, num_chunks, st);
+}
+
+}  // extern "C"

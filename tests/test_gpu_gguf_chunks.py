@@ -1,0 +1,81 @@
+"""Grouped GGUF MoE GEMMs on merged chunks (the tiled route of prompts) against the chunk kernel, on chunk lists
+that do and do not merge."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _lists(total, E):
+    g = torch.Generator().manual_seed(total)
+    merged, at = [], 0
+    for e in range(E):                                  # an expert's rows in full chunks and a remainder; some experts without rows
+        n = 0 if e % 5 == 4 else int(torch.randint(1, 2 * total // E, (1,), generator=g))
+        n = min(n, total - at)
+        merged += [[e, at + t, min(64, n - t)] for t in range(0, n, 64)]
+        at += n
+    odd = [[e, t0, min(n, 37)] for e, t0, n in merged]  # gaps: nothing merges
+    odd += [[E, 0, 5], [-1, 0, 5], [0, -3, 5], [0, total, 5], [1, 3, 0]]       # skipped
+    over = [[0, total - 10, 64], [1, 0, 200], [1, 64, 64], [2, 200, 64], [2, 264, 64], [3, 328, 20]]   # past the end; only 64 rows count
+    return {"merged": merged, "odd": odd, "over": over, "reversed": merged[::-1]}
+
+
+@pytest.mark.parametrize("which", ["merged", "odd", "over", "reversed"])
+@pytest.mark.parametrize("fmt", [2, 5, 6])
+@pytest.mark.parametrize("K,N", [(128, 40), (768, 264), (384, 257)])
+def test_merged_chunks_match_the_chunk_kernel(dev, fmt, which, K, N):
+    """Rows that no chunk names stay untouched; the others agree up to the order of the fp32 sums (weights and their
+    roundings are the same): an fp16 step where a sum sits on the border, 2^-11 of the row's size at most."""
+    from mi355x_qlinear import capi
+    torch.manual_seed(K + N)
+    E, total, nmat = 6, 700, 2 if fmt == 2 else 1
+    u8 = lambda *s: torch.randint(0, 256, s, dtype=torch.uint8, device=dev)
+    h = lambda *s: (torch.rand(*s, device=dev) * 0.01).half()
+    per = 16 if fmt == 6 else 32
+    ql, sc = [u8(E, N, K // 2) for _ in range(nmat)], [h(E, N, K // per) for _ in range(nmat)]
+    mn = [h(E, N, K // 32) for _ in range(nmat)] if fmt != 6 else None
+    qh = [u8(E, N, K // (8 if fmt == 5 else 4))] if fmt != 2 else None
+    x = torch.randn(300, K, device=dev).half()
+    ids = torch.randint(-2, 303, (total,), dtype=torch.int32, device=dev)       # some outside x: rows of zeros
+    chunks = torch.tensor(_lists(total, E)[which], dtype=torch.int32, device=dev)
+    arr = lambda t: capi.ptr_array(t) if t is not None else None
+    outs = [torch.full((total, nmat * N), 7.0, dtype=torch.float16, device=dev) for _ in range(2)]
+    need = ctypes.c_longlong(0)
+    assert capi.lib().mi_moe_gguf_grouped_tiled_workspace(len(chunks), K, ctypes.byref(need)) == 0
+    ws = torch.empty(need.value, dtype=torch.uint8, device=dev)
+    for o, name, tail in ((outs[0], "mi_moe_gguf_grouped", (0,)),
+                          (outs[1], "mi_moe_gguf_grouped_tiled_ws", (capi.ptr(ws), need.value))):
+        capi.call(name, x, fmt, capi.ptr(x), x.shape[0], capi.ptr(ids), nmat, arr(ql), arr(qh), arr(sc), arr(mn), capi.ptr(o),
+                  nmat * N, total, capi.ptr(chunks), len(chunks), E, N, K, *tail)
+    a, b = (o.float() for o in outs)
+    assert torch.equal(a == 7.0, b == 7.0)
+    assert float((a - b).abs().max()) <= 2.0 ** -10 * float(a.abs().max())
+    assert float((a - b).norm() / a.norm()) < 2.0 ** -11
+
+
+def test_many_chunks_and_no_token_list(dev):
+    """More chunks than the table kernel has threads; x in place of a gathered copy."""
+    from mi355x_qlinear import capi
+    E, N, K = 7, 64, 128
+    sizes = [64, 64, 64, 64, 64, 10]
+    chunks, at = [], 0
+    for i in range(3000):
+        n = sizes[i % 6]
+        chunks.append([i // 6 % E, at, n])
+        at += n
+    x = torch.randn(at, K, device=dev).half()
+    ql = torch.randint(0, 256, (E, N, K // 2), dtype=torch.uint8, device=dev)
+    sc, mn = ((torch.rand(E, N, K // 32, device=dev) * 0.01).half() for _ in range(2))
+    c = torch.tensor(chunks, dtype=torch.int32, device=dev)
+    need = ctypes.c_longlong(0)
+    assert capi.lib().mi_moe_gguf_grouped_tiled_workspace(len(c), K, ctypes.byref(need)) == 0
+    ws = torch.empty(need.value, dtype=torch.uint8, device=dev)
+    outs = [torch.zeros(at, N, dtype=torch.float16, device=dev) for _ in range(2)]
+    for o, name, tail in ((outs[0], "mi_moe_gguf_grouped", (0,)),
+                          (outs[1], "mi_moe_gguf_grouped_tiled_ws", (capi.ptr(ws), need.value))):
+        capi.call(name, x, 2, capi.ptr(x), at, None, 1, capi.ptr_array([ql]), None, capi.ptr_array([sc]), capi.ptr_array([mn]),
+                  capi.ptr(o), N, at, capi.ptr(c), len(c), E, N, K, *tail)
+    a, b = (o.float() for o in outs)
+    assert float((a - b).norm() / a.norm()) < 2.0 ** -11
