@@ -6,7 +6,9 @@
 // A function here takes a call when every operand is as the kernels want it.  Any other call - a wrong type, size
 // or device, a non-contiguous operand, a form that needs preparation - goes to the Python implementation of the same
 // operator (registered as mi355x_checked::<name>), which runs it or raises, so that accepted calls, results and
-// error messages are those of that implementation.
+// error messages are those of that implementation.  Only the checks decide that, before anything is enqueued: once an
+// entry of the C ABI has been called, a status other than 0 is raised.  Running the call again would hide a launch that
+// failed and would add to an in-place operand twice (the residual of the norm operators).
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/core/stack.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -37,6 +39,17 @@ Tensor checked(const c10::OperatorHandle& op, const A&... args) {
     static const c10::OperatorHandle op = c10::Dispatcher::singleton().findSchemaOrThrow("mi355x_checked::" name, ""); \
     return checked(op, __VA_ARGS__);                                                                        \
   } while (0)
+
+// Raises what the Python implementations raise for the same status.
+void status(const char* entry, int rc) {
+  if (rc == 0) return;
+  const char* why = rc == -1 ? "invalid argument (null pointer or bad enum)"
+                    : rc == -2 ? "unsupported shape or divisibility"
+                    : rc == -3 ? "kernel launch failed" : nullptr;
+  if (why) TORCH_CHECK(false, entry, " failed: ", why);
+  TORCH_CHECK(false, entry, " failed: ", rc);
+}
+#define CALL(entry, ...) status(#entry, entry(__VA_ARGS__))
 
 // on x's device, contiguous, strided
 bool plain(const Tensor& x, std::initializer_list<const Tensor*> ts) {
@@ -77,7 +90,7 @@ struct Linear {
     long long need = 0;
     bytes = 0;
     for (int i = 0; i < n; ++i) {
-      if (mi_gemm_tiled_workspace_split(M, N[i], K, &need) != 0) need = -1;
+      CALL(mi_gemm_tiled_workspace_split, M, N[i], K, &need);
       bytes = std::max(bytes, need);
     }
     return buffer(x, bytes);
@@ -87,22 +100,21 @@ struct Linear {
 // ---------------------------------------------------------------------------------------- FP8
 enum Scale { kPern = 0, kPert = 1, kBlock = 2 };
 
-int run_fp8(const Tensor& x, Linear& l, Scale mode, bool scale_f16) {
+void run_fp8(const Tensor& x, Linear& l, Scale mode, bool scale_f16) {
   const On on(x);
   const void* xp = x.data_ptr();
   if (l.prefill()) {
     long long bytes;
     const Tensor ws = l.workspace(x, bytes);
     for (int i = 0; i < l.n; ++i)
-      if (int rc = mi_gemm_fp8_tiled_ws(xp, l.w[i], l.s[i], mode, scale_f16, l.o[i], ws.data_ptr(), bytes, l.M, l.N[i], l.K,
-                                        l.adt, on.stream))
-        return rc;
-    return 0;
+      CALL(mi_gemm_fp8_tiled_ws, xp, l.w[i], l.s[i], mode, scale_f16, l.o[i], ws.data_ptr(), bytes, l.M, l.N[i], l.K, l.adt,
+           on.stream);
+    return;
   }
-  if (mode == kPern) return mi_gemm_fp8_pern_multi(xp, l.n, l.w, l.s, l.o, l.N, l.M, l.K, l.adt, scale_f16, on.stream);
   const float* const* s = reinterpret_cast<const float* const*>(l.s);
-  return mode == kPert ? mi_gemm_fp8_pert_multi(xp, l.n, l.w, s, l.o, l.N, l.M, l.K, l.adt, on.stream)
-                       : mi_gemm_fp8_blockscale_multi(xp, l.n, l.w, s, l.o, l.N, l.M, l.K, l.adt, on.stream);
+  if (mode == kPern) CALL(mi_gemm_fp8_pern_multi, xp, l.n, l.w, l.s, l.o, l.N, l.M, l.K, l.adt, scale_f16, on.stream);
+  else if (mode == kPert) CALL(mi_gemm_fp8_pert_multi, xp, l.n, l.w, s, l.o, l.N, l.M, l.K, l.adt, on.stream);
+  else CALL(mi_gemm_fp8_blockscale_multi, xp, l.n, l.w, s, l.o, l.N, l.M, l.K, l.adt, on.stream);
 }
 
 struct Mat { const Tensor &w, &s, &o; int64_t N; };    // N < 0: the weight's rows
@@ -129,7 +141,8 @@ bool fp8_linear(const Tensor& x, std::initializer_list<Mat> mats, int64_t K, Sca
     if (mode == kBlock && (m.s.dim() != 2 || m.s.size(0) != (N + 127) / 128 || m.s.size(1) != K / 128)) return false;
     l.add(m.w, m.s, m.o, N);
   }
-  return run_fp8(x, l, mode, sdt == at::kHalf) == 0;
+  run_fp8(x, l, mode, sdt == at::kHalf);
+  return true;
 }
 
 #define FP8_PERN(name)                                                                                        \
@@ -199,12 +212,16 @@ bool int4_linear(const Tensor& x, std::initializer_list<Mat> mats, const Tensor*
     l.add(m.w, m.s, m.o, N);
   }
   const On on(x);
-  if (!gemm) return mi_gemv_int4_multi(x.data_ptr(), l.n, l.w, l.s, nullptr, l.o, l.N, l.M, l.K, l.adt, on.stream) == 0;
+  if (!gemm) {
+    CALL(mi_gemv_int4_multi, x.data_ptr(), l.n, l.w, l.s, nullptr, l.o, l.N, l.M, l.K, l.adt, on.stream);
+    return true;
+  }
   long long bytes = 0;
   Tensor ws;
   if (l.prefill()) ws = l.workspace(x, bytes);
-  return mi_gemm_int4_ws(x.data_ptr(), l.w[0], l.s[0], zp ? zp->data_ptr() : nullptr, l.o[0], bytes ? ws.data_ptr() : nullptr, bytes,
-                         l.M, l.N[0], l.K, l.adt, on.stream) == 0;
+  CALL(mi_gemm_int4_ws, x.data_ptr(), l.w[0], l.s[0], zp ? zp->data_ptr() : nullptr, l.o[0], bytes ? ws.data_ptr() : nullptr, bytes,
+       l.M, l.N[0], l.K, l.adt, on.stream);
+  return true;
 }
 Tensor esimd_gemv_int4(const Tensor& x, const Tensor& w, const Tensor& s, const Tensor& o) {
   if (int4_linear(x, {{w, s, o, -1}}, nullptr, false)) return o;
@@ -255,16 +272,18 @@ bool gguf_linear(int fmt, const Tensor& x, const Tensor& w, const Tensor* qh, co
   if (gguf_tiled(fmt, l)) {
     long long bytes;
     const Tensor ws = l.workspace(x, bytes);
-    if (fmt == kQ4K) return mi_gemm_q4k_tiled_ws(xp, l.w[0], l.s[0], mp, l.o[0], ws.data_ptr(), bytes, l.M, l.N[0], l.K, on.stream) == 0;
-    return mi_gemm_gguf_tiled_ws(fmt, xp, l.w[0], hp, l.s[0], mp, l.o[0], ws.data_ptr(), bytes, l.M, l.N[0], l.K, on.stream) == 0;
+    if (fmt == kQ4K) CALL(mi_gemm_q4k_tiled_ws, xp, l.w[0], l.s[0], mp, l.o[0], ws.data_ptr(), bytes, l.M, l.N[0], l.K, on.stream);
+    else CALL(mi_gemm_gguf_tiled_ws, fmt, xp, l.w[0], hp, l.s[0], mp, l.o[0], ws.data_ptr(), bytes, l.M, l.N[0], l.K, on.stream);
+    return true;
   }
   switch (fmt) {
-    case kQ4K: return mi_gemv_q4k(xp, l.w[0], l.s[0], mp, l.o[0], l.M, l.N[0], l.K, on.stream) == 0;
-    case kQ40: return mi_gemv_q4_0(xp, l.w[0], l.s[0], l.o[0], l.M, l.N[0], l.K, on.stream) == 0;
-    case kQ80: return mi_gemv_q8_0(xp, l.w[0], l.s[0], l.o[0], l.M, l.N[0], l.K, on.stream) == 0;
-    case kQ5K: return mi_gemv_q5k(xp, l.w[0], hp, l.s[0], mp, l.o[0], l.M, l.N[0], l.K, on.stream) == 0;
-    default: return mi_gemv_q6k(xp, l.w[0], hp, l.s[0], l.o[0], l.M, l.N[0], l.K, on.stream) == 0;
+    case kQ4K: CALL(mi_gemv_q4k, xp, l.w[0], l.s[0], mp, l.o[0], l.M, l.N[0], l.K, on.stream); break;
+    case kQ40: CALL(mi_gemv_q4_0, xp, l.w[0], l.s[0], l.o[0], l.M, l.N[0], l.K, on.stream); break;
+    case kQ80: CALL(mi_gemv_q8_0, xp, l.w[0], l.s[0], l.o[0], l.M, l.N[0], l.K, on.stream); break;
+    case kQ5K: CALL(mi_gemv_q5k, xp, l.w[0], hp, l.s[0], mp, l.o[0], l.M, l.N[0], l.K, on.stream); break;
+    default: CALL(mi_gemv_q6k, xp, l.w[0], hp, l.s[0], l.o[0], l.M, l.N[0], l.K, on.stream);
   }
+  return true;
 }
 Tensor esimd_gemv_q4_k(const Tensor& x, const Tensor& w, const Tensor& s, const Tensor& mn, const Tensor& o) {
   if (gguf_linear(kQ4K, x, w, nullptr, s, &mn, o)) return o;
@@ -308,8 +327,9 @@ bool resadd_norm_gemv(bool int4, const Tensor& x, const Tensor& res, const Tenso
   const void *wp = w.data_ptr(), *sp = s.data_ptr();
   void* op = o.data_ptr();
   const int n = (int)N;
-  return mi_norm_gemv_scaled(x.data_ptr(), res.data_ptr(), nullptr, nw.data_ptr(), normed.data_ptr(), (int)K, (float)eps, 1.0f,
-                             int4 ? 2 : 0, 1, &wp, &sp, &op, &n, (int)K, act(x), on.stream) == 0;
+  CALL(mi_norm_gemv_scaled, x.data_ptr(), res.data_ptr(), nullptr, nw.data_ptr(), normed.data_ptr(), (int)K, (float)eps, 1.0f,
+       int4 ? 2 : 0, 1, &wp, &sp, &op, &n, (int)K, act(x), on.stream);
+  return true;
 }
 #define RESADD_NORM(name, int4)                                                                                        \
   Tensor name(const Tensor& x, const Tensor& res, const Tensor& nw, const Tensor& w, const Tensor& s, const Tensor& o, \
@@ -361,13 +381,13 @@ bool moe_full_decode(const Tensor& x, const Tensor& logits, const Tensor& out, c
   int32_t* ids = (int32_t*)(base + id_at);
   const void* xp = x.data_ptr();
   void* st = on.stream;
-  return mi_moe_topk(logits.data_ptr(), tw, ids, (int)T, (int)E, (int)k, 1, nullptr, xp, gw.data_ptr(), gate, (int)H, adt, st) == 0 &&
-         mi_moe_gemv_fp8_block_routed(xp, (int)k, 0, w13.data_ptr(), s13.data_ptr<float>(), gu, 2 * I, ids, nullptr, (int)P, (int)E,
-                                      sw13.data_ptr(), ss13.data_ptr<float>(), (int)T, 0, (int)(2 * I), (int)H, adt, st) == 0 &&
-         mi_moe_gemv_fp8_block_routed(gu, 1, 1, w2.data_ptr(), s2.data_ptr<float>(), y, H, ids, tw, (int)P, (int)E, sw2.data_ptr(),
-                                      ss2.data_ptr<float>(), (int)T, (int)P, (int)H, (int)I, adt, st) == 0 &&
-         mi_moe_combine_shared(y, nullptr, nullptr, out.data_ptr(), (char*)y + P * H * 2, gate, (int)H, (int)k, (int)T, 0, adt, 0,
-                               st) == 0;
+  CALL(mi_moe_topk, logits.data_ptr(), tw, ids, (int)T, (int)E, (int)k, 1, nullptr, xp, gw.data_ptr(), gate, (int)H, adt, st);
+  CALL(mi_moe_gemv_fp8_block_routed, xp, (int)k, 0, w13.data_ptr(), s13.data_ptr<float>(), gu, 2 * I, ids, nullptr, (int)P, (int)E,
+       sw13.data_ptr(), ss13.data_ptr<float>(), (int)T, 0, (int)(2 * I), (int)H, adt, st);
+  CALL(mi_moe_gemv_fp8_block_routed, gu, 1, 1, w2.data_ptr(), s2.data_ptr<float>(), y, H, ids, tw, (int)P, (int)E, sw2.data_ptr(),
+       ss2.data_ptr<float>(), (int)T, (int)P, (int)H, (int)I, adt, st);
+  CALL(mi_moe_combine_shared, y, nullptr, nullptr, out.data_ptr(), (char*)y + P * H * 2, gate, (int)H, (int)k, (int)T, 0, adt, 0, st);
+  return true;
 }
 Tensor moe_forward_full_fp8_block(const Tensor& x, const Tensor& logits, const Tensor& out, const Tensor& w13, const Tensor& s13,
                                   const Tensor& sw13, const Tensor& ss13, const Tensor& w2, const Tensor& s2, const Tensor& sw2,

@@ -129,3 +129,49 @@ def test_moe_decode_is_the_same(dev, T, dt):
     for op, o in zip((torch.ops.moe_ops, torch.ops.mi355x_checked), outs):
         assert op.moe_forward_full_fp8_block(x, logits, o, *w, k, 1, E) is o
     assert torch.equal(outs[0], outs[1])
+
+
+def _refused(dev):
+    """(Python building block of the operator, call) where the checks pass and the C entry refuses the size before it
+    launches anything: K of no whole granule, and an expert row longer than the LDS holds."""
+    h = lambda *s: torch.zeros(*s, dtype=torch.float16, device=dev)
+    f8 = lambda *s: torch.zeros(*s, dtype=torch.uint8, device=dev)
+    one = torch.ones(1, device=dev)
+    H = 40960
+    moe = [h(1, H), h(1, 2), h(1, H), f8(2, 256, H), torch.ones(2, 2, H // 128, device=dev), f8(256, H),
+           torch.ones(2, H // 128, device=dev), f8(2, H, 128), torch.ones(2, H // 128, 1, device=dev), f8(H, 128),
+           torch.ones(H // 128, 1, device=dev), h(1, H), 1, 1, 2]
+    return {"esimd_gemv_fp8_pern": ("_fp8_pern_multi", lambda: _V.esimd_gemv_fp8_pern(h(1, 48), f8(8, 48), h(8), h(1, 8), 8, 48)),
+            "esimd_gemv_fp8_pert": ("_fp8_pert_multi", lambda: _V.esimd_gemv_fp8_pert(h(1, 48), f8(8, 48), one, h(1, 8))),
+            "esimd_resadd_norm_gemv_fp8_pert": ("_norm_gemv", lambda: _V.esimd_resadd_norm_gemv_fp8_pert(
+                h(1, 24), h(1, 24), h(24), f8(8, 24), one, h(1, 8), h(1, 24), 1e-6)),
+            "moe_forward_full_fp8_block": ("esimd_moe_topk", lambda: torch.ops.moe_ops.moe_forward_full_fp8_block(*moe))}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["esimd_gemv_fp8_pern", "esimd_gemv_fp8_pert", "esimd_resadd_norm_gemv_fp8_pert",
+                                  "moe_forward_full_fp8_block"])
+def test_a_status_is_raised_and_the_call_not_run_again(dev, monkeypatch, name):
+    block, call = _refused(dev)[name]
+    inner, again = getattr(_ops, block), []
+    monkeypatch.setattr(_ops, block, lambda *a, **k: again.append(1) or inner(*a, **k))
+    with pytest.raises(RuntimeError, match="failed: unsupported shape or divisibility"):
+        call()
+    assert not again
+
+
+@pytest.mark.gpu
+def test_a_pending_error_does_not_add_to_the_residual_twice(dev):
+    """An error that something else left on the thread is what the status of the next launch reports: the operator
+    raises it, as its Python implementation does, and has added x to the residual once."""
+    import ctypes
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64.so" in line))
+    args, _ = _args("esimd_resadd_norm_gemv_fp8_pert", 1, 512, 40, torch.float16)
+    want = args[1] + args[0]
+    torch.cuda.synchronize()
+    assert hip.hipSetDevice(1 << 20) != 0                 # no such device: refused on the host
+    with pytest.raises(RuntimeError, match="mi_norm_gemv_scaled failed: kernel launch failed"):
+        _V.esimd_resadd_norm_gemv_fp8_pert(*args)
+    torch.cuda.synchronize()
+    assert torch.equal(args[1], want)
