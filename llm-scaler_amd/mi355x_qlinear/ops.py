@@ -120,6 +120,7 @@ def _fp8_pern_multi(x, ws, ss, os_, Ns, K, who):
              f"{who}: weight_scale must be fp16 or fp32 (all the same), got {s.dtype}")
         _chk(s.numel() == int(N), f"{who}: weight_scale must have N={int(N)} entries")
         _chk(o.numel() == M * int(N), f"{who}: output has {o.numel()} elements, expected M*N={M * int(N)}")
+    ss = [s.contiguous() for s in ss]                  # the kernels read N scales in a row
     if _prefill_route(M, K):
         return _fp8_tiled_multi(x, ws, ss, os_, Ns, M, K, _SC_PERN, sdt == torch.float16)
     capi.call("mi_gemm_fp8_pern_multi", x, capi.ptr(x), len(ws), capi.ptr_array(ws), capi.ptr_array(ss),

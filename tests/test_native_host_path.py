@@ -105,12 +105,20 @@ def test_same_results_and_same_refusals(dev, name):
 
 
 @pytest.mark.gpu
-def test_calls_that_need_preparation_still_run(dev):
-    """Accepted before although not as the kernels want it: a per-channel scale that is a strided view."""
-    args, at = _args("esimd_gemv_fp8_pern", 2, 512, 24, torch.float16)
-    args[2] = args[2].repeat_interleave(2)[::2]
-    out = _V.esimd_gemv_fp8_pern(*args).clone()
-    assert torch.equal(out, torch.ops.mi355x_checked.esimd_gemv_fp8_pern(*args))
+@pytest.mark.parametrize("M", [2, 70])                  # weight-streaming and tiled kernel
+def test_a_strided_scale_is_read_with_its_stride(dev, M):
+    """Accepted although not as the kernels want it: per-channel scales that are views with a stride."""
+    args, at = _args("esimd_gemv_fp8_pern", M, 512, 24, torch.float16)
+    want = _V.esimd_gemv_fp8_pern(*args).clone()
+    assert float(want.abs().max()) > 0
+    wide = torch.stack([args[2], args[2] + 1.0], 1)      # the other column holds other scales
+    args[2] = wide[:, 0]
+    assert not args[2].is_contiguous()
+    assert torch.equal(_V.esimd_gemv_fp8_pern(*args), want)
+    two, at = _args("esimd_gemv_fp8_pern_fused2", M, 512, 24, torch.float16)
+    want = [_V.esimd_gemv_fp8_pern_fused2(*two).clone(), two[7].clone()]
+    two[6] = torch.stack([two[6], two[6] + 1.0], 1)[:, 0]
+    assert torch.equal(_V.esimd_gemv_fp8_pern_fused2(*two), want[0]) and torch.equal(two[7], want[1])
 
 
 @pytest.mark.gpu
