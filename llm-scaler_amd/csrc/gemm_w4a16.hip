@@ -36,17 +36,18 @@ int mi_gemm_int4_ws(const void* x, const void* w, const void* scale, const void*
 
 int mi_gemm_int4(const void* x, const void* w, const void* scale, const void* zp, void* out, int M, int N,
                  int K, int act_dtype, void* stream) {
-  long long bytes = 0;
-  const int rc = mi_gemm_int4_workspace(M, N, K, &bytes);
+  long long one = 0, bytes = 0;
+  const int rc = mi_gemm_int4_workspace(M, N, K, &one);
   if (rc != MI_OK) return rc;
-  if (!bytes) return mi_gemm_int4_ws(x, w, scale, zp, out, nullptr, 0, M, N, K, act_dtype, stream);
+  if (!one) return mi_gemm_int4_ws(x, w, scale, zp, out, nullptr, 0, M, N, K, act_dtype, stream);
   if (mi_gemm_tiled_workspace_split(M, N, K, &bytes) != MI_OK) return MI_ERR_SHAPE;
   // scratch for the re-tiled activations and the K slices' sums: this stream's grow-only buffer (the first
   // call of a size allocates; callers that must never allocate pass their own
-  // workspace through mi_gemm_int4_ws)
-  void* ws = scratch_get((hipStream_t)stream, (size_t)bytes);
+  // workspace through mi_gemm_int4_ws); without room for the sums the GEMM runs in one piece
+  size_t got = 0;
+  void* ws = scratch_get((hipStream_t)stream, (size_t)bytes, (size_t)one, &got);
   if (!ws) return MI_ERR_LAUNCH;
-  return mi_gemm_int4_ws(x, w, scale, zp, out, ws, bytes, M, N, K, act_dtype, stream);
+  return mi_gemm_int4_ws(x, w, scale, zp, out, ws, (long long)got, M, N, K, act_dtype, stream);
 }
 
 }  // extern "C"

@@ -16,19 +16,34 @@ std::map<std::pair<int, hipStream_t>, Buf> g_bufs;
 std::map<std::pair<int, hipStream_t>, unsigned int*> g_counters;
 }  // namespace
 
-void* scratch_get(hipStream_t stream, size_t bytes) {
+void* scratch_get(hipStream_t stream, size_t bytes, size_t least, size_t* got) {
+  if (!got) least = bytes;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
   std::lock_guard<std::mutex> lock(g_mu);
   Buf& b = g_bufs[{dev, stream}];
+  if (got) *got = b.bytes;
   if (b.bytes >= bytes && b.p) return b.p;
+  const bool enough = b.p && b.bytes >= least;
+  if (enough) {                                       // no allocation is even tried in a capture that can do without
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+    if (capture != hipStreamCaptureStatusNone) return b.p;
+  }
   size_t want = 1u << 20;                             // at least 1 MiB, then powers of two
   while (want < bytes) want <<= 1;
   void* p = nullptr;
-  if (hipMalloc(&p, want) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+  if (hipMalloc(&p, want) != hipSuccess) {
+    (void)hipGetLastError();
+    if (enough || least >= bytes) return enough ? b.p : nullptr;
+    want = 1u << 20;
+    while (want < least) want <<= 1;
+    if (hipMalloc(&p, want) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+  }
   // the old buffer stays allocated: kernels already queued may still use it
   b.p = p;
   b.bytes = want;
+  if (got) *got = want;
   return p;
 }
 

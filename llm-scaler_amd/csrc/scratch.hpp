@@ -19,8 +19,10 @@
 
 namespace qlin {
 
-// nullptr when the allocation fails (e.g. under stream capture)
-void* scratch_get(hipStream_t stream, size_t bytes);
+// nullptr when the allocation fails (e.g. under stream capture).  With `least` (0: bytes) and `got`, a call that can do
+// with less gets what the buffer holds, *got bytes, where `bytes` cannot be had: the size a call likes best need not grow
+// with its rows, so a buffer warmed up on the longest prompt may be too small for that of a shorter one.
+void* scratch_get(hipStream_t stream, size_t bytes, size_t least = 0, size_t* got = nullptr);
 
 // A zero-initialised block of 512 32-bit counters per (device, stream) for kernels that
 // count arriving workgroups and leave the counters at zero again when they finish.  The

@@ -88,13 +88,16 @@ static int run(SkinnyArgs a, int act_dtype, hipStream_t st) {
   // prefill: the tiled matrix-core GEMM reads the weight once per 256 rows instead of once per 64
   if constexpr (FMT == 0 || FMT == 2) {
     if (a.M > 64 && a.K % 128 == 0) {
-      long long bytes = 0, need = 0;
+      long long bytes = 0, need = 0, one = 0;
+      if (mi_gemm_tiled_workspace(a.M, a.K, &one) != MI_OK) return MI_ERR_SHAPE;
       for (int i = 0; i < a.nmat; ++i) {
         if (mi_gemm_tiled_workspace_split(a.M, a.N[i], a.K, &need) != MI_OK) return MI_ERR_SHAPE;
         if (need > bytes) bytes = need;
       }
-      void* ws = scratch_get(st, (size_t)bytes);
+      size_t got = 0;                                  // without room for the K slices' sums a matrix runs in one piece
+      void* ws = scratch_get(st, (size_t)bytes, (size_t)one, &got);
       if (!ws) return MI_ERR_LAUNCH;
+      bytes = (long long)got;
       for (int i = 0; i < a.nmat; ++i) {
         const int rc = FMT == 0 ? mi_gemm_fp8_tiled_ws(a.x, a.w[i], a.s[i], SC, a.scale_f16, a.out[i], ws, bytes, a.M,
                                                        a.N[i], a.K, act_dtype, st)

@@ -76,3 +76,52 @@ def test_workspace_without_room_for_the_sums_runs_in_one_piece(v, dev):
     ref = O.matmul_ref(x, O.fp8_dequant_per_channel(w8, s))
     assert all(O.max_rel_err(o, ref) < 1e-2 for o in outs)
     assert float(((outs[0] - outs[1]).norm() / outs[0].norm())) < 2.0 ** -11      # rms of one fp16 rounding each: 2^-12.8
+
+
+@pytest.mark.parametrize("kind", ["int4", "fp8"])
+def test_a_shorter_prompt_captured_after_the_longest(v, dev, kind):
+    """The C entries that keep their own scratch: the K slices' sums can make a problem of few tiles need more than a
+    larger one.  A stream warmed up on the larger (one piece, exactly the re-tiled activations) captures the smaller in
+    one piece; with a workspace for the sums the result differs by their order only."""
+    from mi355x_qlinear import capi
+    M, K, N, wide = 2048, 8192, 512, 4608                 # 4608: 256-row tiles, one piece; 512: split
+    sizes = []
+    for n in (wide, N):
+        need = ctypes.c_longlong(0)
+        assert capi.lib().mi_gemm_tiled_workspace_split(M, n, K, ctypes.byref(need)) == 0
+        sizes.append(need.value)
+    assert sizes[1] > sizes[0] == M * K * 2 == 1 << 25      # the scratch grows in powers of two
+    g = torch.Generator(device=dev).manual_seed(1)
+    x = torch.randn(M, K, generator=g, device=dev).half()
+    if kind == "int4":
+        w = torch.randint(0, 256, (wide, K // 2), dtype=torch.uint8, generator=g, device=dev)
+        s = (torch.rand(wide, K // 128, generator=g, device=dev) * 0.01).half()
+        tail = lambda n: ("mi_gemm_int4", [capi.ptr(s), None], [M, n, K, 0])
+        ws_tail = ("mi_gemm_int4_ws", [capi.ptr(s), None])
+    else:
+        w = torch.randn(wide, K, generator=g, device=dev).to(torch.float8_e4m3fn)
+        s = torch.rand(wide, generator=g, device=dev) * 0.01
+        tail = lambda n: ("mi_gemm_fp8_pern", [capi.ptr(s)], [M, n, K, 0, 0])
+        ws_tail = ("mi_gemm_fp8_tiled_ws", [capi.ptr(s), 0, 0])
+    out = torch.zeros(M, wide, dtype=torch.float16, device=dev)
+
+    def call(n):
+        name, operands, sizes_ = tail(n)
+        capi.call(name, x, capi.ptr(x), capi.ptr(w), *operands, capi.ptr(out), *sizes_)
+
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        call(wide)
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            call(N)
+    ws, want = torch.empty(sizes[1], dtype=torch.uint8, device=dev), torch.empty(M, N, dtype=torch.float16, device=dev)
+    capi.call(ws_tail[0], x, capi.ptr(x), capi.ptr(w), *ws_tail[1], capi.ptr(want), capi.ptr(ws), sizes[1], M, N, K, 0)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.view(-1)[:M * N].view(M, N).float()
+        assert float((got - want.float()).norm() / want.float().norm()) < 2.0 ** -11
