@@ -125,11 +125,44 @@ static int launch_chunk_gemm(GemmArgs p, int nmat, int max_tiles, hipStream_t st
   return launch_status();
 }
 
+// Which of the two kernels a chunk list takes, from what the host knows of it: its length, not its contents.  A list
+// that covers its buffer holds out_rows rows in chunks of which at most one per expert is not full.  Where the buffer is
+// larger than the list can cover, its rows are at least those of the full chunks; where the list is longer, its chunks do
+// not merge.  The experts' tiles follow from the chunks as on average for independent remainders.
+// Time in us.  Tiled: tables and re-tiling, then a chain of K / 64 steps per round of one workgroup per CU, and the
+// multiplications of the live rows.  Chunks: a chain of K steps, and a part per chunk and per 64 rows for every million
+// weights.  Fitted on 1300 launches (1 .. 256 experts, H 1024 .. 6144, I 256 .. 2048, 8 .. 1024 rows per expert; even, drawn
+// and skewed counts): nine in ten within 25 %, so the tiled kernel has to promise 5 %.  Both sides, chunks / tiled in us: E = 8,
+// H = 1024, I = 512, 128 rows per expert, up 20 / 41; E = 16, H = 2048, I = 768, 96 rows 37 / 53; E = 128, same sizes, 60 even
+// rows 123 / 153, 96 rows 226 / 180, 256 rows 517 / 407; E = 256, H = 2048, I = 512, 60 rows 184 / 223, 96 rows 299 / 274.
+static bool chunk_tiles_pay(bool up, long long n, long long out_rows, long long E, long long N, long long K, long long nmat) {
+  if (kChunkRows * n > out_rows + kChunkRows * E) return false;
+  const long long rows = out_rows <= kChunkRows * n ? out_rows : std::max(n, kChunkRows * (n - E));
+  const long long used = std::min(E, n), m_tiles = std::min(n, std::max(used, (2 * n + 3 * used + 7) / 8));
+  const long long cus = device_cu_count_gemm(), n_tiles = nmat * ((N + kGgufBN - 1) / kGgufBN);
+  const double rounds = (double)((m_tiles * n_tiles + cus - 1) / cus), full = (double)(rows * n_tiles) / (double)(kGgufBM * cus);
+  const double steps = (double)(K / 64), weights = (double)(nmat * N * K) / 1e6, r64 = (double)rows / kChunkRows;
+  const double tiled = up ? 17.0 + steps * (0.97 * rounds + 1.64 * full) : 18.0 + steps * (1.11 * rounds + 2.16 * full);
+  const double chunks = up ? 7.0 + 0.41 * steps + weights * (0.12 * (double)n + 0.18 * r64)
+                           : 9.0 + 0.41 * steps + weights * (0.21 * (double)n + 0.18 * r64);
+  return tiled < 0.95 * chunks;
+}
+
 }  // namespace qlin
 
 using namespace qlin;
 
 extern "C" {
+
+int mi_moe_gguf_grouped_tiled_pays(int fmt, int nmat, int num_chunks, int out_rows, int num_experts, int N, int K, int* pays) {
+  if (!pays) return MI_ERR_ARG;
+  if ((fmt != 2 && fmt != 5 && fmt != 6) || nmat < 1 || nmat > 2 || num_experts < 1) return MI_ERR_ARG;
+  if (num_chunks < 0 || out_rows < 0 || N < 0 || K <= 0) return MI_ERR_SHAPE;
+  long long bytes = 0;
+  *pays = !(nmat == 2 && fmt != 2) && mi_moe_gguf_grouped_tiled_workspace(num_chunks, K, &bytes) == MI_OK && num_chunks && N &&
+          chunk_tiles_pay(fmt == 2, num_chunks, out_rows, num_experts, N, K, nmat);
+  return MI_OK;
+}
 
 int mi_moe_gguf_grouped_tiled_workspace(int num_chunks, int K, long long* bytes) {
   if (!bytes) return MI_ERR_ARG;

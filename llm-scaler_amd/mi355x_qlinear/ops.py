@@ -579,18 +579,19 @@ def _chk_chunks(chunks, who):
 
 
 def _grouped_gguf(fmt, x, tok_ids, qls, qhs, scales, mins, out, out_stride, total, chunks, E, N, K, smallm):
-    """One grouped launch over chunks, or, from 60 rows per expert on, the tiled GEMM on merged chunks (128 experts, H = 2048,
-    I = 768, the whole layer: 800 tokens 261 against 292 us, 1024: 315 against 300, 2048: 510 against 404)."""
+    """One grouped launch over chunks or, where the library expects that to be faster (mi_moe_gguf_grouped_tiled_pays: an
+    expert's chunks merge and the tiles fill the CUs), the tiled GEMM on merged chunks."""
     lists = [capi.ptr_array(t) if t is not None else None for t in (qls, qhs, scales, mins)]
     operands = (capi.ptr(x), x.shape[0], capi.ptr(tok_ids), len(qls), *lists, capi.ptr(out), out_stride, total,
                 capi.ptr(chunks), chunks.size(0), E, N, K)
-    aligned = all(t.data_ptr() % 16 == 0 for g in ([x], qls, qhs, scales, mins) if g is not None for t in g)
-    if not smallm and K % 128 == 0 and aligned and total >= 60 * E:
-        need = ctypes.c_longlong(0)
-        if capi.lib().mi_moe_gguf_grouped_tiled_workspace(chunks.size(0), K, ctypes.byref(need)) == 0:
-            ws = torch.empty(need.value, dtype=torch.uint8, device=x.device)
-            capi.call("mi_moe_gguf_grouped_tiled_ws", x, fmt, *operands, capi.ptr(ws), need.value)
-            return
+    pays, need = ctypes.c_int(0), ctypes.c_longlong(0)
+    if not smallm:
+        capi.lib().mi_moe_gguf_grouped_tiled_pays(fmt, len(qls), chunks.size(0), total, E, N, K, ctypes.byref(pays))
+    if pays.value and all(t.data_ptr() % 16 == 0 for g in ([x], qls, qhs, scales, mins) if g is not None for t in g):
+        capi.lib().mi_moe_gguf_grouped_tiled_workspace(chunks.size(0), K, ctypes.byref(need))
+        ws = torch.empty(need.value, dtype=torch.uint8, device=x.device)
+        capi.call("mi_moe_gguf_grouped_tiled_ws", x, fmt, *operands, capi.ptr(ws), need.value)
+        return
     capi.call("mi_moe_gguf_grouped", x, fmt, *operands, 1 if smallm else 0)
 
 

@@ -77,6 +77,32 @@ def test_moe_gguf_grouped_argument_errors():
     assert f(n=0) == 0 and f(rows=0) == 0 and f(x_rows=0) == 0 and f(N=0, stride=0) == 0
 
 
+def test_merged_chunks_are_expected_where_they_were_measured_faster():
+    """mi_moe_gguf_grouped_tiled_pays decides from the length of the chunk list, not from the rows of the caller's
+    buffer alone; geometries where either kernel was measured ahead by 8 % and more."""
+    lib = capi.lib()
+
+    def pays(fmt, n, rows, E, N, K, nmat=None):
+        p = ctypes.c_int(-1)
+        rc = lib.mi_moe_gguf_grouped_tiled_pays(fmt, (2 if fmt == 2 else 1) if nmat is None else nmat, n, rows, E, N, K, ctypes.byref(p))
+        return p.value if rc == 0 else rc
+    for case in ((2, 314, 16384, 128, 768, 2048), (6, 314, 16384, 128, 2048, 768), (5, 231, 9216, 128, 2048, 768),
+                 (2, 513, 24576, 256, 512, 2048), (5, 80, 4096, 32, 2048, 1024), (2, 68, 4096, 8, 1536, 4096)):
+        assert pays(*case) == 1, case
+    for case in ((2, 20, 1024, 8, 512, 1024), (2, 32, 1536, 16, 768, 2048), (2, 128, 7680, 128, 768, 2048),
+                 (2, 328, 15360, 256, 512, 2048), (6, 16, 1024, 8, 1024, 512), (6, 5, 240, 4, 2048, 768)):
+        assert pays(*case) == 0, case
+    # a buffer of the largest size: 64 tokens' chunks stay, a list of full chunks does not
+    assert pays(2, 126, 16384, 128, 768, 2048) == 0 and pays(6, 126, 16384, 128, 2048, 768) == 0
+    assert pays(2, 314, 32768, 128, 768, 2048) == 1
+    assert pays(2, 7680, 7680, 128, 768, 2048) == 0                              # one-row chunks: nothing merges
+    assert pays(2, 314, 16384, 128, 768, 2080) == 0 and pays(2, 200000, 12800000, 8, 768, 2048) == 0    # sizes it does not take
+    assert pays(2, 0, 16384, 128, 768, 2048) == 0 and pays(2, 314, 16384, 128, 0, 2048) == 0
+    assert pays(6, 314, 16384, 128, 2048, 768, nmat=2) == 0
+    assert pays(3, 4, 64, 8, 64, 128) == -1 and pays(2, 4, 64, 0, 64, 128) == -1 and pays(2, -1, 64, 8, 64, 128) == -2
+    assert lib.mi_moe_gguf_grouped_tiled_pays(2, 2, 4, 64, 8, 64, 128, None) == -1
+
+
 def test_moe_grouped_module_matches_the_reference_binding():
     """Names, argument order and defaults of the pybind module the patched SGLang imports
     (S/csrc/moe_grouped/moe_grouped_entry.sycl:108-127, sglang_for_multi_arc.patch:2114)."""

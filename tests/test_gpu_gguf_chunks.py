@@ -79,3 +79,29 @@ def test_many_chunks_and_no_token_list(dev):
                   capi.ptr(o), N, at, capi.ptr(c), len(c), E, N, K, *tail)
     a, b = (o.float() for o in outs)
     assert float((a - b).norm() / a.norm()) < 2.0 ** -11
+
+
+def _record(monkeypatch):
+    """Names of the C entries that the operators call from here on."""
+    from mi355x_qlinear import capi
+    inner, names = capi.call, []
+    monkeypatch.setattr(capi, "call", lambda name, *a: names.append(name) or inner(name, *a))
+    return names
+
+
+@pytest.mark.parametrize("rows,E,per,n_list,want", [
+    (1200, 6, 200, None, "mi_moe_gguf_grouped"),             # few experts, small matrices: the tiles would fill a few CUs
+    (6144, 2, 3072, None, "mi_moe_gguf_grouped_tiled_ws"),
+    (6144, 2, 3072, 6, "mi_moe_gguf_grouped")])              # a buffer of the largest size, a handful of chunks
+def test_which_kernel_the_module_takes(dev, monkeypatch, rows, E, per, n_list, want):
+    from custom_esimd_kernels_sglang import moe_grouped_gguf_xpu as mg
+    H, I = 384, 1536
+    u8 = lambda *s: torch.randint(0, 256, s, dtype=torch.uint8, device=dev)
+    h = lambda *s: (torch.rand(*s, device=dev) * 0.01).half()
+    gate, up = [(u8(E, I, H // 2), h(E, I, H // 32), h(E, I, H // 32)) for _ in range(2)]
+    chunks = torch.tensor([[e, e * per + t, min(64, per - t)] for e in range(E) for t in range(0, per, 64)][:n_list],
+                          dtype=torch.int32, device=dev)
+    x = torch.randn(rows, H, device=dev).half()
+    names = _record(monkeypatch)
+    mg.moe_up_q4k_ggemv(x, *gate, *up, torch.zeros(rows, 2 * I, dtype=torch.float16, device=dev), chunks, H, I)
+    assert names == [want]
