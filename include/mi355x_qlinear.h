@@ -227,7 +227,7 @@ int mi_moe_gguf_grouped(int fmt, const void* x, int x_rows, const int32_t* tok_i
 /* The same for prompts, through the tiled matrix-core GEMM: chunks of one expert that follow each other without a
  * gap are merged into tiles of 256 rows, the rows of x are gathered and re-tiled once.  The operands and results of
  * mi_moe_gguf_grouped with rows16 = 0; K % 128 == 0, x and the stacks 16-byte aligned, two matrices for fmt 2 only,
- * num_chunks x 64 x K x 2 below 2 GiB.  workspace: mi_moe_gguf_grouped_tiled_workspace bytes.
+ * x and num_chunks x 64 x K x 2 below 2 GiB.  workspace: mi_moe_gguf_grouped_tiled_workspace bytes.
  * mi_moe_gguf_grouped_tiled_pays: *pays = 1 where this is expected to be the faster of the two, from the number of
  * chunks and the rows of out (assumed: each expert's chunks full but for the last). */
 int mi_moe_gguf_grouped_tiled_pays(int fmt, int nmat, int num_chunks, int out_rows, int num_experts, int N, int K,

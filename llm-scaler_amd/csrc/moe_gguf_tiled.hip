@@ -183,7 +183,7 @@ int mi_moe_gguf_grouped_tiled_ws(int fmt, const void* x, int x_rows, const int32
   long long need = 0;
   if (const int rc = mi_moe_gguf_grouped_tiled_workspace(num_chunks, K, &need)) return rc;
   if (out_stride < (long long)nmat * N || out_stride >= (1LL << 31)) return MI_ERR_SHAPE;
-  if ((uint64_t)N * (uint64_t)K >= (1ull << 31)) return MI_ERR_SHAPE;
+  if ((uint64_t)N * (uint64_t)K >= (1ull << 31) || (uint64_t)x_rows * (uint64_t)K * 2 >= (1ull << 31)) return MI_ERR_SHAPE;
   for (int i = 0; i < nmat; ++i) {
     if (!ql[i] || !scale[i]) return MI_ERR_ARG;
     if (fmt != 6 && (!qmin || !qmin[i])) return MI_ERR_ARG;

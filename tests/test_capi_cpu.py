@@ -77,6 +77,24 @@ def test_moe_gguf_grouped_argument_errors():
     assert f(n=0) == 0 and f(rows=0) == 0 and f(x_rows=0) == 0 and f(N=0, stride=0) == 0
 
 
+def test_merged_chunks_argument_errors():
+    """The tiled entry refuses what the chunk kernel refuses, whichever of the two a call would take."""
+    lib = capi.lib()
+    ok, arr = ctypes.c_void_p(256), (ctypes.c_void_p * 2)(256, 256)
+
+    def f(**kw):
+        return lib.mi_moe_gguf_grouped_tiled_ws(kw.get("fmt", 2), ok, kw.get("x_rows", 64), None, kw.get("nmat", 2), arr,
+                                                kw.get("qh", None), arr, kw.get("mn", arr), ok, ctypes.c_longlong(kw.get("stride", 1024)),
+                                                64, ok, kw.get("n", 4), 8, kw.get("N", 512), kw.get("K", 2048), kw.get("ws", ok),
+                                                ctypes.c_longlong(kw.get("wsb", 0)), None)
+    assert f(fmt=3) == -1 and f(nmat=0) == -1 and f(mn=None) == -1 and f(fmt=5, nmat=1) == -1 and f(fmt=6, nmat=2, qh=arr) == -1
+    assert f(K=2080) == -2 and f(stride=1023) == -2 and f(n=-1) == -2 and f(n=1 << 14) == -2
+    assert f(N=1 << 20, stride=1 << 22) == -2                                    # N K beyond 2^31
+    assert f(x_rows=1 << 19) == -2                                               # x beyond 2 GiB
+    assert f() == -1 and f(ws=None, wsb=1 << 30) == -1                           # workspace too small / missing
+    assert f(n=0) == 0 and f(x_rows=0) == 0 and f(N=0, stride=0) == 0
+
+
 def test_merged_chunks_are_expected_where_they_were_measured_faster():
     """mi_moe_gguf_grouped_tiled_pays decides from the length of the chunk list, not from the rows of the caller's
     buffer alone; geometries where either kernel was measured ahead by 8 % and more."""
