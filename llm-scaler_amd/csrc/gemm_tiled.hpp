@@ -1129,9 +1129,13 @@ static inline bool gemm_big_tiles(long M, long N) {
 // neighbours' CUs are busy or not, so a problem with few tiles leaves the chip idle: slices up to one workgroup
 // per CU (two per CU share the path from L2 to the CU and gain nothing: Q8_0 1000 x 4096 x 4096, 256 tiles:
 // 61 us in one piece, 65 in two).  Every slice writes and reads fp32 sums of the whole output, 8 bytes per
-// element at about 5 TB/s, which sets the best number where tiles are few.  One slice against this rule's:
-// INT4 128 x 4096 x 4096 44 -> 22 us, Q4_K 100 x 5120 x 5120 63 -> 26 us, Q6_K 129 x 5120 x 5120 71 -> 38 us, INT4
-// 1024 x 6144 x 2048 72 -> 51 us, FP8 70 x 1024 x 1024 13.6 -> 10 us.
+// element at about 5 TB/s, which sets the best number where tiles are few.  The alternative is one piece on tiles of 96
+// columns, about 0.48 us a step; slices have to make up for the second launch and the start of their chains.  Over 1287
+// problems of all formats (M 65 .. 1024, N 128 .. 14336, K 384 .. 8448) that leaves 2 slower in slices by more than 3 % and
+// 17 in one piece (without this line: 53 and none, up to 1.25 times): M x N x K, one piece / slices in us, FP8 block-scaled 320 x
+// 2760 x 1024 15.4 / 19.3 (one piece), INT4 256 x 5688 x 1536 20.1 / 23.9 (one piece).  One slice of 128 columns against
+// the rule's slices (M x K x N): INT4 128 x 4096 x 4096 44 -> 22 us, Q4_K 100 x 5120 x 5120 63 -> 26 us, Q6_K 129 x 5120 x 5120 71 -> 38
+// us, INT4 1024 x 6144 x 2048 72 -> 51 us, FP8 70 x 1024 x 1024 13.6 -> 10 us.
 static inline int gemm_splits(long M, long N, long K) {
   if (M <= 64 || N <= 0 || gemm_big_tiles(M, N)) return 1;
   const long tiles = ((M + 127) / 128) * ((N + 127) / 128);
@@ -1140,7 +1144,8 @@ static inline int gemm_splits(long M, long N, long K) {
   int best = 1;
   for (long s = 2; s <= most; ++s)
     if (chain / s + sums * s < chain / best + (best > 1 ? sums * best : -2.0)) best = (int)s;     // the second launch: 2 us
-  return best;
+  const long steps = (K / 128 + best - 1) / best * 2;                                             // of the longest slice
+  return 2.0 + 0.55 * (double)steps + sums * best < 0.48 * (double)(K / 64) ? best : 1;
 }
 
 // bytes of the re-tiled activations and, behind them, of the slices' sums

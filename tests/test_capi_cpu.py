@@ -77,6 +77,19 @@ def test_moe_gguf_grouped_argument_errors():
     assert f(n=0) == 0 and f(rows=0) == 0 and f(x_rows=0) == 0 and f(N=0, stride=0) == 0
 
 
+@pytest.mark.parametrize("M,N,K,split", [
+    (128, 4096, 4096, True), (100, 5120, 5120, True), (129, 5120, 5120, True), (1024, 2048, 6144, True), (70, 1024, 1024, True),
+    (256, 4936, 1280, False), (320, 2760, 1024, False), (256, 2568, 768, False), (65, 9584, 1024, False), (160, 5120, 1024, False),
+    (256, 5688, 1536, False), (64, 4096, 4096, False), (2048, 14336, 4096, False)])
+def test_k_is_split_where_it_was_measured_faster(M, N, K, split):
+    """Few tiles and a long K: slices.  Short K: one piece (measured 12 to 28 % ahead of slices there)."""
+    lib = capi.lib()
+    one, need = ctypes.c_longlong(-1), ctypes.c_longlong(-1)
+    assert lib.mi_gemm_tiled_workspace(M, K, ctypes.byref(one)) == 0
+    assert lib.mi_gemm_tiled_workspace_split(M, N, K, ctypes.byref(need)) == 0
+    assert (need.value > one.value) == split and need.value >= one.value
+
+
 def test_merged_chunks_argument_errors():
     """The tiled entry refuses what the chunk kernel refuses, whichever of the two a call would take."""
     lib = capi.lib()
