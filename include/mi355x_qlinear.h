@@ -485,7 +485,10 @@ int mi_gemm_q4k_tiled_ws(const void* x, const void* ql, const void* scale, const
 /* The same for the other GGUF formats (fmt 3 = Q4_0, 4 = Q8_0, 5 = Q5_K, 6 = Q6_K, operands as in
  * mi_gemv_q4_0 / _q8_0 / _q5k / _q6k; qh / qmin null where the format has none), fp16 activations;
  * K % 128 == 0 (Q5_K / Q6_K: % 512), x and the weights' N x K below 2 Gi (bytes / elements).
- * workspace: mi_gemm_tiled_workspace bytes. */
+ * workspace: mi_gemm_tiled_workspace bytes.
+ * mi_gemm_gguf_tiled_pays: *pays = 1 where a linear layer of these formats (fmt 2: Q4_K) takes the tiled GEMM; the torch
+ * ops ask it.  Elsewhere the weight-streaming entries are ahead, or the sizes are theirs alone. */
+int mi_gemm_gguf_tiled_pays(int fmt, int M, int N, int K, int* pays);
 int mi_gemm_gguf_tiled_ws(int fmt, const void* x, const void* w, const void* qh, const void* scale, const void* qmin,
                           void* out, void* workspace, long long workspace_bytes, int M, int N, int K, void* stream);
 

@@ -12,11 +12,39 @@ template <class Act, int BN> using WQ80 = WGguf<Act, BN, GT_Q80>;
 template <class Act, int BN> using WQ5K = WGguf<Act, BN, GT_Q5K>;
 template <class Act, int BN> using WQ6K = WGguf<Act, BN, GT_Q6K>;
 
+// 65 .. 128 rows: up to which K two passes of the weight-streaming kernels are ahead.  They are at their best where the
+// weight gives a CU one 16-row block or a little less or more, and on short rows, which the tiles' pipeline does not
+// amortise; the K-sliced kernel takes Q4_0 and Q8_0 further than the others.  Streaming / tiled in us (M x N x K):
+// Q6_K 112 x 4096 x 1024 10.9 / 16.2, 112 x 3072 x 2560 16.6 / 19.3, 112 x 1024 x 2048 13.5 / 12.9, 80 x 10240 x 1024 20.6 / 16.0,
+// 80 x 1024 x 1024 12.8 / 11.0, 128 x 1048 x 1024 10.9 / 13.0; Q8_0 80 x 4096 x 3072 15.2 / 19.2, 128 x 1024 x 3072 17.1 / 13.1;
+// Q4_0 80 x 4096 x 4096 17.8 / 19.7, 128 x 1024 x 4096 20.7 / 14.0.  Over 1512 problems (N 256 .. 10240, K 512 .. 4096) 66 that take the
+// tiles are slower there by more than 3 %, at most 1.17 times.
+static int stream_k(int fmt, long M, long N) {
+  const long cus = device_cu_count_gemm();
+  const bool one_block = N >= 8 * cus && N <= 20 * cus;
+  if (fmt == GT_Q40) return one_block && M <= 96 ? 4096 : 3072;
+  if (fmt == GT_Q80) return one_block ? 3072 : 2048;
+  if (one_block) return M <= 96 ? 2560 : 3072;
+  if (M <= 96 || N > 24 * cus) return 0;
+  return N < 8 * cus ? 1024 : 1536;
+}
+
 }  // namespace qlin
 
 using namespace qlin;
 
 extern "C" {
+
+int mi_gemm_gguf_tiled_pays(int fmt, int M, int N, int K, int* pays) {
+  if (!pays || fmt < 2 || fmt > GT_Q6K) return MI_ERR_ARG;
+  if (M < 0 || N < 0 || K <= 0) return MI_ERR_SHAPE;
+  *pays = M > 64 && N && K % 128 == 0;
+  if (fmt == 2) return MI_OK;
+  if ((uint64_t)(M + 15) * (uint64_t)K * 2 >= (1ull << 31) || (uint64_t)N * (uint64_t)K >= (1ull << 31)) *pays = 0;
+  if ((fmt == GT_Q5K || fmt == GT_Q6K) && K % 512) *pays = 0;
+  if (M <= 128 && K <= stream_k(fmt, M, N)) *pays = 0;
+  return MI_OK;
+}
 
 int mi_gemm_gguf_tiled_ws(int fmt, const void* x, const void* w, const void* qh, const void* scale, const void* qmin,
                           void* out, void* workspace, long long workspace_bytes, int M, int N, int K, void* stream) {

@@ -242,16 +242,12 @@ Tensor esimd_gemm_int4_pgrp_zp(const Tensor& x, const Tensor& w, const Tensor& s
 }
 
 // ---------------------------------------------------------------------------------------- GGUF
-enum Gguf { kQ4K = 2, kQ40 = 3, kQ80 = 4, kQ5K = 5, kQ6K = 6 };   // the format numbers of mi_gemm_gguf_tiled_ws, and Q4_K's
+enum Gguf { kQ4K = 2, kQ40 = 3, kQ80 = 4, kQ5K = 5, kQ6K = 6 };   // the format numbers of mi_gemm_gguf_tiled_pays
 
-// Rows up to which the weight-streaming kernels keep the call: 64, and 128 for Q4_0 / Q8_0 with K within the K-sliced
-// kernel's reach, which covers them in two passes (Q4_0 128 x 1024 x 12000: 14 against 17 us tiled; 66 x 5120 x 1024:
-// 22 against 14; Q8_0 100 x 1024 x 1024: 10 against 11, 80 x 4096 x 4096: 24 against 21).
 bool gguf_tiled(int fmt, const Linear& l) {
-  if (!l.prefill()) return false;
-  if (fmt == kQ4K) return true;
-  if (l.M <= 128 && l.K <= (fmt == kQ40 ? 3072 : fmt == kQ80 ? 2048 : 0)) return false;
-  return ((int64_t)l.M + 15) * l.K * 2 < (1LL << 31) && (int64_t)l.N[0] * l.K < (1LL << 31);
+  int pays = 0;
+  CALL(mi_gemm_gguf_tiled_pays, fmt, l.M, l.N[0], l.K, &pays);
+  return pays;
 }
 bool gguf_linear(int fmt, const Tensor& x, const Tensor& w, const Tensor* qh, const Tensor& s, const Tensor* mn, const Tensor& o) {
   if (w.dim() != 2 || !plain(x, {&w, &s, &o}) || (qh && !plain(x, {qh})) || (mn && !plain(x, {mn}))) return false;

@@ -409,15 +409,15 @@ def _chk_f16(t, numel, nm, who):
          f"{who}: {nm} must be contiguous fp16 with {numel} elements")
 
 
+def _gguf_pays(fmt, M, N, K):
+    pays = ctypes.c_int(0)
+    rc = capi.lib().mi_gemm_gguf_tiled_pays(fmt, M, N, K, ctypes.byref(pays))
+    return rc == 0 and bool(pays.value)
+
+
 def _gguf_tiled(fmt, x, w, qh, scale, qmin, out, M, N, K):
-    """The prefill route of these formats; False where the weight-streaming kernels take the call: K that does not fill
-    the tiles' K steps, operands beyond the 2 Gi that the tiled kernel addresses, or up to 128 rows of Q4_0 and Q8_0 with K
-    within the K-sliced kernel's reach, which covers them in two passes (Q4_0 128 x 1024 x 12000: 14 against 17 us, 66 x
-    5120 x 1024: 22 against 14; Q8_0 100 x 1024 x 1024: 10 against 11, 80 x 4096 x 4096: 24 against 21; Q6_K 120 x 5120 x
-    12288: 74 against 52)."""
-    if M <= 128 and K <= {3: 3072, 4: 2048}.get(fmt, 0):
-        return False
-    if not _prefill_route(M, K) or (M + 15) * K * 2 >= 1 << 31 or N * K >= 1 << 31 or N == 0:
+    """The tiled prefill route of these formats; False where the weight-streaming kernels take the call."""
+    if not _gguf_pays(fmt, M, N, K):
         return False
     buf, nbytes = _tiled_workspace(x, M, [N], K)
     capi.call("mi_gemm_gguf_tiled_ws", x, fmt, capi.ptr(x), capi.ptr(w), capi.ptr(qh), capi.ptr(scale), capi.ptr(qmin),

@@ -90,6 +90,32 @@ def test_k_is_split_where_it_was_measured_faster(M, N, K, split):
     assert (need.value > one.value) == split and need.value >= one.value
 
 
+def test_rows_beyond_64_of_gguf_weights_take_the_measured_route():
+    """mi_gemm_gguf_tiled_pays: one rule for both host paths; either side of its lines, and sizes it does not take."""
+    lib = capi.lib()
+
+    def pays(fmt, M, N, K):
+        p = ctypes.c_int(-1)
+        rc = lib.mi_gemm_gguf_tiled_pays(fmt, M, N, K, ctypes.byref(p))
+        return p.value if rc == 0 else rc
+    q4k, q40, q80, q5k, q6k = 2, 3, 4, 5, 6
+    for fmt in (q40, q80, q5k, q6k):
+        assert pays(fmt, 64, 14336, 14336) == 0 and pays(fmt, 129, 4096, 1024) == 1 and pays(fmt, 65, 10240, 14336) == 1
+        assert pays(fmt, 200, 4096, 96) == 0 and pays(fmt, 200, 1 << 20, 4096) == 0 and pays(fmt, 1 << 20, 256, 4096) == 0
+        assert pays(fmt, 200, 0, 4096) == 0
+    assert pays(q4k, 65, 4096, 1024) == 1 and pays(q4k, 64, 4096, 1024) == 0 and pays(q4k, 65, 4096, 1056) == 0
+    assert pays(q40, 128, 1024, 3072) == 0 and pays(q40, 128, 1024, 3200) == 1
+    assert pays(q40, 96, 4096, 4096) == 0 and pays(q40, 97, 4096, 4096) == 1
+    assert pays(q80, 128, 1024, 2048) == 0 and pays(q80, 128, 1024, 2176) == 1
+    assert pays(q80, 80, 4096, 3072) == 0 and pays(q80, 80, 4096, 3200) == 1
+    for fmt in (q5k, q6k):
+        assert pays(fmt, 96, 4096, 2560) == 0 and pays(fmt, 96, 4096, 3072) == 1 and pays(fmt, 97, 4096, 3072) == 0
+        assert pays(fmt, 97, 1024, 1024) == 0 and pays(fmt, 96, 1024, 1024) == 1 and pays(fmt, 112, 1024, 1536) == 1
+        assert pays(fmt, 128, 6144, 1536) == 0 and pays(fmt, 128, 6152, 1536) == 1 and pays(fmt, 200, 512, 1152) == 0
+    assert pays(7, 200, 512, 512) == -1 and pays(1, 200, 512, 512) == -1 and pays(q80, 1, 1, 0) == -2
+    assert lib.mi_gemm_gguf_tiled_pays(q80, 200, 512, 512, None) == -1
+
+
 def test_merged_chunks_argument_errors():
     """The tiled entry refuses what the chunk kernel refuses, whichever of the two a call would take."""
     lib = capi.lib()

@@ -122,6 +122,27 @@ def test_a_strided_scale_is_read_with_its_stride(dev, M):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name,M,N,K,tiled", [
+    ("esimd_gemm_q4_0", 70, 264, 3072, False), ("esimd_gemm_q4_0", 70, 264, 3200, True),
+    ("esimd_gemv_q8_0_m", 70, 264, 2048, False), ("esimd_gemv_q8_0_m", 70, 264, 2176, True),
+    ("esimd_gemv_q5_k", 97, 264, 1024, False), ("esimd_gemv_q5_k", 96, 264, 1024, True),
+    ("esimd_gemv_q6_k_m", 97, 2056, 3072, False), ("esimd_gemv_q6_k_m", 96, 2056, 3072, True)])
+def test_both_host_paths_take_the_same_route(dev, monkeypatch, name, M, N, K, tiled):
+    """Either side of the lines between streaming and tiled kernels (their sums differ in order, so equal bits are
+    the same route), and the route is the expected one."""
+    torch.manual_seed(K)
+    args, at = _args(name, M, K, N, torch.float16)
+    other = list(args)
+    other[at] = torch.empty_like(args[at])
+    _own(name)(*args)
+    inner, entries = _ops.capi.call, []
+    monkeypatch.setattr(_ops.capi, "call", lambda entry, *a: entries.append(entry) or inner(entry, *a))
+    getattr(torch.ops.mi355x_checked, name)(*other)
+    assert torch.equal(args[at], other[at])
+    assert (entries == ["mi_gemm_gguf_tiled_ws"]) == tiled and len(entries) == 1
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 3, 12, 13])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 def test_moe_decode_is_the_same(dev, T, dt):
