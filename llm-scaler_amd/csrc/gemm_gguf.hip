@@ -17,15 +17,15 @@ template <class Act, int BN> using WQ6K = WGguf<Act, BN, GT_Q6K>;
 // amortise; the K-sliced kernel takes Q4_0 and Q8_0 further than the others.  Streaming / tiled in us (M x N x K):
 // Q6_K 112 x 4096 x 1024 10.9 / 16.2, 112 x 3072 x 2560 16.6 / 19.3, 112 x 1024 x 2048 13.5 / 12.9, 80 x 10240 x 1024 20.6 / 16.0,
 // 80 x 1024 x 1024 12.8 / 11.0, 128 x 1048 x 1024 10.9 / 13.0; Q8_0 80 x 4096 x 3072 15.2 / 19.2, 128 x 1024 x 3072 17.1 / 13.1;
-// Q4_0 80 x 4096 x 4096 17.8 / 19.7, 128 x 1024 x 4096 20.7 / 14.0.  Over 1512 problems (N 256 .. 10240, K 512 .. 4096) 66 that take the
-// tiles are slower there by more than 3 %, at most 1.17 times.
+// Q4_0 80 x 4096 x 4096 17.8 / 19.7, 128 x 1024 x 4096 20.7 / 14.0.  Over 3780 problems (N 256 .. 10240, K 512 .. 4096) 156 that take the
+// tiles are slower there by more than 3 %, at most 1.2 times; with everything on the tiles beyond Q4_0's 3072 and Q8_0's 2048, 634, at most 1.49.
 static int stream_k(int fmt, long M, long N) {
   const long cus = device_cu_count_gemm();
-  const bool one_block = N >= 8 * cus && N <= 20 * cus;
+  const bool one_block = N >= 8 * cus && N <= 16 * cus;
   if (fmt == GT_Q40) return one_block && M <= 96 ? 4096 : 3072;
   if (fmt == GT_Q80) return one_block ? 3072 : 2048;
   if (one_block) return M <= 96 ? 2560 : 3072;
-  if (M <= 96 || N > 24 * cus) return 0;
+  if (M <= 96 || N > 32 * cus) return 0;
   return N < 8 * cus ? 1024 : 1536;
 }
 

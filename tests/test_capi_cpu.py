@@ -107,11 +107,11 @@ def test_rows_beyond_64_of_gguf_weights_take_the_measured_route():
     assert pays(q40, 128, 1024, 3072) == 0 and pays(q40, 128, 1024, 3200) == 1
     assert pays(q40, 96, 4096, 4096) == 0 and pays(q40, 97, 4096, 4096) == 1
     assert pays(q80, 128, 1024, 2048) == 0 and pays(q80, 128, 1024, 2176) == 1
-    assert pays(q80, 80, 4096, 3072) == 0 and pays(q80, 80, 4096, 3200) == 1
+    assert pays(q80, 80, 4096, 3072) == 0 and pays(q80, 80, 4104, 3072) == 1 and pays(q80, 80, 4096, 3200) == 1
     for fmt in (q5k, q6k):
         assert pays(fmt, 96, 4096, 2560) == 0 and pays(fmt, 96, 4096, 3072) == 1 and pays(fmt, 97, 4096, 3072) == 0
         assert pays(fmt, 97, 1024, 1024) == 0 and pays(fmt, 96, 1024, 1024) == 1 and pays(fmt, 112, 1024, 1536) == 1
-        assert pays(fmt, 128, 6144, 1536) == 0 and pays(fmt, 128, 6152, 1536) == 1 and pays(fmt, 200, 512, 1152) == 0
+        assert pays(fmt, 128, 8192, 1536) == 0 and pays(fmt, 128, 8200, 1536) == 1 and pays(fmt, 200, 512, 1152) == 0
     assert pays(7, 200, 512, 512) == -1 and pays(1, 200, 512, 512) == -1 and pays(q80, 1, 1, 0) == -2
     assert lib.mi_gemm_gguf_tiled_pays(q80, 200, 512, 512, None) == -1
 
