@@ -132,7 +132,7 @@ static int launch_chunk_gemm(GemmArgs p, int nmat, int max_tiles, hipStream_t st
 // Time in us.  Tiled: tables and re-tiling, then a chain of K / 64 steps per round of one workgroup per CU, and the
 // multiplications of the live rows.  Chunks: a chain of K steps, and a part per chunk and per 64 rows for every million
 // weights.  Fitted on 1300 launches (1 .. 256 experts, H 1024 .. 6144, I 256 .. 2048, 8 .. 1024 rows per expert; even, drawn
-// and skewed counts): nine in ten within 25 %, so the tiled kernel has to promise 5 %.  Both sides, chunks / tiled in us: E = 8,
+// and skewed counts): nine in ten within 25 %, so the tiled kernel has to promise 5 % (down: 2 %).  Both sides, chunks / tiled in us: E = 8,
 // H = 1024, I = 512, 128 rows per expert, up 20 / 41; E = 16, H = 2048, I = 768, 96 rows 37 / 53; E = 128, same sizes, 60 even
 // rows 123 / 153, 96 rows 226 / 180, 256 rows 517 / 407; E = 256, H = 2048, I = 512, 60 rows 184 / 223, 96 rows 299 / 274.
 static bool chunk_tiles_pay(bool up, long long n, long long out_rows, long long E, long long N, long long K, long long nmat) {
@@ -145,7 +145,7 @@ static bool chunk_tiles_pay(bool up, long long n, long long out_rows, long long 
   const double tiled = up ? 17.0 + steps * (0.97 * rounds + 1.64 * full) : 18.0 + steps * (1.11 * rounds + 2.16 * full);
   const double chunks = up ? 7.0 + 0.41 * steps + weights * (0.12 * (double)n + 0.18 * r64)
                            : 9.0 + 0.41 * steps + weights * (0.21 * (double)n + 0.18 * r64);
-  return tiled < 0.95 * chunks;
+  return tiled < (up ? 0.95 : 0.98) * chunks;
 }
 
 }  // namespace qlin
