@@ -258,7 +258,7 @@ def test_one_hot_activations_return_the_dequantized_weights(ops, dev, kind, M, K
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("M,N,K", [(129, 8, 512),                 # 128 x 128 tiles, a last row tile of one row
                                    (144, 257, 1024),              # odd N: element-wise stores
-                                   (300, 9000, 512),              # 256-row tiles
+                                   (300, 9000, 512),              # 128 x 128 tiles, more than fit one round of 96 columns
                                    (130, 72, 1536),               # three high-bit tiles of 512
                                    (140, 64, 640), (131, 40, 96)])  # Q4_0 / Q8_0 only: K % 128 == 0 (tiled), K % 32 == 0 (streaming)
 def test_prefill_one_hot_rows_return_the_dequantized_weights(ops, dev, kind, M, N, K):

@@ -5,6 +5,9 @@ import ctypes
 import pytest
 import torch
 
+from oracle import qlinear_oracle as O
+from test_gpu_gguf import TOL, _down_stack, _q4k_expert_stacks
+
 pytestmark = pytest.mark.gpu
 
 
@@ -105,3 +108,77 @@ def test_which_kernel_the_module_takes(dev, monkeypatch, rows, E, per, n_list, w
     names = _record(monkeypatch)
     mg.moe_up_q4k_ggemv(x, *gate, *up, torch.zeros(rows, 2 * I, dtype=torch.float16, device=dev), chunks, H, I)
     assert names == [want]
+
+
+def _sorted_rows(counts):
+    """Chunk list of experts with `counts` rows each, and the expert of every row."""
+    chunks, of, at = [], [], 0
+    for e, n in enumerate(counts):
+        chunks += [[e, at + t, min(64, n - t)] for t in range(0, n, 64)]
+        of += [e] * n
+        at += n
+    return torch.tensor(chunks, dtype=torch.int32), torch.tensor(of)
+
+
+@pytest.mark.parametrize("kind", ["q4_k", "q5_k", "q6_k"])
+def test_module_on_merged_chunks_against_the_oracle(dev, monkeypatch, kind):
+    """The module's own call of the tiled route (operands, workspace, decoding of the stacks): one-hot rows return the
+    experts' dequantized weights value for value, random rows agree with the oracle's product.  One expert ends in a full
+    tile, one in a tile of 1 row, one has no rows, and the last rows of the buffer belong to no chunk."""
+    from custom_esimd_kernels_sglang import moe_grouped_gguf_xpu as mg
+    E, K, N = 4, 384, 1536
+    counts = (2048, 0, 1793, 2200)
+    chunks, of = _sorted_rows(counts)
+    rows, total = len(of), len(of) + 40
+    g = torch.Generator().manual_seed(3)
+    if kind == "q4_k":
+        tokens = 900
+        ids = torch.randint(0, tokens, (total,), generator=g).to(torch.int32)
+        reps, deq = _q4k_expert_stacks(E, N, K, (71, 72), torch.arange(E), dev)
+        run = lambda x, out: mg.moe_up_q4k_ggemv(x, *reps[0], *reps[1], out, chunks.to(dev), K, N, ids.to(dev))
+        weights = torch.cat(deq, 1)                       # [E, 2 N, K]
+    else:
+        tokens, ids = total, torch.arange(total)
+        stack, weights = _down_stack(kind, E, N, K, 73, torch.arange(E), dev)
+        fn = mg.moe_down_q5k_ggemv if kind == "q5_k" else mg.moe_down_q6k_ggemv
+        run = lambda x, out: fn(x, *stack, out, chunks.to(dev), K, N)
+    names = _record(monkeypatch)
+    hot = torch.zeros(tokens, K, dtype=torch.float16)
+    ks = (3 + 37 * torch.arange(tokens)) % K
+    hot[torch.arange(tokens), ks] = 1.0
+    out = torch.full((total, weights.shape[1]), 7.0, dtype=torch.float16, device=dev)
+    run(hot.to(dev), out)
+    got = out.cpu().float()
+    assert torch.equal(got[:rows], weights[of, :, ks[ids[:rows].long()]]) and bool((got[rows:] == 7.0).all())
+    x = (torch.randn(tokens, K, generator=g) * 0.1).half()
+    run(x.to(dev), out)
+    xs = x.float()[ids[:rows].long()]
+    want = torch.cat([xs[of == e] @ weights[e].t() for e in range(E)])
+    assert O.max_rel_err(out.cpu()[:rows], want) < TOL
+    assert names == ["mi_moe_gguf_grouped_tiled_ws"] * 2
+    # in a graph: the same bits on every replay
+    eager, stream, graph = out.clone(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    xd, cd, idd = x.to(dev), chunks.to(dev), ids.to(dev)
+    if kind == "q4_k":
+        again = lambda: mg.moe_up_q4k_ggemv(xd, *reps[0], *reps[1], out, cd, K, N, idd)
+    else:
+        again = lambda: fn(xd, *stack, out, cd, K, N)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream), torch.cuda.graph(graph, stream=stream):
+        again()
+    for _ in range(3):
+        out[:rows].fill_(float("nan"))
+        junk = torch.randn(256, 256, device=dev) @ torch.randn(256, 256, device=dev)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        del junk
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16))
+    # activations that are not 16-byte aligned stay on the chunk kernel
+    del names[:]
+    shifted = torch.empty(tokens * K + 4, dtype=torch.float16, device=dev)[4:].view(tokens, K)
+    shifted.copy_(xd)
+    assert shifted.data_ptr() % 16 == 8
+    run(shifted, out)
+    assert names == ["mi_moe_gguf_grouped"]
+    assert O.max_rel_err(out.cpu()[:rows], want) < TOL
