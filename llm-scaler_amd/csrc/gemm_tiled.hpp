@@ -428,8 +428,8 @@ struct WGguf {
         q.o |= q.h1;
       } else if (!kPlainH && part == 1) {
         if constexpr (!kPlainH) {
-        q.h0 = st.h[i][dw >> 1][(dw & 1) * 2] >> st.sh & kField;         // elements 0 1 2 3 of the dword's 8
-        q.h1 = st.h[i][dw >> 1][(dw & 1) * 2 + 1] >> st.sh & kField;     // elements 4 5 6 7
+          q.h0 = st.h[i][dw >> 1][(dw & 1) * 2] >> st.sh & kField;         // elements 0 1 2 3 of the dword's 8
+          q.h1 = st.h[i][dw >> 1][(dw & 1) * 2 + 1] >> st.sh & kField;     // elements 4 5 6 7
         }
       } else if (part == 2) {
         const uint32_t he = __builtin_amdgcn_perm(q.h1, q.h0, 0x06040200u);
