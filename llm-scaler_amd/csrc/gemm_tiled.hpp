@@ -2,8 +2,9 @@
 // fp16 / bf16 activations, templated on the weight format (INT4 group 128, FP8 E4M3 with
 // per-channel / per-tensor / 128x128 block scales, GGUF Q4_K in its repacked representation).
 //
-// MFMA-bound regime (M in the hundreds or thousands).  A workgroup of 4 wavefronts (2 x 2)
-// owns a BM x BN output tile; each wavefront computes a (BM/2) x (BN/2) sub-tile with
+// MFMA-bound regime (M in the hundreds or thousands).  A workgroup of 4 wavefronts (2 x 2; 4 x 1 on
+// the tall, narrow tiles of problems that do not fill the chip otherwise, see gemm_small_tile)
+// owns a BM x BN output tile; each wavefront computes a sub-tile of it with
 // v_mfma_f32_16x16x32_{bf16,f16}, accumulators in the AGPR half of the register file.  What
 // limits this kernel is LDS bandwidth (a CU sustains about 130 B/ns of ds_read_b128 and
 // 75 B/ns of LDS writes, against ~1 us of MFMA work per 64-wide K step), so only the operand
@@ -97,6 +98,12 @@ __device__ __forceinline__ f16x2 nibbles_f16(uint32_t bytes, bool high) {
 __device__ __forceinline__ f16x2 planted_f16(uint32_t bytes, bool high) {
   return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, bytes, high ? 0x04030402u : 0x04010400u));
 }
+template <int DW> using Dwords = std::conditional_t<DW == 4, u32x4, u32x2>;
+template <int DW>
+__device__ __forceinline__ void load_dwords(Dwords<DW>& v, const __amdgpu_buffer_rsrc_t& r, uint32_t off, uint32_t soff) {
+  if constexpr (DW == 4) v = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0);
+  else v = __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0);
+}
 __device__ __forceinline__ f16x2 both(float v) { return f16x2{(_Float16)v, (_Float16)v}; }
 __device__ __forceinline__ f16x2 both_bits(uint32_t v) { return __builtin_bit_cast(f16x2, (v & 0xffffu) * 0x10001u); }
 __device__ __forceinline__ uint32_t bits(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
@@ -112,11 +119,13 @@ __device__ __forceinline__ uint32_t bits(f16x2 v) { return __builtin_bit_cast(ui
 // rounded once; the pairs are (0 2)(1 3)(4 6)(5 7) of a dword's 8 nibbles, and x is re-tiled in that order.
 template <class Act, int BN>
 struct WInt4 {
-  static constexpr int CPR = 2;                       // chunks per row and 64-wide step
+  static constexpr int CPR = BN <= 64 ? 4 : 2;        // chunks per row and 64-wide step: 8 bytes each on narrow tiles,
+  static constexpr int DW = 8 / CPR;                  // so that every thread has one; dwords per chunk
   static constexpr double kWeightBytesPerK = 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256; // chunks per thread
   static constexpr int LPC = 3;                       // load instructions per chunk
-  static constexpr int kPieces = B_CH * 4 * 8;        // 8 pieces per packed dword of 8 nibbles
+  static constexpr int kPieces = B_CH * DW * 8;        // 8 pieces per packed dword of 8 nibbles
+  static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
   static constexpr bool kOutScale = false;
   static constexpr bool kHalf = Act::dt == DT_F16;
   static constexpr bool kPermK = kHalf;
@@ -126,7 +135,7 @@ struct WInt4 {
     int Kg;
   };
   struct Stage {
-    u32x4 b[B_CH];
+    Dwords<DW> b[B_CH];
     uint32_t s[B_CH], z[B_CH];                        // fp16 scale bits, zero-point: 32-bit slots, one register each
   };
   struct Dq {
@@ -147,7 +156,7 @@ struct WInt4 {
   }
   // byte offset of chunk kc of row n at k = 0, and the row's first side-table entry
   static __device__ __forceinline__ void chunk_addr(Res& r, int, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
-    boff = (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * 16);
+    boff = (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * DW * 4);
     soff = (uint32_t)n * (uint32_t)r.Kg;              // in groups; x2 for the fp16 scale
   }
   static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
@@ -155,7 +164,7 @@ struct WInt4 {
     const uint32_t k0 = (uint32_t)kt * kBK;
     const int i = idx / 3, kind = idx % 3;
     if (kind == 0)
-      st.b[i] = __builtin_amdgcn_raw_buffer_load_b128(r.wr, boff[i] | dead, k0 >> 1, 0);
+      load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, k0 >> 1);
     else if (kind == 1)
       st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, ((soff[i] & 0x7fffffffu) * 2u) | (soff[i] & 0x80000000u) | dead,
                                                      (k0 >> 7) * 2u, 0);
@@ -188,7 +197,7 @@ struct WInt4 {
   // piece I of the stage; dst[i] = LDS address of chunk i's 64 output bytes in the target buffer
   static __device__ __forceinline__ void piece(const Stage& st, Dq& q, int I, unsigned char* const (&dst)[B_CH]) {
     const int dword = I >> 3, part = I & 7;
-    const int i = dword / 4, dw = dword % 4;
+    const int i = dword / DW, dw = dword % DW;
     auto pair = [&](float a, float b) {
       return pack2(__builtin_fmaf(a, q.sf[i], q.nzs[i]), __builtin_fmaf(b, q.sf[i], q.nzs[i]));
     };
@@ -227,12 +236,14 @@ struct WInt4 {
 template <class Act, int BN>
 struct WQ4K {
   static_assert(Act::dt == DT_F16, "Q4_K runs in fp16");
-  static constexpr int CPR = 2;
+  static constexpr int CPR = BN <= 64 ? 4 : 2;        // chunks per row and 64-wide step: 8 bytes each on narrow tiles,
+  static constexpr int DW = 8 / CPR;                  // so that every thread has one; dwords per chunk
   static constexpr double kWeightBytesPerK = 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
   static constexpr int LPC = 3;
   static constexpr int PPD = 8;                       // pieces per dword of 8 nibbles
-  static constexpr int kPieces = B_CH * 4 * PPD;
+  static constexpr int kPieces = B_CH * DW * PPD;
+  static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
   static constexpr bool kOutScale = false;
   static constexpr bool kPermK = true;
   struct Res {
@@ -240,7 +251,7 @@ struct WQ4K {
     int Kc;
   };
   struct Stage {
-    u32x4 b[B_CH];
+    Dwords<DW> b[B_CH];
     uint32_t s[B_CH], m[B_CH];                        // fp16 bits (32-bit slots: 16-bit members end up on the stack)
   };
   struct Dq {
@@ -258,14 +269,14 @@ struct WQ4K {
     return r;
   }
   static __device__ __forceinline__ void chunk_addr(Res& r, int, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
-    boff = (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * 16);
-    soff = ((uint32_t)n * (uint32_t)r.Kc + (uint32_t)kc) * 2u;   // bytes: one fp16 per 32 k
+    boff = (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * DW * 4);
+    soff = ((uint32_t)n * (uint32_t)r.Kc + (uint32_t)(DW == 2 ? kc >> 1 : kc)) * 2u;   // bytes: one fp16 per 32 k
   }
   static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
                                                const uint32_t (&soff)[B_CH], int kt, uint32_t dead, int idx) {
     const uint32_t k0 = (uint32_t)kt * kBK;
     const int i = idx / 3, kind = idx % 3;
-    if (kind == 0) st.b[i] = __builtin_amdgcn_raw_buffer_load_b128(r.wr, boff[i] | dead, k0 >> 1, 0);
+    if (kind == 0) load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, k0 >> 1);
     else if (kind == 1) st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, (k0 >> 5) * 2u, 0);
     else st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, (k0 >> 5) * 2u, 0);
   }
@@ -279,7 +290,7 @@ struct WQ4K {
   static __device__ __forceinline__ void piece(const Stage& st, Dq& q, int I, unsigned char* const (&dst)[B_CH]) {
 #pragma clang fp contract(off)
     const int dword = I / PPD, part = I % PPD;
-    const int i = dword / 4, dw = dword % 4;
+    const int i = dword / DW, dw = dword % DW;
     if (part == 0) {
       const uint32_t w = st.b[i][dw];
       q.e = w & 0x0F0F0F0Fu;
@@ -314,12 +325,15 @@ struct WGguf {
   static constexpr bool kPlainH = FMT == GT_Q5P || FMT == GT_Q6P;
   static_assert(Act::dt == DT_F16, "GGUF formats run in fp16");
   static constexpr bool kHigh = F == GT_Q5K || F == GT_Q6K;
-  static constexpr int CPR = F == GT_Q80 ? 4 : 2;
+  static constexpr int CPR = F == GT_Q80 || BN <= 64 ? 4 : 2;
+  static constexpr int DW = F == GT_Q80 ? 4 : 8 / CPR;   // dwords per chunk (nibbles: 8 bytes on narrow tiles, as INT4)
+  static_assert(!kPlainH || DW == 4, "high bits in element order: whole chunks of 32");
   static constexpr double kWeightBytesPerK = F == GT_Q80 ? 1.0 : F == GT_Q6K ? 0.75 : F == GT_Q5K ? 0.625 : 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
-  static constexpr int LPC = (F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2) - (kPlainH ? 1 : 0);
+  static constexpr int LPC = (F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2) - (kPlainH || (kHigh && DW == 2) ? 1 : 0);
   static constexpr int PPD = F == GT_Q5K ? 13 : F == GT_Q6K ? 9 : F == GT_Q40 ? 8 : 3;   // pieces per dword (8 nibbles / 4 bytes)
-  static constexpr int kPieces = B_CH * 4 * PPD;
+  static constexpr int kPieces = B_CH * DW * PPD;
+  static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
   static constexpr bool kOutScale = false;
   static constexpr bool kPermK = F != GT_Q80;            // pairs (0 2)(1 3)(4 6)(5 7); Q8_0 in order
   struct Res {
@@ -328,10 +342,10 @@ struct WGguf {
     uint32_t hoff[kHigh ? B_CH : 1];
   };
   struct Stage {
-    u32x4 b[B_CH];
+    Dwords<DW> b[B_CH];
     uint32_t s[B_CH];
     uint32_t m[F == GT_Q5K ? B_CH : 1];
-    u32x4 h[kHigh && !kPlainH ? B_CH : 1][2];
+    u32x4 h[kHigh && !kPlainH ? B_CH : 1][DW / 2];
     u32x2 hp[kPlainH ? B_CH : 1];
     uint32_t sh;                                      // shift of this step's field of the high-bit bytes (uniform)
   };
@@ -339,7 +353,7 @@ struct WGguf {
     uint32_t e, o, h0, h1;
     f16x2 te, to;
     u32x4 outv;
-    f16x2 sv[B_CH][F == GT_Q6K ? 2 : 1], mv[F == GT_Q5K ? B_CH : 1];
+    f16x2 sv[B_CH][F == GT_Q6K ? DW / 2 : 1], mv[F == GT_Q5K ? B_CH : 1];
   };
   static __device__ __forceinline__ Res make(const GemmArgs& p, int e = 0) {
     Res r;
@@ -352,19 +366,19 @@ struct WGguf {
     return r;
   }
   static __device__ __forceinline__ void chunk_addr(Res& r, int i, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
-    boff = (uint32_t)n * (F == GT_Q80 ? (uint32_t)K : (uint32_t)K >> 1) + (uint32_t)(kc * 16);
-    soff = (uint32_t)n * (uint32_t)r.Ks + (uint32_t)(F == GT_Q80 ? (kc >> 1) * 2 : F == GT_Q6K ? kc * 4 : kc * 2);
+    boff = (uint32_t)n * (F == GT_Q80 ? (uint32_t)K : (uint32_t)K >> 1) + (uint32_t)(kc * DW * 4);
+    soff = (uint32_t)n * (uint32_t)r.Ks + (uint32_t)(F == GT_Q6K ? kc * DW : (CPR == 4 ? kc >> 1 : kc) * 2);
     if constexpr (kHigh) r.hoff[i] = (uint32_t)n * (F == GT_Q6K ? (uint32_t)K >> 2 : (uint32_t)K >> 3) +
-                                     (uint32_t)(kc * (!kPlainH ? 32 : F == GT_Q6K ? 8 : 4));
+                                     (uint32_t)(kc * (!kPlainH ? DW * 8 : F == GT_Q6K ? 8 : 4));
   }
   static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
                                                const uint32_t (&soff)[B_CH], int kt, uint32_t dead, int idx) {
     const uint32_t k0 = (uint32_t)kt * kBK;
     const int i = idx / LPC, kind = idx % LPC;
-    if (kind == 0) st.b[i] = __builtin_amdgcn_raw_buffer_load_b128(r.wr, boff[i] | dead, F == GT_Q80 ? k0 : k0 >> 1, 0);
+    if (kind == 0) load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, F == GT_Q80 ? k0 : k0 >> 1);
     else if (kind == 1) {
-      if constexpr (F == GT_Q6K) st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, k0 >> 3, 0);
-      else st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, k0 >> 4, 0);
+      if constexpr (F == GT_Q6K && DW == 4) st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, k0 >> 3, 0);
+      else st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, F == GT_Q6K ? k0 >> 3 : k0 >> 4, 0);
     } else if (kPlainH && kind == 2) {
       if constexpr (kPlainH && F == GT_Q6K) st.hp[i] = __builtin_amdgcn_raw_buffer_load_b64(r.hr, r.hoff[i] | dead, k0 >> 2, 0);
       else if constexpr (kPlainH) st.hp[i][0] = __builtin_amdgcn_raw_buffer_load_b32(r.hr, r.hoff[i] | dead, k0 >> 3, 0);
@@ -380,14 +394,14 @@ struct WGguf {
 #pragma unroll
     for (int i = 0; i < B_CH; ++i) {
       q.sv[i][0] = both_bits(st.s[i]);
-      if constexpr (F == GT_Q6K) q.sv[i][1] = both_bits(st.s[i] >> 16);
+      if constexpr (F == GT_Q6K && DW == 4) q.sv[i][1] = both_bits(st.s[i] >> 16);
       if constexpr (F == GT_Q5K) q.mv[i] = both_bits(st.m[i]);
     }
   }
   static __device__ __forceinline__ void piece(const Stage& st, Dq& q, int I, unsigned char* const (&dst)[B_CH]) {
 #pragma clang fp contract(off)
     const int dword = I / PPD, part = I % PPD;
-    const int i = dword / 4, dw = dword % 4;
+    const int i = dword / DW, dw = dword % DW;
     const uint32_t w = st.b[i][dw];
     if constexpr (F == GT_Q40) {
       const f16x2 s = q.sv[i][0], m8 = both(-8.0f);
@@ -465,6 +479,7 @@ struct WFp8 {
   static constexpr int LPC = BLOCK ? 2 : 1;
   static constexpr int kPPC = BLOCK ? 10 : 4;         // pieces per chunk
   static constexpr int kPieces = B_CH * kPPC;
+  static constexpr bool kCheapDecode = !BLOCK;
   static constexpr bool kOutScale = !BLOCK;
   static constexpr bool kPermK = false;
   struct Res {
@@ -559,10 +574,11 @@ __device__ __forceinline__ void fold_pieces(std::integer_sequence<int, I...>, F 
 // epilogue writes act(gate) * up (N / 2 output columns).
 // SPLIT: blockIdx.y takes one slice of K and the fp32 sums go to a workspace in accumulator order (1 KiB
 // per store); split_reduce_kernel adds the slices and writes the output.
-template <class Act, class Fmt, int BM, int BN, bool GROUPED = false, bool FUSE = false, bool SPLIT = false>
+template <class Act, class Fmt, int BM, int BN, bool GROUPED = false, bool FUSE = false, bool SPLIT = false, int WR = 2>
 __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   using Elem = typename Act::elem;
-  constexpr int WM = BM / 2, WN = BN / 2;             // wave sub-tile
+  constexpr int WC = 4 / WR;                          // the wavefronts form a WR x WC grid
+  constexpr int WM = BM / WR, WN = BN / WC;           // wave sub-tile
   constexpr int TM = WM / 16, TN = WN / 16;
   constexpr int B_CH = Fmt::B_CH;                     // 16-byte weight chunks of the tile per thread
   constexpr int CPR = Fmt::CPR;
@@ -577,7 +593,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 15, g = lane >> 4;
-  const int wn0 = (wave & 1) * WN;
+  const int wn0 = wave % WC * WN;
 
   // Tile order.  The 8 XCDs take workgroups round-robin and each has its own L2, so the tile of a
   // workgroup is derived from (XCD = id % 8, slot on that XCD = id / 8):
@@ -645,7 +661,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   // fraction of the matrix-core time.  With 8, 4 and 2 alone an expert of 129 .. 160 rows paid for 256: FP8 experts, 2500
   // tokens top 8 of 128, 367 -> 324 us, 2200 334 -> 301; GGUF experts, 2048 tokens, 387 -> 357.  A length of 7 as well made
   // the kernel longer and every size 2 % slower.
-  const int wr = wave >> 1;
+  const int wr = wave / WC;
   auto mtile = [&](int b) { return GROUPED ? 2 * b + wr : wr * TM + b; };
   int live = TM;
   if constexpr (GROUPED) live = __builtin_amdgcn_readfirstlane((((M + 15) >> 4) - wr + 1) >> 1);
@@ -1044,16 +1060,16 @@ __global__ __launch_bounds__(256) void pack_x_grouped_kernel(const uint16_t* __r
 
 // Adds the K slices of a SPLIT launch (in slice order), scales, rounds and writes the output.  A wavefront
 // takes one 16 x 16 accumulator tile: lane 16 g + j holds row j, columns 4 g .. 4 g + 3.  grid (tiles, 4 TN TM / 4).
-template <class Act, class Fmt, int BM, int BN>
+template <class Act, class Fmt, int BM, int BN, int WR>
 __global__ __launch_bounds__(256) void split_reduce_kernel(const GemmArgs p) {
   using Elem = typename Act::elem;
-  constexpr int TM = BM / 32, TN = BN / 32;
+  constexpr int WC = 4 / WR, TM = BM / WR / 16, TN = BN / WC / 16;
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
   const int tile = blockIdx.x;
   const int at = __builtin_amdgcn_readfirstlane(blockIdx.y * 4 + (threadIdx.x >> 6));   // [wave][column tile][row tile]
   const int wave = at / (TN * TM), a = at / TM % TN, b = at % TM;
   const int tn = tile / p.tiles_m, tm = tile - tn * p.tiles_m;
-  const int m = tm * BM + (wave >> 1) * (BM / 2) + b * 16, n = tn * BN + (wave & 1) * (BN / 2) + a * 16 + g * 4;
+  const int m = tm * BM + wave / WC * (BM / WR) + b * 16, n = tn * BN + wave % WC * (BN / WC) + a * 16 + g * 4;
   if (m >= p.M) return;                               // uniform
   const size_t slice = (size_t)p.tiles_m * p.tiles_n * (BM * BN / 4);                   // in f32x4
   const f32x4* src = reinterpret_cast<const f32x4*>(p.partial) + (size_t)tile * (BM * BN / 4) + (size_t)at * 64 + lane;
@@ -1077,7 +1093,7 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const GemmArgs p) {
   }
 }
 
-template <class Act, class Fmt, int BM, int BN, bool SPLIT = false>
+template <class Act, class Fmt, int BM, int BN, bool SPLIT = false, int WR = 2>
 static int launch_gemm_tiled(GemmArgs p, hipStream_t st) {
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
@@ -1094,7 +1110,7 @@ static int launch_gemm_tiled(GemmArgs p, hipStream_t st) {
     }
   }
   const size_t lds = (size_t)2 * (Fmt::B_CH * 256 / Fmt::CPR) * kPitch * 2;
-  auto kern = gemm_tiled_kernel<Act, Fmt, BM, BN, false, false, SPLIT>;
+  auto kern = gemm_tiled_kernel<Act, Fmt, BM, BN, false, false, SPLIT, WR>;
   if (lds > 64 * 1024) {
     static bool raised = false;                       // opt in to > 64 KiB of dynamic LDS once
     if (!raised) {
@@ -1106,7 +1122,7 @@ static int launch_gemm_tiled(GemmArgs p, hipStream_t st) {
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)(SPLIT ? p.splits : 1)), dim3(256), lds, st, p);
   if constexpr (SPLIT)
-    hipLaunchKernelGGL((split_reduce_kernel<Act, Fmt, BM, BN>), dim3((unsigned)(p.tiles_m * p.tiles_n), BM * BN / 1024), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((split_reduce_kernel<Act, Fmt, BM, BN, WR>), dim3((unsigned)(p.tiles_m * p.tiles_n), BM * BN / 1024), dim3(256), 0, st, p);
   return launch_status();
 }
 
@@ -1154,14 +1170,40 @@ static inline int gemm_splits(long M, long N, long K) {
   return 2.0 + 0.55 * (double)steps + sums * best < 0.48 * (double)(K / 64) ? best : 1;
 }
 
+// Tile of a problem that 256-row tiles of 160 and more columns would leave half of the chip idle on, K in one piece.  What a
+// step costs there is not the matrix pipe but the issue of the dequantization (Q6_K 500 x 5120 x 5120 on 128 x 96: 64 us,
+// without the dequantization 34, without the MFMAs 60), and a tile dequantizes its columns whatever its rows.  So tall and
+// narrow: the four wavefronts stack up along M, every one takes all columns of the tile, and x is read once per workgroup
+// instead of once per wavefront column.  Time of a step relative to 256 x 64 with whole rounds of one workgroup per CU (110
+// problems of nine formats, M 66 .. 1024): 256 x 48 0.93, 192 x 64 0.92, 128 x 64 0.89 (four reads of the weight tile from LDS
+// for 128 rows, but the shortest chain), on two wavefront columns 128 x 96 1.15, 128 x 128 1.25; where the decode is one
+// conversion (unscaled FP8), these are 0.90 and 1.10.  M x K x N, 128 x 96 or 128 x 128 against the choice, us: Q6_K 500 x 5120 x 5120
+// 63.6 -> 50.5 (256 x 48), Q5_K 947 x 5120 x 5176 141 -> 88 (256 x 48), Q4_K 352 x 4096 x 13056 89 -> 61 (192 x 64), FP8
+// block-scaled 201 x 2048 x 12288 24.6 -> 21.6 (256 x 48), FP8 per-channel 207 x 5120 x 14168 45.4 -> 41.2 (256 x 64), Q4_K 85 x 1536 x
+// 14080 17.7 -> 14.3 (128 x 64).
+enum SmallTile { kTile128x64, kTile192x64, kTile256x48, kTile256x64, kTile128x96, kTile128x128 };
+static inline SmallTile gemm_small_tile(long M, long N, bool cheap_decode) {
+  const long cus = device_cu_count_gemm();
+  const struct { SmallTile tile; long bm, bn, cost; } shapes[] = {
+      {kTile128x64, 128, 64, 89}, {kTile192x64, 192, 64, 92}, {kTile256x48, 256, 48, 93}, {kTile256x64, 256, 64, 100},
+      {kTile128x96, 128, 96, cheap_decode ? 90 : 115}, {kTile128x128, 128, 128, cheap_decode ? 110 : 125}};
+  SmallTile best = kTile128x64;
+  long least = 0;
+  for (const auto& s : shapes) {
+    const long cost = (((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) + cus - 1) / cus * s.cost;
+    if (!least || cost < least) { least = cost; best = s.tile; }
+  }
+  return best;
+}
+
 // bytes of the re-tiled activations and, behind them, of the slices' sums
 static inline long long gemm_workspace(long M, long N, long K, int splits) {
   const long long packed = ((M + 15) & ~15LL) * K * 2;
   return splits < 2 ? packed : packed + (long long)splits * ((M + 127) / 128) * ((N + 127) / 128) * (128 * 128 * 4);
 }
 
-// Re-tiles x into `workspace` and runs the tile shape that fits the problem: 128 x 128 (or 96) tiles
-// while 256-row tiles would leave more than half of the chip idle, else 256 rows x 256 / 224 /
+// Re-tiles x into `workspace` and runs the tile shape that fits the problem: K slices or one of the small tiles
+// while 256 x 256 tiles would leave more than half of the chip idle, else 256 rows x 256 / 224 /
 // 192 / 160 columns, whichever needs the least time over its rounds of resident workgroups (a
 // 5120-column weight is 32 tiles of 160: with 8 row tiles exactly one round of 256 workgroups,
 // where 256-column tiles fill 160 of the 256 CUs).  FMT is a template taking (Act, BN).
@@ -1172,8 +1214,7 @@ static int run_gemm_tiled(GemmArgs p, const void* x, void* workspace, long long 
   hipLaunchKernelGGL(pack_x_kernel, dim3((unsigned)(((Q + 3) / 4) * (Mp / 16))), dim3(256), 0, st, (const uint16_t*)x,
                      (u32x4*)workspace, p.M, p.K, Q, FMT<Act, 128>::kPermK ? 1 : 0);
   p.x = workspace;
-  // 256-row tiles once they occupy more than half of the CUs (a 128 x 128 tile does a quarter of the
-  // work per weight and activation byte it moves and runs at about a third of the rate)
+  // 256 x 256 and the like once they occupy more than half of the CUs
   const long cus = device_cu_count_gemm();
   const long tiles_m = (p.M + 255) / 256;
   const bool big = gemm_big_tiles(p.M, p.N);
@@ -1183,14 +1224,19 @@ static int run_gemm_tiled(GemmArgs p, const void* x, void* workspace, long long 
       p.split_steps = ((p.K / 128 + splits - 1) / splits) * 2;
       p.splits = (p.K / 64 + p.split_steps - 1) / p.split_steps;
       p.partial = (float*)((char*)workspace + gemm_workspace(p.M, p.N, p.K, 1));
+      // the same tile count and no more row padding on 256 x 64 (0.77 - 1.0 of the time on 128 x 128: Q5_K 145 x 2560 x
+      // 7384 29.7 -> 22.9 us, INT4 387 x 5120 x 1720 26.8 -> 23.9, FP8 block-scaled 978 x 6144 x 1720 42.0 -> 37.1)
+      if ((p.M + 255) / 256 * 2 == (p.M + 127) / 128) return launch_gemm_tiled<Act, FMT<Act, 64>, 256, 64, true, 4>(p, st);
       return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128, true>(p, st);
     }
-    // 96 columns where a whole round of such tiles still fits: the chain of K steps is a quarter shorter in
-    // multiplying and dequantizing, and 129 .. 192 tiles of 128 columns become up to 256 (128 against 96 columns:
-    // FP8 block-scaled 201 x 2048 x 12288 24.2 -> 21.5 us, Q6_K 500 x 5120 x 5120 63.4 -> 59.5, Q5_K 1000 x 3072 x
-    // 2560 47.2 -> 40.6, FP8 900 x 4096 x 2304 38.6 -> 33.9, INT4 bf16 640 x 2048 x 3400 26.0 -> 24.8)
-    if ((long)((p.M + 127) / 128) * ((p.N + 95) / 96) <= cus) return launch_gemm_tiled<Act, FMT<Act, 96>, 128, 96>(p, st);
-    return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128>(p, st);
+    switch (gemm_small_tile(p.M, p.N, FMT<Act, 128>::kCheapDecode)) {
+      case kTile256x48: return launch_gemm_tiled<Act, FMT<Act, 48>, 256, 48, false, 4>(p, st);
+      case kTile256x64: return launch_gemm_tiled<Act, FMT<Act, 64>, 256, 64, false, 4>(p, st);
+      case kTile192x64: return launch_gemm_tiled<Act, FMT<Act, 64>, 192, 64, false, 4>(p, st);
+      case kTile128x64: return launch_gemm_tiled<Act, FMT<Act, 64>, 128, 64, false, 4>(p, st);
+      case kTile128x96: return launch_gemm_tiled<Act, FMT<Act, 96>, 128, 96>(p, st);
+      default: return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128>(p, st);
+    }
   }
   // time ~ rounds of resident workgroups x (columns of a tile + a fixed part per K step)
   auto cost = [&](long bn) { return ((tiles_m * ((p.N + bn - 1) / bn) + cus - 1) / cus) * (bn + kTileFixedCols); };

@@ -1,0 +1,89 @@
+"""Tiled GEMM below the size of 256-row tiles of 160 and more columns: every tile shape of the rule for one K slice, at
+its edges, on every weight format; and the K slices on 256 x 64."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import qlinear_oracle as O
+from test_gpu_gguf import _dequant_oracle, _gemv, _raw_case, _repack_oracle, _t
+from test_gpu_split_k import _call
+from test_gpu_tile_columns import _hot
+
+pytestmark = pytest.mark.gpu
+SHAPES = [(128, 64, 89), (192, 64, 92), (256, 48, 93), (256, 64, 100), (128, 96, 115), (128, 128, 125)]
+
+
+def _tile(M, N, K):
+    from mi355x_qlinear import capi
+    one, split = ctypes.c_longlong(0), ctypes.c_longlong(0)
+    assert capi.lib().mi_gemm_tiled_workspace(M, K, ctypes.byref(one)) == 0
+    assert capi.lib().mi_gemm_tiled_workspace_split(M, N, K, ctypes.byref(split)) == 0
+    if split.value != one.value:
+        return None
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rounds = lambda bm, bn: -(-(-(-M // bm) * -(-N // bn)) // cus)
+    return min(SHAPES, key=lambda t: rounds(*t[:2]) * t[2])[:2]
+
+
+def _weights(kind, dt, M, K, N):
+    if kind == "int4":
+        x, *w = O.make_int4_case(M, K, N, seed=M + K, act_dtype=dt, asym=True)
+        return x, w, O.int4_dequant(w[0], w[1], out_dtype=dt, zp=w[2])
+    if kind == "fp8_channel":
+        x, *w = O.make_fp8_pern_case(M, K, N, seed=M + K, act_dtype=dt)
+        return x, w, O.fp8_dequant_per_channel(*w)
+    if kind == "fp8_block":
+        x, w8, s = O.make_fp8_block_case(M, K, -(-N // 128) * 128, seed=M + K, act_dtype=dt)
+        return x, [w8[:N].contiguous(), s], O.fp8_dequant_block(w8, s, out_dtype=dt)[:N]
+    if kind == "q4_k":
+        x, raw = O.make_q4k_case(M, K, N, seed=M + K)
+        rep = O.q4k_repack(raw)
+        return x, [torch.from_numpy(a) for a in rep], torch.from_numpy(O.q4k_dequant(*rep)).float()
+    rep = _repack_oracle(kind, _raw_case(kind, N, K, seed=N))
+    wd = torch.from_numpy(_dequant_oracle(kind, rep).astype(np.float32))
+    return torch.randn(M, K, generator=torch.Generator().manual_seed(N)).half(), [_t(a) for a in rep], wd
+
+
+def _run(kind, dt, x, w, out):
+    import custom_esimd_kernels_sglang as s
+    import custom_esimd_kernels_vllm as v
+    if kind == "q4_k":
+        s.esimd_gemv_q4_k(x, *w, out)
+    elif kind.startswith("q"):
+        _gemv(s, kind, x, w, out)
+    else:
+        _call(v, kind, dt, x, w, out)
+
+
+KINDS = [("int4", torch.float16), ("int4", torch.bfloat16), ("fp8_channel", torch.bfloat16), ("fp8_block", torch.float16),
+         ("fp8_block", torch.bfloat16)] + [(k, torch.float16) for k in ("q4_k", "q4_0", "q8_0", "q5_k", "q6_k")]
+
+
+def _check(kind, dt, M, N, K, dev):
+    x, w, wd = _weights(kind, dt, M, K, N)
+    wdev = [t.to(dev) for t in w]
+    out = torch.full((M, N), float("nan"), dtype=dt, device=dev)
+    hot, ks = _hot(M, K, dt)
+    _run(kind, dt, hot.to(dev), wdev, out)
+    assert torch.equal(out.cpu().float(), wd.to(dt)[:, ks].t().float())   # one 1.0 per row: the weights value for value
+    _run(kind, dt, x.to(dev), wdev, out)
+    assert O.max_rel_err(out.cpu(), O.matmul_ref(x, wd)) < 1e-2           # the bound of the other tile shapes' tests
+
+
+# first and last rows and columns of a tile, odd N (element-wise stores); K = 512 is one slice here
+@pytest.mark.parametrize("kind,dt", KINDS)
+@pytest.mark.parametrize("M,N,tile", [(129, 3009, (128, 64)), (300, 968, (128, 64)), (192, 8264, (192, 64)), (190, 8257, (192, 64)),
+                                      (256, 8208, (256, 48)), (193, 8257, (256, 48)), (255, 12296, (256, 64)),
+                                      (300, 8300, (128, 128)), (110, 16400, (128, 96))])
+def test_every_tile_of_one_slice(dev, kind, dt, M, N, tile):
+    assert _tile(M, N, 512) == tile
+    _check(kind, dt, M, N, 512, dev)
+
+
+@pytest.mark.parametrize("kind,dt", KINDS)
+@pytest.mark.parametrize("M,N", [(129, 1000), (256, 1001), (500, 520)])
+def test_slices_on_tall_tiles(dev, kind, dt, M, N):
+    assert _tile(M, N, 2048) is None
+    _check(kind, dt, M, N, 2048, dev)

@@ -1,5 +1,5 @@
-"""Tiled GEMM on tiles of 96 columns (problems of one K slice whose tiles of 96 columns fit one round of the CUs), and
-the 256-row tiles of the GGUF formats."""
+"""Tiled GEMM on problems of one K slice whose tiles of 96 columns fit one round of the CUs, and the 256-row tiles of the
+GGUF formats."""
 import ctypes
 
 import numpy as np
@@ -27,7 +27,8 @@ def _hot(M, K, dt):
 
 
 def _tile(M, N, K):
-    """(rows, columns) of the tile that the size rule takes for a problem of one K slice; None where K is split."""
+    """(rows, columns) of the tile on two wavefront columns for a problem of one K slice; None where K is split.  Below 256
+    rows' worth of tiles the launch may prefer a taller, narrower one (test_gpu_tall_tiles.py)."""
     from mi355x_qlinear import capi
     one, split = ctypes.c_longlong(0), ctypes.c_longlong(0)
     assert capi.lib().mi_gemm_tiled_workspace(M, K, ctypes.byref(one)) == 0
