@@ -98,6 +98,11 @@ __device__ __forceinline__ f16x2 nibbles_f16(uint32_t bytes, bool high) {
 __device__ __forceinline__ f16x2 planted_f16(uint32_t bytes, bool high) {
   return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, bytes, high ? 0x04030402u : 0x04010400u));
 }
+// (s0 s1)(s2 s3), (m0 m1)(m2 m3) -> (s0 m0)(s1 m1)(s2 m2)(s3 m3)
+__device__ __forceinline__ u32x4 scale_min_pairs(u32x2 s, u32x2 m) {
+  return u32x4{__builtin_amdgcn_perm(m[0], s[0], 0x05040100u), __builtin_amdgcn_perm(m[0], s[0], 0x07060302u),
+               __builtin_amdgcn_perm(m[1], s[1], 0x05040100u), __builtin_amdgcn_perm(m[1], s[1], 0x07060302u)};
+}
 template <int DW> using Dwords = std::conditional_t<DW == 4, u32x4, u32x2>;
 template <int DW>
 __device__ __forceinline__ void load_dwords(Dwords<DW>& v, const __amdgpu_buffer_rsrc_t& r, uint32_t off, uint32_t soff) {
@@ -123,6 +128,7 @@ struct WInt4 {
   static constexpr int DW = 8 / CPR;                  // so that every thread has one; dwords per chunk
   static constexpr double kWeightBytesPerK = 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256; // chunks per thread
+  static constexpr bool kSide = false;
   static constexpr int LPC = 3;                       // load instructions per chunk
   static constexpr int kPieces = B_CH * DW * 8;        // 8 pieces per packed dword of 8 nibbles
   static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
@@ -233,14 +239,16 @@ struct WInt4 {
 // w = fp16(fp16(nib * scale) - min), the product rounded before the subtraction (two roundings,
 // as the dense dequantization does): one conversion, one packed product and one packed difference per
 // pair of weights.  fp16 activations only; pairs and x in the order of INT4's fp16 form.
-template <class Act, int BN>
+template <class Act, int BN, bool SIDE = false>
 struct WQ4K {
   static_assert(Act::dt == DT_F16, "Q4_K runs in fp16");
   static constexpr int CPR = BN <= 64 ? 4 : 2;        // chunks per row and 64-wide step: 8 bytes each on narrow tiles,
   static constexpr int DW = 8 / CPR;                  // so that every thread has one; dwords per chunk
   static constexpr double kWeightBytesPerK = 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
-  static constexpr int LPC = 3;
+  static constexpr bool kSide = SIDE;                 // scales and mins through the LDS table (see gemm_tiled_kernel)
+  static constexpr int LPC = SIDE ? 1 : 3;
+  struct Side { u32x2 s, m; };                        // a row's scales and mins of 128 k
   static constexpr int PPD = 8;                       // pieces per dword of 8 nibbles
   static constexpr int kPieces = B_CH * DW * PPD;
   static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
@@ -252,7 +260,7 @@ struct WQ4K {
   };
   struct Stage {
     Dwords<DW> b[B_CH];
-    uint32_t s[B_CH], m[B_CH];                        // fp16 bits (32-bit slots: 16-bit members end up on the stack)
+    uint32_t s[SIDE ? 1 : B_CH], m[SIDE ? 1 : B_CH];  // fp16 bits (32-bit slots: 16-bit members end up on the stack)
   };
   struct Dq {
     uint32_t e, o;
@@ -275,10 +283,24 @@ struct WQ4K {
   static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
                                                const uint32_t (&soff)[B_CH], int kt, uint32_t dead, int idx) {
     const uint32_t k0 = (uint32_t)kt * kBK;
-    const int i = idx / 3, kind = idx % 3;
+    const int i = idx / LPC, kind = idx % LPC;
     if (kind == 0) load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, k0 >> 1);
-    else if (kind == 1) st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, (k0 >> 5) * 2u, 0);
-    else st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, (k0 >> 5) * 2u, 0);
+    if constexpr (SIDE) return;
+    if (kind == 1) st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, (k0 >> 5) * 2u, 0);
+    else if (kind == 2) st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, (k0 >> 5) * 2u, 0);
+  }
+  static __device__ __forceinline__ void side_load(const Res& r, Side& d, int n, int pair, uint32_t dead) {
+    const uint32_t off = (uint32_t)n * (uint32_t)r.Kc * 2u | dead;
+    d.s = __builtin_amdgcn_raw_buffer_load_b64(r.sr, off, (uint32_t)pair * 8u, 0);
+    d.m = __builtin_amdgcn_raw_buffer_load_b64(r.mr, off, (uint32_t)pair * 8u, 0);
+  }
+  static __device__ __forceinline__ u32x4 side_entry(const Side& d) { return scale_min_pairs(d.s, d.m); }
+  static __device__ __forceinline__ void begin_side(const uint32_t (&v)[B_CH], Dq& q) {
+#pragma unroll
+    for (int i = 0; i < B_CH; ++i) {
+      q.sv[i] = both_bits(v[i]);
+      q.mv[i] = both_bits(v[i] >> 16);
+    }
   }
   static __device__ __forceinline__ void begin(const Res&, const Stage& st, Dq& q) {
 #pragma unroll
@@ -330,7 +352,8 @@ struct WGguf {
   static_assert(!kPlainH || DW == 4, "high bits in element order: whole chunks of 32");
   static constexpr double kWeightBytesPerK = F == GT_Q80 ? 1.0 : F == GT_Q6K ? 0.75 : F == GT_Q5K ? 0.625 : 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
-  static constexpr int LPC = (F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2) - (kPlainH || (kHigh && DW == 2) ? 1 : 0);
+  static constexpr bool kSide = kPlainH;              // the MoE stacks: scales and mins through the LDS table (see gemm_tiled_kernel)
+  static constexpr int LPC = kPlainH ? 2 : (F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2) - (kHigh && DW == 2 ? 1 : 0);
   static constexpr int PPD = F == GT_Q5K ? 13 : F == GT_Q6K ? 9 : F == GT_Q40 ? 8 : 3;   // pieces per dword (8 nibbles / 4 bytes)
   static constexpr int kPieces = B_CH * DW * PPD;
   static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
@@ -343,8 +366,8 @@ struct WGguf {
   };
   struct Stage {
     Dwords<DW> b[B_CH];
-    uint32_t s[B_CH];
-    uint32_t m[F == GT_Q5K ? B_CH : 1];
+    uint32_t s[kSide ? 1 : B_CH];
+    uint32_t m[F == GT_Q5K && !kSide ? B_CH : 1];
     u32x4 h[kHigh && !kPlainH ? B_CH : 1][DW / 2];
     u32x2 hp[kPlainH ? B_CH : 1];
     uint32_t sh;                                      // shift of this step's field of the high-bit bytes (uniform)
@@ -376,23 +399,47 @@ struct WGguf {
     const uint32_t k0 = (uint32_t)kt * kBK;
     const int i = idx / LPC, kind = idx % LPC;
     if (kind == 0) load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, F == GT_Q80 ? k0 : k0 >> 1);
-    else if (kind == 1) {
-      if constexpr (F == GT_Q6K && DW == 4) st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, k0 >> 3, 0);
+    else if (kind == 1 && !kSide) {
+      if constexpr (kSide) return;
+      else if constexpr (F == GT_Q6K && DW == 4) st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, k0 >> 3, 0);
       else st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, F == GT_Q6K ? k0 >> 3 : k0 >> 4, 0);
-    } else if (kPlainH && kind == 2) {
+    } else if (kPlainH && kind == 1) {
       if constexpr (kPlainH && F == GT_Q6K) st.hp[i] = __builtin_amdgcn_raw_buffer_load_b64(r.hr, r.hoff[i] | dead, k0 >> 2, 0);
       else if constexpr (kPlainH) st.hp[i][0] = __builtin_amdgcn_raw_buffer_load_b32(r.hr, r.hoff[i] | dead, k0 >> 3, 0);
     } else if (kind == LPC - 1 && F == GT_Q5K) {
-      if constexpr (F == GT_Q5K) st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, k0 >> 4, 0);
+      if constexpr (F == GT_Q5K && !kSide) st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, k0 >> 4, 0);
     } else if constexpr (kHigh && !kPlainH) {
       const uint32_t tile = F == GT_Q6K ? (k0 >> 9) * 128u + (k0 & 127u) : (k0 >> 9) * 64u;
       st.h[i][kind - 2] = __builtin_amdgcn_raw_buffer_load_b128(r.hr, r.hoff[i] | dead, tile + (uint32_t)(kind - 2) * 16u, 0);
       st.sh = F == GT_Q6K ? (k0 >> 7 & 3u) * 2u : k0 >> 6 & 7u;
     }
   }
-  static __device__ __forceinline__ void begin(const Res&, const Stage& st, Dq& q) {
+  struct Side { u32x4 s; u32x2 m; };                  // a row's scales (Q6_K 8, Q5_K 4) and mins of 128 k
+  static __device__ __forceinline__ void side_load(const Res& r, Side& d, int n, int pair, uint32_t dead) {
+    const uint32_t off = (uint32_t)n * (uint32_t)r.Ks | dead;
+    if constexpr (F == GT_Q6K) d.s = __builtin_amdgcn_raw_buffer_load_b128(r.sr, off, (uint32_t)pair * 16u, 0);
+    else {
+      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r.sr, off, (uint32_t)pair * 8u, 0);
+      d.s = u32x4{v[0], v[1], 0u, 0u};
+      d.m = __builtin_amdgcn_raw_buffer_load_b64(r.mr, off, (uint32_t)pair * 8u, 0);
+    }
+  }
+  static __device__ __forceinline__ u32x4 side_entry(const Side& d) {
+    if constexpr (F == GT_Q6K) return d.s;            // the two scales of every 32 k
+    else return scale_min_pairs(u32x2{d.s[0], d.s[1]}, d.m);
+  }
+  static __device__ __forceinline__ void begin_side(const uint32_t (&v)[B_CH], Dq& q) {
 #pragma unroll
     for (int i = 0; i < B_CH; ++i) {
+      q.sv[i][0] = both_bits(v[i]);
+      if constexpr (F == GT_Q6K && DW == 4) q.sv[i][1] = both_bits(v[i] >> 16);
+      if constexpr (F == GT_Q5K) q.mv[i] = both_bits(v[i] >> 16);
+    }
+  }
+  static __device__ __forceinline__ void begin(const Res&, const Stage& st, Dq& q) {
+    if constexpr (kSide) return;
+#pragma unroll
+    for (int i = 0; i < (kSide ? 0 : B_CH); ++i) {
       q.sv[i][0] = both_bits(st.s[i]);
       if constexpr (F == GT_Q6K && DW == 4) q.sv[i][1] = both_bits(st.s[i] >> 16);
       if constexpr (F == GT_Q5K) q.mv[i] = both_bits(st.m[i]);
@@ -479,6 +526,7 @@ struct WFp8 {
   static constexpr int LPC = BLOCK ? 2 : 1;
   static constexpr int kPPC = BLOCK ? 10 : 4;         // pieces per chunk
   static constexpr int kPieces = B_CH * kPPC;
+  static constexpr bool kSide = false;
   static constexpr bool kCheapDecode = !BLOCK;
   static constexpr bool kOutScale = !BLOCK;
   static constexpr bool kPermK = false;
@@ -561,6 +609,8 @@ struct WFp8 {
     return p.scale_f16 ? (float)((const _Float16*)r.se)[n] : ((const float*)r.se)[n];
   }
 };
+
+struct NoSide { struct Side {}; };
 
 template <int... I, class F>
 __device__ __forceinline__ void fold_pieces(std::integer_sequence<int, I...>, F f) {
@@ -722,6 +772,30 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
     for (int idx = 0; idx < kLoads; ++idx) load_b1(st, kt, idx);
   };
 
+  // Scales and mins through LDS (Fmt::kSide).  Loaded by the threads that dequantize a chunk they are 2 to 4 bytes of a line per
+  // row, array and step, and the lines of 256 rows do not stay in L1 until the next step: with those loads served from one
+  // line a GGUF layer of 2048 tokens took 306 instead of 363 us.  Thread t loads 128 k of tile row t at once, a 16-byte
+  // table entry (one dword per chunk of 32), every second step; two tables, behind the weight tiles.  In step kt (even) table
+  // kt / 2 + 1 is written; the steps that read it are kt + 1 and kt + 2, and its place was read last in step kt - 2.
+  unsigned char* const side = smem + 2 * (size_t)BNP * kPitch * 2;
+  static_assert(!Fmt::kSide || (GROUPED && !FUSE && BN == 256 && BNP == 256 && CPR == 2), "one table row per thread");
+  auto side_at = [&](int pair) { return side + (pair & 1) * 4096; };
+  auto load_side = [&](auto& d, int pair) {
+    if constexpr (Fmt::kSide)
+      Fmt::side_load(res, d, n0 + tid, pair, (uint32_t)(n0 + tid >= N || 2 * pair >= KT) << 31);
+  };
+  auto begin_stage = [&](const StageB& st, int kt, auto& q) {
+    if constexpr (Fmt::kSide) {
+      uint32_t v[B_CH];
+      const unsigned char* at = side_at(kt >> 1) + (kt & 1) * 8 + (tid >> 1) * 16 + (tid & 1) * 4;
+#pragma unroll
+      for (int i = 0; i < B_CH; ++i) v[i] = *reinterpret_cast<const uint32_t*>(at + i * 2048);
+      Fmt::begin_side(v, q);
+    } else {
+      Fmt::begin(res, st, q);
+    }
+  };
+
   constexpr int kPieces = Fmt::kPieces;
   using DqState = typename Fmt::Dq;
   constexpr size_t kBufBytes = (size_t)BNP * kPitch * 2;
@@ -732,6 +806,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
     Fmt::piece(st, q, I, dst);
   };
 
+  [[maybe_unused]] typename std::conditional_t<Fmt::kSide, Fmt, NoSide>::Side sd;
   // One 64-wide K step: multiply out of LDS buffer `buf` (two 32-wide MFMA steps,
   // ring slots slot0 and slot0 + 1) while the next step's weights (`cur`, loaded one
   // step earlier) are dequantized into the other buffer and the weights two steps
@@ -743,7 +818,13 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
     constexpr int kMfmas = 2 * TN * L;
     const Elem* Bb = Bs + buf * BNP * kPitch;
     DqState q;
-    Fmt::begin(res, cur, q);
+    begin_stage(cur, kt + 1, q);
+    if constexpr (Fmt::kSide) {
+      if (buf == 0) {
+        *reinterpret_cast<u32x4*>(side_at((kt >> 1) + 1) + tid * 16) = Fmt::side_entry(sd);
+        load_side(sd, (kt >> 1) + 2);
+      }
+    }
     auto rd_w = [&](int a, int s) {
       return *reinterpret_cast<const u32x4*>(Bb + (wn0 + a * 16 + j) * kPitch + s * 32 + g * 8);
     };
@@ -782,6 +863,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   };
 
   StageB s0, s1;
+  if constexpr (Fmt::kSide) load_side(sd, 0);
   load_b(s0, kt0);
   __builtin_amdgcn_sched_barrier(0);
   load_b(s1, kt0 + 1);
@@ -790,9 +872,14 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
     __builtin_amdgcn_sched_barrier(0);               // keep the ring's loads in issue order
     load_x(r, 2 * kt0 + r);
   }
+  if constexpr (Fmt::kSide) {
+    *reinterpret_cast<u32x4*>(side_at(0) + tid * 16) = Fmt::side_entry(sd);
+    load_side(sd, 1);
+    __syncthreads();
+  }
   {
     DqState q;
-    Fmt::begin(res, s0, q);
+    begin_stage(s0, kt0, q);
     // a fold, not a loop: the pieces of the longer formats exceed what "#pragma unroll" expands, and a rolled
     // loop would keep the stage on the stack
     fold_pieces(std::make_integer_sequence<int, kPieces>{}, [&](int I) __attribute__((always_inline)) { dq_piece(s0, 0, I, q); });

@@ -10,6 +10,7 @@ namespace qlin {
 
 template <class Act, int BN> using WFp8Plain = WFp8<Act, BN, false>;
 template <class Act, int BN> using WFp8Block = WFp8<Act, BN, true>;
+template <class Act, int BN> using WQ4KDense = WQ4K<Act, BN>;
 
 static inline bool tiled_shape_ok(int M, int N, int K, int wbytes_per_k_num, int wbytes_per_k_den) {
   if (M <= 0 || N <= 0 || K <= 0 || (K % 128)) return false;
@@ -67,7 +68,7 @@ int mi_gemm_q4k_tiled_ws(const void* x, const void* ql, const void* scale, const
   if (!workspace || workspace_bytes < (long long)((M + 15) & ~15) * K * 2) return MI_ERR_ARG;
   GemmArgs p{};
   p.w = ql; p.scale = scale; p.zp = qmin; p.out = out; p.M = M; p.N = N; p.K = K;
-  return run_gemm_tiled<ActF16, WQ4K>(p, x, workspace, workspace_bytes, (hipStream_t)stream);
+  return run_gemm_tiled<ActF16, WQ4KDense>(p, x, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -1,5 +1,6 @@
 """Grouped tiled GEMM: an M-tile of 1 .. 16 live 16-row blocks runs the K loop of the smallest length that covers them."""
 import ctypes
+import math
 
 import pytest
 import torch
@@ -31,18 +32,19 @@ def test_fp8_experts(dev, dt, fuse):
         assert O.max_rel_err(o[at:at + n], ref[at:at + n]) < TOL      # the bound of the other shapes' tests
 
 
+@pytest.mark.parametrize("K,offset", [(256, 0), (384, 0), (128, 1), (640, 3)])   # odd numbers of 128-wide pairs; scales on a 2-byte boundary
 @pytest.mark.parametrize("fmt", [2, 5, 6])
-def test_gguf_experts(dev, fmt):
+def test_gguf_experts(dev, fmt, K, offset):
     """Against the chunk kernel: the same weights, fp32 sums in another order (2^-11 of the result in norm, the fp16 rounding)."""
     from mi355x_qlinear import capi
     torch.manual_seed(fmt)
-    E, N, K, total = len(COUNTS), 264, 256, sum(COUNTS)
+    E, N, total = len(COUNTS), 264, sum(COUNTS)
     rows, at = [], 0
     for e, n in enumerate(COUNTS):
         rows += [[e, at + t, min(64, n - t)] for t in range(0, n, 64)]
         at += n
     u8 = lambda *s: torch.randint(0, 256, s, dtype=torch.uint8, device=dev)
-    h = lambda *s: (torch.rand(*s, device=dev) * 0.01).half()
+    h = lambda *s: (torch.rand(math.prod(s) + offset, device=dev) * 0.01).half()[offset:].view(*s)
     ql, sc = [u8(E, N, K // 2)], [h(E, N, K // (16 if fmt == 6 else 32))]
     mn = [h(E, N, K // 32)] if fmt != 6 else None
     qh = [u8(E, N, K // (8 if fmt == 5 else 4))] if fmt != 2 else None
