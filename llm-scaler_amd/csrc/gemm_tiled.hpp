@@ -349,11 +349,11 @@ struct WGguf {
   static constexpr bool kHigh = F == GT_Q5K || F == GT_Q6K;
   static constexpr int CPR = F == GT_Q80 || BN <= 64 ? 4 : 2;
   static constexpr int DW = F == GT_Q80 ? 4 : 8 / CPR;   // dwords per chunk (nibbles: 8 bytes on narrow tiles, as INT4)
-  static_assert(!kPlainH || DW == 4, "high bits in element order: whole chunks of 32");
+  static_assert(!kPlainH || (DW == 4 && BN > 128), "high bits in element order: whole chunks of 32");
   static constexpr double kWeightBytesPerK = F == GT_Q80 ? 1.0 : F == GT_Q6K ? 0.75 : F == GT_Q5K ? 0.625 : 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
-  static constexpr bool kSide = kPlainH;              // the MoE stacks: scales and mins through the LDS table (see gemm_tiled_kernel)
-  static constexpr int LPC = kPlainH ? 2 : (F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2) - (kHigh && DW == 2 ? 1 : 0);
+  static constexpr bool kSide = kPlainH || (F == GT_Q5K && BN > 128);   // scales and mins through the LDS table (see gemm_tiled_kernel)
+  static constexpr int LPC = kSide ? 1 + (kHigh ? kPlainH ? 1 : 2 : 0) : (F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2) - (kHigh && DW == 2 ? 1 : 0);
   static constexpr int PPD = F == GT_Q5K ? 13 : F == GT_Q6K ? 9 : F == GT_Q40 ? 8 : 3;   // pieces per dword (8 nibbles / 4 bytes)
   static constexpr int kPieces = B_CH * DW * PPD;
   static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
@@ -399,34 +399,34 @@ struct WGguf {
     const uint32_t k0 = (uint32_t)kt * kBK;
     const int i = idx / LPC, kind = idx % LPC;
     if (kind == 0) load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, F == GT_Q80 ? k0 : k0 >> 1);
-    else if (kind == 1 && !kSide) {
-      if constexpr (kSide) return;
-      else if constexpr (F == GT_Q6K && DW == 4) st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, k0 >> 3, 0);
-      else st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, F == GT_Q6K ? k0 >> 3 : k0 >> 4, 0);
-    } else if (kPlainH && kind == 1) {
-      if constexpr (kPlainH && F == GT_Q6K) st.hp[i] = __builtin_amdgcn_raw_buffer_load_b64(r.hr, r.hoff[i] | dead, k0 >> 2, 0);
-      else if constexpr (kPlainH) st.hp[i][0] = __builtin_amdgcn_raw_buffer_load_b32(r.hr, r.hoff[i] | dead, k0 >> 3, 0);
-    } else if (kind == LPC - 1 && F == GT_Q5K) {
+    else if constexpr (kPlainH) {
+      if constexpr (F == GT_Q6K) st.hp[i] = __builtin_amdgcn_raw_buffer_load_b64(r.hr, r.hoff[i] | dead, k0 >> 2, 0);
+      else st.hp[i][0] = __builtin_amdgcn_raw_buffer_load_b32(r.hr, r.hoff[i] | dead, k0 >> 3, 0);
+    } else if (kind == 1 && !kSide) {
+      if constexpr (F == GT_Q6K && DW == 4 && !kSide) st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, k0 >> 3, 0);
+      else if constexpr (!kSide) st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, F == GT_Q6K ? k0 >> 3 : k0 >> 4, 0);
+    } else if (kind == LPC - 1 && F == GT_Q5K && !kSide) {
       if constexpr (F == GT_Q5K && !kSide) st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, k0 >> 4, 0);
-    } else if constexpr (kHigh && !kPlainH) {
+    } else if constexpr (kHigh) {
+      const int piece = kind - (kSide ? 1 : 2);
       const uint32_t tile = F == GT_Q6K ? (k0 >> 9) * 128u + (k0 & 127u) : (k0 >> 9) * 64u;
-      st.h[i][kind - 2] = __builtin_amdgcn_raw_buffer_load_b128(r.hr, r.hoff[i] | dead, tile + (uint32_t)(kind - 2) * 16u, 0);
+      st.h[i][piece] = __builtin_amdgcn_raw_buffer_load_b128(r.hr, r.hoff[i] | dead, tile + (uint32_t)piece * 16u, 0);
       st.sh = F == GT_Q6K ? (k0 >> 7 & 3u) * 2u : k0 >> 6 & 7u;
     }
   }
-  struct Side { u32x4 s; u32x2 m; };                  // a row's scales (Q6_K 8, Q5_K 4) and mins of 128 k
+  struct Side { u32x4 s; u32x2 m; };                  // a row's scales (Q6_K 8, others 4) and mins of 128 k
   static __device__ __forceinline__ void side_load(const Res& r, Side& d, int n, int pair, uint32_t dead) {
     const uint32_t off = (uint32_t)n * (uint32_t)r.Ks | dead;
     if constexpr (F == GT_Q6K) d.s = __builtin_amdgcn_raw_buffer_load_b128(r.sr, off, (uint32_t)pair * 16u, 0);
     else {
       const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r.sr, off, (uint32_t)pair * 8u, 0);
       d.s = u32x4{v[0], v[1], 0u, 0u};
-      d.m = __builtin_amdgcn_raw_buffer_load_b64(r.mr, off, (uint32_t)pair * 8u, 0);
+      if constexpr (F == GT_Q5K) d.m = __builtin_amdgcn_raw_buffer_load_b64(r.mr, off, (uint32_t)pair * 8u, 0);
     }
   }
   static __device__ __forceinline__ u32x4 side_entry(const Side& d) {
     if constexpr (F == GT_Q6K) return d.s;            // the two scales of every 32 k
-    else return scale_min_pairs(u32x2{d.s[0], d.s[1]}, d.m);
+    else return scale_min_pairs(u32x2{d.s[0], d.s[1]}, F == GT_Q5K ? d.m : u32x2{0u, 0u});
   }
   static __device__ __forceinline__ void begin_side(const uint32_t (&v)[B_CH], Dq& q) {
 #pragma unroll
@@ -777,8 +777,10 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   // line a GGUF layer of 2048 tokens took 306 instead of 363 us.  Thread t loads 128 k of tile row t at once, a 16-byte
   // table entry (one dword per chunk of 32), every second step; two tables, behind the weight tiles.  In step kt (even) table
   // kt / 2 + 1 is written; the steps that read it are kt + 1 and kt + 2, and its place was read last in step kt - 2.
+  // The large tiles of dense layers take it for Q5_K alone, the format with five loads per chunk (600 x 5120 x 14336 169 -> 153 us,
+  // 1024 x 4096 x 12288 121 -> 117); Q4_K was 1 to 3 % slower with it there, Q4_0 and Q6_K between 1 % faster and 1.5 % slower.
   unsigned char* const side = smem + 2 * (size_t)BNP * kPitch * 2;
-  static_assert(!Fmt::kSide || (GROUPED && !FUSE && BN == 256 && BNP == 256 && CPR == 2), "one table row per thread");
+  static_assert(!Fmt::kSide || (!FUSE && !SPLIT && BNP == 256 && CPR == 2), "one table row per thread");
   auto side_at = [&](int pair) { return side + (pair & 1) * 4096; };
   auto load_side = [&](auto& d, int pair) {
     if constexpr (Fmt::kSide)
@@ -1196,7 +1198,7 @@ static int launch_gemm_tiled(GemmArgs p, hipStream_t st) {
       if (!p.xcd_m || cost < best) { best = cost; p.xcd_m = a; }
     }
   }
-  const size_t lds = (size_t)2 * (Fmt::B_CH * 256 / Fmt::CPR) * kPitch * 2;
+  const size_t lds = (size_t)2 * (Fmt::B_CH * 256 / Fmt::CPR) * kPitch * 2 + (Fmt::kSide ? 2 * 4096 : 0);
   auto kern = gemm_tiled_kernel<Act, Fmt, BM, BN, false, false, SPLIT, WR>;
   if (lds > 64 * 1024) {
     static bool raised = false;                       // opt in to > 64 KiB of dynamic LDS once

@@ -87,3 +87,19 @@ def test_every_tile_of_one_slice(dev, kind, dt, M, N, tile):
 def test_slices_on_tall_tiles(dev, kind, dt, M, N):
     assert _tile(M, N, 2048) is None
     _check(kind, dt, M, N, 2048, dev)
+
+
+@pytest.mark.parametrize("N", [11008, 14001, 17000, 20001])           # 256-row tiles of 160, 192, 224, 256 columns
+def test_q5k_scales_on_a_two_byte_boundary(dev, N):
+    """The large tiles load 128 k of a row's scales and mins at once: the same bits where the tensors start off an 8-byte boundary."""
+    import custom_esimd_kernels_sglang as s
+    M, K = 520, 1024
+    torch.manual_seed(N)
+    w = [torch.randint(0, 256, (N, K // d), dtype=torch.uint8, device=dev) for d in (2, 8)]
+    sc, mn = ((torch.rand(N, K // 32, device=dev) * 0.01).half() for _ in range(2))
+    off = lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+    x = torch.randn(M, K, device=dev).half()
+    outs = [torch.empty(M, N, dtype=torch.float16, device=dev) for _ in range(2)]
+    s.esimd_gemv_q5_k(x, *w, sc, mn, outs[0])
+    s.esimd_gemv_q5_k(x, *w, off(sc), off(mn), outs[1])
+    assert torch.equal(*outs)
