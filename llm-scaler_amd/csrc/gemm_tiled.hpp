@@ -1240,8 +1240,8 @@ static inline bool gemm_big_tiles(long M, long N) {
 // neighbours' CUs are busy or not, so a problem with few tiles leaves the chip idle: slices up to one workgroup
 // per CU (two per CU share the path from L2 to the CU and gain nothing: Q8_0 1000 x 4096 x 4096, 256 tiles:
 // 61 us in one piece, 65 in two).  Every slice writes and reads fp32 sums of the whole output, 8 bytes per
-// element at about 5 TB/s, which sets the best number where tiles are few.  The alternative is one piece on tiles of 96
-// columns, about 0.48 us a step; slices have to make up for the second launch and the start of their chains.  Over 1287
+// element at about 5 TB/s, which sets the best number where tiles are few.  The alternative is one piece on a smaller
+// tile (gemm_small_tile), 0.45 to 0.5 us a step; slices have to make up for the second launch and the start of their chains.  On tiles of 96 columns and 128 x 128 slices, over 1287
 // problems of all formats (M 65 .. 1024, N 128 .. 14336, K 384 .. 8448) that leaves 2 slower in slices by more than 3 % and
 // 17 in one piece (without this line: 53 and none, up to 1.25 times): M x N x K, one piece / slices in us, FP8 block-scaled 320 x
 // 2760 x 1024 15.4 / 19.3 (one piece), INT4 256 x 5688 x 1536 20.1 / 23.9 (one piece).  One slice of 128 columns against
