@@ -75,9 +75,10 @@ struct GemmArgs {
 
 // MFMA with the accumulator pinned to the AGPR half of the register file and updated in place.
 // Left to the register allocator, the 224-256 accumulator registers of a 128 x 128 wave tile
-// get split and copied around the loop; the constraint keeps them where they are.  The
-// operands of every call come from LDS / global loads (never from a vector-ALU result), and
-// results are only read after the explicit wait at the end of the K loop.
+// get split and copied around the loop; the constraint keeps them where they are.  The compiler does
+// not know that this is an MFMA and keeps no distance from it: the operands of every call come from LDS /
+// global loads (never from a vector-ALU result), and the body of the K loop ends in an explicit wait, so that it lies
+// before whatever the register allocator does with the accumulators behind the loop.
 template <class Act>
 __device__ __forceinline__ void mfma_agpr(f32x4& acc, u32x4 a, u32x4 b) {
   if constexpr (Act::dt == DT_F16)
@@ -861,6 +862,9 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
         }
       }
     }
+    // The last MFMA needs up to 12 wait states until its result may be touched, and exits of the loop begin with copies of
+    // accumulators (also ahead of a wait that stands behind the loop).  Here it runs in the shadow of the LDS writes.
+    if (buf == 1) asm volatile("s_nop 15" ::: "memory");
     __syncthreads();
   };
 
@@ -905,8 +909,6 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
     else k_loop(std::integral_constant<int, 2>{});
   }
 
-  // the last MFMAs are still in the matrix pipe: wait before reading their results
-  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
   // D = W-tile (rows n) x X-tile^T: lane holds n = 4 g + v (v = 0..3), m = j
   if constexpr (SPLIT) {
     f32x4* dst = reinterpret_cast<f32x4*>(p.partial) +
