@@ -477,6 +477,9 @@ int mi_gemm_tiled_workspace(int M, int K, long long* bytes);
  * the chip: the re-tiled activations and the slices' fp32 sums.  With less (down to the sizes above)
  * the same entries run in one piece. */
 int mi_gemm_tiled_workspace_split(int M, int N, int K, long long* bytes);
+/* What those entries launch with that workspace: tiles of *rows x *columns, each in *slices pieces of K.  fmt 0 = INT4,
+ * 1 = FP8 per channel / tensor, 2 .. 6 = the GGUF formats (Q4_K, then as below), 7 = FP8 128x128 blocks. */
+int mi_gemm_tiled_shape(int fmt, int M, int N, int K, int* rows, int* columns, int* slices);
 int mi_gemm_fp8_tiled_ws(const void* x, const void* w, const void* scale, int scale_mode, int scale_is_f16,
                          void* out, void* workspace, long long workspace_bytes, int M, int N, int K,
                          int act_dtype, void* stream);

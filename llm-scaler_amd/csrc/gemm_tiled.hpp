@@ -87,6 +87,9 @@ __device__ __forceinline__ void mfma_agpr(f32x4& acc, u32x4 a, u32x4 b) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
+// What a weight costs on its way into LDS: one conversion per pair of weights, the other formats, high bits in an array of their own.
+enum class GemmDecode { kCheap, kMid, kDear };
+
 constexpr int kBK = 64;
 constexpr int kPitch = kBK + 8;                      // elements per LDS row (144 bytes)
 
@@ -132,7 +135,7 @@ struct WInt4 {
   static constexpr bool kSide = false;
   static constexpr int LPC = 3;                       // load instructions per chunk
   static constexpr int kPieces = B_CH * DW * 8;        // 8 pieces per packed dword of 8 nibbles
-  static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
+  static constexpr GemmDecode kDecode = GemmDecode::kMid;
   static constexpr bool kOutScale = false;
   static constexpr bool kHalf = Act::dt == DT_F16;
   static constexpr bool kPermK = kHalf;
@@ -252,7 +255,7 @@ struct WQ4K {
   struct Side { u32x2 s, m; };                        // a row's scales and mins of 128 k
   static constexpr int PPD = 8;                       // pieces per dword of 8 nibbles
   static constexpr int kPieces = B_CH * DW * PPD;
-  static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
+  static constexpr GemmDecode kDecode = GemmDecode::kMid;
   static constexpr bool kOutScale = false;
   static constexpr bool kPermK = true;
   struct Res {
@@ -357,7 +360,7 @@ struct WGguf {
   static constexpr int LPC = kSide ? 1 + (kHigh ? kPlainH ? 1 : 2 : 0) : (F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2) - (kHigh && DW == 2 ? 1 : 0);
   static constexpr int PPD = F == GT_Q5K ? 13 : F == GT_Q6K ? 9 : F == GT_Q40 ? 8 : 3;   // pieces per dword (8 nibbles / 4 bytes)
   static constexpr int kPieces = B_CH * DW * PPD;
-  static constexpr bool kCheapDecode = false;         // a conversion per pair of weights and nothing else
+  static constexpr GemmDecode kDecode = kHigh ? GemmDecode::kDear : GemmDecode::kMid;
   static constexpr bool kOutScale = false;
   static constexpr bool kPermK = F != GT_Q80;            // pairs (0 2)(1 3)(4 6)(5 7); Q8_0 in order
   struct Res {
@@ -528,7 +531,7 @@ struct WFp8 {
   static constexpr int kPPC = BLOCK ? 10 : 4;         // pieces per chunk
   static constexpr int kPieces = B_CH * kPPC;
   static constexpr bool kSide = false;
-  static constexpr bool kCheapDecode = !BLOCK;
+  static constexpr GemmDecode kDecode = BLOCK ? GemmDecode::kMid : GemmDecode::kCheap;
   static constexpr bool kOutScale = !BLOCK;
   static constexpr bool kPermK = false;
   struct Res {
@@ -1261,30 +1264,59 @@ static inline int gemm_splits(long M, long N, long K) {
   return 2.0 + 0.55 * (double)steps + sums * best < 0.48 * (double)(K / 64) ? best : 1;
 }
 
-// Tile of a problem that 256-row tiles of 160 and more columns would leave half of the chip idle on, K in one piece.  What a
+// Tile of the K slices: 128 x 128, or as many tiles of 256 x 64 where these pad no more rows.  256 x 64 decodes a weight
+// for twice the rows, but every workgroup reads 256 rows of x instead of 128.  It is ahead where x is small beside the weights (one or
+// two row tiles, or no more rows than columns; half of that where the decoding is cheap), where 128 columns would be padding, and where
+// a slice is long enough for the decoding to count.  128 x 128 / 256 x 64 in us, M x N x K: Q5_K 145 x 7384 x 2560 30.2 / 23.7, INT4 387 x
+// 1720 x 5120 27.1 / 24.6, FP8 block-scaled 978 x 1720 x 6144 45.0 / 38.9; Q4_0 1002 x 224 x 2048 13.2 / 16.4, FP8 per-channel 1189 x 528
+// x 8192 33.6 / 41.1, Q4_0 5352 x 280 x 6144 62.4 / 73.8.  Over 1780 problems whose rows pad alike (M 129 .. 6144, N 64 .. 8192) the time
+// over that of the better tile is 1.049 on 128 x 128, 1.019 on 256 x 64 and 1.008 by this line (geometric means); 73 are slower than on
+// 128 x 128 by more than 3 %, at most 1.16 (on 256 x 64 throughout 355, at most 1.35), 94 slower than on 256 x 64, at most 1.23.
+static inline bool gemm_slices_tall(long M, long N, long steps, GemmDecode decode) {
+  if ((M + 255) / 256 * 2 != (M + 127) / 128) return false;
+  const bool cheap = decode == GemmDecode::kCheap, dear = decode == GemmDecode::kDear;
+  if (M <= (cheap ? 256 : 512) || N >= (cheap ? 2 * M : M)) return true;
+  if (N <= 64 || (M > 1280 && N > 128 && N <= 192)) return true;
+  return dear ? steps >= 8 : !cheap && M <= 1024 && steps >= 10;
+}
+
+// Tile of a problem that 256 x 256 tiles would leave half of the chip idle on, K in one piece.  What a
 // step costs there is not the matrix pipe but the issue of the dequantization (Q6_K 500 x 5120 x 5120 on 128 x 96: 64 us,
 // without the dequantization 34, without the MFMAs 60), and a tile dequantizes its columns whatever its rows.  So tall and
 // narrow: the four wavefronts stack up along M, every one takes all columns of the tile, and x is read once per workgroup
 // instead of once per wavefront column.  Time of a step relative to 256 x 64 with whole rounds of one workgroup per CU (110
 // problems of nine formats, M 66 .. 1024): 256 x 48 0.93, 192 x 64 0.92, 128 x 64 0.89 (four reads of the weight tile from LDS
 // for 128 rows, but the shortest chain), on two wavefront columns 128 x 96 1.15, 128 x 128 1.25; where the decode is one
-// conversion (unscaled FP8), these are 0.90 and 1.10.  M x K x N, 128 x 96 or 128 x 128 against the choice, us: Q6_K 500 x 5120 x 5120
-// 63.6 -> 50.5 (256 x 48), Q5_K 947 x 5120 x 5176 141 -> 88 (256 x 48), Q4_K 352 x 4096 x 13056 89 -> 61 (192 x 64), FP8
-// block-scaled 201 x 2048 x 12288 24.6 -> 21.6 (256 x 48), FP8 per-channel 207 x 5120 x 14168 45.4 -> 41.2 (256 x 64), Q4_K 85 x 1536 x
-// 14080 17.7 -> 14.3 (128 x 64).
-enum SmallTile { kTile128x64, kTile192x64, kTile256x48, kTile256x64, kTile128x96, kTile128x128 };
-static inline SmallTile gemm_small_tile(long M, long N, bool cheap_decode) {
+// conversion (unscaled FP8), these are 0.90 and 1.10.  M x K x N, the better of 128 x 96 and 128 x 128 against the choice, us: Q6_K 500 x 5120 x
+// 5120 61.0 -> 46.8 (192 x 64), Q5_K 947 x 5120 x 5176 117 -> 95 (192 x 64; 256 x 48 88), Q4_K 352 x 4096 x 13056 75 -> 60 (192 x 64), FP8
+// block-scaled 201 x 2048 x 12288 23.5 -> 20.6 (256 x 48), FP8 per-channel 207 x 5120 x 14168 46.5 -> 41.9 (256 x 64), Q4_K 85 x 1536 x
+// 14080 17.7 -> 14.2 (128 x 64).  Of 204 problems 13 are more than 3 % off the best of the six, at most 1.13 (unscaled FP8 on 128 x 96).
+struct GemmTile { int rows, columns; };
+static inline GemmTile gemm_small_tile(long M, long N, GemmDecode decode) {
   const long cus = device_cu_count_gemm();
-  const struct { SmallTile tile; long bm, bn, cost; } shapes[] = {
-      {kTile128x64, 128, 64, 89}, {kTile192x64, 192, 64, 92}, {kTile256x48, 256, 48, 93}, {kTile256x64, 256, 64, 100},
-      {kTile128x96, 128, 96, cheap_decode ? 90 : 115}, {kTile128x128, 128, 128, cheap_decode ? 110 : 125}};
-  SmallTile best = kTile128x64;
+  const bool cheap = decode == GemmDecode::kCheap;
+  const struct { GemmTile tile; long cost; } shapes[] = {{{128, 64}, 89},  {{192, 64}, 92},  {{256, 48}, 93},
+                                                         {{256, 64}, 100}, {{128, 96}, cheap ? 90 : 115}, {{128, 128}, cheap ? 110 : 125}};
+  GemmTile best{};
   long least = 0;
   for (const auto& s : shapes) {
-    const long cost = (((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) + cus - 1) / cus * s.cost;
+    const long tiles = ((M + s.tile.rows - 1) / s.tile.rows) * ((N + s.tile.columns - 1) / s.tile.columns);
+    const long cost = (tiles + cus - 1) / cus * s.cost;
     if (!least || cost < least) { least = cost; best = s.tile; }
   }
   return best;
+}
+
+// 256 rows x 256 / 224 / 192 / 160 columns, whichever needs the least time over its rounds of resident workgroups: rounds x
+// (columns of a tile + a fixed part per K step).  A 5120-column weight is 32 tiles of 160: with 8 row tiles exactly one
+// round of 256 workgroups, where 256-column tiles fill 160 of the 256 CUs.
+static inline GemmTile gemm_big_tile(long M, long N) {
+  const long cus = device_cu_count_gemm(), tiles_m = (M + 255) / 256;
+  auto cost = [&](long bn) { return ((tiles_m * ((N + bn - 1) / bn) + cus - 1) / cus) * (bn + kTileFixedCols); };
+  int best = 256;
+  for (int bn : {224, 192, 160})
+    if (cost(bn) < cost(best)) best = bn;
+  return {256, best};
 }
 
 // bytes of the re-tiled activations and, behind them, of the slices' sums
@@ -1293,11 +1325,18 @@ static inline long long gemm_workspace(long M, long N, long K, int splits) {
   return splits < 2 ? packed : packed + (long long)splits * ((M + 127) / 128) * ((N + 127) / 128) * (128 * 128 * 4);
 }
 
-// Re-tiles x into `workspace` and runs the tile shape that fits the problem: K slices or one of the small tiles
-// while 256 x 256 tiles would leave more than half of the chip idle, else 256 rows x 256 / 224 /
-// 192 / 160 columns, whichever needs the least time over its rounds of resident workgroups (a
-// 5120-column weight is 32 tiles of 160: with 8 row tiles exactly one round of 256 workgroups,
-// where 256-column tiles fill 160 of the 256 CUs).  FMT is a template taking (Act, BN).
+// The launch of a problem: its tile, and the slices of K with their length in 64-wide steps.  K slices or a small tile while
+// 256 x 256 tiles would leave more than half of the chip idle, else tiles of 256 rows and 160 and more columns.
+struct GemmPlan { GemmTile tile; int splits, split_steps; };
+static inline GemmPlan gemm_plan(long M, long N, long K, GemmDecode decode, long long workspace_bytes) {
+  if (gemm_big_tiles(M, N)) return {gemm_big_tile(M, N), 1, (int)(K / kBK)};
+  const int most = gemm_splits(M, N, K);
+  if (most < 2 || workspace_bytes < gemm_workspace(M, N, K, most)) return {gemm_small_tile(M, N, decode), 1, (int)(K / kBK)};
+  const int steps = (int)((K / 128 + most - 1) / most) * 2, splits = (int)((K / kBK + steps - 1) / steps);
+  return {gemm_slices_tall(M, N, steps, decode) ? GemmTile{256, 64} : GemmTile{128, 128}, splits, steps};
+}
+
+// Re-tiles x into `workspace` and runs the launch that gemm_plan picks.  FMT is a template taking (Act, BN).
 template <class Act, template <class, int> class FMT>
 static int run_gemm_tiled(GemmArgs p, const void* x, void* workspace, long long workspace_bytes, hipStream_t st) {
   const int Mp = (p.M + 15) & ~15;
@@ -1305,39 +1344,26 @@ static int run_gemm_tiled(GemmArgs p, const void* x, void* workspace, long long 
   hipLaunchKernelGGL(pack_x_kernel, dim3((unsigned)(((Q + 3) / 4) * (Mp / 16))), dim3(256), 0, st, (const uint16_t*)x,
                      (u32x4*)workspace, p.M, p.K, Q, FMT<Act, 128>::kPermK ? 1 : 0);
   p.x = workspace;
-  // 256 x 256 and the like once they occupy more than half of the CUs
-  const long cus = device_cu_count_gemm();
-  const long tiles_m = (p.M + 255) / 256;
-  const bool big = gemm_big_tiles(p.M, p.N);
-  if (!big) {
-    const int splits = gemm_splits(p.M, p.N, p.K);
-    if (splits > 1 && workspace_bytes >= gemm_workspace(p.M, p.N, p.K, splits)) {
-      p.split_steps = ((p.K / 128 + splits - 1) / splits) * 2;
-      p.splits = (p.K / 64 + p.split_steps - 1) / p.split_steps;
-      p.partial = (float*)((char*)workspace + gemm_workspace(p.M, p.N, p.K, 1));
-      // the same tile count and no more row padding on 256 x 64 (0.77 - 1.0 of the time on 128 x 128: Q5_K 145 x 2560 x
-      // 7384 29.7 -> 22.9 us, INT4 387 x 5120 x 1720 26.8 -> 23.9, FP8 block-scaled 978 x 6144 x 1720 42.0 -> 37.1)
-      if ((p.M + 255) / 256 * 2 == (p.M + 127) / 128) return launch_gemm_tiled<Act, FMT<Act, 64>, 256, 64, true, 4>(p, st);
-      return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128, true>(p, st);
-    }
-    switch (gemm_small_tile(p.M, p.N, FMT<Act, 128>::kCheapDecode)) {
-      case kTile256x48: return launch_gemm_tiled<Act, FMT<Act, 48>, 256, 48, false, 4>(p, st);
-      case kTile256x64: return launch_gemm_tiled<Act, FMT<Act, 64>, 256, 64, false, 4>(p, st);
-      case kTile192x64: return launch_gemm_tiled<Act, FMT<Act, 64>, 192, 64, false, 4>(p, st);
-      case kTile128x64: return launch_gemm_tiled<Act, FMT<Act, 64>, 128, 64, false, 4>(p, st);
-      case kTile128x96: return launch_gemm_tiled<Act, FMT<Act, 96>, 128, 96>(p, st);
-      default: return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128>(p, st);
-    }
+  const GemmPlan plan = gemm_plan(p.M, p.N, p.K, FMT<Act, 128>::kDecode, workspace_bytes);
+  if (plan.splits > 1) {
+    p.splits = plan.splits;
+    p.split_steps = plan.split_steps;
+    p.partial = (float*)((char*)workspace + gemm_workspace(p.M, p.N, p.K, 1));
+    if (plan.tile.rows == 256) return launch_gemm_tiled<Act, FMT<Act, 64>, 256, 64, true, 4>(p, st);
+    return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128, true>(p, st);
   }
-  // time ~ rounds of resident workgroups x (columns of a tile + a fixed part per K step)
-  auto cost = [&](long bn) { return ((tiles_m * ((p.N + bn - 1) / bn) + cus - 1) / cus) * (bn + kTileFixedCols); };
-  long best = 256;
-  for (long bn : {224L, 192L, 160L})
-    if (cost(bn) < cost(best)) best = bn;
-  if (best == 160) return launch_gemm_tiled<Act, FMT<Act, 160>, 256, 160>(p, st);
-  if (best == 192) return launch_gemm_tiled<Act, FMT<Act, 192>, 256, 192>(p, st);
-  if (best == 224) return launch_gemm_tiled<Act, FMT<Act, 224>, 256, 224>(p, st);
-  return launch_gemm_tiled<Act, FMT<Act, 256>, 256, 256>(p, st);
+  switch (plan.tile.rows << 16 | plan.tile.columns) {
+    case 128 << 16 | 64: return launch_gemm_tiled<Act, FMT<Act, 64>, 128, 64, false, 4>(p, st);
+    case 192 << 16 | 64: return launch_gemm_tiled<Act, FMT<Act, 64>, 192, 64, false, 4>(p, st);
+    case 256 << 16 | 48: return launch_gemm_tiled<Act, FMT<Act, 48>, 256, 48, false, 4>(p, st);
+    case 256 << 16 | 64: return launch_gemm_tiled<Act, FMT<Act, 64>, 256, 64, false, 4>(p, st);
+    case 128 << 16 | 96: return launch_gemm_tiled<Act, FMT<Act, 96>, 128, 96>(p, st);
+    case 128 << 16 | 128: return launch_gemm_tiled<Act, FMT<Act, 128>, 128, 128>(p, st);
+    case 256 << 16 | 160: return launch_gemm_tiled<Act, FMT<Act, 160>, 256, 160>(p, st);
+    case 256 << 16 | 192: return launch_gemm_tiled<Act, FMT<Act, 192>, 256, 192>(p, st);
+    case 256 << 16 | 224: return launch_gemm_tiled<Act, FMT<Act, 224>, 256, 224>(p, st);
+    default: return launch_gemm_tiled<Act, FMT<Act, 256>, 256, 256>(p, st);
+  }
 }
 
 }  // namespace qlin

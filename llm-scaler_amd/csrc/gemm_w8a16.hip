@@ -38,6 +38,20 @@ int mi_gemm_tiled_workspace_split(int M, int N, int K, long long* bytes) {
   return MI_OK;
 }
 
+int mi_gemm_tiled_shape(int fmt, int M, int N, int K, int* rows, int* columns, int* slices) {
+  static constexpr GemmDecode kDecode[] = {WInt4<ActF16, 128>::kDecode, WFp8Plain<ActF16, 128>::kDecode, WQ4K<ActF16, 128>::kDecode,
+                                           WGguf<ActF16, 128, GT_Q40>::kDecode, WGguf<ActF16, 128, GT_Q80>::kDecode,
+                                           WGguf<ActF16, 128, GT_Q5K>::kDecode, WGguf<ActF16, 128, GT_Q6K>::kDecode,
+                                           WFp8Block<ActF16, 128>::kDecode};
+  if (!rows || !columns || !slices || fmt < 0 || fmt > 7) return MI_ERR_ARG;
+  if (M <= 0 || N <= 0 || K <= 0 || K % 128) return MI_ERR_SHAPE;
+  const GemmPlan plan = gemm_plan(M, N, K, kDecode[fmt], gemm_workspace(M, N, K, gemm_splits(M, N, K)));
+  *rows = plan.tile.rows;
+  *columns = plan.tile.columns;
+  *slices = plan.splits;
+  return MI_OK;
+}
+
 int mi_gemm_fp8_tiled_ws(const void* x, const void* w, const void* scale, int scale_mode, int scale_is_f16,
                          void* out, void* workspace, long long workspace_bytes, int M, int N, int K,
                          int act_dtype, void* stream) {

@@ -478,3 +478,30 @@ def test_names_outside_the_path_raise_when_called():
             fn(torch.zeros(1))
     # guarded sglang sites must keep falling back: no placeholder may shadow them
     assert not hasattr(s, "esimd_gdn_conv_fused_seq") and not hasattr(s, "esimd_qkv_split_norm_rope")
+
+
+def _tile(fmt, M, N, K):
+    """(rows, columns, slices) that the dense tiled GEMM launches; fmt as in mi_gemm_tiled_shape."""
+    out = [ctypes.c_int(0) for _ in range(3)]
+    assert capi.lib().mi_gemm_tiled_shape(fmt, M, N, K, *map(ctypes.byref, out)) == 0
+    return tuple(v.value for v in out)
+
+
+def test_k_slices_take_the_tile_that_was_measured_ahead():
+    """256 x 64 reads twice the rows of x per workgroup: behind 128 x 128 where x is large beside the weights and a slice short."""
+    int4, fp8, q4_k, q4_0, q8_0, q5_k, block = 0, 1, 2, 3, 4, 5, 7
+    for fmt, M, N, K in ((q4_0, 1002, 224, 2048), (fp8, 1189, 528, 8192), (block, 1268, 504, 6144), (q8_0, 997, 224, 2048),
+                         (q4_0, 961, 392, 2688), (int4, 1234, 336, 4992), (fp8, 898, 344, 3712), (q4_0, 5352, 280, 6144),
+                         (int4, 904, 520, 3072), (q4_k, 966, 520, 3072), (block, 904, 520, 3072), (fp8, 501, 960, 3072)):
+        assert _tile(fmt, M, N, K)[:2] == (128, 128) and _tile(fmt, M, N, K)[2] > 1, (fmt, M, N, K)
+    for fmt, M, N, K in ((q5_k, 145, 7384, 2560), (int4, 387, 1720, 5120), (block, 978, 1720, 6144), (q8_0, 150, 3504, 7552),
+                         (q5_k, 1231, 64, 1024), (q8_0, 1955, 192, 2304), (fp8, 488, 1936, 8064), (q4_k, 196, 1400, 4096)):
+        assert _tile(fmt, M, N, K)[:2] == (256, 64) and _tile(fmt, M, N, K)[2] > 1, (fmt, M, N, K)
+    assert _tile(q5_k, 300, 7384, 2560)[:2] != (256, 64)                 # a third row tile of 128: 256 would pad
+
+
+def test_tile_query_refuses_what_the_launch_refuses():
+    v = [ctypes.c_int(0) for _ in range(3)]
+    q = lambda *a: capi.lib().mi_gemm_tiled_shape(*a, *map(ctypes.byref, v))
+    assert q(8, 100, 100, 128) == q(-1, 100, 100, 128) == capi.lib().mi_gemm_tiled_shape(0, 100, 100, 128, None, None, None) != 0
+    assert q(0, 100, 100, 64) == q(0, 0, 100, 128) == -2

@@ -28,7 +28,8 @@ def _call(v, kind, dt, x, w, out):
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K", [(65, 136, 1152),       # slices of unequal length
                                    (129, 257, 640),       # one row in the last row tile, odd N (element-wise stores)
-                                   (128, 96, 4096), (200, 1000, 2048), (70, 40, 128)])
+                                   (128, 96, 4096), (200, 1000, 2048), (70, 40, 128),
+                                   (1001, 105, 1024), (640, 104, 1152)])      # rows that 256 would pad alike, and 128 take
 def test_one_hot_rows_and_random_rows(v, dev, kind, dt, M, N, K):
     """One 1.0 per row returns the dequantized weights value for value (each k is in exactly one slice; the other
     slices add zeros); random rows agree with the oracle."""
