@@ -1,6 +1,6 @@
 """The tiled GEMM's MFMAs are inline assembly: the compiler does not know how long their results stay in the matrix pipe and
 puts no wait states before an instruction that reads or overwrites an accumulator.  The body of the K loops ends in a wait of its
-own (s_nop 15); here the built kernels are followed through every branch: only another MFMA touches an accumulator before it."""
+own (s_nop 7: what the compiler keeps behind the same MFMA as a builtin); here the built kernels are followed through every branch: only another MFMA touches an accumulator before it."""
 import re
 import shutil
 import struct
@@ -55,7 +55,7 @@ def _touched_in_flight(body):
     """Instructions that touch an AGPR which, on some path, is the result of an MFMA with no wait behind it."""
     index = {a: i for i, (a, _, _) in enumerate(body)}
     ops = [t.split(None, 1) + [""] for _, t, _ in body]
-    wait = [o[0] == "s_nop" and o[1].strip() == "15" for o in ops]
+    wait = [o[0] == "s_nop" and int(o[1], 0) >= 7 for o in ops]
     starts, use = [0] * len(body), [0] * len(body)
     for i, o in enumerate(ops):
         if o[0].startswith("v_mfma"):
