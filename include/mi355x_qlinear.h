@@ -461,7 +461,7 @@ int mi_moe_mlp_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_d
 
 /* ---- prefill (M > 64) on FP8 and Q4_K weights: the tiled matrix-core GEMM ---------
  * The same results as mi_gemm_fp8_pern / _pert / _blockscale and mi_gemv_q4k, computed by the
- * 256 x 256 (224, 128) tiled GEMM that also serves mi_gemm_int4, so that a weight byte is read
+ * tiled GEMM that also serves mi_gemm_int4 (256 x 256 tiles, smaller for few rows or columns), so that a weight byte is read
  * once per 256 activation rows.  scale_mode 0 = per output channel (fp32, or fp16 with
  * scale_is_f16), 1 = per tensor (fp32 [1]), 2 = 128 x 128 blocks (fp32 [ceil(N/128), K/128],
  * folded into the weight before its rounding to the activation type).  K % 128 == 0.

@@ -1,6 +1,6 @@
 // Prefill GEMMs on the GGUF formats Q4_0, Q8_0, Q5_K and Q6_K (repacked) for more than 64 activation
 // rows: the tiled matrix-core GEMM of gemm_tiled.hpp, which reads and dequantizes a weight once per
-// 128 or 256 rows of x; the weight-streaming kernel does it once per 64 (M=500, K=N=5120, Q6_K:
+// 128 to 256 rows of x; the weight-streaming kernel does it once per 64 (M=500, K=N=5120, Q6_K:
 // 168 us streaming, 45 us tiled).
 #include "gemm_tiled.hpp"
 #include "../../include/mi355x_qlinear.h"
@@ -15,10 +15,11 @@ template <class Act, int BN> using WQ6K = WGguf<Act, BN, GT_Q6K>;
 // 65 .. 128 rows: up to which K two passes of the weight-streaming kernels are ahead.  They are at their best where the
 // weight gives a CU one 16-row block or a little less or more, and on short rows, which the tiles' pipeline does not
 // amortise; the K-sliced kernel takes Q4_0 and Q8_0 further than the others.  Streaming / tiled in us (M x N x K):
-// Q6_K 112 x 4096 x 1024 10.9 / 16.2, 112 x 3072 x 2560 16.6 / 19.3, 112 x 1024 x 2048 13.5 / 12.9, 80 x 10240 x 1024 20.6 / 16.0,
-// 80 x 1024 x 1024 12.8 / 11.0, 128 x 1048 x 1024 10.9 / 13.0; Q8_0 80 x 4096 x 3072 15.2 / 19.2, 128 x 1024 x 3072 17.1 / 13.1;
-// Q4_0 80 x 4096 x 4096 17.8 / 19.7, 128 x 1024 x 4096 20.7 / 14.0.  Over 3780 problems (N 256 .. 10240, K 512 .. 4096) 156 that take the
-// tiles are slower there by more than 3 %, at most 1.2 times; with everything on the tiles beyond Q4_0's 3072 and Q8_0's 2048, 634, at most 1.49.
+// Q6_K 112 x 4096 x 1024 10.2 / 15.4, 112 x 3072 x 2560 15.8 / 18.3, 112 x 1024 x 2048 12.3 / 11.9, 80 x 10240 x 1024 20.0 / 11.9,
+// 80 x 1024 x 1024 11.8 / 9.9, 128 x 1048 x 1024 10.1 / 12.1; Q8_0 80 x 4096 x 3072 14.6 / 18.6, 128 x 1024 x 3072 16.1 / 12.2;
+// Q4_0 80 x 4096 x 4096 16.7 / 19.3, 128 x 1024 x 4096 19.3 / 13.0.  Of 663 problems that take the tiles (N 256 .. 10240, K 512 .. 4096) 64
+// are slower there by more than 3 %, at most 1.19 times.  The line was drawn before the tall tiles, on the safe side of them now: of 537
+// that stream, 168 would be faster on the tiles by more than 3 %, at most 1.55 times (Q8_0 115 x 10168 x 1152 18.7 / 12.0).
 static int stream_k(int fmt, long M, long N) {
   const long cus = device_cu_count_gemm();
   const bool one_block = N >= 8 * cus && N <= 16 * cus;

@@ -25,8 +25,8 @@
 // weights are the MFMA A operand, so a lane ends up with 4 consecutive output columns of one
 // row and stores them as 8 bytes.
 //
-// A weight format is a policy class: how a 64-wide K step of a weight row is cut into 16-byte
-// chunks, which side loads (scales, zero-points, mins) a chunk needs, the dequantization of a
+// A weight format is a policy class: how a 64-wide K step of a weight row is cut into chunks (16
+// bytes; 8 for nibbles on narrow tiles), which side loads (scales, zero-points, mins) a chunk needs, the dequantization of a
 // chunk as a sequence of small pieces, and an optional factor on the finished sums.
 #pragma once
 #include "qlinear_common.hpp"
@@ -204,7 +204,7 @@ struct WInt4 {
       return __builtin_bit_cast(uint32_t, r);
     }
   }
-  // piece I of the stage; dst[i] = LDS address of chunk i's 64 output bytes in the target buffer
+  // piece I of the stage; dst[i] = LDS address of chunk i's output in the target buffer
   static __device__ __forceinline__ void piece(const Stage& st, Dq& q, int I, unsigned char* const (&dst)[B_CH]) {
     const int dword = I >> 3, part = I & 7;
     const int i = dword / DW, dw = dword % DW;
@@ -634,7 +634,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   constexpr int WC = 4 / WR;                          // the wavefronts form a WR x WC grid
   constexpr int WM = BM / WR, WN = BN / WC;           // wave sub-tile
   constexpr int TM = WM / 16, TN = WN / 16;
-  constexpr int B_CH = Fmt::B_CH;                     // 16-byte weight chunks of the tile per thread
+  constexpr int B_CH = Fmt::B_CH;                     // weight chunks of the tile per thread
   constexpr int CPR = Fmt::CPR;
   constexpr int BNP = B_CH * 256 / CPR;               // LDS rows of the weight tile (>= BN)
   constexpr int kLoads = Fmt::LPC * B_CH;             // load instructions per stage and thread
@@ -781,8 +781,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   // line a GGUF layer of 2048 tokens took 306 instead of 363 us.  Thread t loads 128 k of tile row t at once, a 16-byte
   // table entry (one dword per chunk of 32), every second step; two tables, behind the weight tiles.  In step kt (even) table
   // kt / 2 + 1 is written; the steps that read it are kt + 1 and kt + 2, and its place was read last in step kt - 2.
-  // The large tiles of dense layers take it for Q5_K alone, the format with five loads per chunk (600 x 5120 x 14336 169 -> 153 us,
-  // 1024 x 4096 x 12288 121 -> 117); Q4_K was 1 to 3 % slower with it there, Q4_0 and Q6_K between 1 % faster and 1.5 % slower.
+  // The large tiles of dense layers take it for Q5_K alone, the format with five loads per chunk (M x K x N 600 x 5120 x 14336 169 -> 153
+  // us, 1024 x 4096 x 12288 122 -> 119); Q4_K was 1 to 3 % slower with it there, Q4_0 and Q6_K between 1 % faster and 1.5 % slower.
   unsigned char* const side = smem + 2 * (size_t)BNP * kPitch * 2;
   static_assert(!Fmt::kSide || (!FUSE && !SPLIT && BNP == 256 && CPR == 2), "one table row per thread");
   auto side_at = [&](int pair) { return side + (pair & 1) * 4096; };
@@ -1242,17 +1242,17 @@ static inline bool gemm_big_tiles(long M, long N) {
   return M > 128 && ((M + 255) / 256) * ((N + 255) / 256) * 2 > device_cu_count_gemm();
 }
 
-// K slices of a problem on 128 x 128 tiles.  A tile is a chain of K / 64 steps of about 0.65 us whether its
+// K slices of a problem, counted on 128 x 128 tiles.  A tile is a chain of K / 64 steps of about 0.65 us whether its
 // neighbours' CUs are busy or not, so a problem with few tiles leaves the chip idle: slices up to one workgroup
 // per CU (two per CU share the path from L2 to the CU and gain nothing: Q8_0 1000 x 4096 x 4096, 256 tiles:
-// 61 us in one piece, 65 in two).  Every slice writes and reads fp32 sums of the whole output, 8 bytes per
+// 50 us in one piece, 55 in two).  Every slice writes and reads fp32 sums of the whole output, 8 bytes per
 // element at about 5 TB/s, which sets the best number where tiles are few.  The alternative is one piece on a smaller
-// tile (gemm_small_tile), 0.45 to 0.5 us a step; slices have to make up for the second launch and the start of their chains.  On tiles of 96 columns and 128 x 128 slices, over 1287
-// problems of all formats (M 65 .. 1024, N 128 .. 14336, K 384 .. 8448) that leaves 2 slower in slices by more than 3 % and
-// 17 in one piece (without this line: 53 and none, up to 1.25 times): M x N x K, one piece / slices in us, FP8 block-scaled 320 x
-// 2760 x 1024 15.4 / 19.3 (one piece), INT4 256 x 5688 x 1536 20.1 / 23.9 (one piece).  One slice of 128 columns against
-// the rule's slices (M x K x N): INT4 128 x 4096 x 4096 44 -> 22 us, Q4_K 100 x 5120 x 5120 63 -> 26 us, Q6_K 129 x 5120 x 5120 71 -> 38
-// us, INT4 1024 x 6144 x 2048 72 -> 51 us, FP8 70 x 1024 x 1024 13.6 -> 10 us.
+// tile (gemm_small_tile); slices have to make up for the second launch and the start of their chains.  The line (0.48 us a step in one
+// piece, 0.55 in slices) was drawn on 128 x 96 and 128 x 128, and both sides have become faster since.  One piece / slices as they are now in us, M x N x
+// K: FP8 block-scaled 320 x 2760 x 1024 11.2 / 15.8 and INT4 256 x 5688 x 1536 14.9 / 21.1 (one piece); INT4 128 x 4096 x 4096 29.4 / 20.5, Q4_K 100 x
+// 5120 x 5120 35.0 / 23.7, Q6_K 129 x 5120 x 5120 38.1 / 27.1, INT4 1024 x 2048 x 6144 48.9 / 43.1, FP8 70 x 1024 x 1024 11.1 / 9.6 (slices).
+// Of 696 problems in slices (nine formats, M 65 .. 1024, N 128 .. 14336, K 384 .. 8448) 56 would be faster in one piece by more than 3 %, at
+// most 1.27 times (Q4_0 81 x 13864 x 2560 19.8 / 25.1); of 81 in one piece none in 2 to 4 slices.
 static inline int gemm_splits(long M, long N, long K) {
   if (M <= 64 || N <= 0 || gemm_big_tiles(M, N)) return 1;
   const long tiles = ((M + 127) / 128) * ((N + 127) / 128);

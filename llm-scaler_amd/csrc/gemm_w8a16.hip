@@ -1,6 +1,6 @@
 // Prefill GEMMs on FP8 (per-channel / per-tensor / 128x128 block scales) and GGUF Q4_K weights
 // for more than 64 activation rows: the tiled matrix-core GEMM of gemm_tiled.hpp with the FP8
-// and Q4_K weight formats.  Each weight byte is read once per 256 (or 128) activation rows
+// and Q4_K weight formats.  Each weight byte is read once per 128 to 256 activation rows
 // instead of once per 64 as the weight-streaming kernels would.
 #include "gemm_tiled.hpp"
 #include "scratch.hpp"

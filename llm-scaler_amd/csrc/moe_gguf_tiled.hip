@@ -11,7 +11,7 @@
 namespace qlin {
 
 // 256 x 256 like the FP8 experts' tiles (a wavefront skips the row tiles past the chunk's last): 2048 tokens, top 8 of
-// 128 experts, H = 2048, I = 768: 404 us for the layer against 445 on 128 x 128 and 510 with the chunk kernel.
+// 128 experts, H = 2048, I = 768: 404 us for the layer against 445 on 128 x 128 when the tile was chosen, 334 now; 510 with the chunk kernel.
 constexpr int kGgufBM = 256, kGgufBN = 256;
 constexpr int kChunkRows = 64;                        // rows of a chunk that count
 constexpr int kChunkMapThreads = 1024;
@@ -133,9 +133,12 @@ static int launch_chunk_gemm(GemmArgs p, int nmat, int max_tiles, hipStream_t st
 // Time in us.  Tiled: tables and re-tiling, then a chain of K / 64 steps per round of one workgroup per CU, and the
 // multiplications of the live rows.  Chunks: a chain of K steps, and a part per chunk and per 64 rows for every million
 // weights.  Fitted on 1300 launches (1 .. 256 experts, H 1024 .. 6144, I 256 .. 2048, 8 .. 1024 rows per expert; even, drawn
-// and skewed counts): nine in ten within 25 %, so the tiled kernel has to promise 5 % (down: 2 %).  Both sides, chunks / tiled in us: E = 8,
-// H = 1024, I = 512, 128 rows per expert, up 20 / 41; E = 16, H = 2048, I = 768, 96 rows 37 / 53; E = 128, same sizes, 60 even
-// rows 123 / 153, 96 rows 226 / 180, 256 rows 517 / 407; E = 256, H = 2048, I = 512, 60 rows 184 / 223, 96 rows 299 / 274.
+// and skewed counts): nine in ten within 25 %, so the tiled kernel had to promise 5 % (down: 2 %).  The fit is of the kernel before its further
+// loop lengths and its LDS table, so the line lies on the safe side: of 434 launches 171 take the tiles, 5 of them up to 1.06 times
+// slower by more than 3 %, and 25 of the other 263 would be faster on them, at most 1.8 times.  Chunks / tiled in us, up and down launch: E = 8,
+// H = 1024, I = 512, 128 rows per expert 14 / 32, 11 / 26; E = 16, H = 2048, I = 768, 96 rows 36 / 49, 26 / 30; E = 128, same sizes, 60 even
+// rows 125 / 144, 90 / 95, 96 rows 228 / 160, 163 / 109, 256 rows 421 / 268, 286 / 175; E = 256, H = 2048, I = 512, 60 rows 150 / 182, 117 / 139,
+// 96 rows 285 / 207, 222 / 162.
 static bool chunk_tiles_pay(bool up, long long n, long long out_rows, long long E, long long N, long long K, long long nmat) {
   if (kChunkRows * n > out_rows + kChunkRows * E) return false;
   const long long rows = out_rows <= kChunkRows * n ? out_rows : std::max(n, kChunkRows * (n - E));
