@@ -132,8 +132,9 @@ struct WInt4 {
   static constexpr int DW = 8 / CPR;                  // so that every thread has one; dwords per chunk
   static constexpr double kWeightBytesPerK = 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256; // chunks per thread
-  static constexpr bool kSide = false;
-  static constexpr int LPC = 3;                       // load instructions per chunk
+  static constexpr int kEntry = 4;                    // bytes per row of a scale table: scale, zero-point (see gemm_tiled_kernel)
+  static constexpr bool kHalfEntry = false;
+  static constexpr int LPC = 1;                       // load instructions per chunk
   static constexpr int kPieces = B_CH * DW * 8;        // 8 pieces per packed dword of 8 nibbles
   static constexpr GemmDecode kDecode = GemmDecode::kMid;
   static constexpr bool kOutScale = false;
@@ -146,8 +147,8 @@ struct WInt4 {
   };
   struct Stage {
     Dwords<DW> b[B_CH];
-    uint32_t s[B_CH], z[B_CH];                        // fp16 scale bits, zero-point: 32-bit slots, one register each
   };
+  struct Side { uint32_t s, z; };                     // a row's fp16 scale bits and zero-point of 128 k
   struct Dq {
     uint32_t e, o;
     f32x2 fe, fo;
@@ -164,28 +165,24 @@ struct WInt4 {
     r.has_zp = p.zp != nullptr;
     return r;
   }
-  // byte offset of chunk kc of row n at k = 0, and the row's first side-table entry
-  static __device__ __forceinline__ void chunk_addr(Res& r, int, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
-    boff = (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * DW * 4);
-    soff = (uint32_t)n * (uint32_t)r.Kg;              // in groups; x2 for the fp16 scale
+  // byte offset of chunk kc of row n at k = 0
+  static __device__ __forceinline__ uint32_t chunk_addr(Res&, int, int n, int kc, int K) {
+    return (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * DW * 4);
   }
-  static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
-                                               const uint32_t (&soff)[B_CH], int kt, uint32_t dead, int idx) {
-    const uint32_t k0 = (uint32_t)kt * kBK;
-    const int i = idx / 3, kind = idx % 3;
-    if (kind == 0)
-      load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, k0 >> 1);
-    else if (kind == 1)
-      st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, ((soff[i] & 0x7fffffffu) * 2u) | (soff[i] & 0x80000000u) | dead,
-                                                     (k0 >> 7) * 2u, 0);
-    else          // without zero-points the resource is empty and the load returns 0
-      st.z[i] = __builtin_amdgcn_raw_buffer_load_b8(r.zr, soff[i] | dead, k0 >> 7, 0);
+  static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH], int kt, uint32_t dead, int i) {
+    load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, (uint32_t)kt * (kBK / 2));
   }
-  static __device__ __forceinline__ void begin(const Res& r, const Stage& st, Dq& q) {
+  static __device__ __forceinline__ void side_load(const Res& r, Side& d, int n, int pair, uint32_t dead) {
+    d.s = __builtin_amdgcn_raw_buffer_load_b16(r.sr, (uint32_t)n * (uint32_t)r.Kg * 2u | dead, (uint32_t)pair * 2u, 0);
+    // without zero-points the resource is empty and the load returns 0
+    d.z = __builtin_amdgcn_raw_buffer_load_b8(r.zr, (uint32_t)n * (uint32_t)r.Kg | dead, (uint32_t)pair, 0);
+  }
+  static __device__ __forceinline__ void side_store(const Side& d, unsigned char* at) { *reinterpret_cast<uint32_t*>(at) = d.s | d.z << 16; }
+  static __device__ __forceinline__ void begin(const Res& r, const uint32_t (&v)[B_CH], Dq& q) {
 #pragma unroll
     for (int i = 0; i < B_CH; ++i) {
-      const _Float16 sc = __builtin_bit_cast(_Float16, (uint16_t)st.s[i]);
-      const float z = r.has_zp ? (float)st.z[i] : 8.0f;
+      const _Float16 sc = __builtin_bit_cast(_Float16, (uint16_t)v[i]);
+      const float z = r.has_zp ? (float)(v[i] >> 16) : 8.0f;
       if constexpr (kHalf) {
         q.sh[i] = f16x2{sc, sc};
         q.nz[i] = both(-z);
@@ -243,15 +240,15 @@ struct WInt4 {
 // w = fp16(fp16(nib * scale) - min), the product rounded before the subtraction (two roundings,
 // as the dense dequantization does): one conversion, one packed product and one packed difference per
 // pair of weights.  fp16 activations only; pairs and x in the order of INT4's fp16 form.
-template <class Act, int BN, bool SIDE = false>
+template <class Act, int BN>
 struct WQ4K {
   static_assert(Act::dt == DT_F16, "Q4_K runs in fp16");
   static constexpr int CPR = BN <= 64 ? 4 : 2;        // chunks per row and 64-wide step: 8 bytes each on narrow tiles,
   static constexpr int DW = 8 / CPR;                  // so that every thread has one; dwords per chunk
   static constexpr double kWeightBytesPerK = 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
-  static constexpr bool kSide = SIDE;                 // scales and mins through the LDS table (see gemm_tiled_kernel)
-  static constexpr int LPC = SIDE ? 1 : 3;
+  static constexpr int kEntry = 16, LPC = 1;
+  static constexpr bool kHalfEntry = false;
   struct Side { u32x2 s, m; };                        // a row's scales and mins of 128 k
   static constexpr int PPD = 8;                       // pieces per dword of 8 nibbles
   static constexpr int kPieces = B_CH * DW * PPD;
@@ -264,7 +261,6 @@ struct WQ4K {
   };
   struct Stage {
     Dwords<DW> b[B_CH];
-    uint32_t s[SIDE ? 1 : B_CH], m[SIDE ? 1 : B_CH];  // fp16 bits (32-bit slots: 16-bit members end up on the stack)
   };
   struct Dq {
     uint32_t e, o;
@@ -280,37 +276,23 @@ struct WQ4K {
     r.mr = make_rsrc((const char*)p.zp + (long long)e * p.g_z_stride, (uint32_t)p.N * (uint32_t)r.Kc * 2u);
     return r;
   }
-  static __device__ __forceinline__ void chunk_addr(Res& r, int, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
-    boff = (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * DW * 4);
-    soff = ((uint32_t)n * (uint32_t)r.Kc + (uint32_t)(DW == 2 ? kc >> 1 : kc)) * 2u;   // bytes: one fp16 per 32 k
+  static __device__ __forceinline__ uint32_t chunk_addr(Res&, int, int n, int kc, int K) {
+    return (uint32_t)n * ((uint32_t)K >> 1) + (uint32_t)(kc * DW * 4);
   }
-  static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
-                                               const uint32_t (&soff)[B_CH], int kt, uint32_t dead, int idx) {
-    const uint32_t k0 = (uint32_t)kt * kBK;
-    const int i = idx / LPC, kind = idx % LPC;
-    if (kind == 0) load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, k0 >> 1);
-    if constexpr (SIDE) return;
-    if (kind == 1) st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, (k0 >> 5) * 2u, 0);
-    else if (kind == 2) st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, (k0 >> 5) * 2u, 0);
+  static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH], int kt, uint32_t dead, int i) {
+    load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, (uint32_t)kt * (kBK / 2));
   }
   static __device__ __forceinline__ void side_load(const Res& r, Side& d, int n, int pair, uint32_t dead) {
     const uint32_t off = (uint32_t)n * (uint32_t)r.Kc * 2u | dead;
     d.s = __builtin_amdgcn_raw_buffer_load_b64(r.sr, off, (uint32_t)pair * 8u, 0);
     d.m = __builtin_amdgcn_raw_buffer_load_b64(r.mr, off, (uint32_t)pair * 8u, 0);
   }
-  static __device__ __forceinline__ u32x4 side_entry(const Side& d) { return scale_min_pairs(d.s, d.m); }
-  static __device__ __forceinline__ void begin_side(const uint32_t (&v)[B_CH], Dq& q) {
+  static __device__ __forceinline__ void side_store(const Side& d, unsigned char* at) { *reinterpret_cast<u32x4*>(at) = scale_min_pairs(d.s, d.m); }
+  static __device__ __forceinline__ void begin(const Res&, const uint32_t (&v)[B_CH], Dq& q) {
 #pragma unroll
     for (int i = 0; i < B_CH; ++i) {
       q.sv[i] = both_bits(v[i]);
       q.mv[i] = both_bits(v[i] >> 16);
-    }
-  }
-  static __device__ __forceinline__ void begin(const Res&, const Stage& st, Dq& q) {
-#pragma unroll
-    for (int i = 0; i < B_CH; ++i) {
-      q.sv[i] = both_bits(st.s[i]);
-      q.mv[i] = both_bits(st.m[i]);
     }
   }
   static __device__ __forceinline__ void piece(const Stage& st, Dq& q, int I, unsigned char* const (&dst)[B_CH]) {
@@ -353,11 +335,12 @@ struct WGguf {
   static constexpr bool kHigh = F == GT_Q5K || F == GT_Q6K;
   static constexpr int CPR = F == GT_Q80 || BN <= 64 ? 4 : 2;
   static constexpr int DW = F == GT_Q80 ? 4 : 8 / CPR;   // dwords per chunk (nibbles: 8 bytes on narrow tiles, as INT4)
-  static_assert(!kPlainH || (DW == 4 && BN > 128), "high bits in element order: whole chunks of 32");
+  static_assert(!kPlainH || DW == 4, "high bits in element order: whole chunks of 32");
   static constexpr double kWeightBytesPerK = F == GT_Q80 ? 1.0 : F == GT_Q6K ? 0.75 : F == GT_Q5K ? 0.625 : 0.5;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
-  static constexpr bool kSide = kPlainH || (F == GT_Q5K && BN > 128);   // scales and mins through the LDS table (see gemm_tiled_kernel)
-  static constexpr int LPC = kSide ? 1 + (kHigh ? kPlainH ? 1 : 2 : 0) : (F == GT_Q5K ? 5 : F == GT_Q6K ? 4 : 2) - (kHigh && DW == 2 ? 1 : 0);
+  static constexpr int kEntry = 16;
+  static constexpr bool kHalfEntry = F == GT_Q6K && DW == 2;            // a chunk of 16 k: one of its entry's two scales
+  static constexpr int LPC = 1 + (!kHigh ? 0 : kPlainH ? 1 : DW / 2);
   static constexpr int PPD = F == GT_Q5K ? 13 : F == GT_Q6K ? 9 : F == GT_Q40 ? 8 : 3;   // pieces per dword (8 nibbles / 4 bytes)
   static constexpr int kPieces = B_CH * DW * PPD;
   static constexpr GemmDecode kDecode = kHigh ? GemmDecode::kDear : GemmDecode::kMid;
@@ -370,8 +353,6 @@ struct WGguf {
   };
   struct Stage {
     Dwords<DW> b[B_CH];
-    uint32_t s[kSide ? 1 : B_CH];
-    uint32_t m[F == GT_Q5K && !kSide ? B_CH : 1];
     u32x4 h[kHigh && !kPlainH ? B_CH : 1][DW / 2];
     u32x2 hp[kPlainH ? B_CH : 1];
     uint32_t sh;                                      // shift of this step's field of the high-bit bytes (uniform)
@@ -392,29 +373,21 @@ struct WGguf {
     r.hr = make_rsrc((const char*)p.qh + (long long)e * p.g_h_stride, F == GT_Q6K ? nk / 4 : F == GT_Q5K ? nk / 8 : 0u);
     return r;
   }
-  static __device__ __forceinline__ void chunk_addr(Res& r, int i, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
-    boff = (uint32_t)n * (F == GT_Q80 ? (uint32_t)K : (uint32_t)K >> 1) + (uint32_t)(kc * DW * 4);
-    soff = (uint32_t)n * (uint32_t)r.Ks + (uint32_t)(F == GT_Q6K ? kc * DW : (CPR == 4 ? kc >> 1 : kc) * 2);
+  static __device__ __forceinline__ uint32_t chunk_addr(Res& r, int i, int n, int kc, int K) {
     if constexpr (kHigh) r.hoff[i] = (uint32_t)n * (F == GT_Q6K ? (uint32_t)K >> 2 : (uint32_t)K >> 3) +
                                      (uint32_t)(kc * (!kPlainH ? DW * 8 : F == GT_Q6K ? 8 : 4));
+    return (uint32_t)n * (F == GT_Q80 ? (uint32_t)K : (uint32_t)K >> 1) + (uint32_t)(kc * DW * 4);
   }
-  static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
-                                               const uint32_t (&soff)[B_CH], int kt, uint32_t dead, int idx) {
+  static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH], int kt, uint32_t dead, int idx) {
     const uint32_t k0 = (uint32_t)kt * kBK;
     const int i = idx / LPC, kind = idx % LPC;
     if (kind == 0) load_dwords<DW>(st.b[i], r.wr, boff[i] | dead, F == GT_Q80 ? k0 : k0 >> 1);
     else if constexpr (kPlainH) {
       if constexpr (F == GT_Q6K) st.hp[i] = __builtin_amdgcn_raw_buffer_load_b64(r.hr, r.hoff[i] | dead, k0 >> 2, 0);
       else st.hp[i][0] = __builtin_amdgcn_raw_buffer_load_b32(r.hr, r.hoff[i] | dead, k0 >> 3, 0);
-    } else if (kind == 1 && !kSide) {
-      if constexpr (F == GT_Q6K && DW == 4 && !kSide) st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, k0 >> 3, 0);
-      else if constexpr (!kSide) st.s[i] = __builtin_amdgcn_raw_buffer_load_b16(r.sr, soff[i] | dead, F == GT_Q6K ? k0 >> 3 : k0 >> 4, 0);
-    } else if (kind == LPC - 1 && F == GT_Q5K && !kSide) {
-      if constexpr (F == GT_Q5K && !kSide) st.m[i] = __builtin_amdgcn_raw_buffer_load_b16(r.mr, soff[i] | dead, k0 >> 4, 0);
     } else if constexpr (kHigh) {
-      const int piece = kind - (kSide ? 1 : 2);
       const uint32_t tile = F == GT_Q6K ? (k0 >> 9) * 128u + (k0 & 127u) : (k0 >> 9) * 64u;
-      st.h[i][piece] = __builtin_amdgcn_raw_buffer_load_b128(r.hr, r.hoff[i] | dead, tile + (uint32_t)piece * 16u, 0);
+      st.h[i][kind - 1] = __builtin_amdgcn_raw_buffer_load_b128(r.hr, r.hoff[i] | dead, tile + (uint32_t)(kind - 1) * 16u, 0);
       st.sh = F == GT_Q6K ? (k0 >> 7 & 3u) * 2u : k0 >> 6 & 7u;
     }
   }
@@ -428,25 +401,16 @@ struct WGguf {
       if constexpr (F == GT_Q5K) d.m = __builtin_amdgcn_raw_buffer_load_b64(r.mr, off, (uint32_t)pair * 8u, 0);
     }
   }
-  static __device__ __forceinline__ u32x4 side_entry(const Side& d) {
-    if constexpr (F == GT_Q6K) return d.s;            // the two scales of every 32 k
-    else return scale_min_pairs(u32x2{d.s[0], d.s[1]}, F == GT_Q5K ? d.m : u32x2{0u, 0u});
+  static __device__ __forceinline__ void side_store(const Side& d, unsigned char* at) {
+    if constexpr (F == GT_Q6K) *reinterpret_cast<u32x4*>(at) = d.s;       // the two scales of every 32 k
+    else *reinterpret_cast<u32x4*>(at) = scale_min_pairs(u32x2{d.s[0], d.s[1]}, F == GT_Q5K ? d.m : u32x2{0u, 0u});
   }
-  static __device__ __forceinline__ void begin_side(const uint32_t (&v)[B_CH], Dq& q) {
+  static __device__ __forceinline__ void begin(const Res&, const uint32_t (&v)[B_CH], Dq& q) {
 #pragma unroll
     for (int i = 0; i < B_CH; ++i) {
       q.sv[i][0] = both_bits(v[i]);
       if constexpr (F == GT_Q6K && DW == 4) q.sv[i][1] = both_bits(v[i] >> 16);
       if constexpr (F == GT_Q5K) q.mv[i] = both_bits(v[i] >> 16);
-    }
-  }
-  static __device__ __forceinline__ void begin(const Res&, const Stage& st, Dq& q) {
-    if constexpr (kSide) return;
-#pragma unroll
-    for (int i = 0; i < (kSide ? 0 : B_CH); ++i) {
-      q.sv[i][0] = both_bits(st.s[i]);
-      if constexpr (F == GT_Q6K && DW == 4) q.sv[i][1] = both_bits(st.s[i] >> 16);
-      if constexpr (F == GT_Q5K) q.mv[i] = both_bits(st.m[i]);
     }
   }
   static __device__ __forceinline__ void piece(const Stage& st, Dq& q, int I, unsigned char* const (&dst)[B_CH]) {
@@ -527,10 +491,10 @@ struct WFp8 {
   static constexpr int CPR = 4;
   static constexpr double kWeightBytesPerK = 1.0;
   static constexpr int B_CH = (BN * CPR + 255) / 256;
-  static constexpr int LPC = BLOCK ? 2 : 1;
+  static constexpr int LPC = 1, kEntry = BLOCK ? 4 : 0;
+  static constexpr bool kHalfEntry = false;
   static constexpr int kPPC = BLOCK ? 10 : 4;         // pieces per chunk
   static constexpr int kPieces = B_CH * kPPC;
-  static constexpr bool kSide = false;
   static constexpr GemmDecode kDecode = BLOCK ? GemmDecode::kMid : GemmDecode::kCheap;
   static constexpr bool kOutScale = !BLOCK;
   static constexpr bool kPermK = false;
@@ -541,10 +505,11 @@ struct WFp8 {
   };
   struct Stage {
     u32x4 b[B_CH];
-    uint32_t s[BLOCK ? B_CH : 1];                     // block scale, fp32 bits
   };
+  struct Side { uint32_t s; };                        // block scale, fp32 bits
   struct Dq {
     u32x4 outv;
+    float s[BLOCK ? B_CH : 1];
   };
   // e: expert of a grouped launch (its matrices start e * stride bytes in)
   static __device__ __forceinline__ Res make(const GemmArgs& p, int e = 0) {
@@ -556,18 +521,18 @@ struct WFp8 {
     r.se = (const char*)p.scale + (long long)e * p.g_s_stride;
     return r;
   }
-  static __device__ __forceinline__ void chunk_addr(Res& r, int, int n, int kc, int K, uint32_t& boff, uint32_t& soff) {
-    boff = (uint32_t)n * (uint32_t)K + (uint32_t)(kc * 16);
-    soff = (uint32_t)(n >> 7) * (uint32_t)r.Kb * 4u;  // bytes: the row block's first scale
+  static __device__ __forceinline__ uint32_t chunk_addr(Res&, int, int n, int kc, int K) { return (uint32_t)n * (uint32_t)K + (uint32_t)(kc * 16); }
+  static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH], int kt, uint32_t dead, int i) {
+    st.b[i] = __builtin_amdgcn_raw_buffer_load_b128(r.wr, boff[i] | dead, (uint32_t)kt * kBK, 0);
   }
-  static __device__ __forceinline__ void load1(const Res& r, Stage& st, const uint32_t (&boff)[B_CH],
-                                               const uint32_t (&soff)[B_CH], int kt, uint32_t dead, int idx) {
-    const uint32_t k0 = (uint32_t)kt * kBK;
-    const int i = idx / LPC, kind = idx % LPC;
-    if (kind == 0) st.b[i] = __builtin_amdgcn_raw_buffer_load_b128(r.wr, boff[i] | dead, k0, 0);
-    else st.s[i] = __builtin_amdgcn_raw_buffer_load_b32(r.sr, soff[i] | dead, (k0 >> 7) * 4u, 0);
+  static __device__ __forceinline__ void side_load(const Res& r, Side& d, int n, int pair, uint32_t dead) {
+    d.s = __builtin_amdgcn_raw_buffer_load_b32(r.sr, (uint32_t)(n >> 7) * (uint32_t)r.Kb * 4u | dead, (uint32_t)pair * 4u, 0);
   }
-  static __device__ __forceinline__ void begin(const Res&, const Stage&, Dq&) {}
+  static __device__ __forceinline__ void side_store(const Side& d, unsigned char* at) { *reinterpret_cast<uint32_t*>(at) = d.s; }
+  static __device__ __forceinline__ void begin(const Res&, const uint32_t (&v)[B_CH], Dq& q) {
+#pragma unroll
+    for (int i = 0; i < (BLOCK ? B_CH : 0); ++i) q.s[i] = __builtin_bit_cast(float, v[i]);
+  }
   static __device__ __forceinline__ uint32_t pack2(float a, float b) {
     if constexpr (Act::dt == DT_F16) {
       const f16x2 r = {(_Float16)a, (_Float16)b};
@@ -602,8 +567,7 @@ struct WFp8 {
         const uint32_t w = st.b[i][half * 2 + (sub >> 1)];
         const f32x2 f = (sub & 1) ? __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true)
                                   : __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false);
-        const float sc = __builtin_bit_cast(float, st.s[i]);
-        q.outv[sub] = pack2(f[0] * sc, f[1] * sc);
+        q.outv[sub] = pack2(f[0] * q.s[i], f[1] * q.s[i]);
       }
     }
   }
@@ -614,7 +578,11 @@ struct WFp8 {
   }
 };
 
-struct NoSide { struct Side {}; };
+// LDS of a tile: two weight tiles of 64 k, and behind them two tables of scales (128 k, one entry per row).
+template <class Fmt> struct TileLds {
+  static constexpr int kTileBytes = Fmt::B_CH * 256 / Fmt::CPR * kPitch * 2;
+  static constexpr int kBytes = 2 * kTileBytes + 2 * 256 * Fmt::kEntry;
+};
 
 template <int... I, class F>
 __device__ __forceinline__ void fold_pieces(std::integer_sequence<int, I...>, F f) {
@@ -640,8 +608,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   constexpr int kLoads = Fmt::LPC * B_CH;             // load instructions per stage and thread
   static_assert(WM % 16 == 0 && WN % 16 == 0 && BNP >= BN, "tile shape");
 
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  Elem* Bs = reinterpret_cast<Elem*>(smem);                                   // [2][BNP][kPitch]
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];        // [2][BNP][kPitch], tables of scales
+  using Lds = TileLds<Fmt>;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -749,18 +717,14 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   };
 
   // ---- weights: per-thread chunk addresses at k = 0
-  uint32_t boff[B_CH], soff[B_CH];
+  auto row_live = [&](int row) { return row < BN && (FUSE ? n0 + (row >> 5) * 16 + (row & 15) < p.n_half : n0 + row < N); };
+  uint32_t boff[B_CH];
   unsigned char* blds[B_CH];
 #pragma unroll
   for (int i = 0; i < B_CH; ++i) {
-    const int c = tid + i * 256;
-    const int row = c / CPR, kc = c % CPR;
-    const int n = tile_row(row);
-    const bool live = FUSE ? (n0 + (row >> 5) * 16 + (row & 15) < p.n_half) : (n < N);
-    const uint32_t dead = (uint32_t)(!(live && row < BN)) << 31;
-    Fmt::chunk_addr(res, i, n, kc, K, boff[i], soff[i]);
-    boff[i] |= dead;
-    soff[i] |= dead;
+    const int row = (tid + i * 256) / CPR, kc = (tid + i * 256) % CPR;
+    const uint32_t dead = (uint32_t)!row_live(row) << 31;
+    boff[i] = Fmt::chunk_addr(res, i, tile_row(row), kc, K) | dead;
     blds[i] = smem + (row * kPitch + kc * (kBK / CPR)) * 2;
   }
   using StageB = typename Fmt::Stage;                 // weight chunks of one 64-wide step, in registers
@@ -769,50 +733,49 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   // on each.
   auto load_b1 = [&](StageB& st, int kt, int idx) {
     const uint32_t dead = kt < KT ? 0u : 0x80000000u;
-    Fmt::load1(res, st, boff, soff, kt, dead, idx);
+    Fmt::load1(res, st, boff, kt, dead, idx);
   };
   auto load_b = [&](StageB& st, int kt) {
 #pragma unroll
     for (int idx = 0; idx < kLoads; ++idx) load_b1(st, kt, idx);
   };
 
-  // Scales and mins through LDS (Fmt::kSide).  Loaded by the threads that dequantize a chunk they are 2 to 4 bytes of a line per
-  // row, array and step, and the lines of 256 rows do not stay in L1 until the next step: with those loads served from one
-  // line a GGUF layer of 2048 tokens took 306 instead of 363 us.  Thread t loads 128 k of tile row t at once, a 16-byte
-  // table entry (one dword per chunk of 32), every second step; two tables, behind the weight tiles.  In step kt (even) table
-  // kt / 2 + 1 is written; the steps that read it are kt + 1 and kt + 2, and its place was read last in step kt - 2.
-  // The large tiles of dense layers take it for Q5_K alone, the format with five loads per chunk (M x K x N 600 x 5120 x 14336 169 -> 153
-  // us, 1024 x 4096 x 12288 122 -> 119); Q4_K was 1 to 3 % slower with it there, Q4_0 and Q6_K between 1 % faster and 1.5 % slower.
-  unsigned char* const side = smem + 2 * (size_t)BNP * kPitch * 2;
-  static_assert(!Fmt::kSide || (!FUSE && !SPLIT && BNP == 256 && CPR == 2), "one table row per thread");
-  auto side_at = [&](int pair) { return side + (pair & 1) * 4096; };
-  auto load_side = [&](auto& d, int pair) {
-    if constexpr (Fmt::kSide)
-      Fmt::side_load(res, d, n0 + tid, pair, (uint32_t)(n0 + tid >= N || 2 * pair >= KT) << 31);
+  // Scales and mins through LDS.  Loaded by the threads that dequantize a chunk they are 2 to 4 bytes of a line per row,
+  // array and step, and the lines do not stay in L1 until the next step.  Thread t loads 128 k of tile row t at once, one table
+  // entry, every second step.  In step kt (even) table kt / 2 + 1 is written; the steps that read it are kt + 1 and kt + 2, and
+  // its place was read last in step kt - 2.  With loads per chunk / with the table, us, M x K x N: Q4_K 2048 x 5120 x 5120 112 / 109,
+  // Q5_K 1000 x 4096 x 12288 118 / 113, Q6_K 110 / 106, Q8_0 96.5 / 94, INT4 2048 x 4096 x 14336 201 / 199, Q4_K 500 x 5120 x 10240 75 / 71;
+  // block-scaled FP8 (one load per chunk that a wavefront shares) the same within 1 %.
+  constexpr int kEntry = Fmt::kEntry;
+  unsigned char* const side = smem + 2 * Lds::kTileBytes;
+  auto side_at = [&](int pair) { return side + (pair & 1) * (256 * kEntry); };
+  auto load_side = [&](auto& d, int pair) __attribute__((always_inline)) {
+    if constexpr (kEntry != 0) Fmt::side_load(res, d, tile_row(tid), pair, (uint32_t)(!row_live(tid) || 2 * pair >= KT) << 31);
   };
-  auto begin_stage = [&](const StageB& st, int kt, auto& q) {
-    if constexpr (Fmt::kSide) {
-      uint32_t v[B_CH];
-      const unsigned char* at = side_at(kt >> 1) + (kt & 1) * 8 + (tid >> 1) * 16 + (tid & 1) * 4;
+  auto begin_stage = [&](int kt, auto& q) __attribute__((always_inline)) {
+    uint32_t v[B_CH];
+    if constexpr (kEntry != 0) {
+      const int kc = tid % CPR;
+      const unsigned char* at = side_at(kt >> 1) + tid / CPR * kEntry + (kEntry == 16 ? (kt & 1) * 8 + kc * 2 / CPR * 4 : 0);
 #pragma unroll
-      for (int i = 0; i < B_CH; ++i) v[i] = *reinterpret_cast<const uint32_t*>(at + i * 2048);
-      Fmt::begin_side(v, q);
-    } else {
-      Fmt::begin(res, st, q);
+      for (int i = 0; i < B_CH; ++i) {
+        if constexpr (Fmt::kHalfEntry) v[i] = *reinterpret_cast<const uint16_t*>(at + i * (256 / CPR * kEntry) + (kc & 1) * 2);
+        else v[i] = *reinterpret_cast<const uint32_t*>(at + i * (256 / CPR * kEntry));
+      }
     }
+    Fmt::begin(res, v, q);
   };
 
   constexpr int kPieces = Fmt::kPieces;
   using DqState = typename Fmt::Dq;
-  constexpr size_t kBufBytes = (size_t)BNP * kPitch * 2;
   auto dq_piece = [&](const StageB& st, int buf, int I, DqState& q) {
     unsigned char* dst[B_CH];
 #pragma unroll
-    for (int i = 0; i < B_CH; ++i) dst[i] = blds[i] + buf * kBufBytes;
+    for (int i = 0; i < B_CH; ++i) dst[i] = blds[i] + buf * Lds::kTileBytes;
     Fmt::piece(st, q, I, dst);
   };
 
-  [[maybe_unused]] typename std::conditional_t<Fmt::kSide, Fmt, NoSide>::Side sd;
+  typename Fmt::Side sd;
   // One 64-wide K step: multiply out of LDS buffer `buf` (two 32-wide MFMA steps,
   // ring slots slot0 and slot0 + 1) while the next step's weights (`cur`, loaded one
   // step earlier) are dequantized into the other buffer and the weights two steps
@@ -821,50 +784,46 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   // first MFMA slot with (slot + 1) * kPieces / kMfmas > I
   auto step64 = [&](auto live_c, int kt, int buf, int slot0, StageB& cur, StageB& nxt) __attribute__((always_inline)) {
     constexpr int L = decltype(live_c)::value;        // activation tiles multiplied (<= TM)
-    constexpr int kMfmas = 2 * TN * L;
-    const Elem* Bb = Bs + buf * BNP * kPitch;
+    constexpr int U = 2 * TN, kMfmas = U * L;         // weight operands of the step
+    constexpr int R = L > 6 ? 2 : U < 8 ? 3 : 4;      // operands in registers: read from LDS R - 1 rows of MFMAs ahead
+    constexpr int kLead = L;                          // MFMAs ahead of the first piece, while the scales are read
     DqState q;
-    begin_stage(cur, kt + 1, q);
-    if constexpr (Fmt::kSide) {
+    begin_stage(kt + 1, q);
+    if constexpr (kEntry != 0) {
       if (buf == 0) {
-        *reinterpret_cast<u32x4*>(side_at((kt >> 1) + 1) + tid * 16) = Fmt::side_entry(sd);
+        Fmt::side_store(sd, side_at((kt >> 1) + 1) + tid * kEntry);
         load_side(sd, (kt >> 1) + 2);
       }
     }
-    auto rd_w = [&](int a, int s) {
-      return *reinterpret_cast<const u32x4*>(Bb + (wn0 + a * 16 + j) * kPitch + s * 32 + g * 8);
-    };
-    // the weight operand of row a + 1 is fetched from LDS while row a is multiplied
-    u32x4 wnext = rd_w(0, 0);
+    const unsigned char* const wread = smem + buf * Lds::kTileBytes + ((wn0 + j) * kPitch + g * 8) * 2;
+    auto rd_w = [&](int u) { return *reinterpret_cast<const u32x4*>(wread + (u % TN * 16 * kPitch + u / TN * 32) * 2); };
+    u32x4 wring[R];
+#pragma unroll
+    for (int u = 0; u + 1 < R; ++u) wring[u] = rd_w(u);
     constexpr int kHalf = TN * L;                     // MFMAs per 32-wide step
-    constexpr int kXEvery = kHalf / L;                // one activation load per kXEvery MFMAs
     constexpr int kBEvery = kHalf / kLoads > 0 ? kHalf / kLoads : 1;
+    // a fold, not a loop: the body exceeds what "#pragma unroll" expands, and a rolled loop would keep the rings on the stack
+    fold_pieces(std::make_integer_sequence<int, U>{}, [&](int u) __attribute__((always_inline)) {
+      const int s = u / TN, a = u % TN;
+      if (u + R - 1 < U) wring[(u + R - 1) % R] = rd_w(u + R - 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+      for (int b = 0; b < L; ++b) {
+        mfma_agpr<Act>(acc[a][b], wring[u % R], xring[slot0 + s][b]);
+        const int m = a * L + b, slot = u * L + b;    // MFMA inside this 32-wide step, and inside the step
+        const int p0 = slot < kLead ? 0 : (slot - kLead) * kPieces / (kMfmas - kLead);
+        const int p1 = slot < kLead ? 0 : (slot + 1 - kLead) * kPieces / (kMfmas - kLead);
 #pragma unroll
-      for (int a = 0; a < TN; ++a) {
-        const u32x4 wcur = wnext;
-        if (a + 1 < TN) wnext = rd_w(a + 1, s);
-        else if (s == 0) wnext = rd_w(0, 1);
-#pragma unroll
-        for (int b = 0; b < L; ++b) {
-          mfma_agpr<Act>(acc[a][b], wcur, xring[slot0 + s][b]);
-          const int m = a * L + b;                    // MFMA index inside this 32-wide step
-          const int slot = s * kHalf + m;
-          const int p0 = slot * kPieces / kMfmas, p1 = (slot + 1) * kPieces / kMfmas;
-#pragma unroll
-          for (int I = p0; I < p1; ++I) dq_piece(cur, buf ^ 1, I, q);
-          // global loads, one at a time: the ring slot multiplied in the previous
-          // 32-wide step is refilled 3 steps ahead, and in the first half the weight
-          // chunks two 64-wide steps ahead are fetched
-          if (m % kXEvery == kXEvery / 2 && m / kXEvery < L)
-            load_x1((slot0 + s + 3) & 3, m / kXEvery, 2 * kt + s + 3);
-          if (s == 0 && m % kBEvery == 0 && m / kBEvery < kLoads) load_b1(nxt, kt + 2, m / kBEvery);
-          // keep MFMAs, vector-ALU pieces and memory accesses in this order
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        for (int I = p0; I < p1; ++I) dq_piece(cur, buf ^ 1, I, q);
+        // global loads, one at a time: the ring slot multiplied in the previous
+        // 32-wide step is refilled 3 steps ahead, and in the first half the weight
+        // chunks two 64-wide steps ahead are fetched
+        if (m % TN == TN / 2 && m / TN < L) load_x1((slot0 + s + 3) & 3, m / TN, 2 * kt + s + 3);
+        if (s == 0 && m % kBEvery == 0 && m / kBEvery < kLoads) load_b1(nxt, kt + 2, m / kBEvery);
+        // keep MFMAs, vector-ALU pieces and memory accesses in this order
+        __builtin_amdgcn_sched_barrier(0);
       }
-    }
+    });
     // 8 wait states from the last MFMA until its result may be touched (as the compiler keeps them behind the same instruction as a
     // builtin): exits of the loop begin with copies of accumulators, also ahead of a wait that stands behind the loop.  Here
     // they run in the shadow of the LDS writes (Q6_K 500 x 5120 x 5120 47.0 us with and without; 16 of them cost 0.5 %).
@@ -873,23 +832,26 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   };
 
   StageB s0, s1;
-  if constexpr (Fmt::kSide) load_side(sd, 0);
-  load_b(s0, kt0);
-  __builtin_amdgcn_sched_barrier(0);
-  load_b(s1, kt0 + 1);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    __builtin_amdgcn_sched_barrier(0);               // keep the ring's loads in issue order
-    load_x(r, 2 * kt0 + r);
-  }
-  if constexpr (Fmt::kSide) {
-    *reinterpret_cast<u32x4*>(side_at(0) + tid * 16) = Fmt::side_entry(sd);
-    load_side(sd, 1);
-    __syncthreads();
-  }
   {
+    // everything that the loop waits for is requested ahead of the ring's loads: the loop's waits are those of its first turn
+    typename Fmt::Side sd0;
+    load_side(sd0, kt0 >> 1);
+    load_side(sd, (kt0 >> 1) + 1);
+    load_b(s0, kt0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_b(s1, kt0 + 1);
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      __builtin_amdgcn_sched_barrier(0);             // keep the ring's loads in issue order
+      load_x(r, 2 * kt0 + r);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kEntry != 0) {
+      Fmt::side_store(sd0, side_at(kt0 >> 1) + tid * kEntry);
+      __syncthreads();
+    }
     DqState q;
-    begin_stage(s0, kt0, q);
+    begin_stage(kt0, q);
     // a fold, not a loop: the pieces of the longer formats exceed what "#pragma unroll" expands, and a rolled
     // loop would keep the stage on the stack
     fold_pieces(std::make_integer_sequence<int, kPieces>{}, [&](int I) __attribute__((always_inline)) { dq_piece(s0, 0, I, q); });
@@ -986,7 +948,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   constexpr int RPP = 64 / LPR;                       // rows per store instruction
   constexpr int PASSES = (16 + RPP - 1) / RPP;
   constexpr int OPITCH = WNO * 2 + 16;                // a row of the wave tile + a slot for the row's offset
-  static_assert(WNO % 8 == 0 && 4 * 16 * OPITCH <= 2 * BNP * kPitch * 2, "output staging tile");
+  static_assert(WNO % 8 == 0 && 4 * 16 * OPITCH <= 2 * Lds::kTileBytes, "output staging tile");
   if (((n_out | ld) & 7) == 0 && out_bytes < (1ull << 31) && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0) {
     // Each 16-row tile of results is rounded, turned through a tile in LDS that belongs to this
     // wavefront alone (the weight tiles are free after the K loop's last barrier; the LDS queue of a
@@ -1204,7 +1166,7 @@ static int launch_gemm_tiled(GemmArgs p, hipStream_t st) {
       if (!p.xcd_m || cost < best) { best = cost; p.xcd_m = a; }
     }
   }
-  const size_t lds = (size_t)2 * (Fmt::B_CH * 256 / Fmt::CPR) * kPitch * 2 + (Fmt::kSide ? 2 * 4096 : 0);
+  constexpr size_t lds = TileLds<Fmt>::kBytes;
   auto kern = gemm_tiled_kernel<Act, Fmt, BM, BN, false, false, SPLIT, WR>;
   if (lds > 64 * 1024) {
     static bool raised = false;                       // opt in to > 64 KiB of dynamic LDS once

@@ -120,7 +120,7 @@ static int launch_grouped(GemmArgs p, int max_tiles, hipStream_t st) {
   p.tiles_n = FUSE ? (p.n_half + BN / 2 - 1) / (BN / 2) : (p.N + BN - 1) / BN;
   using F = FMT<Act, BN>;
   auto kern = gemm_tiled_kernel<Act, F, kMoeBM, BN, true, FUSE>;
-  const size_t lds = (size_t)2 * (F::B_CH * 256 / F::CPR) * kPitch * 2;
+  constexpr size_t lds = TileLds<F>::kBytes;
   static bool raised = false;
   if (lds > 64 * 1024 && !raised) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=

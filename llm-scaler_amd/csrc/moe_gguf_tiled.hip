@@ -16,7 +16,6 @@ constexpr int kGgufBM = 256, kGgufBN = 256;
 constexpr int kChunkRows = 64;                        // rows of a chunk that count
 constexpr int kChunkMapThreads = 1024;
 
-template <class Act, int BN> using WQ4KS = WQ4K<Act, BN, true>;
 template <class Act, int BN> using WQ5P = WGguf<Act, BN, GT_Q5P>;
 template <class Act, int BN> using WQ6P = WGguf<Act, BN, GT_Q6P>;
 
@@ -116,7 +115,7 @@ static int launch_chunk_gemm(GemmArgs p, int nmat, int max_tiles, hipStream_t st
   p.tiles_n = nmat * ((p.N + kGgufBN - 1) / kGgufBN);
   if ((long long)p.tiles_m * p.tiles_n >= (1LL << 31)) return MI_ERR_SHAPE;
   auto kern = gemm_tiled_kernel<ActF16, F, kGgufBM, kGgufBN, true, false>;
-  constexpr size_t lds = (size_t)2 * (F::B_CH * 256 / F::CPR) * kPitch * 2 + 2 * 4096;   // weight tiles, tables of scales
+  constexpr size_t lds = TileLds<F>::kBytes;
   if (lds > 64 * 1024) {
     static const int raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess ? MI_OK : MI_ERR_LAUNCH;
@@ -216,7 +215,7 @@ int mi_moe_gguf_grouped_tiled_ws(int fmt, const void* x, int x_rows, const int32
   p.g_z_stride = nk / 16;
   p.g_h_stride = fmt == 5 ? nk / 8 : nk / 4;
   p.x_blocks = max_blocks; p.out_rows = out_rows; p.out_ld = (int)out_stride;
-  if (fmt == 2) return launch_chunk_gemm<WQ4KS>(p, nmat, num_chunks, st);
+  if (fmt == 2) return launch_chunk_gemm<WQ4K>(p, nmat, num_chunks, st);
   return fmt == 5 ? launch_chunk_gemm<WQ5P>(p, nmat, num_chunks, st) : launch_chunk_gemm<WQ6P>(p, nmat, num_chunks, st);
 }
 
