@@ -594,10 +594,11 @@ __device__ __forceinline__ void fold_pieces(std::integer_sequence<int, I...>, F 
 // (MoE: rows sorted by expert, one weight matrix per expert).  FUSE: the tile's weight rows
 // alternate, 16 at a time, between a gate block and the up block n_half rows further on, and the
 // epilogue writes act(gate) * up (N / 2 output columns).
+// OCC: workgroups per CU that the registers have to leave room for.  WR: rows of the grid of wavefronts.
 // SPLIT: blockIdx.y takes one slice of K and the fp32 sums go to a workspace in accumulator order (1 KiB
 // per store); split_reduce_kernel adds the slices and writes the output.
-template <class Act, class Fmt, int BM, int BN, bool GROUPED = false, bool FUSE = false, bool SPLIT = false, int WR = 2>
-__global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
+template <class Act, class Fmt, int BM, int BN, bool GROUPED = false, bool FUSE = false, bool SPLIT = false, int OCC = 1, int WR = 2>
+__global__ __launch_bounds__(256, OCC) void gemm_tiled_kernel(const GemmArgs p) {
   using Elem = typename Act::elem;
   constexpr int WC = 4 / WR;                          // the wavefronts form a WR x WC grid
   constexpr int WM = BM / WR, WN = BN / WC;           // wave sub-tile
@@ -676,17 +677,14 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   GemmArgs mat = p;
   mat.w = mw; mat.scale = ms; mat.zp = mz;
   typename Fmt::Res res = Fmt::make(mat, expert);
-  // 16-row activation tile b of this wavefront inside the BM-row tile.  GROUPED: the two wavefront
-  // rows take the tiles alternately and a wavefront multiplies only the first 8, 6, 5, 4, 3 or 2 of
-  // its tiles, whichever covers the `live` ones with rows of the expert in them (the K loop exists
-  // in these lengths; a branch per MFMA costs more than it saves), so an expert's short last tile costs a
-  // fraction of the matrix-core time.  With 8, 4 and 2 alone an expert of 129 .. 160 rows paid for 256: FP8 experts, 2500
-  // tokens top 8 of 128, 367 -> 324 us, 2200 334 -> 301; GGUF experts, 2048 tokens, 387 -> 357.  A length of 7 as well made
-  // the kernel longer and every size 2 % slower.
+  // 16-row activation tile b of this wavefront inside the BM-row tile.  GROUPED: the wavefronts stacked along M
+  // take the tiles in turn and a wavefront multiplies only the first 4, 3, 2 or 1 of its tiles, as many as have rows of the
+  // expert in them (the K loop exists in these lengths; a branch per MFMA costs more than it saves), so an expert's
+  // short last tile costs a fraction of the matrix-core time.
   const int wr = wave / WC;
-  auto mtile = [&](int b) { return GROUPED ? 2 * b + wr : wr * TM + b; };
+  auto mtile = [&](int b) { return GROUPED ? WR * b + wr : wr * TM + b; };
   int live = TM;
-  if constexpr (GROUPED) live = __builtin_amdgcn_readfirstlane((((M + 15) >> 4) - wr + 1) >> 1);
+  if constexpr (GROUPED) live = __builtin_amdgcn_readfirstlane((((M + 15) >> 4) - wr + WR - 1) / WR);
   // weight row of row r of the LDS tile
   auto tile_row = [&](int r) { return FUSE ? n0 + (r >> 5) * 16 + (r & 15) + ((r >> 4) & 1) * p.n_half : n0 + r; };
 
@@ -866,13 +864,11 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const GemmArgs p) {
   if constexpr (!GROUPED) {
     k_loop(std::integral_constant<int, TM>{});
   } else {
-    static_assert(TM == 8, "loop lengths");
-    if (live > 6) k_loop(std::integral_constant<int, 8>{});
-    else if (live > 5) k_loop(std::integral_constant<int, 6>{});
-    else if (live > 4) k_loop(std::integral_constant<int, 5>{});
-    else if (live > 3) k_loop(std::integral_constant<int, 4>{});
+    static_assert(TM == 4, "loop lengths");
+    if (live > 3) k_loop(std::integral_constant<int, 4>{});
     else if (live > 2) k_loop(std::integral_constant<int, 3>{});
-    else k_loop(std::integral_constant<int, 2>{});
+    else if (live > 1) k_loop(std::integral_constant<int, 2>{});
+    else k_loop(std::integral_constant<int, 1>{});
   }
 
   // D = W-tile (rows n) x X-tile^T: lane holds n = 4 g + v (v = 0..3), m = j
@@ -1167,7 +1163,7 @@ static int launch_gemm_tiled(GemmArgs p, hipStream_t st) {
     }
   }
   constexpr size_t lds = TileLds<Fmt>::kBytes;
-  auto kern = gemm_tiled_kernel<Act, Fmt, BM, BN, false, false, SPLIT, WR>;
+  auto kern = gemm_tiled_kernel<Act, Fmt, BM, BN, false, false, SPLIT, 1, WR>;
   if (lds > 64 * 1024) {
     static bool raised = false;                       // opt in to > 64 KiB of dynamic LDS once
     if (!raised) {

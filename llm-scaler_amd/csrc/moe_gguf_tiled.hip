@@ -10,9 +10,9 @@
 
 namespace qlin {
 
-// 256 x 256 like the FP8 experts' tiles (a wavefront skips the row tiles past the chunk's last): 2048 tokens, top 8 of
-// 128 experts, H = 2048, I = 768: 404 us for the layer against 445 on 128 x 128 when the tile was chosen, 334 now; 510 with the chunk kernel.
-constexpr int kGgufBM = 256, kGgufBN = 256;
+// 256 x 128, two workgroups per CU, like the FP8 experts' tiles (a wavefront skips the row tiles past the chunk's last).  Layer with top 8
+// of 128 experts, H = 2048, I = 768, 256 x 256 (one workgroup per CU) / 256 x 128, us: 1000 tokens 259 / 235, 1500 292 / 270, 2048 332 / 310.
+constexpr int kGgufBM = 256, kGgufBN = 128;
 constexpr int kChunkRows = 64;                        // rows of a chunk that count
 constexpr int kChunkMapThreads = 1024;
 
@@ -114,7 +114,7 @@ static int launch_chunk_gemm(GemmArgs p, int nmat, int max_tiles, hipStream_t st
   p.tiles_m = (max_tiles + 7) / 8 * 8;                // whole rounds of the 8 XCDs (surplus workgroups exit)
   p.tiles_n = nmat * ((p.N + kGgufBN - 1) / kGgufBN);
   if ((long long)p.tiles_m * p.tiles_n >= (1LL << 31)) return MI_ERR_SHAPE;
-  auto kern = gemm_tiled_kernel<ActF16, F, kGgufBM, kGgufBN, true, false>;
+  auto kern = gemm_tiled_kernel<ActF16, F, kGgufBM, kGgufBN, true, false, false, 2, 4>;
   constexpr size_t lds = TileLds<F>::kBytes;
   if (lds > 64 * 1024) {
     static const int raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -142,7 +142,7 @@ static bool chunk_tiles_pay(bool up, long long n, long long out_rows, long long 
   if (kChunkRows * n > out_rows + kChunkRows * E) return false;
   const long long rows = out_rows <= kChunkRows * n ? out_rows : std::max(n, kChunkRows * (n - E));
   const long long used = std::min(E, n), m_tiles = std::min(n, std::max(used, (2 * n + 3 * used + 7) / 8));
-  const long long cus = device_cu_count_gemm(), n_tiles = nmat * ((N + kGgufBN - 1) / kGgufBN);
+  const long long cus = device_cu_count_gemm(), n_tiles = nmat * ((N + 255) / 256);
   const double rounds = (double)((m_tiles * n_tiles + cus - 1) / cus), full = (double)(rows * n_tiles) / (double)(kGgufBM * cus);
   const double steps = (double)(K / 64), weights = (double)(nmat * N * K) / 1e6, r64 = (double)rows / kChunkRows;
   const double tiled = up ? 17.0 + steps * (0.97 * rounds + 1.64 * full) : 18.0 + steps * (1.11 * rounds + 2.16 * full);
