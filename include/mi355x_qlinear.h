@@ -547,6 +547,25 @@ int mi_moe_gemv_fp8_block_routed(const void* x, int x_div, int x_silu, const voi
                                  const float* shared_scale, int shared_rows, int shared_x_first, int N, int K,
                                  int act_dtype, void* stream);
 
+/* Routing and gate_up rows of the same step in one launch: softmax top-k of logits [T, E] (renormalised, lowest index first among
+ * equals) into top_ids / top_w [T, topk], gate[t] = sigmoid(x[t] . gate_weight), and gate_up[t topk + j] = x[t] @
+ * dequant(w[top_ids[t, j]])^T, gate_up[T topk + t] = x[t] @ dequant(shared_w)^T.  w [E, 2 I, H], shared_w [2 I, H] e4m3 with 128 x 128
+ * block scales; H % 128 == 0, I % 128 == 0, E <= 1024, topk <= 64; MI_ERR_LIMIT for H > 4096 (V/csrc/moe_batch/moe.sycl:1509-1582). */
+int mi_moe_gate_up_topk_fp8_block(const void* x, const void* logits, const void* gate_weight, const void* w, const float* w_scale,
+                                  const void* shared_w, const float* shared_scale, void* gate_up, int32_t* top_ids, void* top_w,
+                                  float* gate, int T, int topk, int num_experts, int H, int I, int act_dtype, void* stream);
+
+/* The down projections of the same step and their sum in one launch:
+ * out[t, :] = sum_j top_w[t, j] (act(gate_up[t topk + j, :]) @ dequant(w[top_ids[t, j]])^T)
+ *           + gate[t] (act(gate_up[T topk + t, :]) @ dequant(shared_w)^T), act(row) = silu(gate half) * up half rounded to the
+ * activation type; sums in fp32, one rounding.  gate_up [T topk + T, 2 I], top_w [T, topk] and out [T, H] in the
+ * activation type, gate [T] fp32, w [E, H, I] and shared_w [H, I] e4m3 with 128 x 128 block scales; ids are held into [0, E).
+ * H % 128 == 0, I % 128 == 0; MI_ERR_LIMIT where the token's (topk + 1) I activations exceed 64 KiB
+ * (V/csrc/moe_batch/moe.sycl:1583-1663). */
+int mi_moe_down_sum_fp8_block(const void* gate_up, const void* w, const float* w_scale, const void* shared_w, const float* shared_scale,
+                              const int32_t* top_ids, const void* top_w, const float* gate, void* out, int T, int topk,
+                              int num_experts, int H, int I, int act_dtype, void* stream);
+
 /* The same GEMM with the per-expert-scalar scale of the reference's per-tensor MoE
  * kernels and their epilogues:
  *   scale_per_expert = 1: w_scale is [E] fp32 (one factor per expert); K may then be
