@@ -160,6 +160,16 @@ def test_merged_chunks_are_expected_where_they_were_measured_faster():
     assert lib.mi_moe_gguf_grouped_tiled_pays(2, 2, 4, 64, 8, 64, 128, None) == -1
 
 
+@pytest.mark.parametrize("case, tiles", [((6, 16, 576, 8, 4096, 2048), 1), ((5, 14, 569, 8, 4096, 2048), 1), ((6, 78, 3578, 60, 2560, 1536), 1),
+                                         ((6, 39, 1908, 32, 2048, 1024), 1), ((5, 136, 3003, 128, 2048, 768), 0),
+                                         ((6, 256, 8192, 256, 2048, 512), 0), ((5, 32, 1536, 32, 2048, 1024), 0)])
+def test_down_launches_either_side_of_the_line(case, tiles):
+    """Down launches near the line of mi_moe_gguf_grouped_tiled_pays, where either kernel was measured ahead by 9 % and more."""
+    p = ctypes.c_int(-1)
+    fmt, n, rows, E, N, K = case
+    assert capi.lib().mi_moe_gguf_grouped_tiled_pays(fmt, 1, n, rows, E, N, K, ctypes.byref(p)) == 0 and p.value == tiles
+
+
 def test_moe_grouped_module_matches_the_reference_binding():
     """Names, argument order and defaults of the pybind module the patched SGLang imports
     (S/csrc/moe_grouped/moe_grouped_entry.sycl:108-127, sglang_for_multi_arc.patch:2114)."""
