@@ -181,7 +181,7 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_sum_kernel(const DownSum
   const unsigned per = (unsigned)I >> 4, total = per * (unsigned)(k + 1);      // 16-byte pieces of a route's row, of an output row
   u32x4 wv[RPW][kDownPieces];
   float f[RPW][kDownPieces];                          // block scale x routing weight (or the shared expert's gate)
-  // request the pieces [s0, + 64 x kDownPieces); rows past H and pieces past the end repeat valid ones, with factor 0
+  // request the pieces [s0, + 64 x kDownPieces); rows past H and pieces past the end repeat valid ones
   auto request = [&](unsigned s0) __attribute__((always_inline)) {
     unsigned s[kDownPieces], r[kDownPieces];
     int e[kDownPieces];
@@ -210,9 +210,8 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_sum_kernel(const DownSum
     for (int i = 0; i < kDownPieces; ++i) {
       const bool shared = r[i] >= (unsigned)k;
       const float m = shared ? p.gate[t] : Act::to_f32(((const Elem*)p.route_weight)[(size_t)t * k + (shared ? 0 : r[i])]);
-      const float keep = s0 + i * 64 + lane < total ? m : 0.0f;
 #pragma unroll
-      for (int q = 0; q < RPW; ++q) f[q][i] *= keep;
+      for (int q = 0; q < RPW; ++q) f[q][i] *= m;
     }
   };
   float acc[RPW];
@@ -222,7 +221,8 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_sum_kernel(const DownSum
 #pragma unroll
     for (int i = 0; i < kDownPieces; ++i) {
       unsigned s = s0 + i * 64 + lane;
-      if (s >= total) s = total - 1;
+      const bool mine = s < total;                    // selected, not multiplied by 0: what is repeated may be infinite
+      if (!mine) s = total - 1;
       const u32x4 a0 = *reinterpret_cast<const u32x4*>(smem + (size_t)s * 32), a1 = *reinterpret_cast<const u32x4*>(smem + (size_t)s * 32 + 16);
 #pragma unroll
       for (int q = 0; q < RPW; ++q) {
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_sum_kernel(const DownSum
         for (int j = 0; j < 4; ++j) d = Dot2<Act>::run(b0[j], a0[j], d);
 #pragma unroll
         for (int j = 0; j < 4; ++j) d = Dot2<Act>::run(b1[j], a1[j], d);
-        acc[q] += d * f[q][i];
+        acc[q] += mine ? d * f[q][i] : 0.0f;
       }
     }
   };

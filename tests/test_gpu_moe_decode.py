@@ -43,6 +43,27 @@ def test_down_projections_and_their_sum(dev, dt, T, k, E, H, I):
     assert bool(((out.cpu().double() - ref).abs() <= eps * ref.abs() + (2.0 ** -18 + eps / 16) * scale).all())
 
 
+@pytest.mark.parametrize("T,k,E,H,I", [(1, 8, 16, 256, 768), (3, 1, 2, 128, 128), (12, 4, 8, 1152, 256)])     # 80, 496 and 432 pieces past the end
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_an_infinity_stays_one(dev, dt, T, k, E, H, I):
+    """An activation of the shared expert's last piece overflows: its products are infinite, of the weight's sign, and no lane beyond
+    the sequence's end may turn them into NaN."""
+    from mi355x_qlinear import capi
+    g = torch.Generator().manual_seed(T + k + I)
+    gu = torch.randn(T * k + T, 2 * I, generator=g).to(dt)
+    gu[-1, I - 1], gu[-1, 2 * I - 1] = torch.finfo(dt).max, 4.0          # the last token's shared expert: silu(max) x 4
+    w, ws, _ = _fp8(E, H, I, g=g)
+    sw, sws, swd = _fp8(H, I, g=g)
+    sign = torch.where(torch.arange(H) % 2 == 0, 0x38, 0xB8).to(torch.uint8)    # 1 and -1
+    sw[:, -1] = sign.view(sw.dtype) if sw.dtype != torch.uint8 else sign
+    ids, tw, gate = torch.randint(0, E, (T, k), generator=g).to(torch.int32), torch.rand(T, k, generator=g).to(dt), torch.rand(T, generator=g) + 0.1
+    out = torch.zeros(T, H, dtype=dt, device=dev)
+    d = [t.to(dev) for t in (gu, w, ws, sw, sws, ids, tw, gate)]
+    capi.call("mi_moe_down_sum_fp8_block", d[0], *[capi.ptr(t) for t in d], capi.ptr(out), T, k, E, H, I, capi.act_dtype(d[0]))
+    want = torch.where(torch.arange(H) % 2 == 0, float("inf"), float("-inf")).to(dt)
+    assert torch.equal(out[-1].cpu(), want) and bool(out[:-1].isfinite().all())
+
+
 # x of less than a piece per lane, of whole pieces, and of a partial last one; a wavefront's rows across two experts; 2 to 16 keys per lane
 @pytest.mark.parametrize("T,k,E,H,I", [(1, 1, 1, 128, 128), (1, 8, 128, 2048, 128), (3, 2, 5, 1024, 128), (2, 3, 130, 1152, 128), (4, 64, 65, 256, 128),
                                        (1, 4, 300, 2176, 128), (2, 5, 1024, 4096, 128), (16, 8, 40, 512, 256)])
