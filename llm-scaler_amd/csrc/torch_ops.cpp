@@ -337,9 +337,10 @@ RESADD_NORM(esimd_resadd_norm_gemv_int4_pert, true)
 RESADD_NORM(esimd_resadd_norm_gemv_fp8_pert, false)
 
 // ---------------------------------------------------------------------------------------- MoE decode
-// (token, route) pairs up to which one GEMV runs per route (16 tokens x top 8: 121 us against 133 grouped, 18 tokens 140 against 134;
-// 128 experts, H = 2048, I = 768); beyond, Python's grouped path
-constexpr int64_t kRoutedPairs = 128;
+// (token, route) pairs up to which one GEMV runs per route (12 tokens x top 8); beyond, Python's grouped path, which reads an expert once
+// and rounds once between gate_up and down (16 tokens x top 8 of 128, H = 2048, I = 768: 133 us, 121 with a GEMV per route, whose gate_up rows are rounded
+// before SiLU x up; the routes' error against 64 bits is 1.4 times that)
+constexpr int64_t kRoutedPairs = 96;
 
 bool shape_is(const Tensor& t, at::IntArrayRef s) { return t.sizes() == s; }
 

@@ -1205,7 +1205,7 @@ def moe_gemm_fp8_block(a, a_scale, row_map, weight, weight_scale, expert_start, 
 ROUTED_MAX_PAIRS = 8192       # (token, route) pairs one routed gate_up launch sorts by itself
 GATE_UP_MAX_COLUMNS = 4096       # hidden size up to which the gate_up launch selects the experts itself
 DOWN_SUM_MAX_BYTES = 64 * 1024    # (top_k + 1) activation rows of a token that the one-launch down projection holds
-ROUTED_GEMV_MAX_PAIRS = 128   # (token, route) pairs up to which the fused decode op runs one GEMV per route (16 tokens x top 8)
+ROUTED_GEMV_MAX_PAIRS = 96    # (token, route) pairs up to which the fused decode op runs one GEMV per route (12 tokens x top 8)
 
 
 def moe_gate_up_fp8_routed(xq, xs, top_ids, weight, weight_scale, expert_start, inv, sorted_pairs, output,

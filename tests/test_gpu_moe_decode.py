@@ -131,3 +131,36 @@ def test_a_token_too_long_for_one_launch(dev):
     assert ((out.cpu().float() - ref).abs().mean() / ref.abs().mean()).item() < 3e-3
     p = capi.ptr(out)
     assert getattr(capi.lib(), "mi_moe_down_sum_fp8_block")(p, p, p, p, p, p, p, p, p, T, k, E, H, I, 0, None) == -4
+
+
+@pytest.mark.parametrize("T,k,E", [(13, 8, 16), (16, 8, 128), (97, 1, 8)])     # 104, 128 and 97 pairs
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_pairs_past_the_line_are_rounded_once_between_the_projections(dev, dt, T, k, E):
+    """Above 96 (token, route) pairs the operator's routed part (the shared expert's gate is 0 here) has the error of 64-bit math with the routing
+    weights, SiLU(gate) x up and the output rounded, and not the 1.3 times that of gate_up rows rounded as well."""
+    import custom_esimd_kernels_vllm  # noqa: F401
+    H, I = 512, 256
+    g = torch.Generator().manual_seed(T + E)
+    x, logits, gw = torch.randn(T, H, generator=g).to(dt), (torch.randn(T, E, generator=g) * 0.4).to(dt), torch.zeros(1, H).to(dt)
+    x[:, 0], gw[0, 0] = 8.0, -32.0                          # sigmoid(-256) = 0 in fp32
+    w13, s13, d13 = _fp8(E, 2 * I, H, g=g)
+    w2, s2, d2 = _fp8(E, H, I, g=g)
+    sw13, ss13, _ = _fp8(2 * I, H, g=g)
+    sw2, ss2, _ = _fp8(H, I, g=g)
+    f8 = lambda t: t.view(torch.float8_e4m3fn).to(dev)
+    out = torch.empty(T, H, dtype=dt, device=dev)
+    torch.ops.moe_ops.moe_forward_full_fp8_block(x.to(dev), logits.to(dev), out, f8(w13), s13.to(dev), f8(sw13), ss13.to(dev), f8(w2),
+                                                 s2.to(dev), f8(sw2), ss2.to(dev), gw.to(dev), k, 1, E)
+    top = torch.argsort(logits.double(), dim=1, descending=True, stable=True)[:, :k]
+    tw = torch.softmax(logits.double().gather(1, top), 1)
+    exact, once, twice = (torch.zeros(T, H, dtype=torch.float64) for _ in range(3))
+    rnd, same = (lambda v: v.to(dt).double()), (lambda v: v)
+    for t in range(T):
+        for j in range(k):
+            gu = d13[top[t, j]].double() @ x[t].double()
+            for o, r_gu, r in ((exact, same, same), (once, same, rnd), (twice, rnd, rnd)):
+                a, b = r_gu(gu[:I]), r_gu(gu[I:])
+                o[t] += r(tw[t, j]) * (d2[top[t, j]].double() @ r(a / (1 + torch.exp(-a)) * b))
+    err = lambda o: float((o - exact).norm() / exact.norm())
+    got, lo, hi = err(out.cpu().double()), err(rnd(once)), err(rnd(twice))
+    assert got < (lo + hi) / 2, (got, lo, hi)
