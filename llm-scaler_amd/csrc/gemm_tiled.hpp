@@ -677,7 +677,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tiled_kernel(const GemmArgs p) 
   mat.w = mw; mat.scale = ms; mat.zp = mz;
   typename Fmt::Res res = Fmt::make(mat, expert);
   // 16-row activation tile b of this wavefront inside the BM-row tile.  GROUPED: the wavefronts stacked along M
-  // take the tiles in turn and a wavefront multiplies only the first 5, 4, 3, 2 or 1 of its tiles, as many as have rows of the
+  // take the tiles in turn and a wavefront multiplies only the first 4, 3, 2 or 1 of its tiles, as many as have rows of the
   // expert in them (the K loop exists in these lengths; a branch per MFMA costs more than it saves), so an expert's
   // short last tile costs a fraction of the matrix-core time.
   const int wr = wave / WC;
@@ -863,9 +863,8 @@ __global__ __launch_bounds__(256, OCC) void gemm_tiled_kernel(const GemmArgs p) 
   if constexpr (!GROUPED) {
     k_loop(std::integral_constant<int, TM>{});
   } else {
-    static_assert(TM == 4 || TM == 5, "loop lengths");
-    if (TM > 4 && live > 4) k_loop(std::integral_constant<int, TM>{});
-    else if (live > 3) k_loop(std::integral_constant<int, 4>{});
+    static_assert(TM == 4, "loop lengths");
+    if (live > 3) k_loop(std::integral_constant<int, 4>{});
     else if (live > 2) k_loop(std::integral_constant<int, 3>{});
     else if (live > 1) k_loop(std::integral_constant<int, 2>{});
     else k_loop(std::integral_constant<int, 1>{});

@@ -114,20 +114,15 @@ static inline TiledMoeLayout tiled_moe_layout(int total_rows, int E, int K, int 
 // is decoded once per 256 rows, and a wavefront skips the 16-row tiles past the expert's last row.  128 experts, top 8, H = 2048, I = 768,
 // 256 x 256 (one workgroup per CU) / 256 x 128, us for the layer: 2000 tokens 280 / 264, 2500 309 / 292, 3500 404 / 367, 4096 497 / 457.
 constexpr int kMoeBM = 256, kMoeBN = 128;
-constexpr int kMoeTallBM = 320, kMoeTallBN = 192;
-// 320 x 192 (one workgroup per CU) where experts have 250 to 312 rows on average: most of those past 256 then fit one tile, where 256
-// rows leave a second one that decodes all columns again for a few rows.  Layer of the sizes above, 256 x 128 / 320 x 192, us: 4096 tokens (256
-// rows each) 471 / 424, 4300 520 / 446, 4600 538 / 492, 5000 552 / 545; below and above it is behind: 3700 395 / 396, 5200 592 / 619.  Random
-// routing; the host does not know the counts.  The same number for every expert: 4096 384 / 412, 4300 529 / 448, 5000 546 / 480;
-// skewed counts (experts' logits apart by 0.3 / 1 standard deviation): 4096 450 / 480, 475 / 489, 4600 504 / 505, 521 / 565.
-static inline bool moe_tall(long long rows, int E) { return rows >= 250LL * E && rows <= 312LL * E; }
-
-template <class Act, template <class, int> class FMT, bool FUSE, int BM, int BN, int OCC>
+// Taller tiles (320 x 192, one workgroup per CU, to keep the rows past 256 in one tile) are ahead only where every expert gets about as many
+// rows: 1480 launches (E = 1 .. 256, H 1024 .. 7168, I 512 .. 2048, 96 .. 600 rows per expert; even, random and two skewed counts) 0.78 to 1.85 of the
+// time of these, 1.04 to 1.29 in the mean at 250 to 312 rows per expert whatever the counts.  These are 0.59 to 1.00 of 256 x 256's.
+template <class Act, template <class, int> class FMT, bool FUSE>
 static int launch_grouped(GemmArgs p, int max_tiles, hipStream_t st) {
   p.tiles_m = (max_tiles + 7) / 8 * 8;                // whole rounds of the 8 XCDs (surplus workgroups exit)
-  p.tiles_n = FUSE ? (p.n_half + BN / 2 - 1) / (BN / 2) : (p.N + BN - 1) / BN;
-  using F = FMT<Act, BN>;
-  auto kern = gemm_tiled_kernel<Act, F, BM, BN, true, FUSE, false, OCC, 4>;
+  p.tiles_n = FUSE ? (p.n_half + kMoeBN / 2 - 1) / (kMoeBN / 2) : (p.N + kMoeBN - 1) / kMoeBN;
+  using F = FMT<Act, kMoeBN>;
+  auto kern = gemm_tiled_kernel<Act, F, kMoeBM, kMoeBN, true, FUSE, false, 2, 4>;
   constexpr size_t lds = TileLds<F>::kBytes;
   static bool raised = false;
   if (lds > 64 * 1024 && !raised) {
@@ -140,19 +135,13 @@ static int launch_grouped(GemmArgs p, int max_tiles, hipStream_t st) {
   return launch_status();
 }
 
-template <class Act, template <class, int> class FMT, bool FUSE>
-static int run_grouped_tile(const GemmArgs& p, bool tall, int max_tiles, hipStream_t st) {
-  return tall ? launch_grouped<Act, FMT, FUSE, kMoeTallBM, kMoeTallBN, 1>(p, max_tiles, st)
-              : launch_grouped<Act, FMT, FUSE, kMoeBM, kMoeBN, 2>(p, max_tiles, st);
-}
-
 template <class Act>
-static int run_grouped(const GemmArgs& p, bool per_expert, int fuse, bool tall, int max_tiles, hipStream_t st) {
+static int run_grouped(const GemmArgs& p, bool per_expert, int fuse, int max_tiles, hipStream_t st) {
   if (per_expert)
-    return fuse ? run_grouped_tile<Act, WFp8PlainG, true>(p, tall, max_tiles, st)
-                : run_grouped_tile<Act, WFp8PlainG, false>(p, tall, max_tiles, st);
-  return fuse ? run_grouped_tile<Act, WFp8BlockG, true>(p, tall, max_tiles, st)
-              : run_grouped_tile<Act, WFp8BlockG, false>(p, tall, max_tiles, st);
+    return fuse ? launch_grouped<Act, WFp8PlainG, true>(p, max_tiles, st)
+                : launch_grouped<Act, WFp8PlainG, false>(p, max_tiles, st);
+  return fuse ? launch_grouped<Act, WFp8BlockG, true>(p, max_tiles, st)
+              : launch_grouped<Act, WFp8BlockG, false>(p, max_tiles, st);
 }
 
 }  // namespace qlin
@@ -183,9 +172,7 @@ int mi_moe_gemm_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_
   if (fuse_act && (N % 2)) return MI_ERR_SHAPE;
   if ((uint64_t)N * (uint64_t)K >= (1ull << 31)) return MI_ERR_SHAPE;
   if (!E || !total_rows) return MI_OK;
-  const bool tall = moe_tall(total_rows, E);
-  const int bm = tall ? kMoeTallBM : kMoeBM;
-  const TiledMoeLayout L = tiled_moe_layout(total_rows, E, K, bm);
+  const TiledMoeLayout L = tiled_moe_layout(total_rows, E, K, kMoeBM);
   if ((uint64_t)L.x_bytes >= (1ull << 31)) return MI_ERR_SHAPE;
   if (!workspace || workspace_bytes < L.total) return MI_ERR_ARG;
   hipStream_t st = (hipStream_t)stream;
@@ -193,7 +180,7 @@ int mi_moe_gemm_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_
   int32_t* g_tile = (int32_t*)(ws + L.tile_off);
   int32_t* blk = (int32_t*)(ws + L.blk_off);
   int32_t* counts = (int32_t*)(ws + L.cnt_off);
-  hipLaunchKernelGGL(moe_tile_map_kernel, dim3(1), dim3(kMapThreads), 0, st, expert_start, E, bm, g_tile, blk, counts);
+  hipLaunchKernelGGL(moe_tile_map_kernel, dim3(1), dim3(kMapThreads), 0, st, expert_start, E, kMoeBM, g_tile, blk, counts);
   const int Q = K / 32;
   hipLaunchKernelGGL(pack_x_grouped_kernel<false>, dim3((unsigned)(((Q + kPackQ - 1) / kPackQ) * L.max_blocks)), dim3(256), 0, st, (const uint16_t*)a,
                      row_map, blk, counts, (u32x4*)ws, a_rows, K, Q, row_map_div);
@@ -207,8 +194,8 @@ int mi_moe_gemm_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_
   p.x_blocks = L.max_blocks;
   p.n_half = N / 2; p.gelu = fuse_act == 2;
   p.out_rows = total_rows;
-  return act_dtype == DT_F16 ? run_grouped<ActF16>(p, scale_per_expert != 0, fuse_act, tall, L.max_tiles, st)
-                             : run_grouped<ActBF16>(p, scale_per_expert != 0, fuse_act, tall, L.max_tiles, st);
+  return act_dtype == DT_F16 ? run_grouped<ActF16>(p, scale_per_expert != 0, fuse_act, L.max_tiles, st)
+                             : run_grouped<ActBF16>(p, scale_per_expert != 0, fuse_act, L.max_tiles, st);
 }
 
 int mi_moe_mlp_fp8_tiled_workspace(int total_rows, int E, int H, int I, long long* bytes) {
@@ -237,16 +224,14 @@ int mi_moe_mlp_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_d
   const int rc = mi_moe_mlp_fp8_tiled_workspace(total_rows, E, H, I, &need);
   if (rc != MI_OK) return rc;
   if (!workspace || workspace_bytes < need) return MI_ERR_ARG;
-  const bool tall = moe_tall(total_rows, E);
-  const int bm = tall ? kMoeTallBM : kMoeBM;
-  const TiledMoeLayout L = tiled_moe_layout(total_rows, E, H, bm);
+  const TiledMoeLayout L = tiled_moe_layout(total_rows, E, H, kMoeBM);
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;
   int32_t* g_tile = (int32_t*)(ws + L.tile_off);
   int32_t* blk = (int32_t*)(ws + L.blk_off);
   int32_t* counts = (int32_t*)(ws + L.cnt_off);
   char* inter = ws + L.total;                          // [blocks][I / 32][1 KiB], operand order
-  hipLaunchKernelGGL(moe_tile_map_kernel, dim3(1), dim3(kMapThreads), 0, st, expert_start, E, bm, g_tile, blk, counts);
+  hipLaunchKernelGGL(moe_tile_map_kernel, dim3(1), dim3(kMapThreads), 0, st, expert_start, E, kMoeBM, g_tile, blk, counts);
   const int Q = H / 32;
   hipLaunchKernelGGL(pack_x_grouped_kernel<false>, dim3((unsigned)(((Q + kPackQ - 1) / kPackQ) * L.max_blocks)), dim3(256), 0, st,
                      (const uint16_t*)a, row_map, blk, counts, (u32x4*)ws, a_rows, H, Q, row_map_div);
@@ -259,8 +244,8 @@ int mi_moe_mlp_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_d
   p.x_blocks = L.max_blocks;
   p.n_half = I; p.gelu = fuse_act == 2;
   p.out_rows = L.max_blocks * 16; p.out_packed = 1;
-  int r = act_dtype == DT_F16 ? run_grouped<ActF16>(p, scale_per_expert != 0, fuse_act, tall, L.max_tiles, st)
-                              : run_grouped<ActBF16>(p, scale_per_expert != 0, fuse_act, tall, L.max_tiles, st);
+  int r = act_dtype == DT_F16 ? run_grouped<ActF16>(p, scale_per_expert != 0, fuse_act, L.max_tiles, st)
+                              : run_grouped<ActBF16>(p, scale_per_expert != 0, fuse_act, L.max_tiles, st);
   if (r != MI_OK) return r;
   GemmArgs d{};
   d.x = inter; d.w = w2; d.scale = w2_scale; d.out = out; d.M = total_rows; d.N = H; d.K = I;
@@ -272,8 +257,8 @@ int mi_moe_mlp_fp8_tiled_ws(const void* a, const int32_t* row_map, int row_map_d
   d.x_blocks = L.max_blocks;
   d.n_half = H / 2;
   d.out_rows = total_rows;
-  return act_dtype == DT_F16 ? run_grouped<ActF16>(d, scale_per_expert != 0, 0, tall, L.max_tiles, st)
-                             : run_grouped<ActBF16>(d, scale_per_expert != 0, 0, tall, L.max_tiles, st);
+  return act_dtype == DT_F16 ? run_grouped<ActF16>(d, scale_per_expert != 0, 0, L.max_tiles, st)
+                             : run_grouped<ActBF16>(d, scale_per_expert != 0, 0, L.max_tiles, st);
 }
 
 }  // extern "C"

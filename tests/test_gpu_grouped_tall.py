@@ -1,5 +1,7 @@
-"""Experts with 250 to 312 rows on average run on tiles of 320 rows x 192 columns: rows at the tile's edges (16-row blocks, wavefronts
-of 5, 4 and fewer of them, a second tile of one row) and columns that leave a partial last tile, against fp32 math."""
+"""Experts with 250 to 312 rows on average: rows at the tile's edges (16-row blocks, wavefronts of 4 and fewer of them, a second tile of one
+row) and columns that leave a partial last tile, against fp32 math; tiles of 256 rows whatever the average."""
+import ctypes
+
 import pytest
 import torch
 
@@ -32,3 +34,20 @@ def test_tall_tiles(dev, dt, H, I, counts):
     err = (out.cpu().float() - ref).norm(dim=1) / ref.norm(dim=1)           # per row: a wrong or missing row shows
     # the weights', the intermediate's and the output's roundings, each 2^-9 (bf16) / 2^-12 (fp16) in norm, four times that
     assert err.max().item() < (0.0176 if dt == torch.bfloat16 else 0.0027)
+
+
+@pytest.mark.parametrize("counts", [[250], [257, 250], [300] * 3, [321, 250, 256], [700, 1, 90]])     # 250 to 300 rows on average, and 264
+def test_tiles_have_256_rows(dev, counts):
+    """The table of M-tiles that a launch leaves in its workspace (their number stands in the last 256 bytes): taller tiles in a range
+    of averages were slower on most sizes and counts."""
+    from mi355x_qlinear import capi
+    E, T, H, I = len(counts), sum(counts), 256, 128
+    start = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(dev)
+    x, y = torch.randn(T, H, device=dev).half(), torch.empty(T, I, dtype=torch.float16, device=dev)
+    w, s = torch.zeros(E, I, H, dtype=torch.uint8, device=dev), torch.ones(E, I // 128, H // 128, device=dev)
+    need = ctypes.c_longlong(0)
+    assert capi.lib().mi_moe_gemm_fp8_tiled_workspace(T, E, H, ctypes.byref(need)) == 0
+    ws = torch.zeros(need.value, dtype=torch.uint8, device=dev)
+    capi.call("mi_moe_gemm_fp8_tiled_ws", x, capi.ptr(x), None, 1, capi.ptr(w), capi.ptr(s), 0, capi.ptr(start), capi.ptr(y), None, None,
+              T, T, E, I, H, 0, 0, capi.ptr(ws), need.value)
+    assert int(ws[-256:].view(torch.int32)[0]) == sum(-(-c // 256) for c in counts)
