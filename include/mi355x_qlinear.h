@@ -547,6 +547,15 @@ int mi_moe_gemv_fp8_block_routed(const void* x, int x_div, int x_silu, const voi
                                  const float* shared_scale, int shared_rows, int shared_x_first, int N, int K,
                                  int act_dtype, void* stream);
 
+/* What the fused step launches for T tokens, one bit each; the torch operator and its Python form both ask here.
+ * MI_DECODE_ROUTED: a GEMV per route (else the grouped GEMMs, and no other bit is set).  MI_DECODE_GATE_UP_TOPK: selection and gate_up rows
+ * by mi_moe_gate_up_topk_fp8_block (else mi_moe_topk and mi_moe_gemv_fp8_block_routed).  MI_DECODE_DOWN_SUM: down rows and their
+ * sum by mi_moe_down_sum_fp8_block (else mi_moe_gemv_fp8_block_routed and mi_moe_combine_shared). */
+#define MI_DECODE_ROUTED 1
+#define MI_DECODE_GATE_UP_TOPK 2
+#define MI_DECODE_DOWN_SUM 4
+int mi_moe_decode_plan(int T, int topk, int num_experts, int H, int I, int* plan);
+
 /* Routing and gate_up rows of the same step in one launch: softmax top-k of logits [T, E] (renormalised, lowest index first among
  * equals) into top_ids / top_w [T, topk], gate[t] = sigmoid(x[t] . gate_weight), and gate_up[t topk + j] = x[t] @
  * dequant(w[top_ids[t, j]])^T, gate_up[T topk + t] = x[t] @ dequant(shared_w)^T.  w [E, 2 I, H], shared_w [2 I, H] e4m3 with 128 x 128

@@ -284,11 +284,58 @@ static int launch_down_sum(const DownSumArgs& p, hipStream_t st) {
   return launch_status();
 }
 
+// ---------------------------------------------------------------- which launches
+constexpr int kRoutedPairs = 96;                      // (token, route) pairs up to which one GEMV runs per route
+constexpr int kGateUpColumns = 4096;                  // x of gate_up_topk_kernel is held in registers
+constexpr long long kDownSumBytes = 64 * 1024;        // a token's activations of down_sum_kernel are held in LDS
+
+// The two launches above against the row GEMV's (gemv_rows.hpp, with mi_moe_topk and mi_moe_combine_shared), each half on its own: 4421 problems (17
+// sizes, H 256 .. 5120, I 128 .. 8192, E 8 .. 512, top 1 .. 32, fp16 and bf16) of up to 96 pairs.  By these lines the step takes 0.51 to 1.04 of
+// the four launches' time (0.86 in the mean; the best choice for each 0.82), 1.02 and more on 8; the two launches everywhere 0.51 to 2.22.  On 1965 problems
+// of seven other sizes it takes at most 1.03 (0.85 in the mean, best 0.80; the two launches up to 2.11).
+//
+// Gate_up: ahead up to three tokens, which read hardly any matrix twice.  With more, every token reads the shared expert and, with few
+// experts, those of others again; the row GEMV puts the same rows of all routes on the same XCD where its workgroups per route are a
+// multiple of 4, and reads them from that XCD's L2: E = 8, top 1, H = 4096, I = 1536, gate_up launches in a step of 32 tokens 123 / 166 us (row
+// GEMV / this), of 12 tokens 82 / 76; top 8 of 8, H = 2048, I = 768, 8 tokens 60 / 65.  Every wavefront selects by itself: the rounds times the keys
+// per lane are bounded (top 32 of 512, H = 1024, I = 512, one token 33 / 41).
+static bool gate_up_topk_pays(int T, int k, int E, int H) {
+  const int keys = E <= 128 ? 2 : E <= 256 ? 4 : E <= 512 ? 8 : 16;
+  if (H > kGateUpColumns || k * keys > 64) return false;
+  if (T <= 3) return true;
+  const int routes = T * (k + 1), per_route = (2 * device_cu_count() + routes - 1) / routes;
+  return k >= 4 && (per_route % 4 != 0 || T * k <= E);
+}
+
+// Down: every workgroup stages the token's activations, and a lane has 8 pieces of a row in flight.  Ahead while one batch of pieces makes the
+// row (a second one is a second round trip; short rows per route are worse for the row GEMV, whose spans are 1024 wide) and the
+// workgroups are few rounds of the chip, fewer where the activations are long, more where the row fills the lanes (top 8 and more).
+// Step's time with row GEMVs and sum / with this, us: top 1 of 8, H = 4096, I = 512, 64 tokens 130 / 268; top 8 of 128, H = 2048, I = 768, one token
+// 20.3 / 18.2, 12 tokens 119 / 108; top 3 of 8, H = 2176, I = 2048, two tokens 26.1 / 27.6; top 8 of 64, H = 2048, I = 256, 12 tokens 71 / 52.
+static bool down_sum_pays(int T, int k, int H, int I) {
+  const long long pieces = (long long)(k + 1) * (I / 16), groups = (long long)T * ((H + kDownWaves - 1) / kDownWaves);
+  const long long cus = device_cu_count(), batch = 64 * kDownPieces;
+  if ((long long)(k + 1) * I * 2 > kDownSumBytes || (pieces > batch && I > 640)) return false;
+  return groups <= 2 * cus || (groups <= 4 * cus && I <= 1536) || (groups <= 12 * cus && k >= 8 && pieces <= batch);
+}
+
 }  // namespace qlin
 
 using namespace qlin;
 
 extern "C" {
+
+int mi_moe_decode_plan(int T, int topk, int num_experts, int H, int I, int* plan) {
+  if (!plan) return MI_ERR_ARG;
+  if (T < 0 || topk < 1 || num_experts < 1 || H < 1 || I < 1) return MI_ERR_SHAPE;
+  *plan = 0;
+  if ((long long)T * topk > kRoutedPairs) return MI_OK;
+  *plan = MI_DECODE_ROUTED;
+  if (topk > 64 || num_experts > 64 * kTopkSlots || topk > num_experts || (H % 128) || (I % 128)) return MI_OK;
+  if (gate_up_topk_pays(T, topk, num_experts, H)) *plan |= MI_DECODE_GATE_UP_TOPK;
+  if (down_sum_pays(T, topk, H, I)) *plan |= MI_DECODE_DOWN_SUM;
+  return MI_OK;
+}
 
 int mi_moe_gate_up_topk_fp8_block(const void* x, const void* logits, const void* gate_weight, const void* w, const float* w_scale,
                                   const void* shared_w, const float* shared_scale, void* gate_up, int32_t* top_ids, void* top_w, float* gate,
@@ -297,7 +344,7 @@ int mi_moe_gate_up_topk_fp8_block(const void* x, const void* logits, const void*
   if (act_dtype != DT_F16 && act_dtype != DT_BF16) return MI_ERR_ARG;
   if (T < 0 || T > 65535 || num_experts < 1 || num_experts > 64 * kTopkSlots || topk < 1 || topk > 64 || topk > num_experts) return MI_ERR_SHAPE;
   if (H <= 0 || I <= 0 || (H % 128) || (I % 128) || (long long)(topk + 1) * 2 * I >= (1LL << 31)) return MI_ERR_SHAPE;
-  if (H > 4096) return MI_ERR_LIMIT;
+  if (H > kGateUpColumns) return MI_ERR_LIMIT;
   if (!T) return MI_OK;
   const GateUpArgs p{x, logits, gate_weight, w, shared_w, w_scale, shared_scale, gate_up, top_ids, top_w, gate, T, topk, num_experts, H, 2 * I};
   return act_dtype == DT_F16 ? launch_gate_up<ActF16>(p, (hipStream_t)stream) : launch_gate_up<ActBF16>(p, (hipStream_t)stream);
@@ -309,7 +356,7 @@ int mi_moe_down_sum_fp8_block(const void* gate_up, const void* w, const float* w
   if (!gate_up || !w || !w_scale || !shared_w || !shared_scale || !top_ids || !top_w || !gate || !out) return MI_ERR_ARG;
   if (act_dtype != DT_F16 && act_dtype != DT_BF16) return MI_ERR_ARG;
   if (T < 0 || T > 65535 || topk < 1 || num_experts < 1 || H <= 0 || I <= 0 || (H % 128) || (I % 128)) return MI_ERR_SHAPE;
-  if ((long long)(topk + 1) * I * 2 > 64 * 1024) return MI_ERR_LIMIT;
+  if ((long long)(topk + 1) * I * 2 > kDownSumBytes) return MI_ERR_LIMIT;
   if (!T) return MI_OK;
   const DownSumArgs p{gate_up, w, shared_w, w_scale, shared_scale, top_ids, top_w, gate, out, T, topk, num_experts, H, I};
   return act_dtype == DT_F16 ? launch_down_sum<ActF16>(p, (hipStream_t)stream) : launch_down_sum<ActBF16>(p, (hipStream_t)stream);

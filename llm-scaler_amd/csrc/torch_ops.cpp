@@ -337,27 +337,17 @@ RESADD_NORM(esimd_resadd_norm_gemv_int4_pert, true)
 RESADD_NORM(esimd_resadd_norm_gemv_fp8_pert, false)
 
 // ---------------------------------------------------------------------------------------- MoE decode
-// (token, route) pairs up to which one GEMV runs per route (12 tokens x top 8); beyond, Python's grouped path, which reads an expert once
-// and rounds once between gate_up and down (16 tokens x top 8 of 128, H = 2048, I = 768: 133 us, 121 with a GEMV per route, whose gate_up rows are rounded
-// before SiLU x up; the routes' error against 64 bits is 1.4 times that)
-constexpr int64_t kRoutedPairs = 96;
-
 bool shape_is(const Tensor& t, at::IntArrayRef s) { return t.sizes() == s; }
 
-// a token's activations of mi_moe_down_sum_fp8_block
-constexpr int64_t kDownSumBytes = 64 * 1024;
-// columns of x in registers of mi_moe_gate_up_topk_fp8_block
-constexpr int64_t kGateUpColumns = 4096;
-
-// top-k with the shared expert's gate, and the gate_up rows of all routes and the shared expert | down rows, SiLU(gate) x up
-// applied as they are staged, and their weighted sum.  Two launches; a longer x, or longer activations of a token, than these hold
-// bring one more: top-k apart, or the down rows, each rounded, and their sum.
+// Up to 96 (token, route) pairs: top-k with the shared expert's gate | gate_up rows of all routes and the shared expert | down rows, SiLU(gate) x up
+// applied as they are staged | their weighted sum.  The first two and the last two are one launch each where the plan says so.  More
+// pairs take Python's grouped path, which reads an expert once and rounds once between gate_up and down.
 bool moe_full_decode(const Tensor& x, const Tensor& logits, const Tensor& out, const Tensor& w13, const Tensor& s13,
                      const Tensor& sw13, const Tensor& ss13, const Tensor& w2, const Tensor& s2, const Tensor& sw2,
                      const Tensor& ss2, const Tensor& gw, int64_t k, int64_t shared, int64_t E) {
   if (x.dim() != 2 || x.size(0) < 1 || w13.dim() != 3 || !is16(x) || shared != 1) return false;
   const int64_t T = x.size(0), H = x.size(1), I = w13.size(1) / 2, P = T * k;
-  if (k < 1 || k > 64 || E < k || E > 1024 || P > kRoutedPairs || H < 128 || I < 128 || H % 128 || I % 128 || w13.size(1) % 2)
+  if (k < 1 || k > 64 || E < k || E > 1024 || P > INT32_MAX || H < 128 || I < 128 || H % 128 || I % 128 || w13.size(1) % 2)
     return false;
   if (!plain(x, {&logits, &out, &w13, &s13, &sw13, &ss13, &w2, &s2, &sw2, &ss2, &gw}) || out.data_ptr() == x.data_ptr()) return false;
   const auto dt = x.scalar_type();
@@ -371,12 +361,16 @@ bool moe_full_decode(const Tensor& x, const Tensor& logits, const Tensor& out, c
       !shape_is(s2, {E, H / 128, I / 128}) || !shape_is(ss13, {2 * I / 128, H / 128}) || !shape_is(ss2, {H / 128, I / 128}) ||
       !shape_is(gw, {1, H}))
     return false;
+  int plan = 0;
+  if (H > INT32_MAX || I > INT32_MAX || mi_moe_decode_plan((int)T, (int)k, (int)E, (int)H, (int)I, &plan) != 0 ||
+      !(plan & MI_DECODE_ROUTED))
+    return false;
   const On on(x);
   const int adt = act(x);
   // one allocation: gate_up rows | down rows | routing weights | gates | expert ids, 256 bytes apart
   int64_t at_ = 0;
   auto take = [&](int64_t bytes) { const int64_t here = at_; at_ += (bytes + 255) / 256 * 256; return here; };
-  const bool sum = (k + 1) * I * 2 <= kDownSumBytes;   // the down launch adds the routes up itself
+  const bool sum = plan & MI_DECODE_DOWN_SUM;         // the down launch adds the routes up itself
   const int64_t gu_at = take((P + T) * 2 * I * 2), y_at = take(sum ? 0 : (P + T) * H * 2), tw_at = take(P * 2), g_at = take(T * 4),
                 id_at = take(P * 4);
   const Tensor ws = buffer(x, at_);
@@ -386,7 +380,7 @@ bool moe_full_decode(const Tensor& x, const Tensor& logits, const Tensor& out, c
   int32_t* ids = (int32_t*)(base + id_at);
   const void* xp = x.data_ptr();
   void* st = on.stream;
-  if (H <= kGateUpColumns) {
+  if (plan & MI_DECODE_GATE_UP_TOPK) {
     CALL(mi_moe_gate_up_topk_fp8_block, xp, logits.data_ptr(), gw.data_ptr(), w13.data_ptr(), s13.data_ptr<float>(), sw13.data_ptr(),
          ss13.data_ptr<float>(), gu, ids, tw, gate, (int)T, (int)k, (int)E, (int)H, (int)I, adt, st);
   } else {
@@ -394,7 +388,7 @@ bool moe_full_decode(const Tensor& x, const Tensor& logits, const Tensor& out, c
     CALL(mi_moe_gemv_fp8_block_routed, xp, (int)k, 0, w13.data_ptr(), s13.data_ptr<float>(), gu, 2 * I, ids, nullptr, (int)P, (int)E,
          sw13.data_ptr(), ss13.data_ptr<float>(), (int)T, 0, (int)(2 * I), (int)H, adt, st);
   }
-  if (!y) {
+  if (sum) {
     CALL(mi_moe_down_sum_fp8_block, gu, w2.data_ptr(), s2.data_ptr<float>(), sw2.data_ptr(), ss2.data_ptr<float>(), ids, tw, gate,
          out.data_ptr(), (int)T, (int)k, (int)E, (int)H, (int)I, adt, st);
     return true;

@@ -1203,9 +1203,6 @@ def moe_gemm_fp8_block(a, a_scale, row_map, weight, weight_scale, expert_start, 
 
 
 ROUTED_MAX_PAIRS = 8192       # (token, route) pairs one routed gate_up launch sorts by itself
-GATE_UP_MAX_COLUMNS = 4096       # hidden size up to which the gate_up launch selects the experts itself
-DOWN_SUM_MAX_BYTES = 64 * 1024    # (top_k + 1) activation rows of a token that the one-launch down projection holds
-ROUTED_GEMV_MAX_PAIRS = 96    # (token, route) pairs up to which the fused decode op runs one GEMV per route (12 tokens x top 8)
 
 
 def moe_gate_up_fp8_routed(xq, xs, top_ids, weight, weight_scale, expert_start, inv, sorted_pairs, output,
@@ -1370,19 +1367,22 @@ def moe_forward_full_fp8_block(x, logits, output, gate_up_weight, gate_up_scale,
     top_w = torch.empty(T, k, dtype=x.dtype, device=dev)
     top_ids = torch.empty(T, k, dtype=torch.int32, device=dev)
     gate = torch.empty(T, dtype=torch.float32, device=dev)
-    decode = P <= ROUTED_GEMV_MAX_PAIRS
-    if not (decode and H <= GATE_UP_MAX_COLUMNS):
+    plan = ctypes.c_int(0)
+    rc = capi.lib().mi_moe_decode_plan(T, k, E, H, I, ctypes.byref(plan))
+    _chk(rc == 0, f"{who}: mi_moe_decode_plan: {capi.MI_ERRORS.get(rc, rc)}")
+    decode, topk_gate_up, down_sum = (bool(plan.value & bit) for bit in (1, 2, 4))   # MI_DECODE_*
+    if not topk_gate_up:
         # routing and the shared expert's gate sigmoid(x . w) in one launch
         esimd_moe_topk(logits, top_w, top_ids, T, gate=(x, shared_expert_gate_weight, gate))
     if decode:
         # Decode: one GEMV per (token, route), all routes in one launch per projection (no sort, no
         # grouping: with a handful of rows a grouped launch has work for a few workgroups only and
         # streams each expert's weights at a fraction of the device's rate).  The shared expert's rows
-        # follow the routed ones in the same launches and buffers: two launches in all, one more each where x is
-        # too long for the launch that selects the experts itself, or a token's activations for the one that sums.
+        # follow the routed ones in the same launches and buffers.  Two launches where the plan has the selection in the gate_up
+        # launch and the sum in the down launch, one more for each that it has not.
         adt = capi.act_dtype(x)
         gu = torch.empty(P + T, 2 * I, dtype=x.dtype, device=dev)
-        if H <= GATE_UP_MAX_COLUMNS:                    # routing and gate_up rows in one launch
+        if topk_gate_up:                                # routing and gate_up rows in one launch
             capi.call("mi_moe_gate_up_topk_fp8_block", x, capi.ptr(x), capi.ptr(logits), capi.ptr(shared_expert_gate_weight),
                       capi.ptr(gate_up_weight), capi.ptr(gate_up_scale), capi.ptr(shared_gate_up_weight),
                       capi.ptr(shared_gate_up_scale), capi.ptr(gu), capi.ptr(top_ids), capi.ptr(top_w), capi.ptr(gate),
@@ -1391,7 +1391,7 @@ def moe_forward_full_fp8_block(x, logits, output, gate_up_weight, gate_up_scale,
             capi.call("mi_moe_gemv_fp8_block_routed", x, capi.ptr(x), k, 0, capi.ptr(gate_up_weight), capi.ptr(gate_up_scale),
                       capi.ptr(gu), 2 * I, capi.ptr(top_ids), None, P, E, capi.ptr(shared_gate_up_weight),
                       capi.ptr(shared_gate_up_scale), T, 0, 2 * I, H, adt)
-        if (k + 1) * I * 2 <= DOWN_SUM_MAX_BYTES:       # down projections and their sum in one launch
+        if down_sum:                                    # down projections and their sum in one launch
             capi.call("mi_moe_down_sum_fp8_block", gu, capi.ptr(gu), capi.ptr(down_weight), capi.ptr(down_scale),
                       capi.ptr(shared_down_weight), capi.ptr(shared_down_scale), capi.ptr(top_ids), capi.ptr(top_w), capi.ptr(gate),
                       capi.ptr(output), T, k, E, H, I, adt)

@@ -170,6 +170,25 @@ def test_down_launches_either_side_of_the_line(case, tiles):
     assert capi.lib().mi_moe_gguf_grouped_tiled_pays(fmt, 1, n, rows, E, N, K, ctypes.byref(p)) == 0 and p.value == tiles
 
 
+# (T, top k, E, H, I): us of the step with mi_moe_topk and a row GEMV for gate_up / the selecting launch, a row GEMV and a sum for down / the summing launch
+@pytest.mark.parametrize("case, plan", [((1, 8, 128, 2048, 768), 7),        # 20.3 -> 16.8, -> 18.2
+                                        ((12, 8, 128, 2048, 768), 7),       # 119 -> 103, -> 108
+                                        ((8, 8, 8, 2048, 768), 5),          # 60 -> 65, -> 52
+                                        ((32, 1, 8, 4096, 1536), 1),        # 123 -> 166, -> 205
+                                        ((64, 1, 8, 4096, 512), 1),         # 130 -> 151, -> 268
+                                        ((1, 1, 8, 4096, 1536), 7),         # 18.9 -> 15.9, -> 17.8
+                                        ((2, 3, 8, 2176, 2048), 3),         # 26.1 -> 26.5, -> 27.6
+                                        ((2, 1, 8, 4096, 8192), 3),         # 63 -> 65, -> 68
+                                        ((1, 32, 512, 1024, 512), 5),       # 33 -> 41, -> 33.5
+                                        ((96, 1, 8, 4096, 512), 1), ((97, 1, 8, 4096, 512), 0), ((12, 8, 16, 256, 128), 7), ((13, 8, 16, 256, 128), 0),
+                                        ((1, 8, 9, 4224, 128), 5), ((1, 8, 9, 128, 3712), 3), ((1, 65, 70, 256, 128), 1), ((1, 2, 1025, 256, 128), 1)])
+def test_decode_step_launches_what_was_measured_faster(case, plan):
+    """Either side of the lines of mi_moe_decode_plan: 1 = a GEMV per route, 2 = selection in the gate_up launch, 4 = sum in the down launch."""
+    p = ctypes.c_int(-1)
+    assert capi.lib().mi_moe_decode_plan(*case, ctypes.byref(p)) == 0 and p.value == plan
+    assert capi.lib().mi_moe_decode_plan(*case, None) == -1 and capi.lib().mi_moe_decode_plan(-1, *case[1:], ctypes.byref(p)) == -2
+
+
 def test_moe_grouped_module_matches_the_reference_binding():
     """Names, argument order and defaults of the pybind module the patched SGLang imports
     (S/csrc/moe_grouped/moe_grouped_entry.sycl:108-127, sglang_for_multi_arc.patch:2114)."""

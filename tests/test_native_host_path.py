@@ -160,6 +160,32 @@ def test_moe_decode_is_the_same(dev, T, dt):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,k,E,H,I,plan", [(1, 8, 16, 256, 128, 7), (2, 8, 8, 256, 1024, 3), (8, 1, 8, 256, 128, 5), (64, 1, 8, 256, 128, 1),
+                                            (97, 1, 8, 256, 128, 0)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_moe_decode_launches_the_plan(dev, monkeypatch, T, k, E, H, I, plan, dt):
+    """Each choice of mi_moe_decode_plan: both host paths give the same bits, the entries are the plan's, the result is the oracle's."""
+    from oracle import qlinear_oracle as O
+    g = torch.Generator().manual_seed(T + k)
+    x, logits, gw = torch.randn(T, H, generator=g).to(dt), torch.randn(T, E, generator=g).to(dt), (torch.randn(1, H, generator=g) * 0.1).to(dt)
+    w = [t for s in ((E, 2 * I, H), (2 * I, H), (E, H, I), (H, I)) for t in O.fp8_quantize_block(torch.randn(*s, generator=g) * 0.1)]
+    want = O.moe_forward_full(x, logits, *w, gw, k)
+    args = [t.view(torch.float8_e4m3fn).to(dev) if t.dtype == torch.uint8 else t.to(dev) for t in w] + [gw.to(dev)]
+    x, logits = x.to(dev), logits.to(dev)
+    outs = [torch.empty_like(x) for _ in range(2)]
+    torch.ops.moe_ops.moe_forward_full_fp8_block(x, logits, outs[0], *args, k, 1, E)
+    inner, entries = _ops.capi.call, []
+    monkeypatch.setattr(_ops.capi, "call", lambda entry, *a: entries.append(entry) or inner(entry, *a))
+    torch.ops.mi355x_checked.moe_forward_full_fp8_block(x, logits, outs[1], *args, k, 1, E)
+    assert torch.equal(*outs)
+    gate_up = ["mi_moe_gate_up_topk_fp8_block"] if plan & 2 else ["mi_moe_topk", "mi_moe_gemv_fp8_block_routed"]
+    down = ["mi_moe_down_sum_fp8_block"] if plan & 4 else ["mi_moe_gemv_fp8_block_routed", "mi_moe_combine_shared"]
+    assert entries == gate_up + down if plan else "mi_moe_sort" in entries
+    mean_rel = float((outs[0].cpu().float() - want).abs().mean() / want.abs().mean())
+    assert mean_rel < (3e-3 if dt == torch.float16 else 1e-2)               # the bars of the operator's test
+
+
 def _refused(dev):
     """(Python building block of the operator, call) where the checks pass and the C entry refuses the size before it
     launches anything: K of no whole granule, and an expert row longer than the LDS holds."""
