@@ -426,7 +426,7 @@ int mi_norm_gemv_static(const void* x, void* residual, const void* gate, const v
 /* ---- MoE prefill: grouped FP8 GEMM on the tiled matrix-core kernel ---------------
  * mi_moe_gemm_fp8_grouped in w8a16 mode (no a_scale, output in the activation type) for experts
  * with hundreds of rows: a device-built table of M-tiles per expert, activations gathered and
- * re-tiled per 16-row block, then the 256 x 256 tiled GEMM with one weight matrix per expert, so
+ * re-tiled per 16-row block, then the tiled GEMM (256 x 128 tiles) with one weight matrix per expert, so
  * that an expert's weights are read once per 256 of its rows (a wavefront skips the 16-row tiles
  * past an expert's last row).  Same arguments and
  * results; K % 128 == 0, E <= 1024.  workspace: mi_moe_gemm_fp8_tiled_workspace bytes; that call

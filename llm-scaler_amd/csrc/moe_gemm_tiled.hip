@@ -124,13 +124,7 @@ static int launch_grouped(GemmArgs p, int max_tiles, hipStream_t st) {
   using F = FMT<Act, kMoeBN>;
   auto kern = gemm_tiled_kernel<Act, F, kMoeBM, kMoeBN, true, FUSE, false, 2, 4>;
   constexpr size_t lds = TileLds<F>::kBytes;
-  static bool raised = false;
-  if (lds > 64 * 1024 && !raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
-        hipSuccess)
-      return MI_ERR_LAUNCH;
-    raised = true;
-  }
+  static_assert(lds <= 64 * 1024, "more dynamic LDS has to be asked for");
   hipLaunchKernelGGL(kern, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(256), lds, st, p);
   return launch_status();
 }

@@ -127,11 +127,7 @@ static int launch_chunk_gemm(GemmArgs p, int nmat, int max_tiles, hipStream_t st
   if ((long long)p.tiles_m * p.tiles_n >= (1LL << 31)) return MI_ERR_SHAPE;
   auto kern = gemm_tiled_kernel<ActF16, F, kGgufBM, kGgufBN, true, false, false, 2, 4>;
   constexpr size_t lds = TileLds<F>::kBytes;
-  if (lds > 64 * 1024) {
-    static const int raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess ? MI_OK : MI_ERR_LAUNCH;
-    if (raised != MI_OK) return raised;
-  }
+  static_assert(lds <= 64 * 1024, "more dynamic LDS has to be asked for");
   hipLaunchKernelGGL(kern, dim3((unsigned)(p.tiles_m * p.tiles_n)), dim3(256), lds, st, p);
   return launch_status();
 }
