@@ -43,7 +43,8 @@ def test_down_projections_and_their_sum(dev, dt, T, k, E, H, I):
     assert bool(((out.cpu().double() - ref).abs() <= eps * ref.abs() + (2.0 ** -18 + eps / 16) * scale).all())
 
 
-@pytest.mark.parametrize("T,k,E,H,I", [(1, 8, 16, 256, 768), (3, 1, 2, 128, 128), (12, 4, 8, 1152, 256)])     # 80, 496 and 432 pieces past the end
+# 80, 496 and 432 pieces past the end; 8 of them behind 65 280 bytes of activations, none behind 65 536
+@pytest.mark.parametrize("T,k,E,H,I", [(1, 8, 16, 256, 768), (3, 1, 2, 128, 128), (12, 4, 8, 1152, 256), (1, 50, 51, 128, 640), (1, 63, 64, 128, 512)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 def test_an_infinity_stays_one(dev, dt, T, k, E, H, I):
     """An activation of the shared expert's last piece overflows: its products are infinite, of the weight's sign, and no lane beyond
