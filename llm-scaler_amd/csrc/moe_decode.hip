@@ -174,15 +174,14 @@ template <class Act, int RPW>                         // output rows per wavefro
 __global__ __launch_bounds__(64 * kDownWaves) void down_sum_kernel(const DownSumArgs p) {
   using Elem = typename Act::elem;
   using V8 = typename Act::v8;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];        // [k + 1][I] activations, a piece of zeros where the last batch has lanes left
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];        // [k + 1][I] activations
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int t = blockIdx.y, k = p.k, H = p.H, I = p.I;
   const int n0 = (blockIdx.x * kDownWaves + wave) * RPW;
   const unsigned per = (unsigned)I >> 4, total = per * (unsigned)(k + 1);      // 16-byte pieces of a route's row, of an output row
   u32x4 wv[RPW][kDownPieces];
   float f[RPW][kDownPieces];                          // block scale x routing weight (or the shared expert's gate)
-  // request the pieces [s0, + 64 x kDownPieces); rows past H and pieces past the end repeat valid ones (the latter meet zeros for activations:
-  // those that are repeated may be infinite)
+  // request the pieces [s0, + 64 x kDownPieces); rows past H and pieces past the end repeat valid ones
   auto request = [&](unsigned s0) __attribute__((always_inline)) {
     unsigned s[kDownPieces], r[kDownPieces];
     int e[kDownPieces];
@@ -222,7 +221,8 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_sum_kernel(const DownSum
 #pragma unroll
     for (int i = 0; i < kDownPieces; ++i) {
       unsigned s = s0 + i * 64 + lane;
-      if (s > total) s = total;                       // past the end: zeros
+      const bool mine = s < total;                    // selected, not multiplied by 0: what is repeated may be infinite
+      if (!mine) s = total - 1;
       const u32x4 a0 = *reinterpret_cast<const u32x4*>(smem + (size_t)s * 32), a1 = *reinterpret_cast<const u32x4*>(smem + (size_t)s * 32 + 16);
 #pragma unroll
       for (int q = 0; q < RPW; ++q) {
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_sum_kernel(const DownSum
         for (int j = 0; j < 4; ++j) d = Dot2<Act>::run(b0[j], a0[j], d);
 #pragma unroll
         for (int j = 0; j < 4; ++j) d = Dot2<Act>::run(b1[j], a1[j], d);
-        acc[q] += d * f[q][i];
+        acc[q] = mine ? __builtin_fmaf(d, f[q][i], acc[q]) : acc[q];
       }
     }
   };
@@ -253,7 +253,6 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_sum_kernel(const DownSum
     }
     *reinterpret_cast<u32x4*>(smem + (size_t)i * 16) = __builtin_bit_cast(u32x4, o8);
   }
-  if (total % (64 * kDownPieces) && tid < 2) *reinterpret_cast<u32x4*>(smem + (size_t)total * 32 + tid * 16) = u32x4{0, 0, 0, 0};
   __syncthreads();
   multiply(0);
   for (unsigned s0 = 64 * kDownPieces; s0 < total; s0 += 64 * kDownPieces) {
@@ -269,7 +268,7 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_sum_kernel(const DownSum
 
 template <class Act>
 static int launch_down_sum(const DownSumArgs& p, hipStream_t st) {
-  const size_t acts = (size_t)(p.k + 1) * p.I * 2, lds = acts + (acts % (64 * kDownPieces * 32) ? 32 : 0);   // at most 64 KiB as acts is
+  const size_t lds = (size_t)(p.k + 1) * p.I * 2;
   // A workgroup stages all of its token's activations: a row per wavefront while these fit the chip in one round, else more rows share
   // the staging.  1 / 2 / 4 rows, us for the whole step (sizes as above): one token 18.7 / 19.7 / 22.8, two 28.5 / 27.0 / 29.2, three
   // 37.7 / 38.5 / 34.8, eight 76.5 / 74.0 / 66.9.
