@@ -112,7 +112,7 @@ static inline TiledMoeLayout tiled_moe_layout(int total_rows, int E, int K, int 
 // 256 x 128 tiles of four wavefronts stacked along M, in 256 registers: two workgroups per CU, so that while one waits at a
 // barrier, for its first weights or for its stores, or decodes for an expert's few rows past 256, the other's MFMAs run.  A weight
 // is decoded once per 256 rows, and a wavefront skips the 16-row tiles past the expert's last row.  128 experts, top 8, H = 2048, I = 768,
-// 256 x 256 (one workgroup per CU) / 256 x 128, us for the layer: 2000 tokens 280 / 264, 2500 309 / 292, 3500 404 / 367, 4096 497 / 457.
+// 256 x 256 (one workgroup per CU) / 256 x 128, us for the layer: 2000 tokens 280 / 264, 2500 309 / 292, 3500 404 / 367, 4096 503 / 465.
 constexpr int kMoeBM = 256, kMoeBN = 128;
 // Taller tiles (320 x 192, one workgroup per CU, to keep the rows past 256 in one tile) are ahead only where every expert gets about as many
 // rows: 1480 launches (E = 1 .. 256, H 1024 .. 7168, I 512 .. 2048, 96 .. 600 rows per expert; even, random and two skewed counts) 0.78 to 1.85 of the

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("counts", [[320, 257, 321, 150], [304, 305, 0, 391], [250, 250, 250, 250], [312, 312, 312, 312], [1, 640, 272, 335]])
 @pytest.mark.parametrize("H,I", [(256, 128), (640, 384)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
-def test_tall_tiles(dev, dt, H, I, counts):
+def test_experts_at_a_tiles_edge(dev, dt, H, I, counts):
     import custom_esimd_kernels_vllm as v
     E, T = len(counts), sum(counts)
     assert 250 * E <= T <= 312 * E
